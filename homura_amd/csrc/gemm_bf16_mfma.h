@@ -15,6 +15,8 @@ namespace homura {
 // With parts != NULL the product may be cut along K into up to max_parts slices when M x N alone
 // leaves most of the chip idle: slice s lands in d_c + s * M * N, *parts says how many there are, and
 // the caller adds them up in index order (d_c must hold max_parts * M * N floats).
+// A product comes in more than one slice only while slices times its 128 x 128 tiles stay within gemm_sliced_tiles().
+inline long long gemm_sliced_tiles(int cus) { return 2LL * cus; }
 int gemm_split_nk(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, const uint16_t *d_b_nk, float *d_c, int M, int K,
                   int N, int max_parts = 1, int *parts = nullptr);
 

@@ -2,19 +2,25 @@
 // (sum of B's pieces)^T, A [M][AP Kb], B [N][BP Kb] (piece p in columns [p Kb, (p+1) Kb)).
 //
 // The plain kernel of gemm_bf16_mfma.hip runs one pass over K per product of pieces and loads a B tile
-// again for every A piece. It is bound by what a CU can pull into LDS (about half of its 64 B/clk;
-// the MFMAs of a tile take 40 % of the time the loads do), so this kernel loads every tile once: a
+// again for every A piece. This kernel loads every tile once: a
 // stage holds the tiles of all pieces for 32 values of k, and every product that matters is taken from
 // them: the AP products with a single B (bf16 weights), or the six products (a, b), a + b <= 2, of
 // two three-piece operands (f32 x f32 up to 2^-24). Per product that is a third less (AP = 3, BP = 1)
 // or half (AP = BP = 3) of the bytes, and the operand reads out of LDS shrink the same way.
 //
-// Workgroup tile 128 x 128, eight wavefronts as two k groups of 2 x 2 (group g takes k step g of the
+// Workgroup tile 128 x 128 or 128 x 256 (cut_for), eight wavefronts as two k groups of 2 x 2 (group g takes k step g of the
 // two in a stage), `mfma_f32_32x32x16_bf16`, tiles go global -> LDS directly (global_load_lds_dwordx4:
 // lane l's 16 bytes land at base + 16 l, so an instruction fills sixteen 64-byte rows; the lane that
 // fills slot s of row r fetches chunk s ^ ((r >> 2) & 3), which makes the operand reads conflict
-// free). NB stages rotate through LDS (128 to 144 KiB), one barrier per stage. M, N ragged as in the
-// other kernel; K slices (grid.y) write partial sums the consumer adds in index order.
+// free). NB stages rotate through LDS (96 to 160 KiB), one barrier per stage. M, N ragged as in the
+// other kernel; K slices write partial sums the consumer adds in index order.
+//
+// What bounds it: per 32 k of a 128 x 128 tile the MFMAs of a CU take 0.38 us, the loads into LDS 0.34 us and the operand
+// reads 0.17 us, each measured with the others left out. Issued one after the other behind the barrier they added up to
+// 0.63 us; with a load or an operand read behind every MFMA the stage takes 0.52 us, and 0.70 us for a 128 x 256 tile
+// (twice the MFMAs, 5/4 of the loads), which is what its MFMAs alone take. 512 rows, 3 x 1 pieces, with the slices kept to
+// their dies: 1024 -> 4096 19.6 -> 18.4 us, 2048 -> 1024 15.3 -> 12.9, 1024 -> 6144 27.4 -> 24.9, 3072 -> 1024
+// 19.6 -> 15.3; 2048 rows: 68.2 -> 46.7, 36.1 -> 28.0, 92.4 -> 78.3, 52.9 -> 36.7 (1.1 PFLOP/s of bf16 products).
 //
 // SC (block-scaled B): B holds the integers of a Q8_0 / Q4_0 matrix as bf16 (exact) and every 32-wide block
 // of a row has an f32 scale, scales[k / 32][n] (row stride npad, a multiple of 128). A stage is exactly one
@@ -36,10 +42,11 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int TM = 128, TN = 128, TK = 32;
+constexpr int TM = 128, TK = 32;
 constexpr int ROW_BYTES = TK * 2;               // 64
-constexpr int PIECE_TILE = TM * ROW_BYTES;      // 8 KiB: one piece of one operand for one stage
+constexpr int PIECE_TILE = TM * ROW_BYTES;      // 8 KiB: one piece of 128 rows of one operand for one stage
 constexpr int THREADS = 512;
+constexpr int LDS_MAX = 160 * 1024;
 
 struct PieceDims {
     int M, N, Kb, lda, ldb, ldc;
@@ -48,6 +55,8 @@ struct PieceDims {
     int npad;
     size_t a_batch, b_batch, c_batch;  // grid.z: elements from one problem of a batch to the next
     homura::GroupLists lists;          // GR
+    int tiles, slices;                 // output tiles of a problem, K slices
+    int n_fast;                        // neighbouring tiles: 1 along a row of tiles, 0 along a column
 };
 
 __device__ __forceinline__ int lds_off(int r, int chunk) { return r * ROW_BYTES + ((chunk ^ ((r >> 2) & 3)) << 4); }
@@ -72,21 +81,24 @@ __device__ __forceinline__ float lds_read4(uint32_t addr) {
 
 extern __shared__ __attribute__((aligned(16))) char stage_lds[];
 
-template <int AP, int BP, bool SC = false>
+// NT: 32-wide column tiles of a wavefront (two wavefronts side by side): the workgroup's tile is 128 x 64 NT
+template <int AP, int BP, bool SC = false, int NT = 2>
 struct Shape {
-    static constexpr int TILES = AP + BP;                   // operand tiles per stage
+    static constexpr int TN = 64 * NT;
+    static constexpr int TILES = AP + BP * (NT / 2);        // 128-row operand tiles per stage
     static constexpr int T = TILES + (SC ? 1 : 0);          // loads per wavefront and stage
     static constexpr int STAGE = TILES * PIECE_TILE + (SC ? TN * 4 : 0);  // bytes
-    static constexpr int NB = TILES * PIECE_TILE <= 32 * 1024 ? 4 : 3;    // stages in LDS
-    static constexpr int LDS = NB * STAGE > 64 * 1024 ? NB * STAGE : 64 * 1024;  // the final exchange wants 64 KiB
+    static constexpr int NB = 4 * STAGE <= LDS_MAX && TILES <= 5 ? 4 : 3;  // stages in LDS
+    static constexpr int XCH = NT * 32 * 1024;              // what the final exchange wants
+    static constexpr int LDS = NB * STAGE > XCH ? NB * STAGE : XCH;
 };
 
-template <int AP, int BP, bool SC = false, bool GR = false>
+template <int AP, int BP, bool SC = false, bool GR = false, int NT = 2>
 __global__ __launch_bounds__(THREADS) void gemm_pieces_kernel(const uint16_t *__restrict__ A,
                                                               const uint16_t *__restrict__ B, float *__restrict__ C,
                                                               const PieceDims g) {
-    using S = Shape<AP, BP, SC>;
-    constexpr int T = S::T, NB = S::NB, STAGE = S::STAGE;
+    using S = Shape<AP, BP, SC, NT>;
+    constexpr int T = S::T, NB = S::NB, STAGE = S::STAGE, TN = S::TN;
     static_assert(!SC || BP == 1, "block scales go with a single B operand");
     int M = g.M;  // (GR: of the group)
     const int N = g.N;
@@ -94,11 +106,16 @@ __global__ __launch_bounds__(THREADS) void gemm_pieces_kernel(const uint16_t *__
     const int kgrp = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
     const int l32 = lane & 31, lh = lane >> 5;
 
-    // XCD-aware tile order, as in the other kernel
-    const int mb = GR ? 1 : (M + TM - 1) / TM, total = gridDim.x;
-    int lin = blockIdx.x;
-    if ((total & 7) == 0) lin = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
-    int m0 = (lin % mb) * TM, n0 = (lin / mb) * TN;
+    const int mb = GR ? 1 : (M + TM - 1) / TM, nb_t = (N + TN - 1) / TN, total = g.tiles * g.slices, per = (total + 7) / 8;
+    int lin = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    int slice = 0, m0 = 0, n0 = 0;
+    if (!GR) {
+        if ((int)(blockIdx.x >> 3) >= per || lin >= total) return;
+        slice = lin / g.tiles;
+        lin -= slice * g.tiles;
+        m0 = (g.n_fast ? lin / nb_t : lin % mb) * TM;
+        n0 = (g.n_fast ? lin % nb_t : lin / mb) * TN;
+    }
     const int *list = nullptr;
     if constexpr (GR) {
         const homura::GroupTile t = homura::group_tile(g.lists, blockIdx.x, (N + TN - 1) / TN, TM, TN);
@@ -110,46 +127,51 @@ __global__ __launch_bounds__(THREADS) void gemm_pieces_kernel(const uint16_t *__
         B += (size_t)t.group * g.b_batch;
     }
 
-    f32x16 acc[2][2];
+    f32x16 acc[2][NT];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < NT; j++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
 
-    const int s_first = blockIdx.y * g.stages_per_split;
+    const int s_first = slice * g.stages_per_split;
     const int ns = min(g.stages_per_split, g.Kb / TK - s_first);
     if constexpr (!GR) {
-        C += (size_t)blockIdx.y * M * g.ldc + blockIdx.z * g.c_batch;
+        C += (size_t)slice * M * g.ldc + blockIdx.z * g.c_batch;
         A += blockIdx.z * g.a_batch;
         B += blockIdx.z * g.b_batch;
     }
 
-    // Wavefront w fills rows 16 w .. 16 w + 15 of every tile of a stage, one instruction per tile.
-    const uint16_t *a_src, *b_src;
+    // Wavefront w fills rows 16 w .. 16 w + 15 of every 128-row tile of a stage, one instruction per tile.
+    const uint16_t *a_src, *b_src[NT / 2];
     {
         const int r = wave * 16 + (lane >> 2), s = lane & 3;
         const int c = s ^ ((r >> 2) & 3);
         const int a_row = min(m0 + r, M - 1);
         a_src = A + (size_t)(GR ? list[a_row] % g.lists.a_rows : a_row) * g.lda + c * 8;
-        b_src = B + (size_t)min(n0 + r, N - 1) * g.ldb + c * 8;
+#pragma unroll
+        for (int q = 0; q < NT / 2; q++) b_src[q] = B + (size_t)min(n0 + q * 128 + r, N - 1) * g.ldb + c * 8;
     }
     const int wave_dst = __builtin_amdgcn_readfirstlane(wave * 1024);
-    const int wave_dst64 = __builtin_amdgcn_readfirstlane(wave * 64);
-    const float *s_src = SC ? g.scales + n0 + wave * 16 + (lane & 3) * 4 : nullptr;  // (n0 + 127 < npad)
+    const int wave_dst_s = __builtin_amdgcn_readfirstlane(wave * (TN / 2));
+    const float *s_src = SC ? g.scales + n0 + wave * (TN / 8) + (lane & (TN / 32 - 1)) * 4 : nullptr;  // (n0 + TN - 1 < npad)
     int k_req = s_first * TK;  // k of the next stage to request
     // a stage past the end re-reads the last one (nobody multiplies it): the wait counts stay exact
-    auto request = [&](int buf) {
+    auto request_one = [&](int buf, int o) {  // load o of the T of a stage
         char *base = stage_lds + buf * STAGE + wave_dst;
         const int k = min(k_req, g.Kb - TK);
-#pragma unroll
-        for (int p = 0; p < AP; p++) dma16(a_src + p * g.Kb + k, base + p * PIECE_TILE);
-#pragma unroll
-        for (int p = 0; p < BP; p++) dma16(b_src + p * g.Kb + k, base + (AP + p) * PIECE_TILE);
-        if (SC && lane < 4)  // this wavefront's 16 of the stage's 128 block scales
+        if (o < AP)
+            dma16(a_src + o * g.Kb + k, base + o * PIECE_TILE);
+        else if (o < S::TILES)
+            dma16(b_src[(o - AP) % (NT / 2)] + (o - AP) / (NT / 2) * g.Kb + k, base + o * PIECE_TILE);
+        else if (SC && lane < TN / 32)  // this wavefront's eighth of the stage's block scales
             dma16(reinterpret_cast<const uint16_t *>(s_src + (size_t)(k / TK) * g.npad),
-                  stage_lds + buf * STAGE + S::TILES * PIECE_TILE + wave_dst64);
+                  stage_lds + buf * STAGE + S::TILES * PIECE_TILE + wave_dst_s);
+    };
+    auto request = [&](int buf) {
+#pragma unroll
+        for (int o = 0; o < T; o++) request_one(buf, o);
         k_req += TK;
     };
 #pragma unroll
@@ -158,111 +180,108 @@ __global__ __launch_bounds__(THREADS) void gemm_pieces_kernel(const uint16_t *__
     // this lane's operand addresses inside a stage: piece tiles are PIECE_TILE apart
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)stage_lds;
     const int chunk = kgrp * 2 + lh;  // k step kgrp of the stage, 8 k per half-wavefront
-    uint32_t a_off[2], b_off[2];
+    uint32_t a_off[2], b_off[NT];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        a_off[i] = lds0 + lds_off(wm * 64 + i * 32 + l32, chunk);
-        b_off[i] = lds0 + AP * PIECE_TILE + lds_off(wn * 64 + i * 32 + l32, chunk);
-    }
+    for (int i = 0; i < 2; i++) a_off[i] = lds0 + lds_off(wm * 64 + i * 32 + l32, chunk);
+#pragma unroll
+    for (int j = 0; j < NT; j++) b_off[j] = lds0 + AP * PIECE_TILE + lds_off(wn * (NT * 32) + j * 32 + l32, chunk);
     // operand registers, two sets: the reads of the next stage are in flight during the MFMAs
-    bf16x8 fa[2][AP][2], fb[2][BP][2];
-    float fs[2][2];  // SC: the block scales of this lane's two columns
-    const uint32_t s_off = lds0 + S::TILES * PIECE_TILE + (wn * 64 + l32) * 4;
-    auto read_stage = [&](int set, int buf) {
+    bf16x8 fa[2][AP][2], fb[2][BP][NT];
+    float fs[2][NT];  // SC: the block scales of this lane's columns
+    const uint32_t s_off = lds0 + S::TILES * PIECE_TILE + (wn * (NT * 32) + l32) * 4;
+    constexpr int READS = 2 * AP + NT * BP + (SC ? NT : 0);
+    auto read_one = [&](int set, int buf, int o) {  // operand read o of a stage
         const uint32_t off = (uint32_t)(buf * STAGE);
-        if (SC) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) fs[set][j] = lds_read4(s_off + off + j * 128);
+        if (o < 2 * AP)
+            fa[set][o / 2][o % 2] = lds_read16(a_off[o % 2] + off + (o / 2) * PIECE_TILE);
+        else if (o < 2 * AP + NT * BP) {
+            const int q = o - 2 * AP;
+            fb[set][q / NT][q % NT] = lds_read16(b_off[q % NT] + off + (q / NT) * (NT / 2) * PIECE_TILE);
+        } else if (SC) {
+            const int j = o - 2 * AP - NT * BP;
+            fs[set][j] = lds_read4(s_off + off + j * 128);
         }
+    };
+    auto read_stage = [&](int set, int buf) {
+#pragma unroll
+        for (int o = 0; o < READS; o++) read_one(set, buf, o);
+    };
+    // Wait for every LDS read issued so far (the operand set `set` among them; the empty statements name its
+    // registers so that nothing touches them before the data is there) and for all loads except the youngest
+    // `young`, then meet the other wavefronts.
+    auto settle = [&](int set) {
 #pragma unroll
         for (int p = 0; p < AP; p++)
 #pragma unroll
-            for (int i = 0; i < 2; i++) fa[set][p][i] = lds_read16(a_off[i] + off + p * PIECE_TILE);
+            for (int i = 0; i < 2; i++) asm volatile("" : "+v"(fa[set][p][i])::"memory");
 #pragma unroll
         for (int p = 0; p < BP; p++)
 #pragma unroll
-            for (int i = 0; i < 2; i++) fb[set][p][i] = lds_read16(b_off[i] + off + p * PIECE_TILE);
-    };
-    // Wait for every LDS read issued so far (the operand set `set` among them; the statement names its
-    // registers so that nothing touches them before the data is there) and for all loads except the
-    // youngest (NB - 2) T (DRAIN: for all of them), then meet the other wavefronts.
-#define HM_PIECES_WAIT(CNT, SET)                                                                                    \
-    do {                                                                                                            \
-        if constexpr (SC)                                                                                           \
-            asm volatile("s_waitcnt vmcnt(" #CNT ") lgkmcnt(0)\n\ts_barrier"                                        \
-                         : "+v"(fa[SET][0][0]), "+v"(fa[SET][0][1]), "+v"(fa[SET][1][0]), "+v"(fa[SET][1][1]),      \
-                           "+v"(fa[SET][2][0]), "+v"(fa[SET][2][1]), "+v"(fb[SET][0][0]), "+v"(fb[SET][0][1]),      \
-                           "+v"(fs[SET][0]), "+v"(fs[SET][1])                                                       \
-                         :                                                                                          \
-                         : "memory");                                                                               \
-        else if constexpr (AP == 3 && BP == 3)                                                                      \
-            asm volatile("s_waitcnt vmcnt(" #CNT ") lgkmcnt(0)\n\ts_barrier"                                        \
-                         : "+v"(fa[SET][0][0]), "+v"(fa[SET][0][1]), "+v"(fa[SET][1][0]), "+v"(fa[SET][1][1]),      \
-                           "+v"(fa[SET][2][0]), "+v"(fa[SET][2][1]), "+v"(fb[SET][0][0]), "+v"(fb[SET][0][1]),      \
-                           "+v"(fb[SET][1][0]), "+v"(fb[SET][1][1]), "+v"(fb[SET][2][0]), "+v"(fb[SET][2][1])       \
-                         :                                                                                          \
-                         : "memory");                                                                               \
-        else if constexpr (AP == 1)                                                                                 \
-            asm volatile("s_waitcnt vmcnt(" #CNT ") lgkmcnt(0)\n\ts_barrier"                                        \
-                         : "+v"(fa[SET][0][0]), "+v"(fa[SET][0][1]), "+v"(fb[SET][0][0]), "+v"(fb[SET][0][1])       \
-                         :                                                                                          \
-                         : "memory");                                                                               \
-        else if constexpr (AP == 3)                                                                                 \
-            asm volatile("s_waitcnt vmcnt(" #CNT ") lgkmcnt(0)\n\ts_barrier"                                        \
-                         : "+v"(fa[SET][0][0]), "+v"(fa[SET][0][1]), "+v"(fa[SET][1][0]), "+v"(fa[SET][1][1]),      \
-                           "+v"(fa[SET][2][0]), "+v"(fa[SET][2][1]), "+v"(fb[SET][0][0]), "+v"(fb[SET][0][1])       \
-                         :                                                                                          \
-                         : "memory");                                                                               \
-        else                                                                                                        \
-            asm volatile("s_waitcnt vmcnt(" #CNT ") lgkmcnt(0)\n\ts_barrier"                                        \
-                         : "+v"(fa[SET][0][0]), "+v"(fa[SET][0][1]), "+v"(fa[SET][1][0]), "+v"(fa[SET][1][1]),      \
-                           "+v"(fb[SET][0][0]), "+v"(fb[SET][0][1])                                                 \
-                         :                                                                                          \
-                         : "memory");                                                                               \
-    } while (0)
-    // (NB - 2) T: 3 x 1 pieces 8, 2 x 1 pieces 6, 3 x 3 pieces 6, 1 x 1 pieces 4
-    static_assert(AP != 1 || (BP == 1 && !SC && (NB - 2) * T == 4), "wait count");
-    static_assert(!SC || (AP == 3 && (NB - 2) * T == 10), "wait count");
-    static_assert(SC || (AP == 3 && BP == 1 && (NB - 2) * T == 8) || (AP != 3 || BP != 1), "wait count");
-    static_assert(SC || ((AP == 2 || BP == 3) && (NB - 2) * T == 6) || AP == 1 || (AP == 3 && BP == 1), "wait count");
-    auto wait_and_meet = [&](int set) {
-        if (set == 0) {
-            if constexpr (SC) HM_PIECES_WAIT(10, 0); else if constexpr (AP == 1) HM_PIECES_WAIT(4, 0); else if constexpr (AP == 3 && BP == 1) HM_PIECES_WAIT(8, 0); else HM_PIECES_WAIT(6, 0);
-        } else {
-            if constexpr (SC) HM_PIECES_WAIT(10, 1); else if constexpr (AP == 1) HM_PIECES_WAIT(4, 1); else if constexpr (AP == 3 && BP == 1) HM_PIECES_WAIT(8, 1); else HM_PIECES_WAIT(6, 1);
+            for (int j = 0; j < NT; j++) asm volatile("" : "+v"(fb[set][p][j])::"memory");
+        if constexpr (SC) {
+#pragma unroll
+            for (int j = 0; j < NT; j++) asm volatile("" : "+v"(fs[set][j])::"memory");
         }
     };
-    // the products of one stage: smallest pieces first
-    auto multiply = [&](int set) {
+    auto wait_and_meet = [&](int set) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NB - 2) * T) : "memory");
+        settle(set);
+    };
+    // The products of one stage, smallest pieces first, with the stage's loads and operand reads dealt out between them
+    constexpr int PRODUCTS = BP == 1 ? AP : 6, MFMAS = PRODUCTS * 2 * NT, OPS = T + READS;
+    auto multiply = [&](int set, int buf, int nbuf, bool live) {
+        auto ops_behind = [&](int m) {
+#pragma unroll
+            for (int o = 0; o < OPS; o++)
+                if (o * MFMAS / OPS == m) {
+                    // every other one a load until they are out
+                    if (o < 2 * T && (o & 1)) request_one(buf, o / 2);
+                    else read_one(set ^ 1, nbuf, o < 2 * T ? o / 2 : o - T);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (!live) {
+#pragma unroll
+            for (int m = 0; m < MFMAS; m++) ops_behind(m);
+            k_req += TK;
+            return;
+        }
         if constexpr (SC) {
             // the block's sum on its own (smallest pieces first), then times the block's scale
+            int m = 0;
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
+                for (int j = 0; j < NT; j++) {
                     f32x16 t;
 #pragma unroll
                     for (int v = 0; v < 16; v++) t[v] = 0.f;
 #pragma unroll
-                    for (int pa = AP - 1; pa >= 0; pa--)
+                    for (int pa = AP - 1; pa >= 0; pa--) {
                         t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[set][pa][i], fb[set][0][j], t, 0, 0, 0);
+                        ops_behind(m++);
+                    }
 #pragma unroll
                     for (int v = 0; v < 16; v++) acc[i][j][v] = fmaf(t[v], fs[set][j], acc[i][j][v]);
                 }
-            return;
+        } else {
+            int m = 0;
+#pragma unroll
+            for (int order = AP + BP - 2; order >= 0; order--)
+#pragma unroll
+                for (int pa = AP - 1; pa >= 0; pa--) {
+                    const int pb = order - pa;
+                    if (pb < 0 || pb >= BP || (BP > 1 && order > 2)) continue;
+#pragma unroll
+                    for (int i = 0; i < 2; i++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++) {
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[set][pa][i], fb[set][pb][j], acc[i][j], 0, 0, 0);
+                            ops_behind(m++);
+                        }
+                }
         }
-#pragma unroll
-        for (int order = AP + BP - 2; order >= 0; order--)
-#pragma unroll
-            for (int pa = AP - 1; pa >= 0; pa--) {
-                const int pb = order - pa;
-                if (pb < 0 || pb >= BP || (BP > 1 && order > 2)) continue;
-#pragma unroll
-                for (int i = 0; i < 2; i++)
-#pragma unroll
-                    for (int j = 0; j < 2; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[set][pa][i], fb[set][pb][j], acc[i][j], 0, 0, 0);
-            }
+        k_req += TK;
     };
 
     // stage 0 has landed for everyone (NB - 1 stages of T loads may be in flight)
@@ -276,10 +295,7 @@ __global__ __launch_bounds__(THREADS) void gemm_pieces_kernel(const uint16_t *__
     auto stage = [&](int set, bool live) {
         wait_and_meet(set);
         const int nbuf = buf + 1 == NB ? 0 : buf + 1;
-        request(buf);
-        read_stage(set ^ 1, nbuf);
-        if (live) multiply(set);
-        __builtin_amdgcn_sched_barrier(0);
+        multiply(set, buf, nbuf, live);
         buf = nbuf;
     };
     for (int s = 0; s < ns; s += 2) {
@@ -288,54 +304,77 @@ __global__ __launch_bounds__(THREADS) void gemm_pieces_kernel(const uint16_t *__
     }
 
     // drain what is in flight before the buffers are reused: loads into LDS, and the operand reads of
-    // the stage after the last, which target set 0 (the wait names it, so its registers stay untouched
-    // until the data has arrived). Then the second k group hands its sums over through LDS (64 KiB = 4
-    // wavefronts x 64 x 64 floats, lane-major).
-    HM_PIECES_WAIT(0, 0);
-#undef HM_PIECES_WAIT
-    float *xch = reinterpret_cast<float *>(stage_lds) + (size_t)(wave & 3) * 64 * 64 + lane;
-    if (kgrp == 1) {
+    // the stage after the last, which target set 0 (named behind the wait, so its registers stay untouched
+    // until the data has arrived). Then the two k groups trade halves of their tiles through LDS (lane-major): group g
+    // finishes the 32-row tiles i = g.
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    settle(0);
+    float *xch = reinterpret_cast<float *>(stage_lds) + (size_t)wave * (16 * NT) * 64 + lane;
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+    for (int j = 0; j < NT; j++)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) xch[((i * 2 + j) * 16 + v) * 64] = acc[i][j][v];
-    }
+        for (int v = 0; v < 16; v++) xch[(j * 16 + v) * 64] = kgrp ? acc[0][j][v] : acc[1][j][v];
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (kgrp == 1) return;
+    const float *got = reinterpret_cast<const float *>(stage_lds) + (size_t)(wave ^ 4) * (16 * NT) * 64 + lane;
 
     // accumulator element v of lane l sits at row (v/4)*8 + (l/32)*4 + v%4, column l%32
     const bool interior = m0 + TM <= M && n0 + TN <= N;
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int j = 0; j < NT; j++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int row = m0 + wm * 64 + i * 32 + (v >> 2) * 8 + lh * 4 + (v & 3);
-                const int col = n0 + wn * 64 + j * 32 + l32;
-                const float sum = acc[i][j][v] + xch[((i * 2 + j) * 16 + v) * 64];
-                if constexpr (GR) {
-                    if (row < M && col < N) __builtin_nontemporal_store(sum, C + (size_t)list[row] * g.ldc + col);
-                } else if (interior) {
-                    __builtin_nontemporal_store(sum, C + (size_t)row * g.ldc + col);
-                } else if (row < M && col < N) {
-                    __builtin_nontemporal_store(sum, C + (size_t)row * g.ldc + col);
-                }
+        for (int v = 0; v < 16; v++) {
+            const int row = m0 + wm * 64 + kgrp * 32 + (v >> 2) * 8 + lh * 4 + (v & 3);
+            const int col = n0 + wn * (NT * 32) + j * 32 + l32;
+            const float sum = (kgrp ? acc[1][j][v] : acc[0][j][v]) + got[(j * 16 + v) * 64];
+            if constexpr (GR) {
+                if (row < M && col < N) __builtin_nontemporal_store(sum, C + (size_t)list[row] * g.ldc + col);
+            } else if (interior) {
+                __builtin_nontemporal_store(sum, C + (size_t)row * g.ldc + col);
+            } else if (row < M && col < N) {
+                __builtin_nontemporal_store(sum, C + (size_t)row * g.ldc + col);
             }
+        }
 }
 
-template <int AP, int BP, bool SC = false, bool GR = false>
+template <int AP, int BP, bool SC = false, bool GR = false, int NT = 2>
 int launch(hm_ctx *ctx, const char *who, const uint16_t *a, const uint16_t *b, float *c, const PieceDims &g,
-           unsigned tiles, unsigned slices, unsigned batch = 1) {
-    using S = Shape<AP, BP, SC>;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pieces_kernel<AP, BP, SC, GR>),
+           unsigned grid, unsigned batch = 1) {
+    using S = Shape<AP, BP, SC, NT>;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_pieces_kernel<AP, BP, SC, GR, NT>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
     HM_REQUIRE(ctx, attr == hipSuccess, "%s: cannot reserve %d bytes of LDS: %s", who, S::LDS, hipGetErrorString(attr));
-    hipLaunchKernelGGL((gemm_pieces_kernel<AP, BP, SC, GR>), dim3(tiles, slices, batch), dim3(THREADS), S::LDS, ctx->stream, a, b, c, g);
+    hipLaunchKernelGGL((gemm_pieces_kernel<AP, BP, SC, GR, NT>), dim3(grid, 1, batch), dim3(THREADS), S::LDS, ctx->stream, a, b, c, g);
     HM_LAUNCH_CHECK(ctx);
     return HM_OK;
+}
+
+constexpr int TN = 128;  // of the narrow tile
+
+unsigned whole_dies(long long workgroups) { return (unsigned)((workgroups + 7) / 8 * 8); }
+
+// Tile width and K slices of a product on `cus` CUs (slices: at most max_parts, at least eight stages each): the pair with
+// the least estimated time among those that the callers' buffers hold, in microseconds: 8 around the loop, a stage of a round of workgroups 0.5 (128 wide) or 0.75
+// (256 wide), partial sums written and read again at 7 TB/s. Measured, 3 x 1 pieces, 512 rows: 1024 -> 4096 128 wide in
+// 2 slices 18.4, 256 wide in 4 19.2; 1024 -> 6144 28.6 in 1 and 24.9 in 2; 2048 -> 1024 12.9 and 17.3 in 8; 8960 -> 1536
+// 53.6 in 4 and 44.0 in 8. 2048 rows: 59.0 and 46.7, 88.3 and 83.3 in 1, 30.5 in 2 and 28.0 in 4.
+struct Cut {
+    int nt, slices, stages_per_split;
+};
+Cut cut_for(long long m_tiles, int N, int ns, long long out_bytes, int cus, int max_parts, bool wide_ok) {
+    Cut best{2, 1, (ns + 1) / 2 * 2};
+    double least = 1e30;
+    for (int nt = 2; nt <= (wide_ok ? 4 : 2); nt += 2)
+        for (int want = 1; want <= std::max(1, std::min(max_parts, ns / 8)); want++) {
+            const int per = ((ns + want - 1) / want + 1) / 2 * 2, slices = (ns + per - 1) / per;  // even: stages run in pairs
+            if (slices > 1 && m_tiles * ((N + 127) / 128) * slices > homura::gemm_sliced_tiles(cus)) continue;
+            const long long wgs = m_tiles * ((N + 64 * nt - 1) / (64 * nt)) * slices;
+            const double us = 8 + (double)((wgs + cus - 1) / cus) * per * (nt == 2 ? 0.5 : 0.75) + 2.0 * slices * (double)out_bytes / 7e6;
+            if (us < least) {
+                least = us;
+                best = Cut{nt, slices, per};
+            }
+        }
+    return best;
 }
 
 }  // namespace
@@ -374,7 +413,9 @@ int homura::gemm_pieces_batched(hm_ctx *ctx, const uint16_t *d_a_split, size_t a
     g.a_batch = a_batch;
     g.b_batch = b_batch;
     g.c_batch = c_batch;
-    return launch<3, 1>(ctx, "gemm_pieces_batched", d_a_split, d_b_nk, d_c, g, (unsigned)tiles, 1, (unsigned)batch);
+    g.tiles = (int)tiles;
+    g.slices = 1;
+    return launch<3, 1>(ctx, "gemm_pieces_batched", d_a_split, d_b_nk, d_c, g, whole_dies(tiles), (unsigned)batch);
 }
 
 int homura::gemm_grouped_nk(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, int a_rows, const uint16_t *d_b_nk, float *d_c,
@@ -405,8 +446,8 @@ int homura::gemm_grouped_nk(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, 
     g.stages_per_split = (K / TK + 1) / 2 * 2;
     g.b_batch = (size_t)N * K;
     g.lists = l;
-    if (pieces == 1) return launch<1, 1, false, true>(ctx, "gemm_grouped", d_a_split, d_b_nk, d_c, g, (unsigned)tiles, 1);
-    return launch<3, 1, false, true>(ctx, "gemm_grouped", d_a_split, d_b_nk, d_c, g, (unsigned)tiles, 1);
+    if (pieces == 1) return launch<1, 1, false, true>(ctx, "gemm_grouped", d_a_split, d_b_nk, d_c, g, (unsigned)tiles);
+    return launch<3, 1, false, true>(ctx, "gemm_grouped", d_a_split, d_b_nk, d_c, g, (unsigned)tiles);
 }
 
 int homura::gemm_pieces_any(hm_ctx *ctx, const uint16_t *d_a_split, int a_pieces, const uint16_t *d_b_split, int b_pieces,
@@ -419,8 +460,7 @@ int homura::gemm_pieces_any(hm_ctx *ctx, const uint16_t *d_a_split, int a_pieces
     HM_REQUIRE(ctx, (b_pieces == 1 && (a_pieces == 2 || a_pieces == 3)) || (b_pieces == 3 && a_pieces == 3),
                "%s: %d x %d pieces (2 x 1, 3 x 1 or 3 x 3)", who, a_pieces, b_pieces);
     HM_REQUIRE(ctx, ((uintptr_t)d_a_split % 16) == 0 && ((uintptr_t)d_b_split % 16) == 0, "%s: operands must be 16-byte aligned", who);
-    const long long tiles = (long long)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
-    HM_REQUIRE(ctx, tiles <= 0x7fffffffLL, "%s: too many tiles", who);
+    HM_REQUIRE(ctx, (long long)((M + TM - 1) / TM) * ((N + TN - 1) / TN) <= 0x7fffff00LL, "%s: too many tiles", who);
     PieceDims g{};
     g.M = M;
     g.N = N;
@@ -431,17 +471,21 @@ int homura::gemm_pieces_any(hm_ctx *ctx, const uint16_t *d_a_split, int a_pieces
     g.scales = d_scales;
     g.npad = npad;
     HM_REQUIRE(ctx, g.ldc >= N, "%s: ldc %d below N %d", who, g.ldc, N);
-    // K slices while they still add whole waves of workgroups to a grid smaller than the chip, at least
-    // eight stages (256 k) per slice
-    const int ns_total = K / TK;
-    int want = (int)std::max<long long>(1, ctx->num_cus / tiles);
-    want = std::min(std::min(want, std::max(1, max_parts)), std::max(1, ns_total / 8));
-    if (!parts) want = 1;
-    g.stages_per_split = ((ns_total + want - 1) / want + 1) / 2 * 2;  // even: stages run in pairs
-    const int slices = (ns_total + g.stages_per_split - 1) / g.stages_per_split;
-    if (parts) *parts = slices;
-    if (d_scales) return launch<3, 1, true>(ctx, who, d_a_split, d_b_split, d_c, g, (unsigned)tiles, (unsigned)slices);
-    if (b_pieces == 3) return launch<3, 3>(ctx, who, d_a_split, d_b_split, d_c, g, (unsigned)tiles, (unsigned)slices);
-    if (a_pieces == 3) return launch<3, 1>(ctx, who, d_a_split, d_b_split, d_c, g, (unsigned)tiles, (unsigned)slices);
-    return launch<2, 1>(ctx, who, d_a_split, d_b_split, d_c, g, (unsigned)tiles, (unsigned)slices);
+    const Cut cut = cut_for((M + TM - 1) / TM, N, K / TK, 4LL * M * N, ctx->num_cus, parts ? max_parts : 1,
+                            b_pieces == 1 && !d_scales);  // (a wide scaled tile does not fit the registers)
+    g.stages_per_split = cut.stages_per_split;
+    g.slices = cut.slices;
+    g.tiles = (int)((long long)((M + TM - 1) / TM) * ((N + 64 * cut.nt - 1) / (64 * cut.nt)));
+    // Every die gets a stretch of the tiles, slice by slice: it then reads only its slices' columns of both operands. Within
+    // a slice the larger operand is the one that the dies read parts of (2048 rows, 1024 -> 6144: 83.3 us column by column,
+    // 78.3 row by row).
+    g.n_fast = (long long)a_pieces * M >= (long long)b_pieces * N;
+    if (parts) *parts = cut.slices;
+    const unsigned grid = whole_dies((long long)g.tiles * g.slices);
+    if (d_scales) return launch<3, 1, true>(ctx, who, d_a_split, d_b_split, d_c, g, grid);
+    if (b_pieces == 3) return launch<3, 3>(ctx, who, d_a_split, d_b_split, d_c, g, grid);
+    if (a_pieces == 3) return cut.nt == 4 ? launch<3, 1, false, false, 4>(ctx, who, d_a_split, d_b_split, d_c, g, grid)
+                                          : launch<3, 1>(ctx, who, d_a_split, d_b_split, d_c, g, grid);
+    return cut.nt == 4 ? launch<2, 1, false, false, 4>(ctx, who, d_a_split, d_b_split, d_c, g, grid)
+                       : launch<2, 1>(ctx, who, d_a_split, d_b_split, d_c, g, grid);
 }

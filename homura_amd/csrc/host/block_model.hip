@@ -1116,9 +1116,8 @@ int BlockModel::prepare_prefill() {
     PrefillScratch &p = pf_;
     if (p.rows) return HM_OK;
     const int64_t rows = std::min(chunk_rows_, max_seq_len_);
-    // A product is cut into K slices only while its 128 x 128 tiles times the slices stay within the CUs, so this
-    // holds the slices of a product of any width up to n.
-    auto sliced = [&](int64_t n) { return std::max<int64_t>(rows * n, (int64_t)ctx_->num_cus * 128 * 128); };
+    // holds the slices of a product of any width up to n
+    auto sliced = [&](int64_t n) { return std::max<int64_t>(rows * n, gemm_sliced_tiles(ctx_->num_cus) * 128 * 128); };
     int64_t d1 = wp_, d2 = 32, d3 = 32, f1 = 32, f2 = 32, f3 = 32, split = 2 * wp_, lat = 32, kvf = 32, kws = 32, vws = 32;
     int64_t mm_qk = 32, mm_heads = 1, mm_ahead = 32, mm_values = 32, experts = 1, top = 1;
     for (size_t i = 0; i < cfg_.layers.size(); i++) {

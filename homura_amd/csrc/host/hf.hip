@@ -1878,6 +1878,7 @@ const float *HfModel::weight_f32(const std::string &name) const {
 }
 
 int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
+    constexpr int HEAD_ROWS = 512;  // rows whose logits are held at a time
     const TransformerConfig &c = cfg_;
     const int hidden = c.hidden_size, inter = c.intermediate_size, vocab = c.vocab_size;
     const int H = c.num_attention_heads, kvh = c.kv_heads(), hd = c.head_dim();
@@ -1886,7 +1887,11 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     PrefillScratch &p = pf_;
     const bool quant = dtype_is_quantized(weight_dtype_);
     if (p.rows < n) {
-        const int rows = std::max(n, 128);
+        // powers of two, so that prompts of growing length do not each reallocate
+        int rows = 128;
+        while (rows < n) rows *= 2;
+        rows = std::min(rows, std::max(chunk_rows_, n));
+        auto sliced = [&](int64_t width) { return std::max<int64_t>(rows * width, gemm_sliced_tiles(ctx_->num_cus) * 128 * 128); };
         const int64_t widest = std::max<int64_t>(std::max(hidden, qd), inter);
         hm_sync(ctx_);
         {
@@ -1898,15 +1903,16 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
             grown.icache_off = p.icache_off;
             grown.scache = std::move(p.scache);
             grown.scache_off = p.scache_off;
+            grown.wcache = std::move(p.wcache);
             p = std::move(grown);
         }
         p.ids = Buffer::alloc(ctx_, {rows}, DType::F32);  // int32 ids
         p.h = Buffer::alloc(ctx_, {rows, hidden}, DType::F32);
         p.resid = Buffer::alloc(ctx_, {rows, hidden}, DType::F32);
         p.split = Buffer::alloc(ctx_, {rows, 3 * widest}, DType::BF16);
-        p.qkv = Buffer::alloc(ctx_, {PrefillScratch::MAX_PARTS, rows, nqkv}, DType::F32);
-        p.proj_out = Buffer::alloc(ctx_, {PrefillScratch::MAX_PARTS, rows, hidden}, DType::F32);
-        p.gate_up = Buffer::alloc(ctx_, {PrefillScratch::MAX_PARTS, rows, 2 * (int64_t)inter}, DType::F32);
+        p.qkv = Buffer::alloc(ctx_, {sliced(nqkv)}, DType::F32);
+        p.proj_out = Buffer::alloc(ctx_, {sliced(hidden)}, DType::F32);
+        p.gate_up = Buffer::alloc(ctx_, {sliced(std::max<int64_t>(2 * (int64_t)inter, qd))}, DType::F32);
         if (!p.ids || !p.h || !p.resid || !p.split || !p.qkv || !p.proj_out || !p.gate_up) return HM_ERR_OOM;
         if (quant && widest % 256 == 0) {  // Q8_K rows for K-quant groups (a float holds four of the int8 values)
             p.q8 = Buffer::alloc(ctx_, {rows, widest / 4}, DType::F32);
@@ -1921,7 +1927,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         p.rows = rows;
     }
     if (h_logits && !p.logits) {
-        p.logits = Buffer::alloc(ctx_, {p.rows, vocab}, DType::F32);
+        p.logits = Buffer::alloc(ctx_, {std::min(p.rows, HEAD_ROWS), vocab}, DType::F32);
         if (!p.logits) return HM_ERR_OOM;
     }
     KvCache *kv = plan_->kv_cache();
@@ -2201,26 +2207,29 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     }
     if (h_logits) {  // LM head (reference src/hf/emitter.rs:828-862) for every row
         rc = rmsnorm_split_launch(ctx_, x, res, res_parts, weight_f32("model.norm.weight"), split, np, nullptr, n, hidden, eps);
-        if (rc == HM_OK && !quant)
-            rc = gemm_split_nk(ctx_, split, np, lm_head_packed_.as<uint16_t>(), p.logits.as<float>(), n, hidden, vocab);
-        if (rc == HM_OK && quant) {
-            // the quantised plan's LM head is f32 [vocab][hidden] (reference src/hf/emitter_quant.rs:1390-1437):
-            // slabs of its rows become bf16 pieces in wsplit, as many as fit
-            const int slab = (int)std::min<int64_t>(vocab, (int64_t)(p.wsplit.bytes() / 2) / (3 * (int64_t)hidden) / 128 * 128);
-            if (slab <= 0) return hm_set_error(ctx_, HM_ERR_STATE, "prefill: weight scratch too small for the LM head");
-            const size_t head_rowbytes = lm_head_blocks_ ? lm_head_blocks_.bytes() / (size_t)vocab : 0;
-            for (int v0 = 0; v0 < vocab && rc == HM_OK; v0 += slab) {
-                const int rows = std::min(slab, vocab - v0);
-                if (lm_head_blocks_)  // rows of the output matrix dequantised from its blocks (bit-exact) into the pieces
-                    rc = dequant_split_launch(ctx_, (int)lm_head_blocks_dtype_, lm_head_blocks_.as<uint8_t>() + (size_t)v0 * head_rowbytes,
-                                              rows, (int)hidden, wsplit, 1, 0);
-                else
-                    rc = split_rows_launch(ctx_, lm_head_packed_.as<float>() + (size_t)v0 * hidden, wsplit, 3, (size_t)rows, hidden);
-                if (rc == HM_OK)
-                    rc = gemm_split_split_nk(ctx_, split, wsplit, p.logits.as<float>() + v0, n, hidden, rows, 1, nullptr, vocab);
+        for (int r0 = 0; r0 < n && rc == HM_OK; r0 += HEAD_ROWS) {
+            const int m = std::min(HEAD_ROWS, n - r0);
+            const uint16_t *rows = split + (size_t)r0 * np * hidden;
+            if (!quant) rc = gemm_split_nk(ctx_, rows, np, lm_head_packed_.as<uint16_t>(), p.logits.as<float>(), m, hidden, vocab);
+            else {
+                // the quantised plan's LM head is f32 [vocab][hidden] (reference src/hf/emitter_quant.rs:1390-1437):
+                // slabs of its rows become bf16 pieces in wsplit, as many as fit
+                const int slab = (int)std::min<int64_t>(vocab, (int64_t)(p.wsplit.bytes() / 2) / (3 * (int64_t)hidden) / 128 * 128);
+                if (slab <= 0) return hm_set_error(ctx_, HM_ERR_STATE, "prefill: weight scratch too small for the LM head");
+                const size_t head_rowbytes = lm_head_blocks_ ? lm_head_blocks_.bytes() / (size_t)vocab : 0;
+                for (int v0 = 0; v0 < vocab && rc == HM_OK; v0 += slab) {
+                    const int cols = std::min(slab, vocab - v0);
+                    if (lm_head_blocks_)  // rows of the output matrix dequantised from its blocks (bit-exact) into the pieces
+                        rc = dequant_split_launch(ctx_, (int)lm_head_blocks_dtype_, lm_head_blocks_.as<uint8_t>() + (size_t)v0 * head_rowbytes,
+                                                  cols, (int)hidden, wsplit, 1, 0);
+                    else
+                        rc = split_rows_launch(ctx_, lm_head_packed_.as<float>() + (size_t)v0 * hidden, wsplit, 3, (size_t)cols, hidden);
+                    if (rc == HM_OK)
+                        rc = gemm_split_split_nk(ctx_, rows, wsplit, p.logits.as<float>() + v0, m, hidden, cols, 1, nullptr, vocab);
+                }
             }
+            if (rc == HM_OK) rc = hm_download(ctx_, h_logits + (size_t)r0 * vocab, p.logits.ptr(), (size_t)m * vocab * 4);
         }
-        if (rc == HM_OK) rc = hm_download(ctx_, h_logits, p.logits.ptr(), (size_t)n * vocab * 4);
         if (rc != HM_OK) return rc;
     }
     // one advance after all layers appended (reference src/runtime.rs:1875-1880)
