@@ -412,7 +412,7 @@ int hm_model_run_kv(hm_model *m, const int64_t *h_ids, int n_ids, float *h_logit
 /* The multi-token pass that hm_model_run_kv and hm_model_generate_greedy take for inputs of at
  * least `prefill_min` tokens (reference HfGenerationContext::prefill, src/hf/model.rs:321-336: the
  * whole prompt in one run_kv): projections as GEMMs on the matrix cores, causal attention over
- * cache + chunk, chunks of 512 rows. head_dim 64 or 128; h_logits [n_ids][vocab] or NULL (then the
+ * cache + chunk, chunks of at most 4096 rows. head_dim 64 or 128; h_logits [n_ids][vocab] or NULL (then the
  * LM head is skipped). bf16 models need widths that are multiples of 32. Block-quantised models
  * (the products of hm_gemm_f32_quant_nk) need multiples of 64, and q|k|v as well as gate|up must each
  * be of one kind, Q8_0 / Q4_0 or K-quants, because the members of a group share an activation
