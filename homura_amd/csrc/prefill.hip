@@ -265,8 +265,9 @@ extern __shared__ __attribute__((aligned(16))) char at_lds[];
 // 64, 32 rows, for prompts whose rows x heads alone leave most of the chip idle). A wavefront needs ~150
 // registers, so two or three share a SIMD and one's matrix instructions run under the others' softmax arithmetic.
 // K and V tiles (32 keys) go global -> LDS directly (global_load_lds_dwordx4, no staging registers, no LDS
-// write instructions), row-major and XOR-swizzled on the global side; two sets of KS tile pairs alternate, the
-// next round's tiles arrive while this round is multiplied.
+// write instructions), row-major and XOR-swizzled on the global side; two sets of KS TW tile pairs alternate, the
+// next round's tiles arrive while this round is multiplied. With TW = 2 a wavefront takes two tiles between barriers: the
+// scores of both, one maximum, both products with V (2944 rows behind 3072, 16 heads: 304 -> 283 us with two key groups).
 //   S^T block: A = 16 keys x 32 dims from the K tile, B = the queries' pieces; lane q + 16 c receives keys
 //   4 c .. 4 c + 3 of the block for query q.
 //   O^T block: A = 16 dims x 32 keys, B = the probabilities' pieces. Contraction slot 8 c + i (i < 4) stands
@@ -322,15 +323,17 @@ __device__ __forceinline__ void store_heads4(const PrefillAttnArgs &a, int qrow,
     }
 }
 
-template <int DK, int DV, int NQ, int NP, int KP, int KS, int SETS, bool RING = false>
+template <int DK, int DV, int NQ, int NP, int KP, int KS, int SETS, bool RING = false, int TW = 1>
 __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnArgs a) {
+    static_assert(!RING || TW == 1, "kept rounds are counted in single tiles");
+    constexpr int TILES = KS * TW;                     // tile pairs of a round
     constexpr int KSTEPS = DK / 32;                    // k steps of K . Q
     constexpr int DB = DV / 16;                        // 16-row blocks of O^T
     constexpr int QW = A8_WAVES / KS;                  // 16-row query blocks per workgroup
     constexpr int AT_QROWS = 16 * QW;
     constexpr int KTILE = A8_KEYS * DK * 2, VTILE = A8_KEYS * DV * 2;  // bytes of one piece of a K or V tile
     constexpr int PAIR = KP * (KTILE + VTILE);
-    constexpr int SET = KS * PAIR;                     // the KS tile pairs of a round
+    constexpr int SET = TILES * PAIR;
     constexpr int KCHUNKS = A8_KEYS * DK / 8, VCHUNKS = A8_KEYS * DV / 8;  // 16-byte chunks of a tile
     constexpr int KLOADS = (KCHUNKS + A8_THREADS - 1) / A8_THREADS, VLOADS = (VCHUNKS + A8_THREADS - 1) / A8_THREADS;
 
@@ -339,13 +342,15 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
     // Workgroups are dealt to the eight dies round-robin by their linear index. With a multiple of eight heads
     // every die gets H / 8 neighbouring heads and all their row blocks, so the K and V rows of a KV head are
     // fetched into one die's L2 (or as few as the head grouping allows) instead of all eight.
-    int hx = blockIdx.y, bx = blockIdx.x;
-    if (a.H % 8 == 0) {
-        const int lin = blockIdx.y * gridDim.x + blockIdx.x, per = a.H / 8;
-        hx = (lin & 7) * per + (lin >> 3) % per;
-        bx = (lin >> 3) / per;
-    }
+    // Otherwise all heads of a row block follow one another. Either way the row blocks come in order: within a die
+    // workgroups are dealt to its engines round-robin and wait in line for their engine, so an order in which an engine
+    // always gets the long ones would make the others wait (2000 rows, 12 heads, head by head: 89.8 us with two key groups; this way 49.8).
+    const int lin = blockIdx.y * gridDim.x + blockIdx.x, per = a.H / 8;
+    const bool by_die = a.H % 8 == 0;
+    const int hx = by_die ? (lin & 7) * per + (lin >> 3) % per : lin % a.H;
+    int bx = by_die ? (lin >> 3) / per : lin / a.H;
     const int h = hx, kvhd = h / (a.H / a.kvh);
+    bx = (int)gridDim.x - 1 - bx;  // the row blocks that see the most keys first: the light ones fill the last round
     const int q0 = bx * AT_QROWS;
     const int kv_total = a.past + a.S;
     const uint16_t *kc = a.kcache + (size_t)kvhd * a.max_len * DK;
@@ -354,12 +359,12 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
     const int wg_end = a.past + min(a.S, q0 + AT_QROWS);
     const int wave_end = q0 + qw * 16 < a.S ? a.past + min(a.S, q0 + qw * 16 + 16) : 0;
     const int ntiles = (wg_end + A8_KEYS - 1) / A8_KEYS;
-    const int nrounds_end = (ntiles + KS - 1) / KS;
+    const int nrounds_end = (ntiles + TILES - 1) / TILES;
     const int wave_first = a.past + min(q0 + qw * 16, a.S - 1);
     // first key that the first / the last row of this wavefront sees, and the round the workgroup starts with
     const int wave_lo = a.window ? max(0, wave_first - a.window + 1) : 0;
     const int wave_lo_last = a.window ? a.past + min(q0 + qw * 16 + 15, a.S - 1) - a.window + 1 : 0;
-    const int first_round = a.window ? max(0, a.past + q0 - a.window + 1) / (A8_KEYS * KS) : 0;
+    const int first_round = a.window ? max(0, a.past + q0 - a.window + 1) / (A8_KEYS * TILES) : 0;
     // RING: rounds that hold the kept first keys come ahead of the window's; between the two lie `skip` that nobody sees
     const int keep = RING ? a.keep : 0;
     const int kept_rounds = RING && a.window ? min(first_round, (keep + A8_KEYS * KS - 1) / (A8_KEYS * KS)) : 0;
@@ -367,7 +372,7 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
     // the rounds of this workgroup: all of them, or its share when the keys are cut over gridDim.z workgroups
     const int per_z = (nrounds_end - skip - r_first + (int)gridDim.z - 1) / (int)gridDim.z;
     const int r_begin = r_first + (int)blockIdx.z * per_z, nrounds = min(nrounds_end - skip, r_begin + per_z);
-    auto tile_of = [&](int r, int u) { return (RING && r >= kept_rounds ? r + skip : r) * KS + u; };
+    auto tile_of = [&](int r, int u) { return (RING && r >= kept_rounds ? r + skip : r) * TILES + u; };
     // RING: the slot of a position. What the window sees never spans more than one turn of the ring, so positions
     // count from the turn that holds its first row; rows ahead of that one are masked and may be any.
     int ring_base = 0;
@@ -398,7 +403,7 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
     auto request_round = [&](int r) {
         char *base = at_lds + (SETS == 2 ? (r & 1) * SET : 0) + wave_dst;
 #pragma unroll
-        for (int u = 0; u < KS; u++) {
+        for (int u = 0; u < TILES; u++) {
             const int key0 = tile_of(r, u) * A8_KEYS;
 #pragma unroll
             for (int i = 0; i < KLOADS; i++) {
@@ -464,32 +469,33 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (SETS == 2 && r + 1 < nrounds) request_round(r + 1);
-        const int t = tile_of(r, kh);            // this wavefront's tile of the round
+        const int t = tile_of(r, kh * TW);       // this wavefront's first tile of the round
         // wavefront-uniform: nothing visible to these 16 rows
-        if (t * A8_KEYS >= wave_end || (t * A8_KEYS + A8_KEYS <= wave_lo && (!RING || t * A8_KEYS >= keep))) continue;
-        const char *k_lds = at_lds + (SETS == 2 ? (r & 1) * SET : 0) + kh * PAIR, *v_lds = k_lds + KP * KTILE;
+        if (t * A8_KEYS >= wave_end || (t * A8_KEYS + A8_KEYS * TW <= wave_lo && (!RING || t * A8_KEYS >= keep))) continue;
+        const char *k_lds = at_lds + (SETS == 2 ? (r & 1) * SET : 0) + kh * TW * PAIR, *v_lds = k_lds + KP * KTILE;
 
-        f32x4 s[2];  // key blocks of 16
-        s[0] = s[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        f32x4 s[2 * TW];  // key blocks of 16
+#pragma unroll
+        for (int kb = 0; kb < 2 * TW; kb++) s[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ks++) {
-            bf16x8 kf[KP][2];
+            bf16x8 kf[KP][2 * TW];
 #pragma unroll
             for (int p = 0; p < KP; p++)
 #pragma unroll
-                for (int kb = 0; kb < 2; kb++)
-                    kf[p][kb] = *reinterpret_cast<const bf16x8 *>(k_lds + p * KTILE + k_off<DK>(16 * kb + l16, 4 * ks + c4));
+                for (int kb = 0; kb < 2 * TW; kb++)
+                    kf[p][kb] = *reinterpret_cast<const bf16x8 *>(k_lds + kb / 2 * PAIR + p * KTILE + k_off<DK>(16 * (kb & 1) + l16, 4 * ks + c4));
             piece_products<NQ, KP>([&](int pq, int pk) {
 #pragma unroll
-                for (int kb = 0; kb < 2; kb++)
+                for (int kb = 0; kb < 2 * TW; kb++)
                     s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[pk][kb], qp_[ks][pq], s[kb], 0, 0, 0);
             });
         }
         // value i of block kb belongs to key 16 kb + 4 c4 + i; only tiles that reach past the first row of
         // this wavefront, or back behind the window of its last one, need the mask
-        if (t * A8_KEYS + A8_KEYS - 1 > wave_first || t * A8_KEYS < wave_lo_last) {
+        if (t * A8_KEYS + A8_KEYS * TW - 1 > wave_first || t * A8_KEYS < wave_lo_last) {
 #pragma unroll
-            for (int kb = 0; kb < 2; kb++)
+            for (int kb = 0; kb < 2 * TW; kb++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const int key = t * A8_KEYS + 16 * kb + 4 * c4 + i;
@@ -498,7 +504,7 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
         }
         float mx = -INFINITY;
 #pragma unroll
-        for (int kb = 0; kb < 2; kb++)
+        for (int kb = 0; kb < 2 * TW; kb++)
 #pragma unroll
             for (int i = 0; i < 4; i++) mx = fmaxf(mx, s[kb][i]);
         mx = quad_rows_max(mx);
@@ -510,13 +516,14 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
         // exponential below is 0 and not exp2(inf - inf).
         const float m_new = fmaxf(mx > m_run + 8.0f ? mx : m_run, -1e30f);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        float f[8], psum = 0.f;
+        float f[TW][8], psum = 0.f;
 #pragma unroll
-        for (int kb = 0; kb < 2; kb++)
+        for (int kb = 0; kb < 2 * TW; kb++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                f[4 * kb + i] = __builtin_amdgcn_exp2f(s[kb][i] - m_new);
-                psum += f[4 * kb + i];
+                const float e = __builtin_amdgcn_exp2f(s[kb][i] - m_new);
+                f[kb / 2][4 * (kb & 1) + i] = e;
+                psum += e;
             }
         l_run = l_run * alpha + psum;  // this lane's quarter of the keys; the quarters meet at the end
         m_run = m_new;
@@ -524,25 +531,29 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
 #pragma unroll
             for (int db = 0; db < DB; db++) acc_o[db] *= alpha;
         }
-        bf16x8 pp[NP];
-        split8<NP>(f, pp);
+        bf16x8 pp[TW][NP];
 #pragma unroll
-        for (int db = 0; db < DB; db++) {
-            const int chunk = 2 * db + (v_sub >> 1), within = (v_sub & 1) * 8;
-            bf16x8 vf[KP];
+        for (int u = 0; u < TW; u++) split8<NP>(f[u], pp[u]);
 #pragma unroll
-            for (int p = 0; p < KP; p++) {
-                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (s16x4 __attribute__((address_space(3))) *)(v_lds + p * VTILE + v_off<DV>(v_key, chunk) + within));
-                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (s16x4 __attribute__((address_space(3))) *)(v_lds + p * VTILE + v_off<DV>(16 + v_key, chunk) + within));
-                struct Pair { s16x4 lo, hi; } pr{lo, hi};
-                vf[p] = __builtin_bit_cast(bf16x8, pr);
+        for (int u = 0; u < TW; u++)
+#pragma unroll
+            for (int db = 0; db < DB; db++) {
+                const int chunk = 2 * db + (v_sub >> 1), within = (v_sub & 1) * 8;
+                bf16x8 vf[KP];
+#pragma unroll
+                for (int p = 0; p < KP; p++) {
+                    const char *vt = v_lds + u * PAIR + p * VTILE;
+                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (s16x4 __attribute__((address_space(3))) *)(vt + v_off<DV>(v_key, chunk) + within));
+                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (s16x4 __attribute__((address_space(3))) *)(vt + v_off<DV>(16 + v_key, chunk) + within));
+                    struct Pair { s16x4 lo, hi; } pr{lo, hi};
+                    vf[p] = __builtin_bit_cast(bf16x8, pr);
+                }
+                piece_products<NP, KP>([&](int p, int pv) {
+                    acc_o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[pv], pp[u][p], acc_o[db], 0, 0, 0);
+                });
             }
-            piece_products<NP, KP>([&](int p, int pv) {
-                acc_o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[pv], pp[p], acc_o[db], 0, 0, 0);
-            });
-        }
     }
 
     if (KS > 1) {
@@ -733,6 +744,29 @@ int qkv_post_launch(hm_ctx *ctx, const QkvPostArgs &a) {
     return HM_OK;
 }
 
+// Key groups of a plain cache's attention: the number with the least estimated time, in nanoseconds. A workgroup of 128 / ks
+// rows takes 5000 and 40, 21.5 or 12.8 a key it walks (1, 2, 4 groups; two tiles a wavefront and round with 1 and 2); the
+// grid is over with its longest workgroup or when the CUs have done their share, whichever is later. Measured, 16 heads of
+// 128, us with 1 / 2 / 4 groups: 512 rows 23.3 / 17.0 / 13.4; 1000 36.1 / 28.0 / 28.0; 3072 131.7 / 127.0 / 151.7; 2944 behind
+// 3072 315.5 / 283.8 / 337.4; 4096 190.5 / 193.9 / 240.9.
+static int key_groups_for(const PrefillAttnArgs &a, int cus) {
+    int best = 1;
+    double least = 1e30;
+    for (int ks = 1; ks <= 4; ks *= 2) {
+        const double per_key = ks == 1 ? 40 : ks == 2 ? 21.5 : 12.8;
+        const int rows = 128 / ks;
+        const long long blocks = (a.S + rows - 1) / rows, wgs = blocks * a.H;
+        const double first = a.past + std::min(a.S, rows), last = a.past + a.S;
+        const double share = (first + last) / 2 * (double)wgs / cus + 0.4 * first;
+        const double ns = 5000.0 * (double)((wgs + cus - 1) / cus) + per_key * (wgs <= cus ? last : std::max(last, share));
+        if (ns < least) {
+            least = ns;
+            best = ks;
+        }
+    }
+    return best;
+}
+
 int prefill_attn_launch(hm_ctx *ctx, const PrefillAttnArgs &args) {
     PrefillAttnArgs a = args;
     const bool plain = a.hdv == 0;  // a cache's own rows: keys and values of one width, one piece
@@ -769,12 +803,7 @@ int prefill_attn_launch(hm_ctx *ctx, const PrefillAttnArgs &args) {
     HM_REQUIRE(ctx, a.pieces == 2 || a.pieces == 3, "prefill_attn: %d pieces (2 or 3)", a.pieces);
     int ks = 4;
     if (plain) {
-        // the fewest key groups that still give every CU a workgroup (more groups mean more tile loads)
-        for (int cand = 1; cand < 4; cand *= 2)
-            if ((long long)((a.S + 128 / cand - 1) / (128 / cand)) * a.H >= ctx->num_cus) {
-                ks = cand;
-                break;
-            }
+        ks = key_groups_for(a, ctx->num_cus);
         if (const char *e = getenv("HOMURA_PREFILL_KEY_GROUPS")) {
             const int v = atoi(e);
             if (v == 1 || v == 2 || v == 4) ks = v;
@@ -784,6 +813,7 @@ int prefill_attn_launch(hm_ctx *ctx, const PrefillAttnArgs &args) {
     } else {
         ks = a.hd == 64 ? 4 : 2;
     }
+    const int tw = plain && ks < 4 ? 2 : 1;  // tiles a wavefront takes a round (four groups of two do not fit LDS)
     const int sets = a.hd == 256 && a.kv_pieces == 3 ? 1 : 2;
     const int qrows = 128 / ks;
     dim3 grid((unsigned)((a.S + qrows - 1) / qrows), (unsigned)a.H);
@@ -794,7 +824,7 @@ int prefill_attn_launch(hm_ctx *ctx, const PrefillAttnArgs &args) {
     {
         const long long wgs = (long long)grid.x * grid.y;
         const int keys = a.window ? std::min(a.past + a.S, a.keep + a.window + qrows) : a.past + a.S;  // a row block walks
-        const int rounds = ((keys + A8_KEYS - 1) / A8_KEYS + ks - 1) / ks;
+        const int rounds = ((keys + A8_KEYS - 1) / A8_KEYS + ks - 1) / ks;  // of single tiles
         nz = (int)std::min<long long>(std::min<long long>(32, ctx->num_cus / std::max<long long>(1, wgs)), rounds / 8);
         const size_t per_z = (size_t)a.S * a.H * (a.hdv + 2) * sizeof(float);
         // (callers that carve scratch of their own from the workspace leave its first 16 MiB to the kernels)
@@ -807,9 +837,9 @@ int prefill_attn_launch(hm_ctx *ctx, const PrefillAttnArgs &args) {
             grid.z = (unsigned)nz;
         }
     }
-    // `sets` sets of ks pairs of 32-key tiles; the final exchange of the key groups wants
+    // `sets` sets of ks * tw pairs of 32-key tiles; the final exchange of the key groups wants
     // (ks - 1) * (128 / ks / 16) sets of (hdv / 4 + 2) * 256 bytes
-    const size_t lds = std::max<size_t>((size_t)sets * ks * a.kv_pieces * A8_KEYS * (a.hd + a.hdv) * 2,
+    const size_t lds = std::max<size_t>((size_t)sets * ks * tw * a.kv_pieces * A8_KEYS * (a.hd + a.hdv) * 2,
                                         (size_t)(ks - 1) * (8 / ks) * (a.hdv / 4 + 2) * 256);
     auto launch = [&](auto kernel) -> int {
         if (lds > 64 * 1024) {
@@ -824,8 +854,8 @@ int prefill_attn_launch(hm_ctx *ctx, const PrefillAttnArgs &args) {
     if (plain) {
 #define HM_AT_CASE(HDV, NPV)                                                                          \
     if (a.hd == HDV && a.pieces == NPV) {                                                             \
-        if (ks == 1) rc = launch(prefill_attn16_kernel<HDV, HDV, NPV, NPV, 1, 1, 2>);                 \
-        else if (ks == 2) rc = launch(prefill_attn16_kernel<HDV, HDV, NPV, NPV, 1, 2, 2>);            \
+        if (ks == 1) rc = launch(prefill_attn16_kernel<HDV, HDV, NPV, NPV, 1, 1, 2, false, 2>);       \
+        else if (ks == 2) rc = launch(prefill_attn16_kernel<HDV, HDV, NPV, NPV, 1, 2, 2, false, 2>);  \
         else rc = launch(prefill_attn16_kernel<HDV, HDV, NPV, NPV, 1, 4, 2>);                         \
     }
         HM_AT_CASE(128, 3)

@@ -1,8 +1,10 @@
 """Tiles of the prompt pass's matrix products at the sizes where their choice turns (GPU)."""
+import dataclasses
+
 import numpy as np
 import pytest
 
-from homura_amd import Context, synth
+from homura_amd import Context, synth, synth_model
 
 pytestmark = pytest.mark.gpu
 
@@ -29,4 +31,53 @@ def test_wide_tiles_of_the_piece_product(ctx, M, K, N):
     bound = 3 * K * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
     assert np.all(np.abs(got[:M * N].reshape(M, N) - x64 @ w64.T) <= bound)
     for buf in (dx, dw, dc):
+        buf.free()
+
+
+def test_prompt_longer_than_a_chunk(ctx):
+    """4097 and 4400 tokens go through the layers in two even chunks. The rows they leave in the cache give the logits that
+    the same tokens in portions of other sizes give, up to the cache rows that round to bf16 the other way (one ulp, 0.4 %,
+    of single elements under softmax weights of 1 / 4000 a row)."""
+    cfg = dataclasses.replace(synth_model.TINY, max_position_embeddings=4500)
+    m = synth_model.build_model(ctx, cfg, synth_model.synth_weights(cfg, 5), 4500)
+    for n in (4097, 4400):
+        ids = synth.token_ids(n, n + 1, cfg.vocab_size)
+        got = []
+        for cuts in ((0, n), (0, 1111, 1700, n)):
+            m.reset_kv_cache()
+            for a, b in zip(cuts, cuts[1:]):
+                m.prefill(ids[a:b], want_logits=False)
+            assert m.kv_cache_len() == n
+            got.append(m.run_kv(ids[n:])[0].astype(np.float64))
+        assert np.abs(got[0] - got[1]).max() <= 2e-3 * np.abs(got[1]).max()
+    m.reset_kv_cache()
+    rows = m.prefill(ids[:1100])          # logits of more rows than are held at a time
+    m.reset_kv_cache()
+    m.prefill(ids[:600], want_logits=False)
+    tail = m.prefill(ids[600:1100])
+    assert np.abs(rows[600:] - tail).max() <= 2e-3 * np.abs(tail).max()
+    m.close()
+
+
+@pytest.mark.parametrize("S,past,H,kvh,hd", [(640, 0, 12, 2, 128), (1000, 37, 16, 8, 128), (2111, 0, 14, 2, 64),
+                                             (130, 65, 32, 4, 64), (4096, 0, 8, 8, 64)])
+def test_prompt_attention_over_key_groups(ctx, S, past, H, kvh, hd):
+    """Every number of key groups, heads in eighths and not, ragged row blocks. Keys and values are bf16, queries and
+    probabilities carried whole, sums f32: 2^-20 of the largest value, over a few thousand additions, holds it."""
+    rng = np.random.default_rng(S)
+    L = past + S
+    q = rng.standard_normal((S, H, hd)).astype(np.float32)
+    k, v = (synth.f32_to_bf16_rne(rng.standard_normal((kvh, L, hd)).astype(np.float32)) for _ in range(2))
+    dq, dk, dv, do = ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), ctx.empty(S * H * hd)
+    ctx.gqa_prefill_attn(dq, dk, dv, do, S, H, kvh, hd, L, past, hd ** -0.5)
+    got = do.download(np.float32, (S, H, hd))
+    k64, v64 = synth.bf16_to_f32(k).astype(np.float64), synth.bf16_to_f32(v).astype(np.float64)
+    for i in (0, 1, 15, 16, 127, 128, S // 2, S - 2, S - 1):
+        n = past + i + 1
+        for h in range(0, H, max(1, H // 4)):
+            g = h // (H // kvh)
+            s = k64[g, :n] @ q[i, h].astype(np.float64) * hd ** -0.5
+            p = np.exp(s - s.max())
+            assert np.abs(got[i, h] - (p / p.sum()) @ v64[g, :n]).max() <= 2.0 ** -20 * 6
+    for buf in (dq, dk, dv, do):
         buf.free()
