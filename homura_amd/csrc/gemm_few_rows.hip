@@ -1,0 +1,237 @@
+// Matrix products of a few activation rows (at most 64: a chat turn, the ragged end of a prompt) on the matrix cores:
+// C[M][N] f32 = (sum of A's bf16 pieces) x B[N][K]^T, A [M][AP K] as the prompt pass's row kernels write it.
+//
+// The tile kernel of gemm_pieces_mfma.hip multiplies 128 rows whatever M is and meets at a barrier every 32 k; a product of
+// 37 rows took as long as one of 128. Here a workgroup owns 32 NT rows of B and its eight wavefronts take K in interleaved
+// groups, each for itself: a wavefront brings a group of B's rows and of the activations' pieces (32 MT rows; rows past M
+// repeat the last one) into its own part of LDS (global_load_lds_dwordx4, whole 128- or 64-byte row pieces, XOR-swizzled on
+// the global side), reads its operands, asks for its next group and multiplies. No barrier until the wavefronts' sums meet.
+// `mfma_f32_32x32x16_bf16` with B's rows as its rows: a lane ends up with four neighbouring columns of C.
+// (Operands straight from memory into registers, a 16-byte piece of each of 64 rows a request, took twice as long.)
+//
+// SC: B holds the integers of a Q8_0 / Q4_0 matrix, scales[k / 32][n] the scale of every 32-wide block (row stride npad): a
+// block's products are summed on their own and join the result times the block's scale.
+//
+// What bounds it: latency; a wavefront has one to four groups. Three pieces, weights cold, 24 / 64 rows, us: 2048 -> 1024
+// 4.6 / 4.7, 1024 -> 4096 5.4 / 7.6, 1024 -> 6144 6.5 / 10.0, 896 -> 9728 9.3 / 14.1, 4864 -> 896 6.0 / 8.9, 8960 -> 1536
+// 11.8 / 21.1; the 128-row tiles took 12 to 15 for the shapes of Qwen3-0.6B and Qwen2.5-0.5B.
+#include <algorithm>
+
+#include "gemm_bf16_mfma.h"
+#include "gemm_few_rows.h"
+#include "hm_common.h"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int THREADS = 512, WAVES = 8;
+
+struct FewRowsDims {
+    int M, N, K, lda, ldc;
+    int groups_per_slice;
+    const float *scales;   // SC: [K / 32][npad]
+    int npad;
+};
+
+extern __shared__ __attribute__((aligned(16))) char few_lds[];
+
+__device__ __forceinline__ void dma16(const uint16_t *src, char *dst) {
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1))) *)src,
+                                     (void __attribute__((address_space(3))) *)dst, 16, 0, 0);
+}
+
+template <int AP, int MT, int NT>
+struct Few {
+    static constexpr int GROUP = MT == 1 ? 64 : 32;                     // k of a group
+    static constexpr int ROW = GROUP * 2, CHUNKS = ROW / 16;            // bytes and 16-byte chunks of a row's piece
+    static constexpr int TILE = 32 * ROW;                               // 32 rows of one operand
+    static constexpr int TILES = AP * MT + NT;
+    static constexpr int SUMS = WAVES * MT * NT * 4096;
+    static constexpr int LDS = WAVES * TILES * TILE > SUMS ? WAVES * TILES * TILE : SUMS;
+    // chunk c of row r sits in this slot: the eight (four) rows that a read takes at a time then lie in different banks
+    static __device__ __forceinline__ int slot(int r, int c) { return MT == 1 ? c ^ (r & 7) : c ^ ((r >> 2) & 3); }
+};
+
+template <int AP, int MT, int NT, bool SC>
+__global__ __launch_bounds__(THREADS) void gemm_few_rows_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+                                                                float *__restrict__ C, const FewRowsDims g) {
+    using F = Few<AP, MT, NT>;
+    constexpr int GROUP = F::GROUP, STEPS = GROUP / 16, LOADS = F::TILE / 1024, RPL = 1024 / F::ROW;  // rows of a load
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+    const int n0 = blockIdx.x * (32 * NT);
+    const int groups = (g.K + GROUP - 1) / GROUP;
+    const int g_end = min(groups, (int)(blockIdx.y + 1) * g.groups_per_slice);
+    char *mine = few_lds + wave * (F::TILES * F::TILE);
+
+    // this lane's place in load i of a tile: row RPL i + lane / CHUNKS, slot lane % CHUNKS
+    const int r0 = lane / F::CHUNKS, s0 = lane % F::CHUNKS;
+    auto request = [&](int grp) {
+#pragma unroll
+        for (int i = 0; i < LOADS; i++) {
+            const int r = RPL * i + r0, k = min(grp * GROUP + 8 * F::slot(r, s0), g.K - 8);  // (slot() is its own inverse)
+#pragma unroll
+            for (int t = 0; t < NT; t++) dma16(B + (size_t)min(n0 + t * 32 + r, g.N - 1) * g.K + k, mine + (AP * MT + t) * F::TILE + i * 1024);
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int p = 0; p < AP; p++)
+                    dma16(A + (size_t)min(m * 32 + r, g.M - 1) * g.lda + p * g.K + k, mine + (p * MT + m) * F::TILE + i * 1024);
+        }
+    };
+
+    f32x16 acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[m][t][v] = 0.f;
+
+    int grp = blockIdx.y * g.groups_per_slice + wave;
+    if (grp < g_end) request(grp);
+    for (; grp < g_end; grp += WAVES) {
+        f32x4 sc[NT][GROUP / 32][4];
+        if constexpr (SC) {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int b = 0; b < GROUP / 32; b++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++)  // rows 8 q + 4 half .. + 3 of the tile (npad is a multiple of 128)
+                        sc[t][b][q] = *reinterpret_cast<const f32x4 *>(g.scales + (size_t)min(grp * (GROUP / 32) + b, g.K / 32 - 1) * g.npad +
+                                                                       n0 + t * 32 + 8 * q + 4 * half);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's own tiles: nobody else reads them
+        bf16x8 w[NT][STEPS], x[MT][STEPS][AP];
+#pragma unroll
+        for (int i = 0; i < STEPS; i++) {
+            const int at = l32 * F::ROW + F::slot(l32, 2 * i + half) * 16;
+#pragma unroll
+            for (int t = 0; t < NT; t++) w[t][i] = *reinterpret_cast<const bf16x8 *>(mine + (AP * MT + t) * F::TILE + at);
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int p = 0; p < AP; p++) x[m][i][p] = *reinterpret_cast<const bf16x8 *>(mine + (p * MT + m) * F::TILE + at);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: the tiles may be overwritten
+        if (grp + WAVES < g_end) request(grp + WAVES);
+        const int steps = min(STEPS, (g.K - grp * GROUP) / 16);  // K % 32 == 0: the last group of 64 may be half a group
+        if constexpr (SC) {
+#pragma unroll
+            for (int b = 0; b < STEPS / 2; b++) {
+                if (2 * b >= steps) break;
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int t = 0; t < NT; t++) {
+                        f32x16 s;
+#pragma unroll
+                        for (int v = 0; v < 16; v++) s[v] = 0.f;
+#pragma unroll
+                        for (int p = AP - 1; p >= 0; p--)
+#pragma unroll
+                            for (int i = 2 * b; i < 2 * b + 2; i++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[t][i], x[m][i][p], s, 0, 0, 0);
+#pragma unroll
+                        for (int v = 0; v < 16; v++) acc[m][t][v] = fmaf(s[v], sc[t][b][v >> 2][v & 3], acc[m][t][v]);
+                    }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < STEPS; i++) {
+                if (i >= steps) break;
+#pragma unroll
+                for (int p = AP - 1; p >= 0; p--)
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+#pragma unroll
+                        for (int t = 0; t < NT; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[t][i], x[m][i][p], acc[m][t], 0, 0, 0);
+            }
+        }
+    }
+    __syncthreads();  // nobody reads tiles any more
+
+    // The wavefronts' sums meet in LDS, quarter tiles (four neighbouring n of one m) as units: wavefront w leaves unit q of
+    // tile (m, t) at [w][(m NT + t) 4 + q][lane]; the threads then add eight of them each, in wavefront order.
+    constexpr int UNITS = MT * NT * 4;
+    f32x4 *sums = reinterpret_cast<f32x4 *>(few_lds);
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                sums[(wave * UNITS + (m * NT + t) * 4 + q) * 64 + lane] =
+                    f32x4{acc[m][t][4 * q], acc[m][t][4 * q + 1], acc[m][t][4 * q + 2], acc[m][t][4 * q + 3]};
+    __syncthreads();
+    C += (size_t)blockIdx.y * g.M * g.ldc;
+    for (int u = wave; u < UNITS; u += WAVES) {
+        f32x4 s = sums[u * 64 + lane];
+#pragma unroll
+        for (int o = 1; o < WAVES; o++) s += sums[(o * UNITS + u) * 64 + lane];
+        const int row = (u >> 2) / NT * 32 + l32, col = n0 + (u >> 2) % NT * 32 + 8 * (u & 3) + 4 * half;
+        if (row >= g.M) continue;
+        float *out = C + (size_t)row * g.ldc + col;
+        if (col + 4 <= g.N && (g.ldc & 3) == 0 && ((uintptr_t)C & 15) == 0) {
+            *reinterpret_cast<f32x4 *>(out) = s;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (col + v < g.N) out[v] = s[v];
+        }
+    }
+}
+
+template <int AP, int MT, int NT, bool SC>
+int launch(hm_ctx *ctx, const uint16_t *a, const uint16_t *b, float *c, const FewRowsDims &g, unsigned slices) {
+    constexpr int LDS = Few<AP, MT, NT>::LDS;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_few_rows_kernel<AP, MT, NT, SC>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    HM_REQUIRE(ctx, attr == hipSuccess, "gemm_few_rows: cannot reserve %d bytes of LDS: %s", LDS, hipGetErrorString(attr));
+    hipLaunchKernelGGL((gemm_few_rows_kernel<AP, MT, NT, SC>), dim3((unsigned)((g.N + 32 * NT - 1) / (32 * NT)), slices), dim3(THREADS),
+                       LDS, ctx->stream, a, b, c, g);
+    HM_LAUNCH_CHECK(ctx);
+    return HM_OK;
+}
+
+template <int AP, bool SC>
+int launch_tiles(hm_ctx *ctx, const uint16_t *a, const uint16_t *b, float *c, const FewRowsDims &g, unsigned slices, int nt) {
+    if (g.M <= 32) return nt == 2 ? launch<AP, 1, 2, SC>(ctx, a, b, c, g, slices) : launch<AP, 1, 1, SC>(ctx, a, b, c, g, slices);
+    return nt == 2 ? launch<AP, 2, 2, SC>(ctx, a, b, c, g, slices) : launch<AP, 2, 1, SC>(ctx, a, b, c, g, slices);
+}
+
+}  // namespace
+
+int homura::gemm_few_rows(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, const uint16_t *d_b_nk, const float *d_scales, int npad,
+                          float *d_c, int M, int K, int N, int max_parts, int *parts, int ldc) {
+    HM_CHECK_CTX(ctx);
+    HM_REQUIRE(ctx, d_a_split && d_b_nk && d_c, "gemm_few_rows: NULL pointer");
+    HM_REQUIRE(ctx, M > 0 && M <= FEW_ROWS && N > 0 && K > 0 && K % 32 == 0 && pieces >= 1 && pieces <= 3 && ldc >= N,
+               "gemm_few_rows: need 1 .. %d rows, N > 0, K %% 32 == 0, 1 .. 3 pieces and ldc >= N (M=%d K=%d N=%d)", FEW_ROWS, M, K, N);
+    HM_REQUIRE(ctx, ((uintptr_t)d_a_split % 16) == 0 && ((uintptr_t)d_b_nk % 16) == 0, "gemm_few_rows: operands must be 16-byte aligned");
+    HM_REQUIRE(ctx, !d_scales || (pieces == 3 && npad >= (N + 127) / 128 * 128 && npad % 4 == 0 && ((uintptr_t)d_scales % 16) == 0),
+               "gemm_few_rows: the scales go with three pieces and a row stride of whole tiles");
+    FewRowsDims g{};
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.lda = pieces * K;
+    g.ldc = ldc;
+    g.scales = d_scales;
+    g.npad = npad;
+    const int group = M <= 32 ? 64 : 32, groups = (K + group - 1) / group;
+    const int nt = few_rows_tiles(N, ctx->num_cus);
+    const long long wgs = (N + 32 * nt - 1) / (32 * nt);
+    // K slices while the workgroups still fit the chip at once, a group for every wavefront
+    int want = (int)std::max<long long>(1, ctx->num_cus / wgs);
+    want = std::min(std::min(want, std::max(1, parts ? max_parts : 1)), std::max(1, groups / WAVES));
+    while (want > 1 && (N + 127) / 128 * want > gemm_sliced_tiles(ctx->num_cus)) want--;
+    g.groups_per_slice = (groups + want - 1) / want;
+    const int slices = (groups + g.groups_per_slice - 1) / g.groups_per_slice;
+    if (parts) *parts = slices;
+    if (d_scales) return launch_tiles<3, true>(ctx, d_a_split, d_b_nk, d_c, g, (unsigned)slices, nt);
+    if (pieces == 3) return launch_tiles<3, false>(ctx, d_a_split, d_b_nk, d_c, g, (unsigned)slices, nt);
+    if (pieces == 2) return launch_tiles<2, false>(ctx, d_a_split, d_b_nk, d_c, g, (unsigned)slices, nt);
+    return launch_tiles<1, false>(ctx, d_a_split, d_b_nk, d_c, g, (unsigned)slices, nt);
+}

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "gemm_bf16_mfma.h"
+#include "gemm_few_rows.h"
 #include "grouped_tiles.h"
 #include "hm_common.h"
 
@@ -461,6 +462,9 @@ int homura::gemm_pieces_any(hm_ctx *ctx, const uint16_t *d_a_split, int a_pieces
                "%s: %d x %d pieces (2 x 1, 3 x 1 or 3 x 3)", who, a_pieces, b_pieces);
     HM_REQUIRE(ctx, ((uintptr_t)d_a_split % 16) == 0 && ((uintptr_t)d_b_split % 16) == 0, "%s: operands must be 16-byte aligned", who);
     HM_REQUIRE(ctx, (long long)((M + TM - 1) / TM) * ((N + TN - 1) / TN) <= 0x7fffff00LL, "%s: too many tiles", who);
+    HM_REQUIRE(ctx, ldc <= 0 || ldc >= N, "%s: ldc %d below N %d", who, ldc, N);
+    if (b_pieces == 1 && few_rows_pays(M, N, ctx->num_cus))
+        return gemm_few_rows(ctx, d_a_split, a_pieces, d_b_split, d_scales, npad, d_c, M, K, N, max_parts, parts, ldc > 0 ? ldc : N);
     PieceDims g{};
     g.M = M;
     g.N = N;
@@ -470,7 +474,6 @@ int homura::gemm_pieces_any(hm_ctx *ctx, const uint16_t *d_a_split, int a_pieces
     g.ldc = ldc > 0 ? ldc : N;
     g.scales = d_scales;
     g.npad = npad;
-    HM_REQUIRE(ctx, g.ldc >= N, "%s: ldc %d below N %d", who, g.ldc, N);
     const Cut cut = cut_for((M + TM - 1) / TM, N, K / TK, 4LL * M * N, ctx->num_cus, parts ? max_parts : 1,
                             b_pieces == 1 && !d_scales);  // (a wide scaled tile does not fit the registers)
     g.stages_per_split = cut.stages_per_split;

@@ -4,15 +4,9 @@ import dataclasses
 import numpy as np
 import pytest
 
-from homura_amd import Context, synth, synth_model
+from homura_amd import DTYPE_Q4_0, DTYPE_Q8_0, synth, synth_model
 
 pytestmark = pytest.mark.gpu
-
-
-@pytest.fixture(scope="module")
-def ctx():
-    with Context(0) as c:
-        yield c
 
 
 @pytest.mark.parametrize("M,K,N", [(1100, 32, 4000), (1100, 96, 4000), (1025, 1024, 4001), (2048, 256, 4096), (1153, 64, 3841)])
@@ -80,4 +74,40 @@ def test_prompt_attention_over_key_groups(ctx, S, past, H, kvh, hd):
             p = np.exp(s - s.max())
             assert np.abs(got[i, h] - (p / p.sum()) @ v64[g, :n]).max() <= 2.0 ** -20 * 6
     for buf in (dq, dk, dv, do):
+        buf.free()
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 32, 8), (7, 96, 200), (24, 1024, 6144), (31, 160, 4097), (32, 896, 33), (33, 32, 64), (37, 4864, 896),
+                                   (64, 1056, 1001), (64, 1536, 17920), (64, 2080, 6150)])
+@pytest.mark.parametrize("form", ["f32", "bf16", "q8_0", "q4_0"])
+def test_products_of_few_rows(ctx, oracle, form, M, K, N):
+    """Row tiles of 32 and 64, one and two tiles of B, half a group of 64 k at the end, columns that end inside a vector.
+    Bound as above; the block formats' scales are one rounding more a block."""
+    if form != "f32" and form != "bf16" and K % 64:
+        K = (K + 63) // 64 * 64
+    guard = 512
+    x = synth.normal_f32(31, M * K).reshape(M, K)
+    dc = ctx.to_device(np.full(M * N + guard, -77.0, np.float32))
+    if form in ("q8_0", "q4_0"):
+        raw = {"q8_0": synth.q8_0_blocks, "q4_0": synth.q4_0_blocks}[form](41, N * K // 32, 0.01)
+        w64 = getattr(oracle, "dequant_" + form)(raw).reshape(N, K).astype(np.float64)
+        dx, dw = ctx.to_device(x), ctx.to_device(raw)
+        ctx.gemm_f32_quant_nk(dx, dw, {"q8_0": DTYPE_Q8_0, "q4_0": DTYPE_Q4_0}[form], dc, M, K, N)
+    else:
+        w = synth.normal_bf16(32, K * N, 0.02).reshape(N, K)
+        w64 = synth.bf16_to_f32(w).astype(np.float64)
+        if form == "bf16":
+            bits = synth.f32_to_bf16_rne(x)
+            x = synth.bf16_to_f32(bits)
+            dx, dw = ctx.to_device(bits), ctx.to_device(w)
+            ctx.gemm_bf16_nk(dx, dw, dc, M, K, N)
+        else:
+            dx, dw = ctx.to_device(x), ctx.to_device(w)
+            ctx.gemm_f32_bf16_nk(dx, dw, dc, M, K, N)
+    got = dc.download(np.float32, (M * N + guard,))
+    assert np.all(got[M * N:] == -77.0), "wrote past the end of C"
+    x64 = x.astype(np.float64)
+    bound = 4 * K * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
+    assert np.all(np.abs(got[:M * N].reshape(M, N) - x64 @ w64.T) <= bound)
+    for buf in (dx, dw, dc):
         buf.free()
