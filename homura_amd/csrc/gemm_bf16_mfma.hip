@@ -314,7 +314,11 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_bf16_mfma_kernel(const uint
             }
 }
 
-// ---- [N][K] operand, K tiles aligned: global -> LDS loads without the trip through registers ----
+// ---- K tiles aligned: global -> LDS loads without the trip through registers, B [N][K] or [K][N] ----
+//
+// A [K][N] operand took 4 x 8 blocks through registers and byte permutes into LDS before; its tiles now lie in LDS as they
+// are in memory and the transposing LDS read hands out the operands (512 x 2048 x 8192 35.8 -> 28.6 us, 2048 x 1024 x 4096
+// 39.6 -> 30, 2048 x 2048 x 1024 26.9 -> 18.0; B [N][K]: 24.8, 29.8, 18.0).
 //
 // global_load_lds_dwordx4 writes lane l's 16 bytes to LDS at (wave-uniform base) + 16 l, so one
 // instruction fills eight 128-byte rows. The slot swizzle moves to the global side: the lane that
@@ -322,7 +326,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_bf16_mfma_kernel(const uint
 // live in LDS (DMA_BUFS buffers of 32 KiB), the registers of the ring above are free, and the LDS
 // write instructions are gone.
 constexpr int DMA_BUFS = 4;  // the vmcnt values in the kernel count DMA_BUFS - 1 tiles of four loads in flight
-static_assert(DMA_BUFS == 4, "adjust the wait counts of gemm_nk_dma_kernel");
+static_assert(DMA_BUFS == 4, "adjust the wait counts of gemm_dma_kernel");
 constexpr int DMA_LDS_BYTES = DMA_BUFS * 2 * TILE_BYTES;  // 128 of the CU's 160 KiB
 
 extern __shared__ __attribute__((aligned(16))) char dma_lds[];
@@ -342,10 +346,19 @@ __device__ __forceinline__ bf16x8 lds_read16_imm(uint32_t addr) {
     return v;
 }
 
+template <int IMM>
+__device__ __forceinline__ u32x2 lds_read_tr8_imm(uint32_t addr) {
+    u32x2 v;
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(IMM) : "memory");
+    return v;
+}
+
+// KN: B [K][N]. Its tile lies in LDS as 64 rows of 128 n, chunk c (8 n) of row k in slot c ^ 4 (k % 4), and leaves through the
+// transposing read: lane i of 16 points at 4 n of row i / 4 and receives n = i of the four rows.
 // GR: grouped, see grouped_tiles.h; entry e of a group's list reads row e % a_rows of A and writes row e of C.
 // ACT: neighbouring columns are (gate, up) pairs, and act(weight gate, weight up) of an entry leaves as bf16 in rows of N / 2.
-template <bool GR, bool ACT = false>
-__global__ __launch_bounds__(GEMM_THREADS) void gemm_nk_dma_kernel(const uint16_t *__restrict__ A,
+template <bool GR, bool ACT = false, bool KN = false>
+__global__ __launch_bounds__(GEMM_THREADS) void gemm_dma_kernel(const uint16_t *__restrict__ A,
                                                                    const uint16_t *__restrict__ B,
                                                                    float *__restrict__ C, const GemmDims g) {
     int M = g.M;
@@ -395,7 +408,12 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nk_dma_kernel(const uint16_
         const int c = s ^ (r & 7) ^ ((r >> 3) & 7);
         const int a_row = min(m0 + r, M - 1);
         a_src[j] = A + (size_t)(GR ? list[a_row] % g.lists.a_rows : a_row) * g.lda + c * 8;
-        b_src[j] = B + (size_t)min(n0 + r, N - 1) * g.ldb + c * 8;
+        if (KN) {  // instruction j of wavefront w fills rows 4 (2 w + j) .. + 3
+            const int k = (wave * 2 + j) * 4 + (lane >> 4);
+            b_src[j] = B + (size_t)k * N + min(n0 + ((lane & 15) ^ ((k & 3) << 2)) * 8, N - 8);
+        } else {
+            b_src[j] = B + (size_t)min(n0 + r, N - 1) * g.ldb + c * 8;
+        }
     }
     // where this wavefront's first instruction lands inside an operand tile (scalar: it goes to M0)
     const int wave_dst = __builtin_amdgcn_readfirstlane(wave * 2048);
@@ -403,18 +421,20 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nk_dma_kernel(const uint16_
     // show in the run time). A tile past the end re-reads the last one (nobody multiplies it), so every
     // iteration issues the same four loads and the wait counts below are exact.
     int koff = kt_first * TK;
-    auto request = [&](int buf) {
-        char *base = dma_lds + buf * (2 * TILE_BYTES) + wave_dst;
+    auto request_one = [&](int buf, int o) {  // load o of the four of a tile
+        char *base = dma_lds + buf * (2 * TILE_BYTES) + wave_dst + (o >> 1) * 1024;
         const int k = min(koff, K - TK);
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            dma16(a_src[j] + k, base + j * 1024);
-            dma16(b_src[j] + k, base + TILE_BYTES + j * 1024);
-        }
-        koff += TK;
+        if (o & 1)
+            dma16(b_src[o >> 1] + (KN ? (size_t)k * N : (size_t)k), base + TILE_BYTES);
+        else
+            dma16(a_src[o >> 1] + k, base);
     };
 #pragma unroll
-    for (int d = 0; d < DMA_BUFS; d++) request(d);
+    for (int d = 0; d < DMA_BUFS; d++) {
+#pragma unroll
+        for (int o = 0; o < 4; o++) request_one(d, o);
+        koff += TK;
+    }
     if (GR && tid < TM) {  // for the epilogue
         s_entry[tid] = my_entry;
         if constexpr (ACT) s_weight[tid] = my_weight;
@@ -431,8 +451,14 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nk_dma_kernel(const uint16_
     for (int i = 0; i < 2; i++) {
         a_lo[0][i] = lds0 + lds_off(arow + i * 32, chunk0);
         a_lo[1][i] = lds0 + lds_off(arow + i * 32, chunk1);
-        b_lo[0][i] = lds0 + TILE_BYTES + lds_off(brow + i * 32, chunk0);
-        b_lo[1][i] = lds0 + TILE_BYTES + lds_off(brow + i * 32, chunk1);
+        if (KN) {  // rows 8 lh + (lane % 16) / 4 of the group's k steps, 4 n each; the next four rows are 1 KiB on
+            const int k = kgrp * 32 + 8 * lh + ((lane & 15) >> 2), n = wn * 64 + i * 32 + (lane & 16) + 4 * (lane & 3);
+            b_lo[0][i] = lds0 + TILE_BYTES + k * 256 + ((((n >> 3) ^ ((k & 3) << 2)) << 4) | ((n & 7) << 1));
+            b_lo[1][i] = b_lo[0][i] + 16 * 256;
+        } else {
+            b_lo[0][i] = lds0 + TILE_BYTES + lds_off(brow + i * 32, chunk0);
+            b_lo[1][i] = lds0 + TILE_BYTES + lds_off(brow + i * 32, chunk1);
+        }
 #pragma unroll
         for (int st = 0; st < 2; st++) {
             a_hi[st][i] = a_lo[st][i] + 4 * TILE_BYTES;
@@ -440,50 +466,74 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nk_dma_kernel(const uint16_
         }
     }
     // operand registers, two stages: the reads of the next step are in flight during the MFMAs
-    bf16x8 af[2][2], bfr[2][2];
-    // stage `st` <- k step `st` of buffer `buf` (a compile-time constant in the main loop)
-    auto read_step = [&](int buf, int st) {
+    bf16x8 af[2][2], bfr[KN ? 1 : 2][2];
+    u32x2 bt[KN ? 2 : 1][2][2];
+    // operand `o` (A's rows 0, 1, then B's) of stage `st` <- k step `st` of buffer `buf` (a compile-time constant in the main loop)
+    auto read_one = [&](int buf, int st, int o) {
+        const int i = o & 1;
+        const uint32_t pa = buf < 2 ? a_lo[st][i] : a_hi[st][i], pb = buf < 2 ? b_lo[st][i] : b_hi[st][i];
+        if (o < 2) {
+            af[st][i] = (buf & 1) ? lds_read16_imm<2 * TILE_BYTES>(pa) : lds_read16_imm<0>(pa);
+        } else if constexpr (KN) {
+            bt[st][i][0] = (buf & 1) ? lds_read_tr8_imm<2 * TILE_BYTES>(pb) : lds_read_tr8_imm<0>(pb);
+            bt[st][i][1] = (buf & 1) ? lds_read_tr8_imm<2 * TILE_BYTES + 1024>(pb) : lds_read_tr8_imm<1024>(pb);
+        } else {
+            bfr[st][i] = (buf & 1) ? lds_read16_imm<2 * TILE_BYTES>(pb) : lds_read16_imm<0>(pb);
+        }
+    };
+    // names the registers of a stage behind the wait for its reads, so that nothing touches them before
+    auto settle = [&](int st) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
-            const uint32_t pa = buf < 2 ? a_lo[st][i] : a_hi[st][i], pb = buf < 2 ? b_lo[st][i] : b_hi[st][i];
-            if (buf & 1) {
-                af[st][i] = lds_read16_imm<2 * TILE_BYTES>(pa);
-                bfr[st][i] = lds_read16_imm<2 * TILE_BYTES>(pb);
+            asm volatile("" : "+v"(af[st][i])::"memory");
+            if constexpr (KN) {
+                asm volatile("" : "+v"(bt[st][i][0])::"memory");
+                asm volatile("" : "+v"(bt[st][i][1])::"memory");
             } else {
-                af[st][i] = lds_read16_imm<0>(pa);
-                bfr[st][i] = lds_read16_imm<0>(pb);
+                asm volatile("" : "+v"(bfr[st][i])::"memory");
             }
         }
     };
+    auto product = [&](int st, int i, int j) {
+        bf16x8 b;
+        if constexpr (KN) {
+            struct Pair { u32x2 lo, hi; } pr{bt[st][j][0], bt[st][j][1]};
+            b = __builtin_bit_cast(bf16x8, pr);
+        } else {
+            b = bfr[st][j];
+        }
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[st][i], b, acc[i][j], 0, 0, 0);
+    };
     // tiles 1..3 (four loads each) may still be in flight; tile 0 has landed for everyone
     asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");
-    read_step(0, 0);
+#pragma unroll
+    for (int o = 0; o < 4; o++) read_one(0, 0, o);
 
-    // one K tile out of buffer `buf`
+    // One K tile out of buffer `buf`. An operand read, or a load and an operand read, follow every MFMA: issued in front of
+    // them, the MFMAs of both wavefronts of a SIMD waited for the issue (2048 x 768 x 3072: 20.3 us, 19.5 this way).
     auto tile = [&](int buf) {
-        read_step(buf, 1);
-        // the four reads above may be in flight; the four before them (stage 0) have arrived
-        asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(af[0][0]), "+v"(af[0][1]), "+v"(bfr[0][0]), "+v"(bfr[0][1]));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        settle(0);
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[0][i], bfr[0][j], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);  // these MFMAs go out before the wait: it hides behind them
+        for (int o = 0; o < 4; o++) {
+            product(0, o >> 1, o & 1);
+            __builtin_amdgcn_sched_barrier(0);
+            read_one(buf, 1, o);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         // every wavefront has read its last operands of this tile, and the next tile has landed for
         // everyone (the two after it may be in flight): this tile's buffer takes tile kt + 4
-        asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier"
-                     : "+v"(af[1][0]), "+v"(af[1][1]), "+v"(bfr[1][0]), "+v"(bfr[1][1])
-                     :
-                     : "memory");
-        request(buf);
-        read_step((buf + 1) % DMA_BUFS, 0);
+        asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        settle(1);
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[1][i], bfr[1][j], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int o = 0; o < 4; o++) {
+            product(1, o >> 1, o & 1);
+            __builtin_amdgcn_sched_barrier(0);
+            read_one((buf + 1) % DMA_BUFS, 0, o);
+            request_one(buf, o);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        koff += TK;
     };
     // whole rounds of four tiles: every buffer index is a constant, the body is one basic block
     int kt = 0;
@@ -502,12 +552,10 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nk_dma_kernel(const uint16_
     }
 
     // drain what is in flight before the buffers are reused for the exchange: the loads into LDS, and
-    // the operand reads of the tile after the last (stage 0; the wait names its registers so that they
+    // the operand reads of the tile after the last (stage 0; named behind the wait, so that its registers
     // stay untouched until the data has arrived)
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier"
-                 : "+v"(af[0][0]), "+v"(af[0][1]), "+v"(bfr[0][0]), "+v"(bfr[0][1])
-                 :
-                 : "memory");
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    settle(0);
     // each group hands over its sums for the other's 32 rows of every block of 64 (lane-major: 4 blocks x 2 groups x 32 x 64)
     float *xch = reinterpret_cast<float *>(dma_lds) + (size_t)(wave & 3) * 2 * 32 * 64 + lane;
 #pragma unroll
@@ -547,12 +595,12 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nk_dma_kernel(const uint16_
     }
 }
 
-template <bool GR, bool ACT = false>
+template <bool GR, bool ACT = false, bool KN = false>
 int gemm_dma_launch(hm_ctx *ctx, const char *who, dim3 grid, const uint16_t *a, const uint16_t *b, float *c, const GemmDims &g) {
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_nk_dma_kernel<GR, ACT>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_dma_kernel<GR, ACT, KN>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, DMA_LDS_BYTES);
     HM_REQUIRE(ctx, attr == hipSuccess, "%s: cannot reserve %d bytes of LDS: %s", who, DMA_LDS_BYTES, hipGetErrorString(attr));
-    hipLaunchKernelGGL((gemm_nk_dma_kernel<GR, ACT>), grid, dim3(GEMM_THREADS), DMA_LDS_BYTES, ctx->stream, a, b, c, g);
+    hipLaunchKernelGGL((gemm_dma_kernel<GR, ACT, KN>), grid, dim3(GEMM_THREADS), DMA_LDS_BYTES, ctx->stream, a, b, c, g);
     return HM_OK;
 }
 
@@ -587,6 +635,9 @@ int gemm_launch(hm_ctx *ctx, const char *who, const uint16_t *a, const uint16_t 
     const bool aligned = g.K % TK == 0 && g.Kb % TK == 0;
     if (b_nk && aligned) {
         const int rc = gemm_dma_launch<false>(ctx, who, grid, a, b, c, g);
+        if (rc != HM_OK) return rc;
+    } else if (aligned && a_pieces == 1) {
+        const int rc = gemm_dma_launch<false, false, true>(ctx, who, grid, a, b, c, g);
         if (rc != HM_OK) return rc;
     } else if (b_nk)
         hipLaunchKernelGGL((gemm_bf16_mfma_kernel<true, false>), grid, dim3(GEMM_THREADS), 0, ctx->stream, a, b, c, g);
