@@ -21,6 +21,9 @@ int pack_quant_planes(hm_ctx *ctx, bool q4, const uint8_t *d_blocks, uint8_t *d_
 int gemv_planes_fused(hm_ctx *ctx, bool q4, const float *d_x, const uint8_t *d_planes, float *d_out, int K, int N,
                       const QuantFuse &fuse);
 
+// out[N] = W[N][K] . x, W as raw Q8_0 blocks, rows cut across the wavefronts of a workgroup; K <= 8192
+int gemv_q8_0_blocks_cut(hm_ctx *ctx, const float *d_x, const uint8_t *d_blocks, float *d_out, int K, int N);
+
 // Workgroups gemv_planes_fused launches for this shape (= argmax candidates it leaves when asked to).
 int gemv_planes_workgroups(const hm_ctx *ctx, bool q4, int K, int N);
 

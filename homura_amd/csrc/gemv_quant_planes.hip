@@ -95,6 +95,8 @@ typedef const uint32_t __attribute__((address_space(1))) *global_u32_ptr;
 typedef const u32x2 __attribute__((address_space(1))) *global_u32x2_ptr;
 typedef const uint16_t __attribute__((address_space(1))) *global_u16_ptr;
 typedef const u32x4 __attribute__((address_space(1))) *global_u32x4_ptr;
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef const u32x4_a2 __attribute__((address_space(1))) *global_u32x4_a2_ptr;
 
 template <int QT>
 __device__ __forceinline__ QWords<QT> load_quarter(const uint8_t *q) {
@@ -326,7 +328,9 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_kernel(const float *__re
 // (SiLU pair, residual add) are applied to the pieces in registers; the four partial sums of a row meet in
 // LDS and are added in wavefront order. No RMSNorm here (rows that long are normalised by their own launch).
 // MODE 0: plain row. 1: a second operand (x2 or res_in). 2: RMSNorm, with or without res_in.
-template <int QT, int R, int NC, int MODE, int WPS>
+// RAW: `quants` are the blocks as the file has them (34 or 18 bytes, f16 scale first): a unit's 16 bytes start at an even
+// address, which one 16-byte load takes as well.
+template <int QT, int R, int NC, int MODE, int WPS, bool RAW = false>
 __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const float *__restrict__ x, const uint8_t *__restrict__ quants,
                                                                       const uint16_t *__restrict__ scales, float *__restrict__ out,
                                                                       int K, int N, const QuantFuse fuse_arg) {
@@ -366,8 +370,14 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int row = min(row0 + r, N - 1);  // rows past the end re-read the last one
-            qw[c][r] = __builtin_nontemporal_load((global_u32x4_ptr)(quants + (size_t)row * qrow + (QT == 0 ? kc : kc / 2)));
-            sc[c][r] = __builtin_nontemporal_load((global_u16_ptr)(scales + (size_t)row * nb + kc / 32));
+            if constexpr (RAW) {
+                const uint8_t *blk = quants + ((size_t)row * nb + kc / 32) * PlaneTraits<QT>::BLOCK;
+                qw[c][r] = __builtin_nontemporal_load((global_u32x4_a2_ptr)(blk + 2 + (QT == 0 ? (kc & 16) : 0)));
+                sc[c][r] = __builtin_nontemporal_load((global_u16_ptr)blk);
+            } else {
+                qw[c][r] = __builtin_nontemporal_load((global_u32x4_ptr)(quants + (size_t)row * qrow + (QT == 0 ? kc : kc / 2)));
+                sc[c][r] = __builtin_nontemporal_load((global_u16_ptr)(scales + (size_t)row * nb + kc / 32));
+            }
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above goes out before any arithmetic below
@@ -421,15 +431,19 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
     for (int r = 0; r < R; r++) a[r] = 0.f;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-        float xv[KPL], sx = 0.f;
+        float xv[KPL], sx = 0.f, sx_first = 0.f;
 #pragma unroll
         for (int j = 0; j < XV; j++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
+                if (RAW && j == XV / 2 && e == 0) {
+                    sx_first = sx;
+                    sx = 0.f;
+                }
                 xv[4 * j + e] = xr[c][j][e];
                 sx += xr[c][j][e];
             }
-        const float sx_off = sx * (QT == 0 ? 128.f : 8.f);
+        const float sx_off = sx * (QT == 0 ? 128.f : 8.f), sx_off_first = sx_first * 128.f;
         if (QT == 1) {
 #pragma unroll
             for (int j = 0; j < KPL; j++) xv[j] *= NIBBLE_FP8_UNIT;
@@ -441,7 +455,13 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
             float t = 0.f;
             if (QT == 0) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) t = dot4_bytes(w[i] ^ 0x80808080u, xv + 4 * i, t);  // int8 -> biased unsigned
+                for (int i = 0; i < 4; i++) {
+                    if (RAW && i == 2) {  // the offset comes off every eight weights: the biased sums stay small
+                        a[r] += d * (t - sx_off_first);
+                        t = 0.f;
+                    }
+                    t = dot4_bytes(w[i] ^ 0x80808080u, xv + 4 * i, t);  // int8 -> biased unsigned
+                }
             } else {
                 // byte i of the block's 16: low nibble = weight i, high nibble = weight 16 + i
 #pragma unroll
@@ -1011,6 +1031,35 @@ int homura::gemv_planes_fused(hm_ctx *ctx, bool q4, const float *d_x, const uint
                               const QuantFuse &fuse) {
     return q4 ? planes_launch<1>(ctx, "gemv_planes[q4_0]", d_x, d_planes, d_out, 1, K, N, fuse)
               : planes_launch<0>(ctx, "gemv_planes[q8_0]", d_x, d_planes, d_out, 1, K, N, fuse);
+}
+
+// Rows a set: as many as leave seven hundred workgroups (every set re-reads the activation pieces), two at least. us with
+// 2 / 4 / 8 / 16: 1024 -> 6144 3.62 / 3.89 / 3.94 / 5.75, 2048 -> 5632 5.38 / 5.10 / 5.89 / 6.39, 768 -> 32000 10.94 / 9.87 /
+// 9.81 / 10.13, 4096 -> 32000 47.8 / 41.9 / 41.3 / 40.5; the kernel that stages blocks in LDS took 4.54, 6.74, 12.75 and
+// 53.4. (Q4_0 blocks are no faster this way: 2048 -> 5632 4.69 at best against 4.40.)
+int homura::gemv_q8_0_blocks_cut(hm_ctx *ctx, const float *d_x, const uint8_t *d_blocks, float *d_out, int K, int N) {
+    const int chunk_k = WAVE * 16, wps = K <= chunk_k ? 1 : (K <= 2 * chunk_k ? 2 : 4), nc = (K + wps * chunk_k - 1) / (wps * chunk_k);
+    HM_REQUIRE(ctx, nc <= 2, "gemv_q8_0_blocks_cut: K=%d above 8192", K);
+    const int sets = PWAVES / wps;
+    int r = nc == 1 ? 16 : 8;
+    while (r > 2 && N / (r * sets) < 700) r /= 2;
+    const dim3 grid((unsigned)((N + r * sets - 1) / (r * sets)));
+#define HM_CUT(RR, CC, WW)                                                                                              \
+    hipLaunchKernelGGL((gemv_planes_splitk_kernel<0, RR, CC, 0, WW, true>), grid, dim3(PTHREADS), 0, ctx->stream, d_x,  \
+                       d_blocks, (const uint16_t *)nullptr, d_out, K, N, homura::QuantFuse())
+#define HM_CUT_R(CC, WW)                                                                                                \
+    do {                                                                                                                \
+        if (r == 8) HM_CUT(8, CC, WW); else if (r == 4) HM_CUT(4, CC, WW); else HM_CUT(2, CC, WW);                      \
+    } while (0)
+    if (nc == 2) HM_CUT_R(2, 4);
+    else if (r == 16) { if (wps == 1) HM_CUT(16, 1, 1); else if (wps == 2) HM_CUT(16, 1, 2); else HM_CUT(16, 1, 4); }
+    else if (wps == 1) HM_CUT_R(1, 1);
+    else if (wps == 2) HM_CUT_R(1, 2);
+    else HM_CUT_R(1, 4);
+#undef HM_CUT_R
+#undef HM_CUT
+    HM_LAUNCH_CHECK(ctx);
+    return HM_OK;
 }
 
 int homura::pack_quant_planes(hm_ctx *ctx, bool q4, const uint8_t *d_blocks, uint8_t *d_planes, int N, int K) {

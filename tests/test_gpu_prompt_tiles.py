@@ -111,3 +111,24 @@ def test_products_of_few_rows(ctx, oracle, form, M, K, N):
     assert np.all(np.abs(got[:M * N].reshape(M, N) - x64 @ w64.T) <= bound)
     for buf in (dx, dw, dc):
         buf.free()
+
+
+@pytest.mark.parametrize("K,N", [(32, 1), (32, 2801), (992, 5603), (1024, 11203), (1024, 45001), (1056, 1401), (2048, 22403), (2080, 703),
+                                 (4096, 11201), (4128, 701), (7680, 5601)])
+def test_q8_0_rows_straight_from_blocks(ctx, oracle, K, N):
+    """One, two and four wavefronts a row, one and two chunks each, every number of rows a set, rows and units past the end.
+    A block's sum is 32 f32 additions of exact integers times activations, the blocks' sums as many again as there are."""
+    raw = synth.q8_0_blocks(51, N * K // 32, 0.01)
+    x = synth.normal_f32(52, 2 * K).reshape(2, K)
+    dx, dw, dout = ctx.to_device(x), ctx.to_device(raw), ctx.to_device(np.full(2 * N + 64, -77.0, np.float32))
+    ctx.gemv_q8_0(dx, dw, dout, 2, K, N)
+    got = dout.download(np.float32, (2 * N + 64,))
+    assert np.all(got[2 * N:] == -77.0), "wrote past the end"
+    w64, x64 = oracle.dequant_q8_0(raw).reshape(N, K).astype(np.float64), x.astype(np.float64)
+    blocks = raw.reshape(-1, 34)
+    scale = np.abs(blocks[:, :2].copy().view(np.float16).astype(np.float64)).reshape(N, K // 32)
+    # quants enter as q + 128 and the offset is taken off a block: magnitudes of up to 256 scales
+    mags = np.abs(x64).reshape(2, K // 32, 32).sum(2) @ (256 * scale).T
+    assert np.all(np.abs(got[:2 * N].reshape(2, N) - x64 @ w64.T) <= (64 + K / 16) * 2.0 ** -24 * mags)
+    for buf in (dx, dw, dout):
+        buf.free()
