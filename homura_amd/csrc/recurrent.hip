@@ -1,6 +1,8 @@
 // Recurrent mixers (see recurrent.h): convolution rows, selective scan, gated linear recurrence.
 #include "recurrent.h"
 
+#include <algorithm>
+
 #include "row_pieces.h"
 
 namespace {
@@ -162,21 +164,44 @@ __device__ __forceinline__ void store_taps(const RowSource &in, const TapRing &r
 // way into registers while this one is scanned out of LDS, four tokens a read (token-minor rows of SCAN_T + 4
 // floats: the 16-byte reads of 16 neighbouring rows touch every bank once). Rows behind the chunk's end scan as dt = 0, which
 // leaves the state as it is.
-template <int SPL>
-__global__ __launch_bounds__(256) void selective_scan_kernel(SelectiveScanArgs a) {
+//
+// A workgroup walks its tokens one after the other (45 ns a token: the latency of an exponential and a multiply-add, LDS reads and the sum
+// over the states, with one wavefront a SIMD), so a long chunk is cut into segments (grid.y) and scanned by two launches.
+// ENDS: every segment but the last from a zero state (the first one from the chunk's) to its end, states only; left in
+// g.ends, with the segment's sum of steps: the segment multiplies a state by e^(A sum). Then every segment folds the ends
+// ahead of it into the state it starts from and is scanned in full. 2048 tokens, 2048 channels of 16 states: 91 us in one
+// segment, 33 + 19 in eight.
+struct ScanSegments {
+    int rows = 0;                    // of a segment, a multiple of the tile; 0: the chunk is one segment
+    float *ends = nullptr;           // [segments][inner][state_pad]: slot 0 the chunk's first state, slot g + 1 the end of segment g
+    float *steps = nullptr;          // [segments][inner]: slot g + 1 the sum of segment g's steps
+};
+
+template <int SPL, bool ENDS>
+__global__ __launch_bounds__(256) void selective_scan_kernel(SelectiveScanArgs a, ScanSegments g) {
     constexpr int SCAN_T = SPL <= 2 ? 64 : 32, SCAN_LD = SCAN_T + 4;  // (longer tiles hide the loads of the next one)
     constexpr int SP = 16 * SPL;
     constexpr int E = SCAN_T * 16 / 256, EB = SCAN_T * SP / 256;
     __shared__ __attribute__((aligned(16))) float s_dt[16][SCAN_LD], s_dx[16][SCAN_LD], s_y[16][SCAN_LD];
     __shared__ __attribute__((aligned(16))) float s_b[SP][SCAN_LD], s_c[SP][SCAN_LD];
-    const int tid = threadIdx.x, ch = tid >> 4, l = tid & 15, c0 = blockIdx.x * 16, n = a.n;
+    const int tid = threadIdx.x, ch = tid >> 4, l = tid & 15, c0 = blockIdx.x * 16;
+    const int seg = blockIdx.y, t_first = seg * g.rows, n = g.rows ? min(a.n, t_first + g.rows) : a.n;  // tokens t_first .. n - 1
+    const size_t states = (size_t)a.inner * SP;
     float A[SPL], S[SPL];
 #pragma unroll
     for (int k = 0; k < SPL; k++) {
         const size_t at = (size_t)(c0 + ch) * SP + l + 16 * k;
         A[k] = a.a_log2[at];
-        S[k] = a.past ? a.state[at] : 0.f;
+        if (ENDS || !g.rows) {
+            S[k] = a.past && seg == 0 ? a.state[at] : 0.f;
+            if (ENDS && seg == 0) g.ends[at] = S[k];  // (the other launch's last segment writes a.state while its first one starts)
+        } else {
+            S[k] = g.ends[at + (seg > 0 ? states : 0)];
+            for (int q = 2; q <= seg; q++)
+                S[k] = fmaf(__builtin_amdgcn_exp2f(A[k] * g.steps[(size_t)q * a.inner + c0 + ch]), S[k], g.ends[at + q * states]);
+        }
     }
+    float dt_sum = 0.f;
     const int ec = c0 + l, er = tid >> 4;  // this thread's channel and first row in loads and stores
     const bool odd = l & 1, upper = l & 2;
     const float d_c = a.d[ec], dt_bias = a.dt_bias[ec];
@@ -187,25 +212,26 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(SelectiveScanArgs a
             const size_t at = (size_t)min(t0 + er + e * 16, n - 1) * a.inner + ec;
             r_dt[e] = a.dt[at];
             r_x[e] = a.x[at];
-            r_z[e] = a.z[at];
+            if (!ENDS) r_z[e] = a.z[at];
         }
 #pragma unroll
         for (int e = 0; e < EB; e++) {
             const int i = tid + e * 256;
             const size_t at = (size_t)min(t0 + i / SP, n - 1) * a.bc_ld + i % SP;
             r_b[e] = a.b[at];
-            r_c[e] = a.c[at];
+            if (!ENDS) r_c[e] = a.c[at];
         }
     };
-    load_tile(0);
-    for (int t0 = 0; t0 < n; t0 += SCAN_T) {
+    load_tile(t_first);
+    for (int t0 = t_first; t0 < n; t0 += SCAN_T) {
         float x[E], z[E];
 #pragma unroll
         for (int e = 0; e < E; e++) {
             float dt = softplus_dev(r_dt[e] + dt_bias);
             if (t0 + er + e * 16 >= n) dt = 0.f;
             x[e] = r_x[e];
-            z[e] = r_z[e];
+            if (!ENDS) z[e] = r_z[e];
+            dt_sum += dt;
             s_dt[l][er + e * 16] = dt;
             s_dx[l][er + e * 16] = dt * x[e];
         }
@@ -213,7 +239,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(SelectiveScanArgs a
         for (int e = 0; e < EB; e++) {
             const int i = tid + e * 256;
             s_b[i % SP][i / SP] = r_b[e];
-            s_c[i % SP][i / SP] = r_c[e];
+            if (!ENDS) s_c[i % SP][i / SP] = r_c[e];
         }
         __syncthreads();
         if (t0 + SCAN_T < n) load_tile(t0 + SCAN_T);
@@ -226,7 +252,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(SelectiveScanArgs a
 #pragma unroll
             for (int k = 0; k < SPL; k++) {
                 b[set][k] = *reinterpret_cast<const f32x4 *>(&s_b[l + 16 * k][t]);
-                c[set][k] = *reinterpret_cast<const f32x4 *>(&s_c[l + 16 * k][t]);
+                if (!ENDS) c[set][k] = *reinterpret_cast<const f32x4 *>(&s_c[l + 16 * k][t]);
             }
         };
         read(0, 0);
@@ -238,18 +264,19 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(SelectiveScanArgs a
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int k = 0; k < SPL; k++) {
-                float g[4], h[4];
+                float keep[4], h[4];
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    g[u] = __builtin_amdgcn_exp2f(dt[set][u] * A[k]);
+                    keep[u] = __builtin_amdgcn_exp2f(dt[set][u] * A[k]);
                     h[u] = dx[set][u] * b[set][k][u];
                 }
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    S[k] = fmaf(g[u], S[k], h[u]);
-                    acc[u] = fmaf(S[k], c[set][k][u], acc[u]);
+                    S[k] = fmaf(keep[u], S[k], h[u]);
+                    if (!ENDS) acc[u] = fmaf(S[k], c[set][k][u], acc[u]);
                 }
             }
+            if (ENDS) continue;
             // lane l receives the sum over the 16 lanes for token l % 4
             const float p0 = (odd ? acc[1] : acc[0]) + dpp_move<0xB1, 0xF>(odd ? acc[0] : acc[1], 0.f);
             const float p1 = (odd ? acc[3] : acc[2]) + dpp_move<0xB1, 0xF>(odd ? acc[2] : acc[3], 0.f);
@@ -260,6 +287,7 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(SelectiveScanArgs a
             if ((t & 15) == 12) s_y[ch][t - 12 + l] = y;
         }
         __syncthreads();
+        if (ENDS) continue;
 #pragma unroll
         for (int e = 0; e < E; e++) {
             const int r = er + e * 16;
@@ -268,6 +296,20 @@ __global__ __launch_bounds__(256) void selective_scan_kernel(SelectiveScanArgs a
         }
         // (the next tile's staging writes none of what is read here: s_y is written behind its barrier)
     }
+    if constexpr (ENDS) {
+#pragma unroll
+        for (int k = 0; k < SPL; k++) g.ends[(seg + 1) * states + (size_t)(c0 + ch) * SP + l + 16 * k] = S[k];
+        s_y[l][er] = dt_sum;  // (nobody else uses s_y here)
+        __syncthreads();
+        if (tid < 16) {
+            float sum = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; r++) sum += s_y[tid][r];
+            g.steps[(size_t)(seg + 1) * a.inner + c0 + tid] = sum;
+        }
+        return;
+    }
+    if (n < a.n) return;
 #pragma unroll
     for (int k = 0; k < SPL; k++) a.state[(size_t)(c0 + ch) * SP + l + 16 * k] = S[k];
     store_taps(a.conv_in, a.ring, c0, n, a.past);
@@ -460,14 +502,40 @@ int selective_scan_launch(hm_ctx *ctx, const SelectiveScanArgs &a) {
     HM_REQUIRE(ctx, a.x && a.dt && a.dt_bias && a.z && a.b && a.c && a.a_log2 && a.d && a.state && a.out_split && a.ring.ring && a.n > 0 && a.past >= 0, "selective_scan: bad arguments");
     HM_REQUIRE(ctx, a.inner > 0 && a.inner % 16 == 0 && a.ring.width == a.inner && a.bc_ld >= a.state_pad && a.pieces >= 1 && a.pieces <= 3 &&
                         !bad_source(a.conv_in, a.inner), "selective_scan: bad shape");
-    const dim3 g(a.inner / 16), b(256);
+    // Segments of 128 tokens at least while the workgroups leave the chip short of four a CU (the 2048 tokens of a prompt of a
+    // model with 30 such layers of 2048 channels: 13.11 ms in one segment, 12.66 / 12.05 / 11.58 / 11.56 in 2 / 4 / 8 / 16)
+    const int tile = a.state_pad <= 32 ? 64 : 32, wgs = a.inner / 16;
+    int segs = std::min(4 * ctx->num_cus / wgs, a.n / 128);
+    const size_t per = (size_t)a.inner * (a.state_pad + 1) * sizeof(float);
+    segs = (int)std::min<size_t>((size_t)std::max(segs, 1), ((size_t)16 << 20) / per);  // (the kernels' part of the workspace)
+    ScanSegments s;
+    const dim3 b(256);
+    dim3 g(wgs);
+    if (segs > 1) {
+        s.rows = ((a.n + segs - 1) / segs + tile - 1) / tile * tile;
+        segs = (a.n + s.rows - 1) / s.rows;
+        s.ends = static_cast<float *>(ctx->workspace);
+        s.steps = s.ends + (size_t)segs * a.inner * a.state_pad;
+        g.y = segs;
+    }
+    if (segs <= 1) {
+        s = ScanSegments();
+        g.y = 1;
+    }
+    const dim3 ge(wgs, g.y - 1);
+#define HM_SCAN(SPL)                                                                                              \
+    do {                                                                                                          \
+        if (g.y > 1) hipLaunchKernelGGL((selective_scan_kernel<SPL, true>), ge, b, 0, ctx->stream, a, s);         \
+        hipLaunchKernelGGL((selective_scan_kernel<SPL, false>), g, b, 0, ctx->stream, a, s);                      \
+    } while (0)
     switch (a.state_pad) {
-    case 16: hipLaunchKernelGGL(selective_scan_kernel<1>, g, b, 0, ctx->stream, a); break;
-    case 32: hipLaunchKernelGGL(selective_scan_kernel<2>, g, b, 0, ctx->stream, a); break;
-    case 64: hipLaunchKernelGGL(selective_scan_kernel<4>, g, b, 0, ctx->stream, a); break;
-    case 128: hipLaunchKernelGGL(selective_scan_kernel<8>, g, b, 0, ctx->stream, a); break;
+    case 16: HM_SCAN(1); break;
+    case 32: HM_SCAN(2); break;
+    case 64: HM_SCAN(4); break;
+    case 128: HM_SCAN(8); break;
     default: return hm_set_error(ctx, HM_ERR_INVALID, "selective_scan: %d padded states", a.state_pad);
     }
+#undef HM_SCAN
     HM_LAUNCH_CHECK(ctx);
     return HM_OK;
 }

@@ -4,7 +4,7 @@ import dataclasses
 import numpy as np
 import pytest
 
-from homura_amd import DTYPE_Q4_0, DTYPE_Q8_0, synth, synth_model
+from homura_amd import DTYPE_F32, DTYPE_Q4_0, DTYPE_Q8_0, synth, synth_model
 
 pytestmark = pytest.mark.gpu
 
@@ -132,3 +132,24 @@ def test_q8_0_rows_straight_from_blocks(ctx, oracle, K, N):
     assert np.all(np.abs(got[:2 * N].reshape(2, N) - x64 @ w64.T) <= (64 + K / 16) * 2.0 ** -24 * mags)
     for buf in (dx, dw, dout):
         buf.free()
+
+
+@pytest.mark.parametrize("n", [127, 255, 256, 300, 1025, 2048])
+def test_selective_scan_in_segments(ctx, n):
+    """A chunk scanned in segments leaves the logits that the same tokens give one portion of at most 100 after the other
+    (those are one segment each), on an empty state and behind one."""
+    cfg = {"architecture": "Nokuvik", "vocab": 96, "width": 64, "embedding": {"scale": 1.0}, "norm": {"eps": 1e-5}, "loop": None,
+           "layers": [{"type": "mamba1", "mlp": None, "mixer": {"inner": 128, "conv": 4, "dt_rank": 8, "state": s}} for s in (16, 24, 40)]}
+    m = synth_model.build_block_model(ctx, cfg, 3, 4096, DTYPE_F32)
+    ids = synth.token_ids(n, n + 51, cfg["vocab"])
+    for past in (0, 50):
+        got = []
+        for step in (n, 100):
+            m.reset_kv_cache()
+            if past:
+                m.prefill(ids[:past], want_logits=False)
+            out = [m.prefill(ids[at:min(at + step, past + n)]) for at in range(past, past + n, step)]
+            got.append((np.concatenate(out).astype(np.float64), m.run_kv(ids[past + n:past + n + 1])[0].astype(np.float64)))
+        for a, b in zip(*got):
+            assert np.abs(a - b).max() <= 2e-4 * np.abs(b).max()
+    m.close()
