@@ -310,6 +310,8 @@ __global__ __launch_bounds__(256) void quantize_q8k_rows_kernel(const float *__r
 
 namespace homura {
 
+int kq_i8_min_slices(int K) { return (K / 256 + MAXB - 1) / MAXB; }
+
 int kq_i8_pack(hm_ctx *ctx, int hm_dtype, const uint8_t *d_blocks, int rows, int K, int8_t *d_planes, float *d_scales,
                int N_total, int row_mult, int row_off) {
     HM_CHECK_CTX(ctx);
@@ -357,7 +359,7 @@ int gemm_q8k_kquant_nk(hm_ctx *ctx, const int8_t *d_aq, const float *d_ascale, c
     // a slice's scales must fit their LDS tables
     const int KB = K / 256;
     int want = (int)std::max<long long>(1, ctx->num_cus / tiles);
-    want = std::min(std::min(want, std::max(1, max_parts)), KB);
+    want = std::min(std::min(std::max(want, kq_i8_min_slices(K)), std::max(1, max_parts)), KB);
     if (!parts) want = 1;
     g.blocks_per_split = (KB + want - 1) / want;
     HM_REQUIRE(ctx, g.blocks_per_split <= MAXB, "%s: K = %d needs %d K slices (%d allowed)", who, K, (KB + MAXB - 1) / MAXB,

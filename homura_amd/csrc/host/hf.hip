@@ -1891,7 +1891,9 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         int rows = 128;
         while (rows < n) rows *= 2;
         rows = std::min(rows, std::max(chunk_rows_, n));
-        auto sliced = [&](int64_t width) { return std::max<int64_t>(rows * width, gemm_sliced_tiles(ctx_->num_cus) * 128 * 128); };
+        auto sliced = [&](int64_t width, int K) {
+            return std::max<int64_t>((quant ? kq_i8_min_slices(K) : 1) * rows * width, gemm_sliced_tiles(ctx_->num_cus) * 128 * 128);
+        };
         const int64_t widest = std::max<int64_t>(std::max(hidden, qd), inter);
         hm_sync(ctx_);
         {
@@ -1910,9 +1912,9 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         p.h = Buffer::alloc(ctx_, {rows, hidden}, DType::F32);
         p.resid = Buffer::alloc(ctx_, {rows, hidden}, DType::F32);
         p.split = Buffer::alloc(ctx_, {rows, 3 * widest}, DType::BF16);
-        p.qkv = Buffer::alloc(ctx_, {sliced(nqkv)}, DType::F32);
-        p.proj_out = Buffer::alloc(ctx_, {sliced(hidden)}, DType::F32);
-        p.gate_up = Buffer::alloc(ctx_, {sliced(std::max<int64_t>(2 * (int64_t)inter, qd))}, DType::F32);
+        p.qkv = Buffer::alloc(ctx_, {sliced(nqkv, hidden)}, DType::F32);
+        p.proj_out = Buffer::alloc(ctx_, {sliced(hidden, std::max(qd, inter))}, DType::F32);
+        p.gate_up = Buffer::alloc(ctx_, {sliced(std::max<int64_t>(2 * (int64_t)inter, qd), hidden)}, DType::F32);
         if (!p.ids || !p.h || !p.resid || !p.split || !p.qkv || !p.proj_out || !p.gate_up) return HM_ERR_OOM;
         if (quant && widest % 256 == 0) {  // Q8_K rows for K-quant groups (a float holds four of the int8 values)
             p.q8 = Buffer::alloc(ctx_, {rows, widest / 4}, DType::F32);

@@ -153,3 +153,22 @@ def test_selective_scan_in_segments(ctx, n):
         for a, b in zip(*got):
             assert np.abs(a - b).max() <= 2e-4 * np.abs(b).max()
     m.close()
+
+
+def test_long_k_quant_prompt_with_wide_rows(ctx):
+    """Rows of 18 blocks need two K slices (a workgroup's tables hold 16), also where the tiles alone fill the chip."""
+    cfg = synth_model.TransformerConfig(hidden_size=2048, intermediate_size=4608, num_attention_heads=16, num_hidden_layers=1, vocab_size=512,
+                                        num_key_value_heads=4, head_dim=64, max_position_embeddings=2048, tie_word_embeddings=False)
+    types = synth_model.q4_k_m_mix(cfg)
+    m = synth_model.build_model(ctx, cfg, synth_model.synth_weights(cfg, 9, DTYPE_Q8_0, False, proj_dtypes=types), 2048, DTYPE_Q8_0, False,
+                                proj_dtypes=types)
+    ids = synth.token_ids(6, 1501, cfg.vocab_size)
+    got = []
+    for cuts in ((0, 1500), (0, 400, 800, 1200, 1500)):
+        m.reset_kv_cache()
+        for a, b in zip(cuts, cuts[1:]):
+            m.prefill(ids[a:b], want_logits=False)
+        got.append(m.run_kv(ids[1500:])[0].astype(np.float64))
+    # one layer: the sums are integers, only rows whose norm rounds the other way are quantised differently (1 / 127 of a value)
+    assert np.abs(got[0] - got[1]).max() <= 1e-2 * np.abs(got[1]).max()
+    m.close()
