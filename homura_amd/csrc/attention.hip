@@ -560,6 +560,32 @@ __global__ __launch_bounds__(GROUPS ? FOLD_THREADS : HD) void gqa_decode_fold_ke
     const float *aml = part_ml + (pair * nsplit * G + gi) * 2;
     constexpr int FB = FOLD_BATCH;
     float o[FB];
+    if constexpr (!GROUPS) {
+        // At most 32 splits: lane s holds split s's (max, sum), one exponential a lane gives every weight, and the weights are
+        // read across lanes. (Each thread walked the pairs through LDS
+        // with an exponential a split before: 8 sequences x 12 heads, 16 splits, 14.0 -> 12.5 us for both launches; 32 steps of
+        // Qwen2.5-1.5B behind 700 rows 45.5 -> 44.4 ms.)
+        const int lane = threadIdx.x & (WAVE - 1);
+        const float m = lane < nsplit ? aml[(size_t)lane * G * 2] : -INFINITY, l = lane < nsplit ? aml[(size_t)lane * G * 2 + 1] : 0.f;
+#pragma unroll
+        for (int u0 = 0; u0 < FB; u0 += 8)
+            if (u0 < nsplit) {
+#pragma unroll
+                for (int u = u0; u < u0 + 8; u++) o[u] = ao[(size_t)min(u, nsplit - 1) * G * HD];
+            }
+        const float M = wave_max(m);
+        const float w = lane < nsplit ? expf(m - M) : 0.f;
+        const float L = wave_sum(w * l);
+        float O = 0.f;
+#pragma unroll
+        for (int u0 = 0; u0 < FB; u0 += 8)
+            if (u0 < nsplit) {
+#pragma unroll
+                for (int u = u0; u < u0 + 8; u++) O = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u)), o[u], O);
+            }
+        out[((size_t)b * H + kvhd * G + gi) * HD + d] = O / L;
+        return;
+    }
 #pragma unroll
     for (int u = 0; u < FB; u++) {
         const int sp = sg + u * SG;
@@ -618,8 +644,8 @@ template <int HD, int G>
 int launch_fold(hm_ctx *ctx, const AttnArgs &a, const float *part_o, const float *part_ml, int nsplit, int chunk,
                 const DecodeState *state) {
     const bool groups = nsplit > FOLD_BATCH;
-    const int sg = groups ? FOLD_THREADS / HD : 1;
-    const size_t fold_lds = ((size_t)sg * (HD + 2) + (size_t)nsplit * 2) * sizeof(float);
+    const int sg = groups ? FOLD_THREADS / HD : 0;
+    const size_t fold_lds = groups ? ((size_t)sg * (HD + 2) + (size_t)nsplit * 2) * sizeof(float) : 0;
     HM_REQUIRE(ctx, fold_lds <= 64 * 1024, "gqa_decode_attn: too many splits (%d)", nsplit);
     if (groups)
         hipLaunchKernelGGL((gqa_decode_fold_kernel<HD, G, true>), dim3(a.kvh * G, a.B), dim3(FOLD_THREADS), fold_lds,

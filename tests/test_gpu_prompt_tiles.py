@@ -172,3 +172,25 @@ def test_long_k_quant_prompt_with_wide_rows(ctx):
     # one layer: the sums are integers, only rows whose norm rounds the other way are quantised differently (1 / 127 of a value)
     assert np.abs(got[0] - got[1]).max() <= 1e-2 * np.abs(got[1]).max()
     m.close()
+
+
+@pytest.mark.parametrize("B,H,kvh,hd,kv_len", [(1, 7, 1, 64, 65), (1, 4, 2, 128, 513), (2, 12, 2, 128, 1025), (1, 8, 1, 64, 2047), (3, 32, 4, 64, 577)])
+def test_fold_of_a_few_splits(ctx, B, H, kvh, hd, kv_len):
+    """Two to thirty-two splits, one far ahead of the others: the weights of the fold span the whole range of exp."""
+    rng = np.random.default_rng(kv_len)
+    q = rng.standard_normal((B, H, hd)).astype(np.float32)
+    k, v = rng.standard_normal((2, B, kvh, kv_len, hd)).astype(np.float32)
+    k[:, :, kv_len // 2] *= 20.0
+    kb, vb = synth.f32_to_bf16_rne(k), synth.f32_to_bf16_rne(v)
+    dq, dk, dv, do = ctx.to_device(q), ctx.to_device(kb), ctx.to_device(vb), ctx.empty(B * H * hd)
+    ctx.gqa_decode_attn(dq, dk, dv, do, B, H, kvh, hd, kv_len, kv_len, hd ** -0.5)
+    got = do.download(np.float32, (B, H, hd))
+    k64, v64 = synth.bf16_to_f32(kb).astype(np.float64), synth.bf16_to_f32(vb).astype(np.float64)
+    for b in range(B):
+        for h in range(H):
+            s = k64[b, h // (H // kvh)] @ q[b, h].astype(np.float64) * hd ** -0.5
+            p = np.exp(s - s.max())
+            # scores up to about 60 in f32: an exponential is off by 2^-24 of its exponent
+            assert np.abs(got[b, h] - (p / p.sum()) @ v64[b, h // (H // kvh)]).max() <= 5e-5
+    for buf in (dq, dk, dv, do):
+        buf.free()
