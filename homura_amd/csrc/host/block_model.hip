@@ -195,7 +195,6 @@ std::unique_ptr<BlockModel> BlockModel::create(hm_ctx *ctx, const BlockConfig &c
     m->compute_ = compute;
     m->prefill_pieces_ = compute == DType::F32 ? 3 : 1;
     m->chunk_rows_ = MAX_CHUNK;
-    m->even_chunks_ = false;
     m->wp_ = pad32(cfg.width);
     m->runs_ = cfg.runs();
     for (size_t r = 0; r < m->runs_.size(); r++) {

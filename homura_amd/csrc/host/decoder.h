@@ -108,9 +108,9 @@ class DecoderModel {
     int prefill_pieces_ = 3;
     // Rows of the prompt pass that go through the layers together at most: a product of 2048 rows and more fills the CUs
     // with 128 x 256 tiles and few K slices (6000 tokens of the Qwen3-0.6B shape and 16 steps in chunks of 512 rows 60.9 ms, of
-    // 3072 46.5; 1000 tokens in Q8_0 7.8 and 6.4)
+    // 3072 46.5; 1000 tokens in Q8_0 7.8 and 6.4). A longer prompt takes full chunks and a rest, which is few products' worth:
+    // cut into equal chunks 4200, 5000 and 6001 tokens take 22.6, 27.8 and 33.8 ms, so 21.1, 25.2 and 31.8
     int chunk_rows_ = 4096;
-    bool even_chunks_ = true;  // a prompt of several chunks is cut evenly, in steps of 128 rows
 
   private:
     // the bodies of the calls of the same name (see guarded)

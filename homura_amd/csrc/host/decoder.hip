@@ -77,13 +77,8 @@ int DecoderModel::prefill(const int64_t *h_ids, int n_ids, float *h_logits) {
     std::vector<int32_t> ids;
     int rc = check_ids(h_ids, n_ids, ids);
     if (rc != HM_OK) return rc;
-    int rows = chunk_rows_;
-    if (even_chunks_) {
-        const int chunks = (n_ids - 1) / chunk_rows_ + 1;
-        rows = std::min(chunk_rows_, ((n_ids - 1) / chunks / 128 + 1) * 128);
-    }
-    for (int at = 0; at < n_ids; at += rows) {
-        const int n = std::min(rows, n_ids - at);
+    for (int at = 0; at < n_ids; at += chunk_rows_) {
+        const int n = std::min(chunk_rows_, n_ids - at);
         rc = prefill_chunk(ids.data() + at, n, h_logits ? h_logits + (size_t)at * vocab_size() : nullptr);
         if (rc != HM_OK) return rc;
     }
