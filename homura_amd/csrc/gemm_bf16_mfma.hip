@@ -2,18 +2,21 @@
 // [K][N] (the reference's weight layout, src/hf/weights.rs:225-261) or [N][K] (the K-contiguous
 // stream layout the decode GEMVs use).
 //
-// The only MFMA kernel of the path (everything at batch 1 is HBM-bound). Workgroup tile 128x128,
-// eight wavefronts: two groups of 2x2, each wavefront owning 64x64 = 2x2 accumulator tiles of
-// v_mfma_f32_32x32x16_bf16 over half of the k steps. K advances 64 at a time. Four K tiles travel
-// global -> registers while the current one is multiplied out of LDS; two LDS buffers, one
-// barrier per tile.
+// Workgroup tile 128x128, eight wavefronts: two groups of 2x2, each wavefront owning 64x64 = 2x2
+// accumulator tiles of v_mfma_f32_32x32x16_bf16 over half of the k steps; K advances 64 at a time.
+// Two kernels:
+// gemm_dma_kernel (K a multiple of 64, operands on 16 bytes): global -> LDS without registers, four
+// buffers; a [K][N] tile keeps its rows in LDS and is transposed by the reads.
+// gemm_bf16_mfma_kernel (everything else, and [K][N] with A as several pieces): four K tiles travel
+// global -> registers while the current one is multiplied out of LDS; two LDS buffers, one barrier per tile.
 //
-// LDS holds both operands K-contiguous: row r (an m of A or an n of B) is 128 bytes = eight 16-byte
-// chunks of 8 k; chunk c of row r lives at slot c ^ (r & 7) ^ ((r >> 3) & 7). The MFMA operand read
-// (32 consecutive rows, one chunk each, 16 bytes per lane) then touches every bank once per 8 lanes,
-// and the transposing writes of a [K][N] tile (rows 8 apart per instruction) spread as well.
-// A [K][N] tile is transposed in registers: a thread loads a 4(k) x 8(n) block as four 16-byte rows,
-// regroups it with byte permutes into eight 8-byte columns and writes those.
+// LDS holds both operands K-contiguous (gemm_dma_kernel's [K][N] tile apart): row r (an m of A or an n
+// of B) is 128 bytes = eight 16-byte chunks of 8 k; chunk c of row r lives at slot
+// c ^ (r & 7) ^ ((r >> 3) & 7). The MFMA operand read (32 consecutive rows, one chunk each, 16 bytes
+// per lane) then touches every bank once per 8 lanes, and the transposing writes of a [K][N] tile
+// (rows 8 apart per instruction) spread as well: in gemm_bf16_mfma_kernel a thread loads a
+// 4(k) x 8(n) block as four 16-byte rows, regroups it with byte permutes into eight 8-byte columns and
+// writes those.
 //
 // Workgroups that share a B column block (the M/128 row blocks) get consecutive ids on one XCD, so
 // B is fetched from HBM once and served to the others from that XCD's L2.
