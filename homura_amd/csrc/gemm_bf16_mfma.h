@@ -14,8 +14,8 @@ namespace homura {
 // K-contiguous stream layout of the model weights. K % 32 == 0, pieces 1..3.
 // With parts != NULL the product may be cut along K into up to max_parts slices when M x N alone
 // leaves most of the chip idle: slice s lands in d_c + s * M * N, *parts says how many there are, and
-// the caller adds them up in index order (d_c must hold max_parts * M * N floats).
-// A product comes in more than one slice only while slices times its 128 x 128 tiles stay within gemm_sliced_tiles().
+// the caller adds them up in index order. A product comes in more than one slice only while slices times
+// its 128 x 128 tiles stay within gemm_sliced_tiles(): d_c holds M * N floats, and that many tiles at least.
 inline long long gemm_sliced_tiles(int cus) { return 2LL * cus; }
 int gemm_split_nk(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, const uint16_t *d_b_nk, float *d_c, int M, int K,
                   int N, int max_parts = 1, int *parts = nullptr);
@@ -60,6 +60,8 @@ int gemm_grouped_nk(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, int a_ro
 // up to 128). C = sum over blocks of scale * (A x ints^T over the block). Slices and ldc as above.
 int gemm_pieces_scaled_nk(hm_ctx *ctx, const uint16_t *d_a_split, const uint16_t *d_b_ints, const float *d_scales, int npad,
                           float *d_c, int M, int K, int N, int max_parts = 1, int *parts = nullptr, int ldc = 0);
+// The K slices that a product of activation pieces with b_pieces (1 or 3) pieces of B, or with a block-scaled B, comes in
+int gemm_pieces_slices(int b_pieces, bool scaled, int M, int K, int N, int cus, int max_parts);
 int gemm_pieces_any(hm_ctx *ctx, const uint16_t *d_a_split, int a_pieces, const uint16_t *d_b_split, int b_pieces,
                     const float *d_scales, int npad, float *d_c, int M, int K, int N, int max_parts, int *parts, int ldc);
 

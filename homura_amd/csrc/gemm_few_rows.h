@@ -20,6 +20,9 @@ inline bool few_rows_pays(int M, int N, int cus) {
     return M <= 32 || (M <= FEW_ROWS && (N + 32 * nt - 1) / (32 * nt) <= cus);
 }
 
+// K slices of such a product, at most max_parts: while the workgroups still fit the chip at once, a group for every wavefront
+int few_rows_slices(int M, int K, int N, int cus, int max_parts);
+
 // C[M][N] f32 (row stride ldc) = (sum of the pieces of A [M][pieces K])  x  B [N][K]^T, M <= FEW_ROWS, K % 32 == 0; with d_scales
 // (pieces = 3) B holds the integers of a block format and d_scales [K / 32][npad] the scale of every 32-wide block, npad >= N
 // rounded up to 128. With parts the result may come as up to max_parts K slices, slice s at d_c + s * M * ldc.

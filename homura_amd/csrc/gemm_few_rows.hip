@@ -201,7 +201,22 @@ int launch_tiles(hm_ctx *ctx, const uint16_t *a, const uint16_t *b, float *c, co
     return nt == 2 ? launch<AP, 2, 2, SC>(ctx, a, b, c, g, slices) : launch<AP, 2, 1, SC>(ctx, a, b, c, g, slices);
 }
 
+int few_rows_cut(int M, int K, int N, int cus, int max_parts, int *groups_per_slice) {
+    const int group = M <= 32 ? 64 : 32, groups = (K + group - 1) / group, nt = homura::few_rows_tiles(N, cus);
+    const long long wgs = (N + 32 * nt - 1) / (32 * nt);
+    int want = (int)std::max<long long>(1, cus / wgs);
+    want = std::min(std::min(want, std::max(1, max_parts)), std::max(1, groups / WAVES));
+    while (want > 1 && (N + 127) / 128 * want > homura::gemm_sliced_tiles(cus)) want--;
+    *groups_per_slice = (groups + want - 1) / want;
+    return (groups + *groups_per_slice - 1) / *groups_per_slice;
+}
+
 }  // namespace
+
+int homura::few_rows_slices(int M, int K, int N, int cus, int max_parts) {
+    int per = 0;
+    return few_rows_cut(M, K, N, cus, max_parts, &per);
+}
 
 int homura::gemm_few_rows(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, const uint16_t *d_b_nk, const float *d_scales, int npad,
                           float *d_c, int M, int K, int N, int max_parts, int *parts, int ldc) {
@@ -220,15 +235,8 @@ int homura::gemm_few_rows(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, co
     g.ldc = ldc;
     g.scales = d_scales;
     g.npad = npad;
-    const int group = M <= 32 ? 64 : 32, groups = (K + group - 1) / group;
     const int nt = few_rows_tiles(N, ctx->num_cus);
-    const long long wgs = (N + 32 * nt - 1) / (32 * nt);
-    // K slices while the workgroups still fit the chip at once, a group for every wavefront
-    int want = (int)std::max<long long>(1, ctx->num_cus / wgs);
-    want = std::min(std::min(want, std::max(1, parts ? max_parts : 1)), std::max(1, groups / WAVES));
-    while (want > 1 && (N + 127) / 128 * want > gemm_sliced_tiles(ctx->num_cus)) want--;
-    g.groups_per_slice = (groups + want - 1) / want;
-    const int slices = (groups + g.groups_per_slice - 1) / g.groups_per_slice;
+    const int slices = few_rows_cut(M, K, N, ctx->num_cus, parts ? max_parts : 1, &g.groups_per_slice);
     if (parts) *parts = slices;
     if (d_scales) return launch_tiles<3, true>(ctx, d_a_split, d_b_nk, d_c, g, (unsigned)slices, nt);
     if (pieces == 3) return launch_tiles<3, false>(ctx, d_a_split, d_b_nk, d_c, g, (unsigned)slices, nt);

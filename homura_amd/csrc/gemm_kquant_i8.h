@@ -33,8 +33,10 @@ int quantize_q8k_rows_launch(hm_ctx *ctx, const float *d_x, int8_t *d_q, float *
 
 // C [M][N] f32 (row stride ldc, 0 = N) = Q8_K rows x K-quant matrix^T. With `parts`, K may be cut into up to
 // max_parts slices of whole blocks written as [parts][M][ldc], to be added in index order by the consumer.
-// (the LDS tables of a workgroup hold 16 blocks: wider rows come in this many slices at least, however many tiles there are)
+// (the LDS tables of a workgroup hold 16 blocks: wider rows come in kq_i8_min_slices at least, however many tiles there are;
+// more than that only while slices times the 128 x 128 tiles stay within the CUs)
 int kq_i8_min_slices(int K);
+int kq_i8_slices(int M, int K, int N, int cus, int max_parts);
 int gemm_q8k_kquant_nk(hm_ctx *ctx, const int8_t *d_aq, const float *d_ascale, const int8_t *d_planes,
                        const float *d_scales, float *d_c, int M, int K, int N, int max_parts = 1, int *parts = nullptr,
                        int ldc = 0);

@@ -310,7 +310,18 @@ __global__ __launch_bounds__(256) void quantize_q8k_rows_kernel(const float *__r
 
 namespace homura {
 
-int kq_i8_min_slices(int K) { return (K / 256 + MAXB - 1) / MAXB; }
+int kq_i8_min_slices(int K) { return std::max(1, (K / 256 + MAXB - 1) / MAXB); }
+
+int kq_i8_slices(int M, int K, int N, int cus, int max_parts) {
+    // slices of whole blocks while they still add whole waves of workgroups to a grid smaller than the chip;
+    // a slice's scales must fit their LDS tables
+    const long long tiles = (long long)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
+    const int KB = K / 256;
+    int want = (int)std::max<long long>(1, cus / tiles);
+    want = std::min(std::min(std::max(want, kq_i8_min_slices(K)), std::max(1, max_parts)), KB);
+    const int per = (KB + want - 1) / want;
+    return (KB + per - 1) / per;
+}
 
 int kq_i8_pack(hm_ctx *ctx, int hm_dtype, const uint8_t *d_blocks, int rows, int K, int8_t *d_planes, float *d_scales,
                int N_total, int row_mult, int row_off) {
@@ -355,16 +366,10 @@ int gemm_q8k_kquant_nk(hm_ctx *ctx, const int8_t *d_aq, const float *d_ascale, c
     g.K = K;
     g.ldc = ldc > 0 ? ldc : N;
     HM_REQUIRE(ctx, g.ldc >= N, "%s: ldc %d below N %d", who, g.ldc, N);
-    // K slices of whole blocks while they still add whole waves of workgroups to a grid smaller than the chip;
-    // a slice's scales must fit their LDS tables
-    const int KB = K / 256;
-    int want = (int)std::max<long long>(1, ctx->num_cus / tiles);
-    want = std::min(std::min(std::max(want, kq_i8_min_slices(K)), std::max(1, max_parts)), KB);
-    if (!parts) want = 1;
-    g.blocks_per_split = (KB + want - 1) / want;
-    HM_REQUIRE(ctx, g.blocks_per_split <= MAXB, "%s: K = %d needs %d K slices (%d allowed)", who, K, (KB + MAXB - 1) / MAXB,
+    const int KB = K / 256, slices = kq_i8_slices(M, K, N, ctx->num_cus, parts ? max_parts : 1);
+    g.blocks_per_split = (KB + slices - 1) / slices;
+    HM_REQUIRE(ctx, g.blocks_per_split <= MAXB, "%s: K = %d needs %d K slices (%d allowed)", who, K, kq_i8_min_slices(K),
                parts ? max_parts : 1);
-    const int slices = (KB + g.blocks_per_split - 1) / g.blocks_per_split;
     if (parts) *parts = slices;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_q8k_kquant_kernel),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES);

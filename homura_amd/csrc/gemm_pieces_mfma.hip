@@ -380,6 +380,11 @@ Cut cut_for(long long m_tiles, int N, int ns, long long out_bytes, int cus, int 
 
 }  // namespace
 
+int homura::gemm_pieces_slices(int b_pieces, bool scaled, int M, int K, int N, int cus, int max_parts) {
+    if (b_pieces == 1 && few_rows_pays(M, N, cus)) return few_rows_slices(M, K, N, cus, max_parts);
+    return cut_for((M + TM - 1) / TM, N, K / TK, 4LL * M * N, cus, max_parts, b_pieces == 1 && !scaled).slices;
+}
+
 int homura::gemm_pieces_scaled_nk(hm_ctx *ctx, const uint16_t *d_a_split, const uint16_t *d_b_ints, const float *d_scales,
                                   int npad, float *d_c, int M, int K, int N, int max_parts, int *parts, int ldc) {
     HM_CHECK_CTX(ctx);

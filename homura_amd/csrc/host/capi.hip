@@ -499,6 +499,13 @@ int hm_model_shape(hm_model *m, int *vocab_size, int *hidden_size, int *num_laye
 
 int hm_model_is_transformer(hm_model *m) { return m && dynamic_cast<HfModel *>(m->impl.get()) ? 1 : 0; }
 
+int hm_test_prompt_product(int hm_dtype, int rows, int m, int k, int n, int cus, long long *floats_held, long long *floats_written) {
+    if (!floats_held || !floats_written || m < 1 || m > rows || k < 32 || k % 32 || n < 1 || cus < 1) return HM_ERR_INVALID;
+    *floats_held = prompt_product_floats((DType)hm_dtype, rows, k, n, cus);
+    *floats_written = (long long)prompt_product_slices((DType)hm_dtype, m, k, n, cus) * m * n;
+    return HM_OK;
+}
+
 int hm_model_capture_residuals(hm_model *m, int on) {
     BlockModel *b = m ? dynamic_cast<BlockModel *>(m->impl.get()) : nullptr;
     return b ? b->capture_residuals(on != 0) : HM_ERR_INVALID;

@@ -159,7 +159,6 @@ class HfModel : public DecoderModel {
     std::shared_ptr<PlanScratch> scratch_;
     // prefill pass: activations of one chunk of rows
     struct PrefillScratch {
-        static constexpr int MAX_PARTS = 8;  // K slices a projection result may come in
         int rows = 0;
         Buffer ids, h, resid, split, qkv, proj_out, gate_up, logits;
         Buffer wsplit;  // block formats: the matrices of one group of projections as three bf16 pieces per weight
@@ -182,5 +181,11 @@ class HfModel : public DecoderModel {
     PrefillScratch pf_;
     size_t prefill_weight_cache_bytes_ = (size_t)32 << 30;
 };
+
+constexpr int PROMPT_PARTS = 8;  // K slices a projection result of the prompt pass may come in
+// Floats that hold the result of a prompt product of up to `rows` rows with an [N][K] matrix of a format, in all the K slices
+// it may come in; and the most slices that one of M rows does come in.
+int64_t prompt_product_floats(DType dtype, int64_t rows, int K, int64_t N, int cus);
+int prompt_product_slices(DType dtype, int M, int K, int N, int cus);
 
 }  // namespace homura

@@ -1877,6 +1877,20 @@ const float *HfModel::weight_f32(const std::string &name) const {
     return it == slot_by_name_.end() ? nullptr : weight_bufs_[it->second].as<float>();
 }
 
+int64_t prompt_product_floats(DType dtype, int64_t rows, int K, int64_t N, int cus) {
+    const bool kquant = dtype == DType::Q4_K || dtype == DType::Q6_K;
+    return std::max<int64_t>((kquant ? kq_i8_min_slices(K) : 1) * rows * N, gemm_sliced_tiles(cus) * 128 * 128);
+}
+
+int prompt_product_slices(DType dtype, int M, int K, int N, int cus) {
+    const int MP = PROMPT_PARTS;
+    if (dtype == DType::BF16) return gemm_pieces_slices(1, false, M, K, N, cus, MP);
+    const bool kquant = dtype == DType::Q4_K || dtype == DType::Q6_K;
+    // (weights as pieces where the integers do not fit the budget)
+    const int pieces = gemm_pieces_slices(3, false, M, K, N, cus, MP);
+    return std::max(pieces, kquant ? (K % 256 ? 1 : kq_i8_slices(M, K, N, cus, MP)) : gemm_pieces_slices(1, true, M, K, N, cus, MP));
+}
+
 int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     constexpr int HEAD_ROWS = 512;  // rows whose logits are held at a time
     const TransformerConfig &c = cfg_;
@@ -1891,8 +1905,12 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         int rows = 128;
         while (rows < n) rows *= 2;
         rows = std::min(rows, std::max(chunk_rows_, n));
-        auto sliced = [&](int64_t width, int K) {
-            return std::max<int64_t>((quant ? kq_i8_min_slices(K) : 1) * rows * width, gemm_sliced_tiles(ctx_->num_cus) * 128 * 128);
+        // the f32 results of a group of projections (`first` names its members' format, the same in every layer or not)
+        auto sliced = [&](int first, int K, int64_t width) {
+            int64_t most = 0;
+            for (int l = 0; l < c.num_hidden_layers; l++)
+                most = std::max(most, prompt_product_floats(proj_dtype(l, first), rows, K, width, ctx_->num_cus));
+            return most;
         };
         const int64_t widest = std::max<int64_t>(std::max(hidden, qd), inter);
         hm_sync(ctx_);
@@ -1912,9 +1930,9 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         p.h = Buffer::alloc(ctx_, {rows, hidden}, DType::F32);
         p.resid = Buffer::alloc(ctx_, {rows, hidden}, DType::F32);
         p.split = Buffer::alloc(ctx_, {rows, 3 * widest}, DType::BF16);
-        p.qkv = Buffer::alloc(ctx_, {sliced(nqkv, hidden)}, DType::F32);
-        p.proj_out = Buffer::alloc(ctx_, {sliced(hidden, std::max(qd, inter))}, DType::F32);
-        p.gate_up = Buffer::alloc(ctx_, {sliced(std::max<int64_t>(2 * (int64_t)inter, qd), hidden)}, DType::F32);
+        p.qkv = Buffer::alloc(ctx_, {sliced(0, hidden, nqkv)}, DType::F32);
+        p.proj_out = Buffer::alloc(ctx_, {std::max(sliced(3, qd, hidden), sliced(6, inter, hidden))}, DType::F32);
+        p.gate_up = Buffer::alloc(ctx_, {std::max<int64_t>(sliced(4, hidden, 2 * (int64_t)inter), (int64_t)rows * qd)}, DType::F32);
         if (!p.ids || !p.h || !p.resid || !p.split || !p.qkv || !p.proj_out || !p.gate_up) return HM_ERR_OOM;
         if (quant && widest % 256 == 0) {  // Q8_K rows for K-quant groups (a float holds four of the int8 values)
             p.q8 = Buffer::alloc(ctx_, {rows, widest / 4}, DType::F32);
@@ -1940,7 +1958,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     float *proj_out = p.proj_out.as<float>(), *gate_up = p.gate_up.as<float>();
     uint16_t *split = p.split.as<uint16_t>();
     const int np = quant ? 3 : prefill_pieces_;
-    const int MP = PrefillScratch::MAX_PARTS;
+    const int MP = PROMPT_PARTS;
     int parts = 1;  // K slices of the latest projection
     uint16_t *wsplit = quant ? p.wsplit.as<uint16_t>() : nullptr;
     static const char *const proj_name[7] = {"self_attn.q_proj.weight", "self_attn.k_proj.weight", "self_attn.v_proj.weight",

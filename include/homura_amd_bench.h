@@ -56,6 +56,10 @@ int hm_bench_launch_floor(hm_ctx *ctx, int n_kernels, int chained, int replays, 
  * variable HOMURA_ALLOC_FILL=<byte>, read when the first buffer is allocated. */
 int hm_test_fill_lds(hm_ctx *ctx, uint32_t word);
 
+/* Test support: the floats that the prompt pass sets aside for the product of up to `rows` rows with an [n][k] matrix of a
+ * weight format on a chip of `cus` CUs, and the most that the product of m <= rows rows writes (all its K slices). Host only. */
+int hm_test_prompt_product(int hm_dtype, int rows, int m, int k, int n, int cus, long long *floats_held, long long *floats_written);
+
 /* Phase trace of the latest whole-step decode launch: device-clock ticks (100 MHz) taken by workgroup
  * 0 at 11 points per layer (both workgroup barriers of the Q|K|V, attention, O, gate|up and down
  * phases; the end of the fold follows attention's second barrier) and one at the end of the kernel, then

@@ -174,6 +174,26 @@ def test_long_k_quant_prompt_with_wide_rows(ctx):
     m.close()
 
 
+@pytest.mark.parametrize("fmt", [DTYPE_Q8_0, DTYPE_Q4_0])
+def test_long_block_format_prompt_of_a_narrow_model(ctx, fmt):
+    """A width below a K-quant block and a wide MLP: 1100 rows of 8192 gate and up values are more than the least that a product's
+    scratch holds. The same tokens in short portions leave the same rows, up to cache elements that round the other way."""
+    cfg = synth_model.TransformerConfig(hidden_size=128, intermediate_size=4096, num_attention_heads=2, num_hidden_layers=2, vocab_size=256,
+                                        num_key_value_heads=1, head_dim=64, max_position_embeddings=1200, tie_word_embeddings=False)
+    types = [fmt] * 7 * cfg.num_hidden_layers
+    m = synth_model.build_model(ctx, cfg, synth_model.synth_weights(cfg, 11, DTYPE_Q8_0, False, proj_dtypes=types), 1200, DTYPE_Q8_0, False,
+                                proj_dtypes=types)
+    ids = synth.token_ids(7, 1101, cfg.vocab_size)
+    got = []
+    for step in (1100, 100):
+        m.reset_kv_cache()
+        rows = [m.prefill(ids[at:at + step]) for at in range(0, 1100, step)]
+        got.append((np.concatenate(rows).astype(np.float64), m.run_kv(ids[1100:])[0].astype(np.float64)))
+    for a, b in zip(*got):
+        assert np.abs(a - b).max() <= 2e-3 * np.abs(b).max()
+    m.close()
+
+
 @pytest.mark.parametrize("B,H,kvh,hd,kv_len", [(1, 7, 1, 64, 65), (1, 4, 2, 128, 513), (2, 12, 2, 128, 1025), (1, 8, 1, 64, 2047), (3, 32, 4, 64, 577)])
 def test_fold_of_a_few_splits(ctx, B, H, kvh, hd, kv_len):
     """Two to thirty-two splits, one far ahead of the others: the weights of the fold span the whole range of exp."""
