@@ -581,7 +581,8 @@ __global__ __launch_bounds__(GROUPS ? FOLD_THREADS : HD) void gqa_decode_fold_ke
         for (int u0 = 0; u0 < FB; u0 += 8)
             if (u0 < nsplit) {
 #pragma unroll
-                for (int u = u0; u < u0 + 8; u++) O = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u)), o[u], O);
+                for (int u = u0; u < u0 + 8; u++)  // (past the last split: not its sum again, 0 times infinity is NaN)
+                    O = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u)), u < nsplit ? o[u] : 0.f, O);
             }
         out[((size_t)b * H + kvhd * G + gi) * HD + d] = O / L;
         return;

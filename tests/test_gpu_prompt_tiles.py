@@ -214,3 +214,18 @@ def test_fold_of_a_few_splits(ctx, B, H, kvh, hd, kv_len):
             assert np.abs(got[b, h] - (p / p.sum()) @ v64[b, h // (H // kvh)]).max() <= 5e-5
     for buf in (dq, dk, dv, do):
         buf.free()
+
+
+@pytest.mark.parametrize("H,kvh,hd,kv_len", [(8, 2, 128, 577), (4, 2, 64, 300), (12, 2, 128, 200), (32, 4, 64, 2047)])
+def test_fold_keeps_an_infinite_value(ctx, H, kvh, hd, kv_len):
+    """An infinite element of the last split's values makes its own column infinite, however many splits there are, and no other."""
+    rng = np.random.default_rng(kv_len)
+    q = rng.standard_normal((1, H, hd)).astype(np.float32)
+    k, v = (synth.f32_to_bf16_rne(rng.standard_normal((1, kvh, kv_len, hd)).astype(np.float32)) for _ in range(2))
+    v[:, :, kv_len - 1, 5] = 0x7F80
+    dq, dk, dv, do = ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), ctx.empty(H * hd)
+    ctx.gqa_decode_attn(dq, dk, dv, do, 1, H, kvh, hd, kv_len, kv_len, hd ** -0.5)
+    got = do.download(np.float32, (H, hd))
+    assert np.all(got[:, 5] == np.inf) and np.all(np.isfinite(np.delete(got, 5, 1)))
+    for buf in (dq, dk, dv, do):
+        buf.free()
