@@ -431,6 +431,7 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
     for (int r = 0; r < R; r++) a[r] = 0.f;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
+        const bool live = ((c * WPS + wis) * WAVE + lane) * KPL < K;
         float xv[KPL], sx = 0.f, sx_first = 0.f;
 #pragma unroll
         for (int j = 0; j < XV; j++)
@@ -450,7 +451,8 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const float d = f16_bits_to_f32((uint16_t)sc[c][r]);
+            float d = f16_bits_to_f32((uint16_t)sc[c][r]);
+            if (RAW && !live) d = 0.f;  // (a unit past the row's end: an infinite scale times its zero activations would be NaN)
             const uint32_t w[4] = {qw[c][r].x, qw[c][r].y, qw[c][r].z, qw[c][r].w};
             float t = 0.f;
             if (QT == 0) {

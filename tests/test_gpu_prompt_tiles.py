@@ -134,6 +134,27 @@ def test_q8_0_rows_straight_from_blocks(ctx, oracle, K, N):
         buf.free()
 
 
+@pytest.mark.parametrize("K", [32, 544, 1056, 2080, 4128])
+def test_q8_0_row_with_an_infinite_scale(ctx, K):
+    """A first block with an infinite scale and positive products makes its row infinite, also where the row's last units are
+    past its end; the other rows are what they are without it."""
+    N = 5
+    raw = synth.q8_0_blocks(51, N * K // 32, 0.01).reshape(N, K // 32, 34).copy()
+    x = np.abs(synth.normal_f32(52, K)) + np.float32(0.1)
+    dx, dout = ctx.to_device(x), ctx.empty(N)
+    got = []
+    for inf in (False, True):
+        if inf:
+            raw[2, 0, :2], raw[2, 0, 2:] = (0x00, 0x7C), 3
+        dw = ctx.to_device(raw)
+        ctx.gemv_q8_0(dx, dw, dout, 1, K, N)
+        got.append(dout.download(np.float32, (N,)))
+        dw.free()
+    assert got[1][2] == np.inf and np.array_equal(np.delete(got[0], 2), np.delete(got[1], 2))
+    for buf in (dx, dout):
+        buf.free()
+
+
 @pytest.mark.parametrize("n", [127, 255, 256, 300, 1025, 2048])
 def test_selective_scan_in_segments(ctx, n):
     """A chunk scanned in segments leaves the logits that the same tokens give one portion of at most 100 after the other
