@@ -535,7 +535,10 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
 #pragma unroll
         for (int u = 0; u < TW; u++) split8<NP>(f[u], pp[u]);
 #pragma unroll
-        for (int u = 0; u < TW; u++)
+        for (int u = 0; u < TW; u++) {
+            // a second tile that none of these 16 rows sees stays out: its weights are zero, but a value in it may be infinite
+            // (1905 rows of 16 heads of 128 behind 4096 219.8 -> 223.2 us, 4096 rows of 32 heads of 64 187 -> 183)
+            if (u > 0 && __builtin_expect((t + u) * A8_KEYS >= wave_end, 0)) break;
 #pragma unroll
             for (int db = 0; db < DB; db++) {
                 const int chunk = 2 * db + (v_sub >> 1), within = (v_sub & 1) * 8;
@@ -554,6 +557,7 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
                     acc_o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[pv], pp[u][p], acc_o[db], 0, 0, 0);
                 });
             }
+        }
     }
 
     if (KS > 1) {

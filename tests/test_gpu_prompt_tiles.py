@@ -77,6 +77,24 @@ def test_prompt_attention_over_key_groups(ctx, S, past, H, kvh, hd):
         buf.free()
 
 
+@pytest.mark.parametrize("groups", [1, 2, 4])
+@pytest.mark.parametrize("H,kvh,hd", [(16, 8, 128), (14, 2, 64)])
+def test_prompt_rows_ahead_of_an_infinite_value(ctx, monkeypatch, groups, H, kvh, hd):
+    """Rows of 16 that see none of the 32 keys around an infinite value stay finite, whatever a wavefront takes between barriers."""
+    monkeypatch.setenv("HOMURA_PREFILL_KEY_GROUPS", str(groups))
+    S = 300
+    rng = np.random.default_rng(groups)
+    q = rng.standard_normal((S, H, hd)).astype(np.float32)
+    k, v = (synth.f32_to_bf16_rne(rng.standard_normal((kvh, S, hd)).astype(np.float32)) for _ in range(2))
+    v[:, 190, 5] = 0x7F80
+    dq, dk, dv, do = ctx.to_device(q), ctx.to_device(k), ctx.to_device(v), ctx.empty(S * H * hd)
+    ctx.gqa_prefill_attn(dq, dk, dv, do, S, H, kvh, hd, S, 0, hd ** -0.5)
+    got = do.download(np.float32, (S, H, hd))
+    assert np.all(np.isfinite(got[:160])) and np.all(np.isfinite(np.delete(got, 5, 2))) and not np.any(np.isfinite(got[190:, :, 5]))
+    for buf in (dq, dk, dv, do):
+        buf.free()
+
+
 @pytest.mark.parametrize("M,K,N", [(1, 32, 8), (7, 96, 200), (24, 1024, 6144), (31, 160, 4097), (32, 896, 33), (33, 32, 64), (37, 4864, 896),
                                    (64, 1056, 1001), (64, 1536, 17920), (64, 2080, 6150)])
 @pytest.mark.parametrize("form", ["f32", "bf16", "q8_0", "q4_0"])
