@@ -1,6 +1,6 @@
 // GGUF block-quantised weights: dequant-GEMV (Q8_0, Q4_0) and bit-exact block dequantisation.
 //
-// (A plain Q8_0 product goes through gemv_q8_0_blocks_cut instead.)
+// (A plain Q8_0 product goes through gemv_q8_0_blocks_cut instead, unless staged_rows_pay.)
 //
 // Weights stay in HBM as the raw GGUF block bytes, rows of K/32 blocks. A workgroup takes a
 // contiguous run of rows, which is a contiguous byte range of the weight buffer, and copies
@@ -412,6 +412,18 @@ QuantShape quant_shape(const hm_ctx *ctx, int K, int N) {
     return sh;
 }
 
+// Whether a plain Q8_0 product stages its blocks in LDS: where gemv_q8_0_blocks_cut leaves lanes without a unit (a quarter of
+// them at 1536, three eighths at 2560, an eighth at 3584), a row's quarters fill this kernel's rounds of lanes, and there are
+// so many rows that the stream counts and not its start. us here / there, weights cold: 1536 -> 65536 32.8 / 34.1, 1536 ->
+// 151936 68.4 / 75.3, 2432 -> 17000 17.2 / 19.0, 2560 -> 24000 21.6 / 24.6, 2560 -> 151936 111 / 137, 3584 -> 65536 68.1 / 70.0;
+// but 1536 -> 32000 19.4 / 18.5, 1504 -> 65536 33.6 / 32.7, 2560 -> 10000 13.4 / 12.0, 2304 -> 65536 63.5 / 58.4, 2688 -> 65536
+// 64 / 61, 3072 -> 65536 73.3 / 65.0, 3552 -> 65536 67.7 / 67.1.
+bool staged_rows_pay(int K, int N) {
+    if (K <= 1536) return K > 1088 && K % 64 == 0 && N >= 60000;
+    if (K <= 2560) return K >= 2432 && N >= 16500;
+    return K >= 3264 && K <= 3584 && K % 64 == 0 && N >= 60000;
+}
+
 template <int QT>
 int gemv_quant_launch(hm_ctx *ctx, const char *name, const float *d_x, const uint8_t *d_w,
                       float *d_out, int M, int K, int N, const homura::QuantFuse &fuse = homura::QuantFuse()) {
@@ -443,7 +455,7 @@ int gemv_quant_launch(hm_ctx *ctx, const char *name, const float *d_x, const uin
         return rc;
     }
     const bool fused = fuse.x2 || fuse.res_in || fuse.norm_w || fuse.res_out_add || fuse.cand_v;
-    if (QT == 0 && !fused) {  // straight from the blocks into registers (2048 -> 5632 6.74 -> 5.10 us)
+    if (QT == 0 && !fused && !staged_rows_pay(K, N)) {  // straight from the blocks into registers (2048 -> 5632 6.74 -> 5.10 us)
         int rc = HM_OK;
         for (int m = 0; m < M && rc == HM_OK; m++)
             rc = homura::gemv_q8_0_blocks_cut(ctx, d_x + (size_t)m * K, d_w, d_out + (size_t)m * N, K, N);
@@ -462,7 +474,7 @@ int gemv_quant_launch(hm_ctx *ctx, const char *name, const float *d_x, const uin
         if (fused)                                                                                        \
             hipLaunchKernelGGL((gemv_quant_kernel<QT, C, true>), dim3(grid), dim3(QTHREADS), lds, ctx->stream, xm, \
                                d_w, om, K, N, rows, fuse);                                                \
-        else if constexpr (QT == 1)                                                                       \
+        else if constexpr (QT == 1 || C == 3 || C == 5 || C == 7) /* (see staged_rows_pay) */             \
             hipLaunchKernelGGL((gemv_quant_kernel<QT, C, false>), dim3(grid), dim3(QTHREADS), lds, ctx->stream, xm, \
                                d_w, om, K, N, rows, fuse);                                                \
     } while (0)

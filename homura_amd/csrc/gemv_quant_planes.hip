@@ -98,6 +98,15 @@ typedef const u32x4 __attribute__((address_space(1))) *global_u32x4_ptr;
 typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 typedef const u32x4_a2 __attribute__((address_space(1))) *global_u32x4_a2_ptr;
 
+// sum over the 32 lanes of a half wavefront, in its last lane
+__device__ __forceinline__ float half_sum(float v) {
+    v += dpp_move<0xB1, 0xF>(v, 0.f);   // quad_perm [1,0,3,2]
+    v += dpp_move<0x4E, 0xF>(v, 0.f);   // quad_perm [2,3,0,1]
+    v += dpp_move<0x141, 0xF>(v, 0.f);  // row_half_mirror
+    v += dpp_move<0x140, 0xF>(v, 0.f);  // row_mirror: every lane of a row of 16 holds its total
+    return v + dpp_move<0x142, 0xA>(v, 0.f);  // row_bcast15 into rows 1 and 3
+}
+
 template <int QT>
 __device__ __forceinline__ QWords<QT> load_quarter(const uint8_t *q) {
     QWords<QT> r;
@@ -330,22 +339,24 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_kernel(const float *__re
 // MODE 0: plain row. 1: a second operand (x2 or res_in). 2: RMSNorm, with or without res_in.
 // RAW: `quants` are the blocks as the file has them (34 or 18 bytes, f16 scale first): a unit's 16 bytes start at an even
 // address, which one 16-byte load takes as well.
-template <int QT, int R, int NC, int MODE, int WPS, bool RAW = false>
+// L: lanes a row takes of a wavefront; with 32 a request of the wavefront covers two rows (R then counts pairs of rows).
+template <int QT, int R, int NC, int MODE, int WPS, bool RAW = false, int L = WAVE>
 __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const float *__restrict__ x, const uint8_t *__restrict__ quants,
                                                                       const uint16_t *__restrict__ scales, float *__restrict__ out,
                                                                       int K, int N, const QuantFuse fuse_arg) {
     constexpr bool FUSED = MODE >= 1;
     const QuantFuse fuse = FUSED ? fuse_arg : QuantFuse();
     constexpr int KPL = QT == 0 ? 16 : 32, XV = KPL / 4;  // weights and f32x4 activation pieces of a unit
-    __shared__ float part[PWAVES][R];
+    constexpr int ROWS = R * (WAVE / L);  // of a set
+    __shared__ float part[PWAVES][ROWS];
     __shared__ float red[PWAVES];
-    const int lane = threadIdx.x & (WAVE - 1);
+    const int lane = threadIdx.x & (WAVE - 1), ul = lane & (L - 1), sub = lane / L;  // this lane's unit of its row
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    // WPS wavefronts (as many as a row has chunks, so that none idles) share a set of R rows; a workgroup works
+    // WPS wavefronts (as many as a row has chunks, so that none idles) share a set of rows; a workgroup works
     // on PWAVES / WPS sets
     constexpr int SETS = PWAVES / WPS;
     const int set = wave / WPS, wis = wave % WPS;
-    const int row0 = (blockIdx.x * SETS + set) * R;
+    const int row0 = (blockIdx.x * SETS + set) * ROWS;
     const size_t qrow = QT == 0 ? (size_t)K : (size_t)K / 2;
     const int nb = K / 32;
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
@@ -355,7 +366,7 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
     const float *second = fuse.x2 ? fuse.x2 : fuse.res_in;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-        const int k = ((c * WPS + wis) * WAVE + lane) * KPL;
+        const int k = ((c * WPS + wis) * L + ul) * KPL;
 #pragma unroll
         for (int j = 0; j < XV; j++) {
             xr[c][j] = k < K ? *reinterpret_cast<const f32x4 *>(x + k + 4 * j) : zero4;
@@ -365,11 +376,11 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
     }
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-        const int k = ((c * WPS + wis) * WAVE + lane) * KPL;
+        const int k = ((c * WPS + wis) * L + ul) * KPL;
         const int kc = k < K ? k : 0;  // units past the row end re-read its first one against activations of zero
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const int row = min(row0 + r, N - 1);  // rows past the end re-read the last one
+            const int row = min(row0 + r * (WAVE / L) + sub, N - 1);  // rows past the end re-read the last one
             if constexpr (RAW) {
                 const uint8_t *blk = quants + ((size_t)row * nb + kc / 32) * PlaneTraits<QT>::BLOCK;
                 qw[c][r] = __builtin_nontemporal_load((global_u32x4_a2_ptr)(blk + 2 + (QT == 0 ? (kc & 16) : 0)));
@@ -393,7 +404,7 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
         } else if (fuse.res_in) {
 #pragma unroll
             for (int c = 0; c < NC; c++) {
-                const int k = ((c * WPS + wis) * WAVE + lane) * KPL;
+                const int k = ((c * WPS + wis) * L + ul) * KPL;
 #pragma unroll
                 for (int j = 0; j < XV; j++) {
                     xr[c][j] += ar[c][j];
@@ -431,7 +442,7 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
     for (int r = 0; r < R; r++) a[r] = 0.f;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-        const bool live = ((c * WPS + wis) * WAVE + lane) * KPL < K;
+        const bool live = ((c * WPS + wis) * L + ul) * KPL < K;
         float xv[KPL], sx = 0.f, sx_first = 0.f;
 #pragma unroll
         for (int j = 0; j < XV; j++)
@@ -452,7 +463,8 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
 #pragma unroll
         for (int r = 0; r < R; r++) {
             float d = f16_bits_to_f32((uint16_t)sc[c][r]);
-            if (RAW && !live) d = 0.f;  // (a unit past the row's end: an infinite scale times its zero activations would be NaN)
+            // a unit past the row's end (there is none but in the last chunk): an infinite scale times its zero activations would be NaN
+            if (RAW && c == NC - 1 && !live) d = 0.f;
             const uint32_t w[4] = {qw[c][r].x, qw[c][r].y, qw[c][r].z, qw[c][r].w};
             float t = 0.f;
             if (QT == 0) {
@@ -475,15 +487,16 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
         }
     }
 #pragma unroll
-    for (int r = 0; r < R; r++) a[r] = wave_sum(a[r]);
-    if (lane == 0) {
+    for (int r = 0; r < R; r++) a[r] = L == WAVE ? wave_sum(a[r]) : half_sum(a[r]);
+    if (ul == L - 1) {
 #pragma unroll
-        for (int r = 0; r < R; r++) part[wave][r] = a[r];
+        for (int r = 0; r < R; r++) part[wave][r * (WAVE / L) + sub] = a[r];
     }
     __syncthreads();
     const int t = threadIdx.x;
-    if (t < SETS * R) {
-        const int ts = t / R, tr = t % R, row = (blockIdx.x * SETS + ts) * R + tr;
+    static_assert(SETS * ROWS <= PTHREADS, "a thread a row");
+    if (t < SETS * ROWS) {
+        const int ts = t / ROWS, tr = t % ROWS, row = (blockIdx.x * SETS + ts) * ROWS + tr;
         if (row < N) {
             float v = part[ts * WPS][tr];
 #pragma unroll
@@ -1037,23 +1050,33 @@ int homura::gemv_planes_fused(hm_ctx *ctx, bool q4, const float *d_x, const uint
 
 // Rows a set: as many as leave seven hundred workgroups (every set re-reads the activation pieces), two at least. us with
 // 2 / 4 / 8 / 16: 1024 -> 6144 3.62 / 3.89 / 3.94 / 5.75, 2048 -> 5632 5.38 / 5.10 / 5.89 / 6.39, 768 -> 32000 10.94 / 9.87 /
-// 9.81 / 10.13, 4096 -> 32000 47.8 / 41.9 / 41.3 / 40.5; the kernel that stages blocks in LDS took 4.54, 6.74, 12.75 and
-// 53.4. (Q4_0 blocks are no faster this way: 2048 -> 5632 4.69 at best against 4.40.)
+// 9.81 / 10.13, 4096 -> 32000 47.8 / 41.9 / 41.3 / 40.5; with four wavefronts a row sixteen only from 19000 rows on (3584 ->
+// 18000 22.1 with eight, 23.3 with sixteen, 20000 24.1 and 23.7). Rows of up to 512: half a wavefront a row, one to four pairs
+// of rows (256 -> 10000 3.8 us, 4.8 with a whole one, 512 -> 32000 6.6 and 9.6). Many rows of 4353 .. 5120: a wavefront a row,
+// five chunks (4608 -> 32000 53.1, 59.4 with four wavefronts and two chunks).
+// The kernel that stages blocks in LDS took 4.54, 6.74, 12.75, 53.4; 22.7, 36.7; 4.5, 8.4; 57.2 (see staged_rows_pay). Q4_0
+// blocks are no faster this way: 2048 -> 5632 4.69 at best against 4.40.
 int homura::gemv_q8_0_blocks_cut(hm_ctx *ctx, const float *d_x, const uint8_t *d_blocks, float *d_out, int K, int N) {
     const int chunk_k = WAVE * 16, wps = K <= chunk_k ? 1 : (K <= 2 * chunk_k ? 2 : 4), nc = (K + wps * chunk_k - 1) / (wps * chunk_k);
     HM_REQUIRE(ctx, nc <= 2, "gemv_q8_0_blocks_cut: K=%d above 8192", K);
-    const int sets = PWAVES / wps;
+    const bool half = K <= 512, five = K > 4352 && K <= 5 * chunk_k && N >= 15000;
+    const int sets = five ? PWAVES : PWAVES / wps;
     int r = nc == 1 ? 16 : 8;
-    while (r > 2 && N / (r * sets) < 700) r /= 2;
-    const dim3 grid((unsigned)((N + r * sets - 1) / (r * sets)));
-#define HM_CUT(RR, CC, WW)                                                                                              \
-    hipLaunchKernelGGL((gemv_planes_splitk_kernel<0, RR, CC, 0, WW, true>), grid, dim3(PTHREADS), 0, ctx->stream, d_x,  \
-                       d_blocks, (const uint16_t *)nullptr, d_out, K, N, homura::QuantFuse())
+    while (r > 2 && (N / (r * sets) < 700 || (r == 16 && wps == 4 && N < 19000))) r /= 2;
+    if (half) r = N >= 20000 ? 4 : N >= 4000 ? 2 : 1;
+    if (five) r = 4;
+    const int rows = r * sets * (half ? 2 : 1);
+    const dim3 grid((unsigned)((N + rows - 1) / rows));
+#define HM_CUT(RR, CC, WW, ...)                                                                                         \
+    hipLaunchKernelGGL((gemv_planes_splitk_kernel<0, RR, CC, 0, WW, true, ##__VA_ARGS__>), grid, dim3(PTHREADS), 0,     \
+                       ctx->stream, d_x, d_blocks, (const uint16_t *)nullptr, d_out, K, N, homura::QuantFuse())
 #define HM_CUT_R(CC, WW)                                                                                                \
     do {                                                                                                                \
         if (r == 8) HM_CUT(8, CC, WW); else if (r == 4) HM_CUT(4, CC, WW); else HM_CUT(2, CC, WW);                      \
     } while (0)
-    if (nc == 2) HM_CUT_R(2, 4);
+    if (half) { if (r == 4) HM_CUT(4, 1, 1, 32); else if (r == 2) HM_CUT(2, 1, 1, 32); else HM_CUT(1, 1, 1, 32); }
+    else if (five) HM_CUT(4, 5, 1);
+    else if (nc == 2) HM_CUT_R(2, 4);
     else if (r == 16) { if (wps == 1) HM_CUT(16, 1, 1); else if (wps == 2) HM_CUT(16, 1, 2); else HM_CUT(16, 1, 4); }
     else if (wps == 1) HM_CUT_R(1, 1);
     else if (wps == 2) HM_CUT_R(1, 2);

@@ -132,9 +132,11 @@ def test_products_of_few_rows(ctx, oracle, form, M, K, N):
 
 
 @pytest.mark.parametrize("K,N", [(32, 1), (32, 2801), (992, 5603), (1024, 11203), (1024, 45001), (1056, 1401), (2048, 22403), (2080, 703),
-                                 (4096, 11201), (4128, 701), (7680, 5601)])
+                                 (4096, 11201), (4128, 701), (7680, 5601), (64, 3999), (480, 4003), (512, 20001), (1152, 60000), (1536, 60001),
+                                 (2432, 16500), (2560, 16501), (3264, 60000), (3584, 60001), (4384, 15000), (5120, 15001)])
 def test_q8_0_rows_straight_from_blocks(ctx, oracle, K, N):
-    """One, two and four wavefronts a row, one and two chunks each, every number of rows a set, rows and units past the end.
+    """Half a, one, two and four wavefronts a row, one, two and five chunks each, every number of rows a set, rows and units past the
+    end; and the sizes from which rows go through LDS.
     A block's sum is 32 f32 additions of exact integers times activations, the blocks' sums as many again as there are."""
     raw = synth.q8_0_blocks(51, N * K // 32, 0.01)
     x = synth.normal_f32(52, 2 * K).reshape(2, K)
