@@ -438,10 +438,18 @@ int gemv_quant_launch(hm_ctx *ctx, const char *name, const float *d_x, const uin
     HM_REQUIRE(ctx, ((uintptr_t)fuse.x2 % 16) == 0 && ((uintptr_t)fuse.res_in % 16) == 0 && ((uintptr_t)fuse.resid_out % 16) == 0 &&
                         ((uintptr_t)fuse.norm_w % 16) == 0, "%s: fused operands must be 16-byte aligned", name);
     HM_REQUIRE(ctx, M == 1 || (!fuse.x2 && !fuse.res_in && !fuse.norm_w && !fuse.res_out_add), "%s: fused light ops need M == 1", name);
+    const bool fused = fuse.x2 || fuse.res_in || fuse.norm_w || fuse.res_out_add || fuse.cand_v;
+    if (QT == 0 && !fused && K <= 8192 && !staged_rows_pay(K, N)) {  // straight from the blocks into registers (2048 -> 5632 6.74 -> 5.10 us)
+        int rc = HM_OK;
+        for (int m = 0; m < M && rc == HM_OK; m++)
+            rc = homura::gemv_q8_0_blocks_cut(ctx, d_x + (size_t)m * K, d_w, d_out + (size_t)m * N, K, N);
+        return rc;
+    }
     const size_t rowbytes = (size_t)(K / 32) * BB;
     const size_t x_bytes = (size_t)K * 4;
     if (!(x_bytes + QWAVES * rowbytes + 32 <= 64 * 1024 && QWAVES * rowbytes + 32 <= (size_t)STAGE_BYTES)) {
-        // Rows too long for the LDS stage (above about 7700 for Q8_0, 14500 for Q4_0): the blocks are re-packed
+        // Rows too long for the LDS stage (above about 7700 for Q8_0 with light ops around the product, 14500 for Q4_0) or,
+        // plain Q8_0, for the registers of gemv_q8_0_blocks_cut (above 8192): the blocks are re-packed
         // into planes in the workspace and multiplied by the cut-row kernel, two launches a call. (A caller that
         // keeps its weights on the device packs them once and calls the planes entry points.)
         const size_t need = homura::quant_planes_bytes(QT == 1, N, K);
@@ -452,13 +460,6 @@ int gemv_quant_launch(hm_ctx *ctx, const char *name, const float *d_x, const uin
         int rc = homura::pack_quant_planes(ctx, QT == 1, d_w, planes, N, K);
         for (int m = 0; m < M && rc == HM_OK; m++)
             rc = homura::gemv_planes_fused(ctx, QT == 1, d_x + (size_t)m * K, planes, d_out + (size_t)m * N, K, N, fuse);
-        return rc;
-    }
-    const bool fused = fuse.x2 || fuse.res_in || fuse.norm_w || fuse.res_out_add || fuse.cand_v;
-    if (QT == 0 && !fused && !staged_rows_pay(K, N)) {  // straight from the blocks into registers (2048 -> 5632 6.74 -> 5.10 us)
-        int rc = HM_OK;
-        for (int m = 0; m < M && rc == HM_OK; m++)
-            rc = homura::gemv_q8_0_blocks_cut(ctx, d_x + (size_t)m * K, d_w, d_out + (size_t)m * N, K, N);
         return rc;
     }
     const QuantShape sh = quant_shape<QT>(ctx, K, N);
