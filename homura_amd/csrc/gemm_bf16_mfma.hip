@@ -682,7 +682,7 @@ int homura::gemm_split_nk(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, co
     HM_REQUIRE(ctx, pieces >= 1 && pieces <= 3, "gemm_split_nk: %d pieces (1..3)", pieces);
     if (pieces >= 2)  // every tile once, all piece products per stage
         return gemm_pieces_nk(ctx, d_a_split, pieces, d_b_nk, 1, d_c, M, K, N, max_parts, parts);
-    if (M > 0 && N > 0 && few_rows_pays(M, N, ctx->num_cus)) return gemm_few_rows(ctx, d_a_split, 1, d_b_nk, nullptr, 0, d_c, M, K, N, max_parts, parts, N);
+    if (M > 0 && N > 0 && few_rows_pays(1, M, N, ctx->num_cus)) return gemm_few_rows(ctx, d_a_split, 1, d_b_nk, nullptr, 0, d_c, M, K, N, max_parts, parts, N);
     // K slices while they still add whole waves of workgroups to a grid smaller than the chip (the
     // slices cost a write and a read of C each), at least 4 K tiles per slice
     const long long tiles = (long long)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
@@ -713,7 +713,7 @@ extern "C" int hm_gemm_bf16_nk(hm_ctx *ctx, const uint16_t *d_a_mk, const uint16
                                int M, int K, int N) {
     HM_CHECK_CTX(ctx);
     const bool vectors = ((uintptr_t)d_a_mk | (uintptr_t)d_b_nk) % 16 == 0 && K > 0 && K % 32 == 0;
-    if (d_a_mk && d_b_nk && d_c && vectors && M > 0 && N > 0 && homura::few_rows_pays(M, N, ctx->num_cus))
+    if (d_a_mk && d_b_nk && d_c && vectors && M > 0 && N > 0 && homura::few_rows_pays(1, M, N, ctx->num_cus))
         return homura::gemm_few_rows(ctx, d_a_mk, 1, d_b_nk, nullptr, 0, d_c, M, K, N, 1, nullptr, N);
     return gemm_launch(ctx, "hm_gemm_bf16_nk", d_a_mk, d_b_nk, d_c, M, K, N, true);
 }

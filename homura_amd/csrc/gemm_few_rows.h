@@ -13,11 +13,16 @@ constexpr int FEW_ROWS = 64;
 // (24 rows: 1024 -> 4096 5.4 us with one and 6.2 with two, 1024 -> 6144 7.3 and 6.5)
 inline int few_rows_tiles(int N, int cus) { return (N + 31) / 32 * 4 > 3 * (long long)cus ? 2 : 1; }
 
-// Whether a product goes this way: always up to 32 rows, up to 64 while its workgroups are one round (64 rows, 1536 -> 17920:
-// 40 us in two rounds, 32 in 128-row tiles)
-inline bool few_rows_pays(int M, int N, int cus) {
+// Whether a product goes this way: up to 64 rows while its workgroups are one round (64 rows, 1536 -> 17920: 40 us in two
+// rounds, 32 in 128-row tiles); more rounds with up to 32 rows, always with two or three pieces and with one where the last
+// round is nearly full. Weights cold, 24 rows, us here / in 128-row tiles, three pieces: 1536 -> 17920 26.7 / 34.3, 1024 ->
+// 65536 41.2 / 56.1, 1536 -> 151936 132 / 191, 3072 -> 24576 46.7 / 65.4; one piece: 1536 -> 17920 (1.1 rounds) 17.8 / 17.5,
+// 3072 -> 24576 (1.5) 34.2 / 33.0, 2048 -> 32000 (1.95) 30.9 / 34.4, 1024 -> 65536 (4) 30.9 / 36.4, 1536 -> 151936 (9.3) 104 / 104.
+inline bool few_rows_pays(int pieces, int M, int N, int cus) {
     const int nt = few_rows_tiles(N, cus);
-    return M <= 32 || (M <= FEW_ROWS && (N + 32 * nt - 1) / (32 * nt) <= cus);
+    const long long wgs = (N + 32 * nt - 1) / (32 * nt), rounds = (wgs + cus - 1) / cus;
+    if (rounds <= 1) return M <= FEW_ROWS;
+    return M <= 32 && (pieces > 1 || 10 * wgs >= 9 * rounds * cus);
 }
 
 // K slices of such a product, at most max_parts: while the workgroups still fit the chip at once, a group for every wavefront

@@ -381,7 +381,7 @@ Cut cut_for(long long m_tiles, int N, int ns, long long out_bytes, int cus, int 
 }  // namespace
 
 int homura::gemm_pieces_slices(int b_pieces, bool scaled, int M, int K, int N, int cus, int max_parts) {
-    if (b_pieces == 1 && few_rows_pays(M, N, cus)) return few_rows_slices(M, K, N, cus, max_parts);
+    if (b_pieces == 1 && few_rows_pays(3, M, N, cus)) return few_rows_slices(M, K, N, cus, max_parts);
     return cut_for((M + TM - 1) / TM, N, K / TK, 4LL * M * N, cus, max_parts, b_pieces == 1 && !scaled).slices;
 }
 
@@ -468,7 +468,7 @@ int homura::gemm_pieces_any(hm_ctx *ctx, const uint16_t *d_a_split, int a_pieces
     HM_REQUIRE(ctx, ((uintptr_t)d_a_split % 16) == 0 && ((uintptr_t)d_b_split % 16) == 0, "%s: operands must be 16-byte aligned", who);
     HM_REQUIRE(ctx, (long long)((M + TM - 1) / TM) * ((N + TN - 1) / TN) <= 0x7fffff00LL, "%s: too many tiles", who);
     HM_REQUIRE(ctx, ldc <= 0 || ldc >= N, "%s: ldc %d below N %d", who, ldc, N);
-    if (b_pieces == 1 && few_rows_pays(M, N, ctx->num_cus))
+    if (b_pieces == 1 && few_rows_pays(a_pieces, M, N, ctx->num_cus))
         return gemm_few_rows(ctx, d_a_split, a_pieces, d_b_split, d_scales, npad, d_c, M, K, N, max_parts, parts, ldc > 0 ? ldc : N);
     PieceDims g{};
     g.M = M;
