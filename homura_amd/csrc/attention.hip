@@ -529,64 +529,75 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_stream_kernel(
 // Second half of the split attention: one workgroup per (batch, query head) folds that head's partial
 // (o, max, sum) triples. A separate launch instead of a "last workgroup to arrive" fold: the kernel boundary
 // orders the partial writes, so no device-scope fence (a full L2 write-back + invalidate on this chip) is needed.
-// The workgroup is SG groups of HD threads (thread = output element d of group sg). Group sg takes splits sg,
-// sg + SG, ... in ascending order against the maximum of its own splits, up to 32 loads a thread in flight; the
-// groups' (max, sum, o) then meet in LDS and are merged in group order. One group (grids of at most 32 splits) is the
-// plain ascending fold; a grid of hundreds of splits (tens of thousands of cached rows) folded by one group took
-// 57 us, longer than the attention itself.
 constexpr int FOLD_BATCH = 32;      // splits fetched per batch, all loads of a batch in flight together
-constexpr int FOLD_THREADS = 1024;  // of a workgroup with groups
+constexpr int FOLD_THREADS = 1024;  // of a workgroup with groups (one of 1024 threads costs about 2 us more to start than one of 64 or 128)
 
-// GROUPS false: one group of HD threads (grids of at most FOLD_BATCH splits: a workgroup of 1024 threads costs about
-// 2 us more to start than one of 64 or 128). GROUPS true: FOLD_THREADS / HD groups; with few splits live (a grid
-// sized for a long cache with few rows in it yet) one group folds and the others leave at once.
-template <int HD, int G, bool GROUPS>
-__global__ __launch_bounds__(GROUPS ? FOLD_THREADS : HD) void gqa_decode_fold_kernel(
+// Grids of at most FOLD_BATCH splits: thread = output element. Lane s of every wavefront holds split s's (max, sum), one
+// exponential a lane gives every weight, the weights are added up across the lanes and read from them in turn. (Each thread
+// walked the pairs through LDS with an exponential a split before: 8 sequences x 12 heads, 16 splits, 14.0 -> 12.5 us for both
+// launches; 32 steps of Qwen2.5-1.5B behind 700 rows 45.5 -> 44.4 ms.)
+template <int HD, int G>
+__global__ __launch_bounds__(HD) void gqa_decode_fold_kernel(float *__restrict__ out, const float *__restrict__ part_o,
+                                                             const float *__restrict__ part_ml, int kvh, int kv_len_arg, int chunk,
+                                                             const DecodeState *__restrict__ state) {
+    static_assert(HD % WAVE == 0, "wave_max and wave_sum want whole wavefronts");
+    static_assert(FOLD_BATCH <= WAVE && FOLD_BATCH % 8 == 0, "a split a lane, eight requested at a time");
+    const int d = threadIdx.x, lane = threadIdx.x & (WAVE - 1);
+    const int gi = blockIdx.x % G, kvhd = blockIdx.x / G, b = blockIdx.y;
+    const int H = kvh * G;
+    const int kv_len = state ? state->pos + 1 : kv_len_arg;
+    const int nsplit = (kv_len + chunk - 1) / chunk;
+    if (nsplit == 1) return;  // the attention kernel wrote the final result itself
+    const size_t pair = (size_t)b * kvh + kvhd;
+    const float *ao = part_o + (pair * nsplit * G + gi) * HD + d;
+    const float *aml = part_ml + (pair * nsplit * G + gi) * 2;
+    float o[FOLD_BATCH];
+    const float m = lane < nsplit ? aml[(size_t)lane * G * 2] : -INFINITY, l = lane < nsplit ? aml[(size_t)lane * G * 2 + 1] : 0.f;
+#pragma unroll
+    for (int u0 = 0; u0 < FOLD_BATCH; u0 += 8)
+        if (u0 < nsplit) {
+#pragma unroll
+            for (int u = u0; u < u0 + 8; u++) o[u] = ao[(size_t)min(u, nsplit - 1) * G * HD];
+        }
+    const float M = wave_max(m);
+    const float w = lane < nsplit ? expf(m - M) : 0.f;
+    const float L = wave_sum(w * l);
+    float O = 0.f;
+#pragma unroll
+    for (int u0 = 0; u0 < FOLD_BATCH; u0 += 8)
+        if (u0 < nsplit) {
+#pragma unroll
+            for (int u = u0; u < u0 + 8; u++)  // (past the last split: not its sum again, 0 times infinity is NaN)
+                O = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u)), u < nsplit ? o[u] : 0.f, O);
+        }
+    out[((size_t)b * H + kvhd * G + gi) * HD + d] = O / L;
+}
+
+// Larger grids: the workgroup is SG groups of HD threads (thread = output element d of group sg). Group sg takes splits sg,
+// sg + SG, ... in ascending order against the maximum of its own splits, up to FOLD_BATCH loads a thread in flight; the
+// groups' (max, sum, o) then meet in LDS and are merged in group order (a grid of hundreds of splits, tens of thousands of
+// cached rows, folded by one group took 57 us, longer than the attention itself). With few splits live (a grid sized for a
+// long cache with few rows in it yet) one group folds and the others leave at once.
+template <int HD, int G>
+__global__ __launch_bounds__(FOLD_THREADS) void gqa_decode_fold_groups_kernel(
     float *__restrict__ out, const float *__restrict__ part_o, const float *__restrict__ part_ml,
     int kvh, int kv_len_arg, int chunk, const DecodeState *__restrict__ state) {
-    constexpr int SGMAX = GROUPS ? FOLD_THREADS / HD : 1;
+    constexpr int SGMAX = FOLD_THREADS / HD;
     extern __shared__ float s_fold[];  // [SGMAX][HD + 2] group results, then [nsplit][2] (max, sum) of this head
-    const int d = GROUPS ? threadIdx.x % HD : threadIdx.x, sg = GROUPS ? threadIdx.x / HD : 0;
+    const int d = threadIdx.x % HD, sg = threadIdx.x / HD;
     float *s_grp = s_fold, *s_ml = s_fold + SGMAX * (HD + 2);
     const int gi = blockIdx.x % G, kvhd = blockIdx.x / G, b = blockIdx.y;
     const int H = kvh * G;
     const int kv_len = state ? state->pos + 1 : kv_len_arg;
     const int nsplit = (kv_len + chunk - 1) / chunk;
     if (nsplit == 1) return;  // the attention kernel wrote the final result itself
-    const int SG = GROUPS && nsplit > FOLD_BATCH / 2 ? SGMAX : 1;
+    const int SG = nsplit > FOLD_BATCH / 2 ? SGMAX : 1;
     if (sg >= SG) return;
     const size_t pair = (size_t)b * kvh + kvhd;
     const float *ao = part_o + (pair * nsplit * G + gi) * HD + d;
     const float *aml = part_ml + (pair * nsplit * G + gi) * 2;
     constexpr int FB = FOLD_BATCH;
     float o[FB];
-    if constexpr (!GROUPS) {
-        // At most 32 splits: lane s holds split s's (max, sum), one exponential a lane gives every weight, and the weights are
-        // read across lanes. (Each thread walked the pairs through LDS
-        // with an exponential a split before: 8 sequences x 12 heads, 16 splits, 14.0 -> 12.5 us for both launches; 32 steps of
-        // Qwen2.5-1.5B behind 700 rows 45.5 -> 44.4 ms.)
-        const int lane = threadIdx.x & (WAVE - 1);
-        const float m = lane < nsplit ? aml[(size_t)lane * G * 2] : -INFINITY, l = lane < nsplit ? aml[(size_t)lane * G * 2 + 1] : 0.f;
-#pragma unroll
-        for (int u0 = 0; u0 < FB; u0 += 8)
-            if (u0 < nsplit) {
-#pragma unroll
-                for (int u = u0; u < u0 + 8; u++) o[u] = ao[(size_t)min(u, nsplit - 1) * G * HD];
-            }
-        const float M = wave_max(m);
-        const float w = lane < nsplit ? expf(m - M) : 0.f;
-        const float L = wave_sum(w * l);
-        float O = 0.f;
-#pragma unroll
-        for (int u0 = 0; u0 < FB; u0 += 8)
-            if (u0 < nsplit) {
-#pragma unroll
-                for (int u = u0; u < u0 + 8; u++)  // (past the last split: not its sum again, 0 times infinity is NaN)
-                    O = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), u)), u < nsplit ? o[u] : 0.f, O);
-            }
-        out[((size_t)b * H + kvhd * G + gi) * HD + d] = O / L;
-        return;
-    }
 #pragma unroll
     for (int u = 0; u < FB; u++) {
         const int sp = sg + u * SG;
@@ -645,14 +656,13 @@ template <int HD, int G>
 int launch_fold(hm_ctx *ctx, const AttnArgs &a, const float *part_o, const float *part_ml, int nsplit, int chunk,
                 const DecodeState *state) {
     const bool groups = nsplit > FOLD_BATCH;
-    const int sg = groups ? FOLD_THREADS / HD : 0;
-    const size_t fold_lds = groups ? ((size_t)sg * (HD + 2) + (size_t)nsplit * 2) * sizeof(float) : 0;
+    const size_t fold_lds = groups ? ((size_t)(FOLD_THREADS / HD) * (HD + 2) + (size_t)nsplit * 2) * sizeof(float) : 0;
     HM_REQUIRE(ctx, fold_lds <= 64 * 1024, "gqa_decode_attn: too many splits (%d)", nsplit);
     if (groups)
-        hipLaunchKernelGGL((gqa_decode_fold_kernel<HD, G, true>), dim3(a.kvh * G, a.B), dim3(FOLD_THREADS), fold_lds,
+        hipLaunchKernelGGL((gqa_decode_fold_groups_kernel<HD, G>), dim3(a.kvh * G, a.B), dim3(FOLD_THREADS), fold_lds,
                            ctx->stream, a.out, part_o, part_ml, a.kvh, a.kv_len, chunk, state);
     else
-        hipLaunchKernelGGL((gqa_decode_fold_kernel<HD, G, false>), dim3(a.kvh * G, a.B), dim3(HD), fold_lds, ctx->stream,
+        hipLaunchKernelGGL((gqa_decode_fold_kernel<HD, G>), dim3(a.kvh * G, a.B), dim3(HD), 0, ctx->stream,
                            a.out, part_o, part_ml, a.kvh, a.kv_len, chunk, state);
     HM_LAUNCH_CHECK(ctx);
     return HM_OK;
