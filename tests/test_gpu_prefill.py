@@ -84,8 +84,7 @@ def test_run_kv_and_generate_route_long_inputs_through_prefill(ctx):
 
 
 def test_prefill_in_chunks_and_cache_limits(ctx):
-    """600 tokens in one call = a chunk of 512 and one of 88; the second attends to the first through
-    the cache. Then 60 more on top."""
+    """600 tokens in one call, 60 more that attend to them through the cache, and a prompt that does not fit."""
     import dataclasses
     cfg = dataclasses.replace(synth_model.TINY, max_position_embeddings=1024)
     weights = synth_model.synth_weights(cfg, 5)
@@ -106,6 +105,33 @@ def test_prefill_in_chunks_and_cache_limits(ctx):
     assert gm.kv_cache_len() == 660 and logit_err(got2, want2) < TOL
     with pytest.raises(HomuraError):
         gm.prefill([cfg.vocab_size], want_logits=False)   # id outside the vocabulary
+    gm.close()
+
+
+@pytest.mark.parametrize("which", ["bf16", "q8_0", "q4_k"])
+def test_prompt_over_two_chunks(ctx, which):
+    """4160 tokens in one call = a chunk of 4096 and one of 64, with the logits of every row: the second chunk attends to the first
+    through the cache. K-quants against the oracle with the GPU's own rounding decisions (see the test of the quantised pass)."""
+    import dataclasses
+    n = 4160
+    cfg = {"bf16": synth_model.TINY, "q8_0": synth_model.TINY_LLAMA, "q4_k": synth_model.TINY_K}[which]
+    cfg = dataclasses.replace(cfg, max_position_embeddings=n + 16, num_hidden_layers=2)
+    kw = {} if which == "bf16" else dict(has_qk_norm=False, proj_dtypes=[{"q8_0": 2, "q4_k": 5}[which]] * 14)
+    weights = synth_model.synth_weights(cfg, 77, **kw)
+    gm = synth_model.build_model(ctx, cfg, weights, n + 16, **kw)
+    om = mf.build_oracle_model(cfg, weights, n + 16, **kw)
+    ids = synth.token_ids(12, n, cfg.vocab_size)
+    if which == "q4_k":
+        gm.prefill_capture_q8k_inputs(n)
+    got = gm.prefill(ids)
+    assert gm.kv_cache_len() == n
+    if which == "q4_k":
+        om.set_q8k_inputs(gm.prefill_captured_q8k_inputs(), n, 0)
+        gm.prefill_capture_q8k_inputs(0)
+    want = om.run_kv(ids) if which == "bf16" else np.concatenate([om.run_kv(ids[i:i + 1]) for i in range(n)])
+    errs = [logit_err(got[i], want[i]) for i in range(n)]
+    say(f"{which}: worst rel err {max(errs):.1e}, rows 4095, 4096, 4097 {[f'{errs[i]:.1e}' for i in (4095, 4096, 4097)]}")
+    assert max(errs) < (2e-5 if which == "q4_k" else TOL)
     gm.close()
 
 

@@ -29,7 +29,7 @@ def test_wide_tiles_of_the_piece_product(ctx, M, K, N):
 
 
 def test_prompt_longer_than_a_chunk(ctx):
-    """4097 and 4400 tokens go through the layers in two even chunks. The rows they leave in the cache give the logits that
+    """4097 and 4400 tokens go through the layers in a chunk of 4096 and a rest. The rows they leave in the cache give the logits that
     the same tokens in portions of other sizes give, up to the cache rows that round to bf16 the other way (one ulp, 0.4 %,
     of single elements under softmax weights of 1 / 4000 a row)."""
     cfg = dataclasses.replace(synth_model.TINY, max_position_embeddings=4500)
@@ -53,11 +53,32 @@ def test_prompt_longer_than_a_chunk(ctx):
     m.close()
 
 
+@pytest.mark.parametrize("M,K,N", [(130, 192, 264), (37, 448, 8), (200, 320, 136), (129, 256, 120), (65, 576, 392), (257, 704, 1032), (64, 1216, 72)])
+def test_kn_products_between_whole_rounds(ctx, M, K, N):
+    """[K, N] weights: none to three K tiles of 64 behind whole rounds of four, with and without a round ahead of them, columns
+    that end inside a tile. Bound as above."""
+    guard = 512
+    a, b = synth.normal_bf16(61, M * K, 1.0).reshape(M, K), synth.normal_bf16(62, K * N, 0.02).reshape(K, N)
+    da, db, dc = ctx.to_device(a), ctx.to_device(b), ctx.to_device(np.full(M * N + guard, -77.0, np.float32))
+    ctx.gemm_bf16(da, db, dc, M, K, N)
+    got = dc.download(np.float32, (M * N + guard,))
+    assert np.all(got[M * N:] == -77.0), "wrote past the end of C"
+    a64, b64 = synth.bf16_to_f32(a).astype(np.float64), synth.bf16_to_f32(b).astype(np.float64)
+    assert np.all(np.abs(got[:M * N].reshape(M, N) - a64 @ b64) <= 3 * K * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64)))
+    for buf in (da, db, dc):
+        buf.free()
+
+
+@pytest.mark.parametrize("groups", [None, 1, 2, 4])
 @pytest.mark.parametrize("S,past,H,kvh,hd", [(640, 0, 12, 2, 128), (1000, 37, 16, 8, 128), (2111, 0, 14, 2, 64),
-                                             (130, 65, 32, 4, 64), (4096, 0, 8, 8, 64)])
-def test_prompt_attention_over_key_groups(ctx, S, past, H, kvh, hd):
-    """Every number of key groups, heads in eighths and not, ragged row blocks. Keys and values are bf16, queries and
+                                             (130, 65, 32, 4, 64), (4096, 0, 8, 8, 64), (4096, 0, 16, 8, 128), (4000, 0, 14, 2, 64)])
+def test_prompt_attention_over_key_groups(ctx, monkeypatch, S, past, H, kvh, hd, groups):
+    """The chosen number of key groups and each of them, heads in eighths and not, ragged row blocks, more than one round of
+    workgroups with each. Keys and values are bf16, queries and
     probabilities carried whole, sums f32: 2^-20 of the largest value, over a few thousand additions, holds it."""
+    monkeypatch.delenv("HOMURA_PREFILL_KEY_GROUPS", raising=False)
+    if groups:
+        monkeypatch.setenv("HOMURA_PREFILL_KEY_GROUPS", str(groups))
     rng = np.random.default_rng(S)
     L = past + S
     q = rng.standard_normal((S, H, hd)).astype(np.float32)
