@@ -107,6 +107,8 @@ struct PrefillAttnArgs {
     const float *gate = nullptr;
     int gate_ld = 0, gate_parts = 1;
     size_t gate_stride = 0;
+    // set by prefill_attn_launch: the grid is heads x row blocks instead of row blocks x heads (a grid's y ends at 65535)
+    int heads_x = 0;
     // set by prefill_attn_launch when few query rows face a long cache: the keys are cut over gridDim.z
     // workgroups, which leave their (O, max, sum) here for a second kernel to join
     float *part_o = nullptr, *part_ml = nullptr;

@@ -17,6 +17,7 @@
 #include "row_pieces.h"
 
 #include <algorithm>
+#include <utility>
 #include <cstdlib>
 
 #include "gemm_bf16_mfma.h"
@@ -342,15 +343,18 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
     // Workgroups are dealt to the eight dies round-robin by their linear index. With a multiple of eight heads
     // every die gets H / 8 neighbouring heads and all their row blocks, so the K and V rows of a KV head are
     // fetched into one die's L2 (or as few as the head grouping allows) instead of all eight.
-    // Otherwise all heads of a row block follow one another. Either way the row blocks come in order: within a die
+    // Otherwise all heads of a row block follow one another (heads along x). Either way the row blocks come in order: within a die
     // workgroups are dealt to its engines round-robin and wait in line for their engine, so an order in which an engine
     // always gets the long ones would make the others wait (2000 rows, 12 heads, head by head: 89.8 us with two key groups; this way 49.8).
-    const int lin = blockIdx.y * gridDim.x + blockIdx.x, per = a.H / 8;
-    const bool by_die = a.H % 8 == 0;
-    const int hx = by_die ? (lin & 7) * per + (lin >> 3) % per : lin % a.H;
-    int bx = by_die ? (lin >> 3) / per : lin / a.H;
+    const int gx = blockIdx.x, gy = blockIdx.y, blocks = a.heads_x ? (int)gridDim.y : (int)gridDim.x;
+    int hx = a.heads_x ? gx : gy, bx = a.heads_x ? gy : gx;
+    if (a.H % 8 == 0) {
+        const int lin = gy * (int)gridDim.x + gx, per = a.H / 8;
+        hx = (lin & 7) * per + (lin >> 3) % per;
+        bx = (lin >> 3) / per;
+    }
     const int h = hx, kvhd = h / (a.H / a.kvh);
-    bx = (int)gridDim.x - 1 - bx;  // the row blocks that see the most keys first: the light ones fill the last round
+    bx = blocks - 1 - bx;  // the row blocks that see the most keys first: the light ones fill the last round
     const int q0 = bx * AT_QROWS;
     const int kv_total = a.past + a.S;
     const uint16_t *kc = a.kcache + (size_t)kvhd * a.max_len * DK;
@@ -752,7 +756,10 @@ int qkv_post_launch(hm_ctx *ctx, const QkvPostArgs &a) {
 // rows takes 5000 and 40, 21.5 or 12.8 a key it walks (1, 2, 4 groups; two tiles a wavefront and round with 1 and 2); the
 // grid is over with its longest workgroup or when the CUs have done their share, whichever is later. Measured, 16 heads of
 // 128, us with 1 / 2 / 4 groups: 512 rows 23.3 / 17.0 / 13.4; 1000 36.1 / 28.0 / 28.0; 3072 131.7 / 127.0 / 151.7; 2944 behind
-// 3072 315.5 / 283.8 / 337.4; 4096 190.5 / 193.9 / 240.9.
+// 3072 315.5 / 283.8 / 337.4; 4096 190.5 / 193.9 / 240.9. Other shapes share the constants, which then miss the best of the
+// three by up to a fifth (chosen first): 14 heads of 64, 1000 rows 17.5 (2) and 15.9 (4), 4096 rows 110 (1) and 92.6 (2);
+// 9 heads of 64, 3072 rows 49.0 (2) and 43.7 (4); 32 heads of 128, 512 rows behind 2000 65.6 (4) and 58.2 (2). Against the
+// fewest groups that give every CU a workgroup, which this replaced, none of 171 shapes is slower by more than the runs differ.
 static int key_groups_for(const PrefillAttnArgs &a, int cus) {
     int best = 1;
     double least = 1e30;
@@ -821,6 +828,8 @@ int prefill_attn_launch(hm_ctx *ctx, const PrefillAttnArgs &args) {
     const int sets = a.hd == 256 && a.kv_pieces == 3 ? 1 : 2;
     const int qrows = 128 / ks;
     dim3 grid((unsigned)((a.S + qrows - 1) / qrows), (unsigned)a.H);
+    a.heads_x = a.H % 8 != 0 && grid.x <= 65535;
+    if (a.heads_x) std::swap(grid.x, grid.y);
     // Few query rows in front of a long cache (a chat turn behind a long conversation) leave most CUs without a
     // workgroup while each workgroup walks every key: the keys are then cut over nz workgroups, eight rounds of
     // tiles each at least, which leave their (O, max, sum) in the workspace for a second kernel to join.
