@@ -320,7 +320,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_bf16_mfma_kernel(const uint
 // ---- K tiles aligned: global -> LDS loads without the trip through registers, B [N][K] or [K][N] ----
 //
 // A [K][N] operand took 4 x 8 blocks through registers and byte permutes into LDS before; its tiles now lie in LDS as they
-// are in memory and the transposing LDS read hands out the operands (512 x 2048 x 8192 35.8 -> 28.6 us, 2048 x 1024 x 4096
+// are in memory and the transposing LDS read hands out the operands (weights cold, 512 x 2048 x 8192 35.8 -> 28.6 us, 2048 x 1024 x 4096
 // 39.6 -> 30, 2048 x 2048 x 1024 26.9 -> 18.0; B [N][K]: 24.8, 29.8, 18.0).
 //
 // global_load_lds_dwordx4 writes lane l's 16 bytes to LDS at (wave-uniform base) + 16 l, so one

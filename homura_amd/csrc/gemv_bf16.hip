@@ -615,8 +615,11 @@ bool try_splitk(hm_ctx *ctx, const GemvArgs &a, int epi, int *rc) {
     // pieces itself (4 bytes per k, 12 with residual and norm weights, against 2 R of weights), so a prologue
     // wants more rows; few short rows want one.
     const size_t bytes = (size_t)2 * a.K * a.N;
+    // With a prologue, us with 4 / 8 rows over 24 gate|up shapes of K 512 .. 3072: 512 -> 12288 8.2 / 7.0, 512 -> 24576 12.9 / 10.7,
+    // 1024 -> 8192 6.8 / 6.9, 1024 -> 12288 9.3 / 8.4, 2048 -> 8192 9.2 / 8.6, 3072 -> 8192 13.0 / 11.4, 3072 -> 24576 32.4 / 27.4;
+    // 16 rows gain nothing more (32 steps of Qwen2.5-1.5B, 1536 -> 17920: 40.8 ms with 4, 40.1 with 8, 40.7 with 16).
     int r;
-    if (pro) r = a.N >= 8192 ? 8 : 4;  // (Qwen2.5-1.5B with 4 rows for its 1536 -> 17920: 40.8 ms for 32 steps, with 8 40.1, with 16 40.7)
+    if (pro) r = a.N >= 8192 ? 8 : 4;
     else r = (a.K >= 4096 && a.N >= 2048) ? 4 : ((a.N <= 1536 && bytes < ((size_t)17 << 19)) ? 1 : 2);
     if (epi == GEMV_EPI_SILU_MUL_PAIRS && r == 1) r = 2;
 #define HM_SPLITK(RR, CC) \
