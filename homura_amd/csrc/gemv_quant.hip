@@ -416,11 +416,13 @@ QuantShape quant_shape(const hm_ctx *ctx, int K, int N) {
 // them at 1536, three eighths at 2560, an eighth at 3584), a row's quarters fill this kernel's rounds of lanes, and there are
 // so many rows that the stream counts and not its start. us here / there, weights cold: 1536 -> 65536 32.8 / 34.1, 1536 ->
 // 151936 68.4 / 75.3, 2432 -> 17000 17.2 / 19.0, 2560 -> 24000 21.6 / 24.6, 2560 -> 151936 111 / 137, 3584 -> 65536 68.1 / 70.0;
-// but 1536 -> 32000 19.4 / 18.5, 1504 -> 65536 33.6 / 32.7, 2560 -> 10000 13.4 / 12.0, 2304 -> 65536 63.5 / 58.4, 2688 -> 65536
+// (2560 and 2432 also where five workgroups a CU of the other kernel's eight rows do not hold them: 2560 -> 10000 12.9 / 11.7, 11008
+// 13.0 / 13.3, 12288 13.1 / 13.5, 14000 15.3 / 15.4, 15000 15.3 / 16.9, 2432 -> 11008 12.9 / 13.2, but 2496 -> 14000 15.6 / 15.3);
+// but 1536 -> 32000 19.4 / 18.5, 1504 -> 65536 33.6 / 32.7, 2304 -> 65536 63.5 / 58.4, 2688 -> 65536
 // 64 / 61, 3072 -> 65536 73.3 / 65.0, 3552 -> 65536 67.7 / 67.1.
 bool staged_rows_pay(int K, int N) {
     if (K <= 1536) return K > 1088 && K % 64 == 0 && N >= 60000;
-    if (K <= 2560) return K >= 2432 && N >= 16500;
+    if (K <= 2560) return K >= 2432 && N >= (K % 128 ? 16500 : 10241);
     return K >= 3264 && K <= 3584 && K % 64 == 0 && N >= 60000;
 }
 

@@ -1052,14 +1052,14 @@ int homura::gemv_planes_fused(hm_ctx *ctx, bool q4, const float *d_x, const uint
 // 2 / 4 / 8 / 16: 1024 -> 6144 3.62 / 3.89 / 3.94 / 5.75, 2048 -> 5632 5.38 / 5.10 / 5.89 / 6.39, 768 -> 32000 10.94 / 9.87 /
 // 9.81 / 10.13, 4096 -> 32000 47.8 / 41.9 / 41.3 / 40.5; with four wavefronts a row sixteen only from 19000 rows on (3584 ->
 // 18000 22.1 with eight, 23.3 with sixteen, 20000 24.1 and 23.7). Rows of up to 512: half a wavefront a row, one to four pairs
-// of rows (256 -> 10000 3.8 us, 4.8 with a whole one, 512 -> 32000 6.6 and 9.6). Many rows of 4353 .. 5120: a wavefront a row,
-// five chunks (4608 -> 32000 53.1, 59.4 with four wavefronts and two chunks).
+// of rows (256 -> 10000 3.8 us, 4.8 with a whole one, 512 -> 32000 6.6 and 9.6). Many rows of 4097 .. 5120: a wavefront a row,
+// five chunks (4128 -> 32000 48.1, 50.1 with four wavefronts and two chunks; 4352 -> 16384 27.3 and 31.6, 4608 -> 32000 53.1 and 59.4).
 // The kernel that stages blocks in LDS took 4.54, 6.74, 12.75, 53.4; 22.7, 36.7; 4.5, 8.4; 57.2 (see staged_rows_pay). Q4_0
 // blocks are no faster this way: 2048 -> 5632 4.69 at best against 4.40.
 int homura::gemv_q8_0_blocks_cut(hm_ctx *ctx, const float *d_x, const uint8_t *d_blocks, float *d_out, int K, int N) {
     const int chunk_k = WAVE * 16, wps = K <= chunk_k ? 1 : (K <= 2 * chunk_k ? 2 : 4), nc = (K + wps * chunk_k - 1) / (wps * chunk_k);
     HM_REQUIRE(ctx, nc <= 2, "gemv_q8_0_blocks_cut: K=%d above 8192", K);
-    const bool half = K <= 512, five = K > 4352 && K <= 5 * chunk_k && N >= 15000;
+    const bool half = K <= 512, five = K > 4 * chunk_k && K <= 5 * chunk_k && N >= 15000;
     const int sets = five ? PWAVES : PWAVES / wps;
     int r = nc == 1 ? 16 : 8;
     while (r > 2 && (N / (r * sets) < 700 || (r == 16 && wps == 4 && N < 19000))) r /= 2;

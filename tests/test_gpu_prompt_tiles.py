@@ -155,7 +155,7 @@ def test_products_of_few_rows(ctx, oracle, form, M, K, N):
 
 @pytest.mark.parametrize("K,N", [(32, 1), (32, 2801), (992, 5603), (1024, 11203), (1024, 45001), (1056, 1401), (2048, 22403), (2080, 703),
                                  (4096, 11201), (4128, 701), (7680, 5601), (64, 3999), (480, 4003), (512, 20001), (1152, 60000), (1536, 60001),
-                                 (2432, 16500), (2560, 16501), (3264, 60000), (3584, 60001), (4384, 15000), (5120, 15001),
+                                 (2432, 16500), (2432, 10241), (2496, 10241), (2560, 10240), (2560, 16501), (3264, 60000), (3584, 60001), (4128, 15003), (4352, 14999), (4384, 15000), (5120, 15001),
                                  (7712, 1001), (8192, 5601), (8192, 8003)])
 def test_q8_0_rows_straight_from_blocks(ctx, oracle, K, N):
     """Half a, one, two and four wavefronts a row, one, two and five chunks each, every number of rows a set, rows and units past the
