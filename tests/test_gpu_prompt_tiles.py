@@ -203,7 +203,7 @@ def test_selective_scan_in_segments(ctx, n):
     """A chunk scanned in segments leaves the logits that the same tokens give one portion of at most 100 after the other
     (those are one segment each), on an empty state and behind one."""
     cfg = {"architecture": "Nokuvik", "vocab": 96, "width": 64, "embedding": {"scale": 1.0}, "norm": {"eps": 1e-5}, "loop": None,
-           "layers": [{"type": "mamba1", "mlp": None, "mixer": {"inner": 128, "conv": 4, "dt_rank": 8, "state": s}} for s in (16, 24, 40)]}
+           "layers": [{"type": "mamba1", "mlp": None, "mixer": {"inner": 128, "conv": 4, "dt_rank": 8, "state": s}} for s in (16, 24, 40, 100)]}
     m = synth_model.build_block_model(ctx, cfg, 3, 4096, DTYPE_F32)
     ids = synth.token_ids(n, n + 51, cfg["vocab"])
     for past in (0, 50):
