@@ -17,6 +17,7 @@
 #include "row_pieces.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 #include <cstdlib>
 
@@ -538,29 +539,42 @@ __global__ __launch_bounds__(A8_THREADS) void prefill_attn16_kernel(PrefillAttnA
         bf16x8 pp[TW][NP];
 #pragma unroll
         for (int u = 0; u < TW; u++) split8<NP>(f[u], pp[u]);
+        auto mix = [&](auto first, auto end) {  // with tiles first .. end - 1
 #pragma unroll
-        for (int u = 0; u < TW; u++) {
-            // a second tile that none of these 16 rows sees stays out: its weights are zero, but a value in it may be infinite
-            // (1905 rows of 16 heads of 128 behind 4096 219.8 -> 223.2 us, 4096 rows of 32 heads of 64 187 -> 183)
-            if (u > 0 && __builtin_expect((t + u) * A8_KEYS >= wave_end, 0)) break;
+            for (int u = decltype(first)::value; u < decltype(end)::value; u++)
 #pragma unroll
-            for (int db = 0; db < DB; db++) {
-                const int chunk = 2 * db + (v_sub >> 1), within = (v_sub & 1) * 8;
-                bf16x8 vf[KP];
+                for (int db = 0; db < DB; db++) {
+                    const int chunk = 2 * db + (v_sub >> 1), within = (v_sub & 1) * 8;
+                    bf16x8 vf[KP];
 #pragma unroll
-                for (int p = 0; p < KP; p++) {
-                    const char *vt = v_lds + u * PAIR + p * VTILE;
-                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (s16x4 __attribute__((address_space(3))) *)(vt + v_off<DV>(v_key, chunk) + within));
-                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (s16x4 __attribute__((address_space(3))) *)(vt + v_off<DV>(16 + v_key, chunk) + within));
-                    struct Pair { s16x4 lo, hi; } pr{lo, hi};
-                    vf[p] = __builtin_bit_cast(bf16x8, pr);
+                    for (int p = 0; p < KP; p++) {
+                        const char *vt = v_lds + u * PAIR + p * VTILE;
+                        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (s16x4 __attribute__((address_space(3))) *)(vt + v_off<DV>(v_key, chunk) + within));
+                        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (s16x4 __attribute__((address_space(3))) *)(vt + v_off<DV>(16 + v_key, chunk) + within));
+                        struct Pair { s16x4 lo, hi; } pr{lo, hi};
+                        vf[p] = __builtin_bit_cast(bf16x8, pr);
+                    }
+                    piece_products<NP, KP>([&](int p, int pv) {
+                        acc_o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[pv], pp[u][p], acc_o[db], 0, 0, 0);
+                    });
                 }
-                piece_products<NP, KP>([&](int p, int pv) {
-                    acc_o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[pv], pp[u][p], acc_o[db], 0, 0, 0);
-                });
-            }
+        };
+        // A second tile that none of these 16 rows sees stays out: its weights are zero, but a value in it may be infinite.
+        // Heads of 128 have both tiles in one block of code and the first alone in another, heads of 64 the second behind a
+        // branch: the one lets both tiles' reads and products overlap (1905 rows behind 4096, 16 heads of 128: 225 us behind a
+        // branch, 207 this way), the other keeps 128 registers and so two workgroups a CU (4096 rows, 32 heads of 64: 184, 217).
+        constexpr std::integral_constant<int, 0> zero;
+        constexpr std::integral_constant<int, 1> one;
+        constexpr std::integral_constant<int, TW> all;
+        const bool seen = TW == 1 || __builtin_expect((t + TW - 1) * A8_KEYS < wave_end, 1);
+        if constexpr (DV >= 128) {
+            if (seen) mix(zero, all);
+            else mix(zero, one);
+        } else {
+            mix(zero, one);
+            if (TW > 1 && seen) mix(one, all);
         }
     }
 
