@@ -68,6 +68,11 @@ int hm_test_prompt_product(int hm_dtype, int rows, int m, int k, int n, int cus,
 int hm_test_prompt_rows(hm_ctx *ctx, int front, const float *x, const float *norm_w, int dtype, const void *w, int half, int m, int k,
                         int n, float *out, float *row_factor, int *parts, int copies, int rounds, float *us);
 
+/* Test support: the tail of the prompt pass's q|k|v projection for S rows [S][(H + 2 kvh) * hd] at positions past ..: q rotated in
+ * place, k and v into caches [kvh][max_len][hd]. d_qw and d_kw [hd], or both NULL. hd 64 or 128. */
+int hm_test_qkv_tail(hm_ctx *ctx, float *d_qkv, const float *d_qw, const float *d_kw, const float *d_cos, const float *d_sin,
+                     uint16_t *d_kcache, uint16_t *d_vcache, int S, int H, int kvh, int hd, int max_len, int past, float eps);
+
 /* Phase trace of the latest whole-step decode launch: device-clock ticks (100 MHz) taken by workgroup
  * 0 at 11 points per layer (both workgroup barriers of the Q|K|V, attention, O, gate|up and down
  * phases; the end of the fold follows attention's second barrier) and one at the end of the kernel, then

@@ -748,6 +748,36 @@ def test_qknorm_rope(ctx, oracle, S, H, kvh, hd, qk_norm):
     assert rel_err(dk.download(np.float32, k.shape), wk) < 1e-4
 
 
+@pytest.mark.parametrize("S,H,kvh,hd,qk_norm", [(1, 16, 8, 128, True), (37, 14, 2, 64, False), (67, 16, 8, 128, True), (129, 4, 4, 64, True),
+                                                 (5, 3, 1, 128, False)])
+def test_prompt_tail_has_the_bits_of_the_decode_kernel(ctx, oracle, S, H, kvh, hd, qk_norm):
+    """Norm, rotation and cache append of a chunk's q, k and v rows, bit for bit what the one-row kernel makes of them: the sums of a
+    norm join in the same order, so that a token's cache row does not depend on which of the two passes it came through."""
+    past, L, eps = 5, S + 9, 1e-6
+    x = synth.normal_f32(15, S * (H + 2 * kvh) * hd).reshape(S, H + 2 * kvh, hd)
+    qw, kw = synth.normal_f32(7, hd), synth.normal_f32(8, hd)
+    cos, sin = oracle.rope_tables(hd, 2048, 1e6)
+    at = slice(past, past + S)
+    dqw, dkw = (ctx.to_device(qw), ctx.to_device(kw)) if qk_norm else (None, None)
+    rows = [ctx.to_device(a) for a in (x[:, :H], x[:, H:H + kvh], cos[at], sin[at])]
+    ctx.qknorm_rope(rows[0], rows[1], dqw, dkw, rows[2], rows[3], S, H, kvh, hd, eps)
+    q, k = rows[0].download(np.float32, (S, H, hd)), rows[1].download(np.float32, (S, kvh, hd))
+    dev = [ctx.to_device(a) for a in (x, cos, sin)] + [ctx.to_device(np.full((kvh, L, hd), 0x1234, np.uint16)) for _ in range(2)]
+    ctx._check(ctx.lib.hm_test_qkv_tail(ctx.h, dev[0].ptr, dqw.ptr if dqw else None, dkw.ptr if dkw else None, dev[1].ptr, dev[2].ptr,
+                                        dev[3].ptr, dev[4].ptr, S, H, kvh, hd, L, past, eps))
+    got = dev[0].download(np.float32, x.shape)[:, :H]
+    kc, vc = (b.download(np.uint16, (kvh, L, hd)) for b in dev[3:])
+
+    def bf16(v):
+        u = np.ascontiguousarray(v).view(np.uint32)
+        return ((u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16).transpose(1, 0, 2)
+    assert np.array_equal(got.view(np.uint32), q.view(np.uint32))
+    assert np.array_equal(kc[:, at], bf16(k)) and np.array_equal(vc[:, at], bf16(x[:, H + kvh:]))
+    assert np.all(kc[:, :past] == 0x1234) and np.all(vc[:, past + S:] == 0x1234)  # nothing beside its rows
+    for b in rows + dev + ([dqw, dkw] if qk_norm else []):
+        b.free()
+
+
 def test_silu_add_embed(ctx, oracle, golden):
     g = synth.normal_f32(10, 3072) * 3
     u = synth.normal_f32(11, 3072)
