@@ -99,6 +99,28 @@ def test_scales_follow_the_values(ctx, dtype):
     assert np.all(np.linalg.norm(got - want, axis=1) <= 1e-6 * np.linalg.norm(want, axis=1))
 
 
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_Q8_0])
+def test_rows_whose_squares_overflow(ctx, dtype):
+    """A finite row whose sum of squares f32 cannot hold is divided by infinity: zeros, as the three bf16 pieces and the decode kernels
+    leave it, and no NaN. Its neighbours, one just below that size among them, are what they are."""
+    rng = np.random.default_rng(8)
+    m, k, n = 70, 512, 40
+    norm_w = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    raw, w = weights(dtype, n, k, rng)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    over = [2, 31, 32, 69]
+    x[over] *= 2.0 ** 66
+    x[5] *= 2.0 ** 58   # 512 squares of 2^116 and less: 2^125
+    x[6, 7] = 2.0 ** 120  # a single entry
+    over.append(6)
+    want = rows_of(0, x, norm_w) @ w.T.astype(np.float64)
+    want[over] = 0
+    for half in (1, 0):
+        got = product(ctx, 0, x, norm_w, dtype, raw, n, half)
+        assert np.all(got[over] == 0)
+        assert np.all(np.linalg.norm(got - want, axis=1) <= 1e-6 * np.linalg.norm(want, axis=1))
+
+
 def test_weights_that_f16_would_round_are_refused(ctx):
     """bf16 values more than 31 binades below their row's largest, and norm weights that would spread a block of integers too far."""
     rng = np.random.default_rng(6)
