@@ -121,6 +121,28 @@ def test_rows_whose_squares_overflow(ctx, dtype):
         assert np.all(np.linalg.norm(got - want, axis=1) <= 1e-6 * np.linalg.norm(want, axis=1))
 
 
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_Q8_0])
+@pytest.mark.parametrize("k", [512, 2048])
+def test_gated_rows_of_every_finite_size(ctx, dtype, k):
+    """Rows of SiLU(gate) * up whose largest value runs from 2^-127 to f32's last binade: each as exact as a row around one, up to the
+    2^-149 that a value below 2^-126 is off by in f32 already."""
+    rng = np.random.default_rng(9)
+    n = 40
+    raw, w = weights(dtype, n, k, rng)
+    size = np.concatenate([np.arange(-126, -96), np.arange(-96, 96, 8), np.arange(113, 129)])
+    g = np.empty((len(size), 2 * k), np.float32)
+    g[:, 0::2] = 20  # SiLU(20) = 20 (1 - 2e-9)
+    u = rng.uniform(-0.1, 0.1, (len(size), k))
+    u[:, 3] = 1.5
+    g[:, 1::2] = u * 2.0 ** (size[:, None] - 5.0)  # the largest: 0.94 2^size
+    rows = rows_of(1, g, np.ones(k))
+    want = rows @ w.T.astype(np.float64)
+    assert max(np.abs(rows).max(), np.abs(want).max()) < 0.95 * 2.0 ** 128
+    got = product(ctx, 1, g, np.ones(k, np.float32), dtype, raw, n).astype(np.float64)
+    lost = 2.0 ** -149 * np.linalg.norm(np.abs(w.astype(np.float64)).sum(1) + 1)
+    assert np.all(np.linalg.norm(got - want, axis=1) <= 1e-6 * np.linalg.norm(want, axis=1) + lost)
+
+
 def test_weights_that_f16_would_round_are_refused(ctx):
     """bf16 values more than 31 binades below their row's largest, and norm weights that would spread a block of integers too far."""
     rng = np.random.default_rng(6)
