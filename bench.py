@@ -242,8 +242,11 @@ def main() -> int:
         if not args.no_prefill:
             ptoks = synth.token_ids(seed + 0x300, 512, cfg.vocab_size)
             prefill = {"tokens": 512, "unit": "tok/s"}
-            for pieces in (3, 2):
-                model.set_prefill_pieces(pieces)
+            for what in ("f16x2", "bf16x3", "bf16x2"):
+                if what == "f16x2":
+                    model.set_prefill_f16(True)
+                else:
+                    model.set_prefill_pieces(int(what[-1]))
                 model.reset_kv_cache()
                 model.prefill(ptoks, want_logits=False)   # warm-up (allocates the chunk's scratch)
                 best = None
@@ -254,10 +257,11 @@ def main() -> int:
                     model.prefill(ptoks, want_logits=False)
                     dt = time.perf_counter() - t0
                     best = dt if best is None or dt < best else best
-                prefill[f"bf16x{pieces}"] = {"value": round(512 / best, 1), "ms": round(best * 1e3, 3)}
-            model.set_prefill_pieces(3)
-            prefill["what"] = ("HfModel.prefill of 512 prompt tokens, empty cache, no LM head; bf16x3 = every f32 "
-                               "activation as three bf16 pieces (default, exact), bf16x2 = two pieces")
+                prefill[what] = {"value": round(512 / best, 1), "ms": round(best * 1e3, 3)}
+            model.set_prefill_f16(True)
+            prefill["what"] = ("HfModel.prefill of 512 prompt tokens, empty cache, no LM head; f16x2 = every f32 activation as "
+                               "two f16 pieces (default where the weights are f16 without loss, 23 to 24 bits), bf16x3 = three "
+                               "bf16 pieces (every bit), bf16x2 = two")
         launches = model.launches_per_step()
         device = ctx.device_name()
         model.close()

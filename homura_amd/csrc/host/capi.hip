@@ -94,6 +94,20 @@ int hm_model_set_prefill_pieces(hm_model *m, int pieces) {
     return m->impl->set_prefill_pieces(pieces);
 }
 
+int hm_model_set_prefill_f16(hm_model *m, int on) {
+    if (!m) return HM_ERR_INVALID;
+    HfModel *hf = m->hf("hm_model_set_prefill_f16");
+    return hf ? hf->set_prefill_f16(on != 0) : HM_ERR_INVALID;
+}
+
+int hm_test_prefill_f16_copies(hm_model *m, size_t *bytes, int *groups) {
+    if (!m || !bytes || !groups) return HM_ERR_INVALID;
+    HfModel *hf = m->hf("hm_test_prefill_f16_copies");
+    if (!hf) return HM_ERR_INVALID;
+    hf->prefill_f16_copies(bytes, groups);
+    return HM_OK;
+}
+
 int hm_model_set_prefill_chunk(hm_model *m, int rows) {
     if (!m) return HM_ERR_INVALID;
     return m->impl->set_prefill_chunk(rows);

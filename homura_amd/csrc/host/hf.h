@@ -71,9 +71,13 @@ class HfModel : public DecoderModel {
 
     // The prompt pass: causal attention over cache + chunk. bf16 plan, head_dim 64 or 128.
     bool prefill_available() const override;
-    // bf16 pieces per f32 activation in the prefill pass: 3 (all 24 significant bits, default) or 2
-    // (16 bits, two thirds of the matrix-core work)
+    // What the prefill pass carries an f32 activation as. Default: two f16 pieces (23 to 24 bits, half_weights.h) where the weights are
+    // f16 without loss, three bf16 pieces elsewhere. set_prefill_pieces: that many bf16 pieces everywhere, 3 (all 24 bits, at any
+    // size) or 2 (16 bits; block formats keep 3), and no f16 copies of the weights; set_prefill_f16(true) returns to the default.
     int set_prefill_pieces(int n) override;
+    int set_prefill_f16(bool on);
+    // Test support: the bytes of the f16 copies held and the groups of projections (four a layer) that multiply with them.
+    void prefill_f16_copies(size_t *bytes, int *groups) const;
     // Block-quantised models: HBM the prompt pass may keep for the dequantised projections (three bf16
     // pieces per weight, 6 bytes). When all of them fit, they are written once and stay; otherwise
     // (or with 0) every chunk dequantises them again into one scratch matrix.
@@ -191,6 +195,8 @@ class HfModel : public DecoderModel {
     static size_t half_matrix_bytes(int64_t N, int64_t K) { return ((size_t)N * K * 2 + 255) / 256 * 256; }
     size_t half_bytes() const;
     int build_half_weights();
+    int refresh_half_weights();
+    bool half_wanted_ = true;
     size_t prefill_weight_cache_bytes_ = (size_t)32 << 30;
 };
 

@@ -556,7 +556,7 @@ int HfModel::finalize(int max_seq_len) {
     mask_view_ = Buffer::view(plan_->state(), sizeof(DecodeState), {1, 1, 1, DIM_DYNAMIC}, {1, 1, 1, 1},
                               DType::F32);
     finalized_ = true;
-    if ((rc = build_half_weights()) != HM_OK) return rc;
+    if ((rc = refresh_half_weights()) != HM_OK) return rc;
     return hm_sync(ctx_);
 }
 
@@ -1842,8 +1842,24 @@ int HfModel::check_status_words(const uint32_t *h_ctl) {
 
 int HfModel::set_prefill_pieces(int n) {
     if (n != 2 && n != 3) return hm_set_error(ctx_, HM_ERR_INVALID, "prefill pieces must be 2 or 3");
+    const int rc = set_prefill_f16(false);
     prefill_pieces_ = n;
-    return HM_OK;
+    return rc;
+}
+
+int HfModel::set_prefill_f16(bool on) {
+    half_wanted_ = on;
+    if (on) prefill_pieces_ = 3;
+    return refresh_half_weights();
+}
+
+// The f16 copies as the settings want them: none, or built.
+int HfModel::refresh_half_weights() {
+    if (!finalized_ || half_.empty() == !half_wanted_) return HM_OK;
+    if (half_wanted_) return build_half_weights();
+    const int rc = hm_sync(ctx_);
+    half_.clear();
+    return rc;
 }
 
 const char *HfModel::prefill_needs() const {
@@ -1874,7 +1890,7 @@ void HfModel::set_prefill_weight_cache(size_t bytes) {
     pf_.wcache.clear();
     if (pf_.rows > 0) return;  // the integers and planes of the first prompt stay, and so do the f16 matrices
     if (half_bytes() > bytes) half_.clear();
-    else if (half_.empty() && finalized_) (void)build_half_weights();
+    else (void)refresh_half_weights();
 }
 
 size_t HfModel::half_bytes() const {
@@ -1882,6 +1898,13 @@ size_t HfModel::half_bytes() const {
     for (const HalfLayer &h : half_)
         for (const Buffer &b : h.w) sum += b ? b.bytes() : 0;
     return sum;
+}
+
+void HfModel::prefill_f16_copies(size_t *bytes, int *groups) const {
+    *bytes = half_bytes();
+    *groups = 0;
+    for (const HalfLayer &h : half_)
+        for (bool ok : h.ok) *groups += ok;
 }
 
 // Groups of bf16 projections, or of Q8_0 / Q4_0 ones, whose weights are f16 without loss. Everything is enqueued, then one
@@ -2198,7 +2221,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         return &slot;
     };
     // group g of layer l multiplies f16 pieces with f16 weights
-    auto half = [&](int l, int g) { return np == 3 && !half_.empty() && half_[l].ok[g] && (g != 1 || !kv_given_); };
+    auto half = [&](int l, int g) { return !half_.empty() && half_[l].ok[g] && (g != 1 || !kv_given_); };
     const Buffer *i8 = nullptr;  // the planes of the group about to be multiplied, if it takes that path
     int8_t *q8 = p.q8 ? p.q8.as<int8_t>() : nullptr;
     float *q8s = p.q8s ? p.q8s.as<float>() : nullptr;

@@ -445,7 +445,8 @@ class DecoderModel:
         return out[:n.value].copy()
 
     def set_prefill_pieces(self, pieces: int):
-        """bf16 numbers per f32 activation in the prefill pass: 3 (exact), 2, and where the model takes it 1."""
+        """bf16 numbers per f32 activation in the prefill pass: 3 (exact), 2, and where the model takes it 1. A transformer's
+        default is two f16 numbers where its weights allow it (HfModel.set_prefill_f16)."""
         self._check(self.lib.hm_model_set_prefill_pieces(self.h, pieces))
 
     def generate_greedy(self, prompt_ids, n_new: int) -> np.ndarray:
@@ -598,6 +599,11 @@ class HfModel(DecoderModel):
         f32 lm_head.weight slot (hm_model_set_lm_head_blocks)."""
         a = np.ascontiguousarray(blocks, np.uint8).reshape(-1)
         self._check(self.lib.hm_model_set_lm_head_blocks(self.h, int(dtype), a.ctypes.data, a.nbytes))
+
+    def set_prefill_f16(self, on: bool):
+        """True (the default): the prefill pass carries f32 activations as two f16 numbers (23 to 24 bits) where the weights are f16
+        without loss. False, or set_prefill_pieces: bf16 numbers only, and no f16 copies of the weights."""
+        self._check(self.lib.hm_model_set_prefill_f16(self.h, int(on)))
 
     def set_prefill_weight_cache(self, nbytes: int):
         """Block-quantised models: HBM the prompt pass may keep for dequantised projections (0 = none)."""

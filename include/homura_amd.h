@@ -417,12 +417,16 @@ int hm_model_run_kv(hm_model *m, const int64_t *h_ids, int n_ids, float *h_logit
  * (the products of hm_gemm_f32_quant_nk) need multiples of 64, and q|k|v as well as gate|up must each
  * be of one kind, Q8_0 / Q4_0 or K-quants, because the members of a group share an activation
  * matrix; other models keep stepping token by token. hm_model_set_prefill_min: 0 = always token by
- * token (default 8). hm_model_set_prefill_pieces (bf16 models): bf16 numbers per f32 activation on the
- * matrix cores, 3 (default, every bit of the f32; as two f16 numbers where the weights are f16 without loss) or 2 (16 bits; K/V
- * rows then round to a neighbouring bf16 now and then). */
+ * token (default 8). On the matrix cores an f32 activation is by default two f16 numbers where the weights are f16 without loss
+ * (23 to 24 bits; fewer for a value more than 2^15 below the largest that the weights allow in its place, or, of SiLU(gate) * up,
+ * below its row's largest), and three bf16 numbers elsewhere. hm_model_set_prefill_pieces (bf16 models): bf16 numbers everywhere, 3 (every bit of the
+ * f32 at any size) or 2 (16 bits; K/V rows then round to a neighbouring bf16 now and then), and the f16 copies of the weights are
+ * given back; 3 does the same for block-quantised models. hm_model_set_prefill_f16(m, 1) returns to the default, 0 leaves the bf16
+ * numbers as last set (transformers only). */
 int hm_model_prefill(hm_model *m, const int64_t *h_ids, int n_ids, float *h_logits);
 int hm_model_set_prefill_min(hm_model *m, int n_tokens);
 int hm_model_set_prefill_pieces(hm_model *m, int pieces);
+int hm_model_set_prefill_f16(hm_model *m, int on);
 /* HBM the prompt pass may keep for copies of the projections (default 32 GiB): f16 copies of bf16, Q8_0 and Q4_0 projections (2 bytes
  * a weight), made by hm_model_finalize; for block-quantised models also the dequantised ones (three bf16
  * pieces = 6 bytes per weight). Takes effect until the first prompt pass. If all projections fit, and an eighth of the device

@@ -68,6 +68,10 @@ int hm_test_prompt_product(int hm_dtype, int rows, int m, int k, int n, int cus,
 int hm_test_prompt_rows(hm_ctx *ctx, int front, const float *x, const float *norm_w, int dtype, const void *w, int half, int m, int k,
                         int n, float *out, float *row_factor, int *parts, int copies, int rounds, float *us);
 
+/* Test support: the bytes of f16 weight copies that a transformer's prompt pass holds, and how many of its groups of projections
+ * (q|k|v, o, gate|up, down of every layer) multiply with them. */
+int hm_test_prefill_f16_copies(hm_model *m, size_t *bytes, int *groups);
+
 /* Test support: the tail of the prompt pass's q|k|v projection for S rows [S][(H + 2 kvh) * hd] at positions past ..: q rotated in
  * place, k and v into caches [kvh][max_len][hd]. d_qw and d_kw [hd], or both NULL. hd 64 or 128. */
 int hm_test_qkv_tail(hm_ctx *ctx, float *d_qkv, const float *d_qw, const float *d_kw, const float *d_cos, const float *d_sin,

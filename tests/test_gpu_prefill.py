@@ -1,6 +1,8 @@
 """The multi-token pass (prompt chunks as matrices on the matrix cores) against the CPU oracle's
 batched run_kv (reference HfGenerationContext::prefill -> run_kv with seq > 1, src/hf/model.rs:321-336)
 and against the token-by-token path. Logits within TOL below, greedy tokens identical."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -263,6 +265,58 @@ def test_resident_and_per_chunk_dequantisation_agree(ctx):
         runs.append(gm.prefill(ids))
     for r in runs[1:]:
         assert np.array_equal(r.view(np.uint32), runs[0].view(np.uint32))
+    gm.close()
+
+
+def f16_copies(gm):
+    """(bytes held, groups of projections that multiply with f16 copies)"""
+    nbytes, groups = C.c_size_t(), C.c_int()
+    gm._check(gm.lib.hm_test_prefill_f16_copies(gm.h, C.byref(nbytes), C.byref(groups)))
+    return nbytes.value, groups.value
+
+
+@pytest.mark.parametrize("how", ["pieces", "budget"])
+@pytest.mark.parametrize("which", ["bf16", "q8_0", "q4_0_wide_vocab", "q8_0_and_k_quants_by_group"])
+def test_prompt_pass_without_f16_copies(ctx, which, how):
+    """The bf16 pieces behind the f16 products, asked for by name (three of them, Q8_0 / Q4_0 groups as integers with block scales) and
+    by a weight budget of 0 (Q8_0 / Q4_0 groups dequantised for every chunk): the oracle's rows, and no copies held. Back to the default,
+    the copies are there again and the rows agree with the oracle as closely."""
+    cfg, mix = (synth_model.TINY, None) if which == "bf16" else _quant_case(which)
+    kw = {} if mix is None else dict(has_qk_norm=False, proj_dtypes=mix)
+    weights = synth_model.synth_weights(cfg, 51, **kw)
+    gm = synth_model.build_model(ctx, cfg, weights, 96, **kw)
+    om = mf.build_oracle_model(cfg, weights, 96, **kw)
+    plain = 4 if mix is None else sum(mix[j] in (2, 3) for j in (0, 3, 4, 6))
+    default = f16_copies(gm)
+    assert default[0] > 0 and default[1] == plain * cfg.num_hidden_layers
+    ids = synth.token_ids(14, 70, cfg.vocab_size)
+    if mix is not None and any(t in (5, 6) for t in mix):
+        want = None  # rows of Q8_K values: compared with each other below
+    else:
+        want = om.run_kv(ids) if mix is None else np.concatenate([om.run_kv(ids[i:i + 1]) for i in range(len(ids))])
+
+    def rows():
+        gm.reset_kv_cache()
+        got = gm.prefill(ids)
+        if want is not None:
+            err = logit_err(got, want)
+            say(f"{which} {how}: rel err {err:.1e}, copies {f16_copies(gm)}")
+            assert err < TOL
+        return got
+    if how == "pieces":
+        gm.set_prefill_pieces(3)
+    else:
+        gm.set_prefill_weight_cache(0)
+    assert f16_copies(gm) == (0, 0)
+    exact = rows()
+    if how == "pieces":
+        gm.set_prefill_f16(True)
+        assert f16_copies(gm) == default
+        pairs = rows()
+        assert not np.array_equal(pairs, exact)     # another path it was
+        assert logit_err(pairs, exact) < (TOL if want is not None else 2e-2)
+        gm.set_prefill_f16(False)
+        assert f16_copies(gm) == (0, 0) and np.array_equal(rows(), exact)
     gm.close()
 
 
