@@ -123,8 +123,7 @@ int hm_model_set_prefill_weight_cache(hm_model *m, size_t bytes) {
 
 int hm_model_set_prefill_min(hm_model *m, int n_tokens) {
     if (!m || n_tokens < 0) return HM_ERR_INVALID;
-    m->impl->set_prefill_min(n_tokens);
-    return HM_OK;
+    return m->impl->set_prefill_min(n_tokens);
 }
 
 int hm_model_num_weight_slots(hm_model *m) {

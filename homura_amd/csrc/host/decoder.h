@@ -59,7 +59,10 @@ class DecoderModel {
     int prefill(const int64_t *h_ids, int n_ids, float *h_logits);
     virtual bool prefill_available() const = 0;
     // Inputs of at least this many tokens take the prefill pass (0 = never). Default 8.
-    void set_prefill_min(int n) { prefill_min_ = n; }
+    virtual int set_prefill_min(int n) {
+        prefill_min_ = n;
+        return HM_OK;
+    }
     int prefill_min() const { return prefill_min_; }
     // bf16 pieces per f32 activation in the prefill pass; HM_ERR_INVALID when the model does not take that many
     virtual int set_prefill_pieces(int n) = 0;

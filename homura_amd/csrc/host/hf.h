@@ -76,6 +76,7 @@ class HfModel : public DecoderModel {
     // size) or 2 (16 bits; block formats keep 3), and no f16 copies of the weights; set_prefill_f16(true) returns to the default.
     int set_prefill_pieces(int n) override;
     int set_prefill_f16(bool on);
+    int set_prefill_min(int n) override;  // 0 gives the f16 copies back until a prompt pass comes all the same
     // Test support: the bytes of the f16 copies held and the groups of projections (four a layer) that multiply with them.
     void prefill_f16_copies(size_t *bytes, int *groups) const;
     // Block-quantised models: HBM the prompt pass may keep for the dequantised projections (three bf16
@@ -196,7 +197,8 @@ class HfModel : public DecoderModel {
     size_t half_bytes() const;
     int build_half_weights();
     int refresh_half_weights();
-    bool half_wanted_ = true;
+    bool half_wanted_ = true;   // set_prefill_f16
+    bool half_waits_ = false;   // not built for want of prompt passes (set_prefill_min(0)): the next one builds them
     size_t prefill_weight_cache_bytes_ = (size_t)32 << 30;
 };
 

@@ -1853,10 +1853,18 @@ int HfModel::set_prefill_f16(bool on) {
     return refresh_half_weights();
 }
 
+int HfModel::set_prefill_min(int n) {
+    prefill_min_ = n;
+    return refresh_half_weights();
+}
+
 // The f16 copies as the settings want them: none, or built.
 int HfModel::refresh_half_weights() {
-    if (!finalized_ || half_.empty() == !half_wanted_) return HM_OK;
-    if (half_wanted_) return build_half_weights();
+    if (!finalized_) return HM_OK;
+    const bool wanted = half_wanted_ && prefill_min_ > 0;
+    half_waits_ = half_wanted_ && !wanted;
+    if (half_.empty() == !wanted) return HM_OK;
+    if (wanted) return build_half_weights();
     const int rc = hm_sync(ctx_);
     half_.clear();
     return rc;
@@ -2028,6 +2036,10 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     const int H = c.num_attention_heads, kvh = c.kv_heads(), hd = c.head_dim();
     const int qd = c.q_dim(), kvd = c.kv_dim(), nqkv = qd + 2 * kvd;
     const float eps = (float)c.rms_norm_eps;
+    if (half_waits_) {
+        half_waits_ = false;
+        if (const int built = build_half_weights(); built != HM_OK) return built;
+    }
     PrefillScratch &p = pf_;
     const bool quant = dtype_is_quantized(weight_dtype_);
     if (p.rows < n) {

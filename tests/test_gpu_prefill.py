@@ -8,7 +8,7 @@ import pytest
 
 import model_fixture as mf
 from homura_amd import HomuraError, synth, synth_model
-from homura_amd.runtime import DTYPE_Q8_0
+from homura_amd.runtime import DTYPE_BF16, DTYPE_Q8_0
 
 pytestmark = pytest.mark.gpu
 
@@ -317,6 +317,31 @@ def test_prompt_pass_without_f16_copies(ctx, which, how):
         assert logit_err(pairs, exact) < (TOL if want is not None else 2e-2)
         gm.set_prefill_f16(False)
         assert f16_copies(gm) == (0, 0) and np.array_equal(rows(), exact)
+    gm.close()
+
+
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_Q8_0])
+def test_no_f16_copies_while_prompts_go_token_by_token(ctx, dtype):
+    """set_prefill_min(0) gives the copies back; a prompt pass by name builds them again, and so does a larger minimum. The rows are
+    the same bits whenever they were built."""
+    cfg = synth_model.TINY if dtype == DTYPE_BF16 else synth_model.TINY_LLAMA
+    kw = {} if dtype == DTYPE_BF16 else dict(has_qk_norm=False)
+    gm = synth_model.build_model(ctx, cfg, synth_model.synth_weights(cfg, 53, dtype, **kw), 96, dtype, **kw)
+    ids, default = synth.token_ids(15, 40, cfg.vocab_size), f16_copies(gm)
+    want = gm.prefill(ids)
+    assert default[0] > 0
+    for again in ("prefill", "minimum"):
+        gm.set_prefill_min(0)
+        assert f16_copies(gm) == (0, 0)
+        gm.reset_kv_cache()
+        step_by_step = gm.run_kv(ids)
+        assert f16_copies(gm) == (0, 0) and logit_err(step_by_step, want) < TOL
+        if again == "minimum":
+            gm.set_prefill_min(8)
+            assert f16_copies(gm) == default
+        gm.reset_kv_cache()
+        got = gm.prefill(ids)
+        assert f16_copies(gm) == default and np.array_equal(got, want)
     gm.close()
 
 
