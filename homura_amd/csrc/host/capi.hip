@@ -117,8 +117,7 @@ int hm_model_set_prefill_weight_cache(hm_model *m, size_t bytes) {
     if (!m) return HM_ERR_INVALID;
     HfModel *hf = m->hf("hm_model_set_prefill_weight_cache");
     if (!hf) return HM_ERR_INVALID;
-    hf->set_prefill_weight_cache(bytes);
-    return HM_OK;
+    return hf->set_prefill_weight_cache(bytes);
 }
 
 int hm_model_set_prefill_min(hm_model *m, int n_tokens) {

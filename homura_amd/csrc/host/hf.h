@@ -79,10 +79,11 @@ class HfModel : public DecoderModel {
     int set_prefill_min(int n) override;  // 0 gives the f16 copies back until a prompt pass comes all the same
     // Test support: the bytes of the f16 copies held and the groups of projections (four a layer) that multiply with them.
     void prefill_f16_copies(size_t *bytes, int *groups) const;
-    // Block-quantised models: HBM the prompt pass may keep for the dequantised projections (three bf16
-    // pieces per weight, 6 bytes). When all of them fit, they are written once and stay; otherwise
-    // (or with 0) every chunk dequantises them again into one scratch matrix.
-    void set_prefill_weight_cache(size_t bytes);
+    // HBM the prompt pass may keep for f16 copies of the projections (2 bytes a weight) and, of block formats, for the dequantised
+    // ones (three bf16 pieces, 6 bytes). What fits is written once and stays. Otherwise (or with 0) every chunk dequantises the
+    // projections again into one scratch matrix; f16 copies are then not used at all, or, once a prompt has used them, made again
+    // for every chunk too.
+    int set_prefill_weight_cache(size_t bytes);
     int init_kv_cache(const float *const *h_kv, int seq_len);
     int reset_kv_cache() override;
     // The whole-step decode launch (one kernel for the embedding row and all layers) instead of one
@@ -186,15 +187,27 @@ class HfModel : public DecoderModel {
     PrefillScratch pf_;
     // The projections as f16 for the prompt pass (half_weights.h), built by finalize() within the prompt pass's weight budget. Per
     // layer: the groups' matrices (q|k|v, o, gate|up, down; rows interleaved as in the packed bf16 matrices) followed by their row
-    // factors or block scales, the two norms' weights times their columns' factors, and the value rows' factors.
+    // factors or block scales, the two norms' weights times their columns' factors, and the value rows' factors. A group that is
+    // ok without a matrix has it made in half_scratch_ for every chunk (a budget made smaller behind the first prompt).
     struct HalfLayer {
         Buffer w[4], norms, values;
         bool ok[4] = {false, false, false, false};
     };
+    struct HalfGroup {
+        int first, count, K, N;
+        size_t factors, bytes;  // where the factors begin, and the whole
+    };
     std::vector<HalfLayer> half_;
+    Buffer half_exps_, half_flags_, half_scratch_;
     bool kv_given_ = false;  // the cache holds rows of the caller's: nothing bounds its values
     static size_t half_matrix_bytes(int64_t N, int64_t K) { return ((size_t)N * K * 2 + 255) / 256 * 256; }
     size_t half_bytes() const;
+    HalfGroup half_group(int g) const;
+    bool half_takes(int l, int g) const;
+    bool half_fits(size_t need) const;
+    int make_half_group(int l, int g, char *dst);
+    int keep_half_weights();
+    void drop_half_weights();
     int build_half_weights();
     int refresh_half_weights();
     bool half_wanted_ = true;   // set_prefill_f16

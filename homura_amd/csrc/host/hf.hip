@@ -1866,7 +1866,7 @@ int HfModel::refresh_half_weights() {
     if (half_.empty() == !wanted) return HM_OK;
     if (wanted) return build_half_weights();
     const int rc = hm_sync(ctx_);
-    half_.clear();
+    drop_half_weights();
     return rc;
 }
 
@@ -1892,13 +1892,33 @@ bool HfModel::prefill_available() const {
     return true;
 }
 
-void HfModel::set_prefill_weight_cache(size_t bytes) {
+int HfModel::set_prefill_weight_cache(size_t bytes) {
     prefill_weight_cache_bytes_ = bytes;
-    if (ctx_) hm_sync(ctx_);
+    int rc = hm_sync(ctx_);
     pf_.wcache.clear();
-    if (pf_.rows > 0) return;  // the integers and planes of the first prompt stay, and so do the f16 matrices
-    if (half_bytes() > bytes) half_.clear();
-    else (void)refresh_half_weights();
+    // Until the first prompt the budget decides whether there are f16 products at all. Later (the integers and planes of the first
+    // prompt stay) only whether their matrices are kept or made again for every chunk: results do not change under a caller.
+    if (half_bytes() > bytes) {
+        if (pf_.rows == 0) {
+            drop_half_weights();
+            return rc;
+        }
+        size_t most = 0;
+        for (HalfLayer &h : half_)
+            for (int g = 0; g < 4; g++)
+                if (h.ok[g]) {
+                    h.w[g] = Buffer();
+                    most = std::max(most, half_group(g).bytes);
+                }
+        half_scratch_ = Buffer::alloc(ctx_, {(int64_t)(most + 3) / 4}, DType::F32);
+        if (!half_scratch_) {
+            (void)hipGetLastError();
+            drop_half_weights();
+        }
+        return rc;
+    }
+    if (rc == HM_OK) rc = half_scratch_ ? keep_half_weights() : refresh_half_weights();
+    return rc;
 }
 
 size_t HfModel::half_bytes() const {
@@ -1915,48 +1935,117 @@ void HfModel::prefill_f16_copies(size_t *bytes, int *groups) const {
         for (bool ok : h.ok) *groups += ok;
 }
 
-// Groups of bf16 projections, or of Q8_0 / Q4_0 ones, whose weights are f16 without loss. Everything is enqueued, then one
-// synchronisation reads which groups are not. No memory, or not enough budget: the prompt pass keeps its bf16 pieces.
-int HfModel::build_half_weights() {
+void HfModel::drop_half_weights() {
     half_.clear();
+    half_exps_ = Buffer();
+    half_flags_ = Buffer();
+    half_scratch_ = Buffer();
+}
+
+HfModel::HalfGroup HfModel::half_group(int g) const {
     const TransformerConfig &c = cfg_;
-    const int L = c.num_hidden_layers, hidden = c.hidden_size, inter = c.intermediate_size, hd = c.head_dim();
-    const int qd = c.q_dim(), kvd = c.kv_dim(), nqkv = qd + 2 * kvd;
-    if (!prefill_available() || prefill_weight_cache_bytes_ == 0) return HM_OK;
-    const bool bf16 = weight_dtype_ == DType::BF16;
-    const int first[4] = {0, 3, 4, 6}, count[4] = {3, 1, 2, 1};
-    const int K[4] = {hidden, qd, hidden, inter}, N[4] = {nqkv, hidden, 2 * inter, hidden};
+    const int hidden = c.hidden_size, inter = c.intermediate_size, qd = c.q_dim(), nqkv = qd + 2 * c.kv_dim();
+    const int first[4] = {0, 3, 4, 6}, count[4] = {3, 1, 2, 1}, K[4] = {hidden, qd, hidden, inter}, N[4] = {nqkv, hidden, 2 * inter, hidden};
+    HalfGroup hg{first[g], count[g], K[g], N[g], half_matrix_bytes(N[g], K[g]), 0};
+    hg.bytes = hg.factors + (weight_dtype_ == DType::BF16 ? (size_t)N[g] * 4 : (size_t)(K[g] / 32) * half_scale_cols(N[g]) * 4);
+    return hg;
+}
+
+// Groups of bf16 projections, or of Q8_0 / Q4_0 ones, with an activation whose size is bounded (half_weights.h)
+bool HfModel::half_takes(int l, int g) const {
+    auto plain = [&](int j) { return weight_dtype_ == DType::BF16 || proj_dtype(l, j) == DType::Q8_0 || proj_dtype(l, j) == DType::Q4_0; };
+    const HalfGroup hg = half_group(g);
+    for (int j = hg.first; j < hg.first + hg.count; j++)
+        if (!plain(j)) return false;
+    return hg.K % 64 == 0 && (g != 1 || plain(2)) && (g != 3 || cfg_.intermediate_size <= SILU_HALF_MAX);
+}
+
+// The matrix of a group and its factors or block scales, written to dst
+int HfModel::make_half_group(int l, int g, char *dst) {
+    const int hidden = cfg_.hidden_size, inter = cfg_.intermediate_size, qd = cfg_.q_dim(), kvd = cfg_.kv_dim();
     const int rows[7] = {qd, kvd, kvd, hidden, inter, inter, hidden};
     static const char *const name[7] = {"self_attn.q_proj.weight", "self_attn.k_proj.weight", "self_attn.v_proj.weight",
                                         "self_attn.o_proj.weight", "mlp.gate_proj.weight", "mlp.up_proj.weight", "mlp.down_proj.weight"};
-    auto plain = [&](int l, int j) { return bf16 || proj_dtype(l, j) == DType::Q8_0 || proj_dtype(l, j) == DType::Q4_0; };
-    auto wanted = [&](int l, int g) {
-        for (int j = first[g]; j < first[g] + count[g]; j++)
-            if (!plain(l, j)) return false;
-        return K[g] % 64 == 0 && (g != 1 || plain(l, 2)) && (g != 3 || inter <= SILU_HALF_MAX);
-    };
-    auto bytes_of = [&](int g) {
-        return half_matrix_bytes(N[g], K[g]) + (bf16 ? (size_t)N[g] * 4 : (size_t)(K[g] / 32) * half_scale_cols(N[g]) * 4);
-    };
-    size_t need = 0, free_b = 0, total_b = 0;
-    for (int l = 0; l < L; l++)
-        for (int g = 0; g < 4; g++) need += wanted(l, g) ? bytes_of(g) : 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = total_b = 0;
-    if (need == 0 || need > prefill_weight_cache_bytes_ || need + total_b / 8 > free_b) return HM_OK;
+    const HalfGroup hg = half_group(g);
+    const int *e = half_exps_.as<int>() + (size_t)l * (2 * hidden + qd);
+    const int *col[4] = {e, e + 2 * hidden, e + hidden, nullptr};
+    int *flag = half_flags_.as<int>() + l * 4 + g;
+    uint16_t *w = reinterpret_cast<uint16_t *>(dst);
+    float *factors = reinterpret_cast<float *>(dst + hg.factors);
+    if (weight_dtype_ == DType::BF16) {
+        const LayerPacked &lp = packed_[l];
+        const Buffer *packed[4] = {&lp.qkv, &lp.o, &lp.gate_up, &lp.down};
+        return half_rows(ctx_, packed[g]->as<uint16_t>(), col[g], hg.N, hg.K, w, factors, flag);
+    }
+    int rc = HM_OK;
+    for (int j = hg.first, row = 0; j < hg.first + hg.count && rc == HM_OK; row += rows[j], j++) {
+        const uint8_t *raw = weight_bufs_[slot_by_name_.at("model.layers." + std::to_string(l) + "." + name[j])].as<uint8_t>();
+        rc = half_ints(ctx_, (int)proj_dtype(l, j), raw, col[g], rows[j], hg.K, g == 2 ? w : w + (size_t)row * hg.K,
+                       g == 2 ? factors : factors + row, half_scale_cols(hg.N), g == 2 ? 2 : 1, g == 2 ? j - hg.first : 0, flag);
+    }
+    return rc;
+}
 
-    Buffer exps = Buffer::alloc(ctx_, {(int64_t)L * (2 * hidden + qd)}, DType::F32), flags = Buffer::alloc(ctx_, {(int64_t)L * 4}, DType::F32);
-    if (!exps || !flags) {
+// Whether `need` bytes of copies are within the budget and leave enough of the device
+bool HfModel::half_fits(size_t need) const {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = total_b = 0;
+    return need <= prefill_weight_cache_bytes_ && need + total_b / 8 <= free_b;
+}
+
+// The f16 products' matrices, which a smaller budget had made again for every chunk, kept once more if they fit.
+int HfModel::keep_half_weights() {
+    size_t need = 0;
+    for (const HalfLayer &h : half_)
+        for (int g = 0; g < 4; g++) need += h.ok[g] ? half_group(g).bytes : 0;
+    if (!half_fits(need)) return HM_OK;
+    int rc = HM_OK;
+    bool all = true;
+    for (int l = 0; l < (int)half_.size() && rc == HM_OK && all; l++)
+        for (int g = 0; g < 4 && rc == HM_OK && all; g++) {
+            if (!half_[l].ok[g]) continue;
+            half_[l].w[g] = Buffer::alloc(ctx_, {(int64_t)(half_group(g).bytes + 3) / 4}, DType::F32);
+            all = (bool)half_[l].w[g];
+            if (all) rc = make_half_group(l, g, half_[l].w[g].as<char>());
+        }
+    const int synced = hm_sync(ctx_);
+    if (!all || rc != HM_OK) {
         (void)hipGetLastError();
+        for (HalfLayer &h : half_)
+            for (Buffer &b : h.w) b = Buffer();
+    } else {
+        half_scratch_ = Buffer();
+    }
+    return rc != HM_OK ? rc : synced;
+}
+
+// Everything is enqueued, then one synchronisation reads which groups have weights that f16 would round. No memory, or not enough
+// budget: the prompt pass keeps its bf16 pieces.
+int HfModel::build_half_weights() {
+    drop_half_weights();
+    const TransformerConfig &c = cfg_;
+    const int L = c.num_hidden_layers, hidden = c.hidden_size, hd = c.head_dim(), qd = c.q_dim(), kvd = c.kv_dim();
+    if (!prefill_available() || prefill_weight_cache_bytes_ == 0) return HM_OK;
+    const bool bf16 = weight_dtype_ == DType::BF16;
+    size_t need = 0;
+    for (int l = 0; l < L; l++)
+        for (int g = 0; g < 4; g++) need += half_takes(l, g) ? half_group(g).bytes : 0;
+    if (need == 0 || !half_fits(need)) return HM_OK;
+
+    half_exps_ = Buffer::alloc(ctx_, {(int64_t)L * (2 * hidden + qd)}, DType::F32);
+    half_flags_ = Buffer::alloc(ctx_, {(int64_t)L * 4}, DType::F32);
+    if (!half_exps_ || !half_flags_) {
+        (void)hipGetLastError();
+        drop_half_weights();
         return HM_OK;
     }
-    HM_HIP(ctx_, hipMemsetAsync(flags.ptr(), 0, (size_t)L * 16, ctx_->stream));
+    HM_HIP(ctx_, hipMemsetAsync(half_flags_.ptr(), 0, (size_t)L * 16, ctx_->stream));
     half_.resize((size_t)L);
     int rc = HM_OK;
     for (int l = 0; l < L && rc == HM_OK; l++) {
         HalfLayer &h = half_[l];
         const std::string pre = "model.layers." + std::to_string(l) + ".";
-        int *e1 = exps.as<int>() + (size_t)l * (2 * hidden + qd), *e2 = e1 + hidden, *eo = e2 + hidden, *flag = flags.as<int>() + l * 4;
-        const int *col[4] = {e1, eo, e2, nullptr};
+        int *e1 = half_exps_.as<int>() + (size_t)l * (2 * hidden + qd), *e2 = e1 + hidden, *eo = e2 + hidden, *flag = half_flags_.as<int>() + l * 4;
         const float *w1 = weight_f32(pre + "input_layernorm.weight"), *w2 = weight_f32(pre + "post_attention_layernorm.weight");
         h.norms = Buffer::alloc(ctx_, {2 * (int64_t)hidden}, DType::F32);
         h.values = Buffer::alloc(ctx_, {kvd}, DType::F32);
@@ -1966,39 +2055,25 @@ int HfModel::build_half_weights() {
         }
         rc = half_norm_scales(ctx_, w1, hidden, h.norms.as<float>(), e1, flag + 0);
         if (rc == HM_OK) rc = half_norm_scales(ctx_, w2, hidden, h.norms.as<float>() + hidden, e2, flag + 2);
-        auto raw = [&](int j) { return weight_bufs_[slot_by_name_.at(pre + name[j])].as<uint8_t>(); };
         const LayerPacked &lp = packed_[l];
-        if (rc == HM_OK && wanted(l, 1))
+        if (rc == HM_OK && half_takes(l, 1))
             rc = half_value_scales(ctx_, bf16 ? HM_DTYPE_BF16 : (int)proj_dtype(l, 2),
-                                   bf16 ? (const void *)(lp.qkv.as<uint16_t>() + (size_t)(qd + kvd) * hidden) : raw(2), w1,
-                                   lp.qkv_bias ? lp.qkv_bias.as<float>() + qd + kvd : nullptr, kvd, hidden, c.num_attention_heads, hd,
+                                   bf16 ? (const void *)(lp.qkv.as<uint16_t>() + (size_t)(qd + kvd) * hidden)
+                                        : weight_bufs_[slot_by_name_.at(pre + "self_attn.v_proj.weight")].ptr(),
+                                   w1, lp.qkv_bias ? lp.qkv_bias.as<float>() + qd + kvd : nullptr, kvd, hidden, c.num_attention_heads, hd,
                                    h.values.as<float>(), eo, flag + 1);
-        const Buffer *packed[4] = {&lp.qkv, &lp.o, &lp.gate_up, &lp.down};
         for (int g = 0; g < 4 && rc == HM_OK; g++) {
-            if (!wanted(l, g)) continue;
-            h.w[g] = Buffer::alloc(ctx_, {(int64_t)(bytes_of(g) + 3) / 4}, DType::F32);
-            if (!h.w[g]) {
-                rc = HM_ERR_OOM;
-                break;
-            }
-            uint16_t *w = h.w[g].as<uint16_t>();
-            float *scales = reinterpret_cast<float *>(h.w[g].as<char>() + half_matrix_bytes(N[g], K[g]));
-            if (bf16) {
-                rc = half_rows(ctx_, packed[g]->as<uint16_t>(), col[g], N[g], K[g], w, scales, flag + g);
-                continue;
-            }
-            const int npad = half_scale_cols(N[g]);
-            for (int j = first[g], row = 0; j < first[g] + count[g] && rc == HM_OK; row += rows[j], j++)
-                rc = half_ints(ctx_, (int)proj_dtype(l, j), raw(j), col[g], rows[j], K[g], g == 2 ? w : w + (size_t)row * K[g],
-                               g == 2 ? scales : scales + row, npad, g == 2 ? 2 : 1, g == 2 ? j - first[g] : 0, flag + g);
+            if (!half_takes(l, g)) continue;
+            h.w[g] = Buffer::alloc(ctx_, {(int64_t)(half_group(g).bytes + 3) / 4}, DType::F32);
+            rc = h.w[g] ? make_half_group(l, g, h.w[g].as<char>()) : HM_ERR_OOM;
         }
     }
     std::vector<int> bad((size_t)L * 4, 1);
-    if (rc == HM_OK) rc = hm_download(ctx_, bad.data(), flags.ptr(), (size_t)L * 16);
+    if (rc == HM_OK) rc = hm_download(ctx_, bad.data(), half_flags_.ptr(), (size_t)L * 16);
     const int synced = hm_sync(ctx_);
     if (rc == HM_ERR_OOM) {
         (void)hipGetLastError();
-        half_.clear();
+        drop_half_weights();
         return synced;
     }
     if (rc != HM_OK) return rc;
@@ -2241,9 +2316,12 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         int N = 0;
         for (int j = first; j < first + count; j++) N += proj_n[j];
         if (const int g = first == 0 ? 0 : first == 3 ? 1 : first == 4 ? 2 : 3; half(l, g)) {
-            const Buffer &w = half_[l].w[g];
-            const float *f = reinterpret_cast<const float *>(w.as<char>() + half_matrix_bytes(N, K));
-            return gemm_half_nk(ctx_, split, w.as<uint16_t>(), HalfProduct{quant ? nullptr : f}, quant ? f : nullptr,
+            const Buffer &kept = half_[l].w[g];
+            char *w = kept ? kept.as<char>() : half_scratch_.as<char>();
+            if (!kept)
+                if (const int made = make_half_group(l, g, w); made != HM_OK) return made;
+            const float *f = reinterpret_cast<const float *>(w + half_matrix_bytes(N, K));
+            return gemm_half_nk(ctx_, split, reinterpret_cast<const uint16_t *>(w), HalfProduct{quant ? nullptr : f}, quant ? f : nullptr,
                                 quant ? half_scale_cols(N) : 0, out, n, K, N, MP, &parts);
         }
         if (!quant) return gemm_split_nk(ctx_, split, np, packed.as<uint16_t>(), out, n, K, N, MP, &parts);

@@ -345,6 +345,27 @@ def test_no_f16_copies_while_prompts_go_token_by_token(ctx, dtype):
     gm.close()
 
 
+@pytest.mark.parametrize("which", ["bf16", "q8_0", "q4_0_wide_vocab"])
+def test_a_smaller_budget_gives_the_f16_copies_back(ctx, which):
+    """Behind a first prompt: no copies within a budget of 0 (or one byte too few), and the bits that the resident ones gave, from
+    matrices made for every chunk; kept again when the budget allows it."""
+    cfg, mix = (synth_model.TINY, None) if which == "bf16" else _quant_case(which)
+    kw = {} if mix is None else dict(has_qk_norm=False, proj_dtypes=mix)
+    gm = synth_model.build_model(ctx, cfg, synth_model.synth_weights(cfg, 52, **kw), 96, **kw)
+    ids, default = synth.token_ids(16, 66, cfg.vocab_size), f16_copies(gm)
+    want = gm.prefill(ids)
+    for budget, held in ((0, 0), (default[0] - 1, 0), (default[0], default[0]), (0, 0), (1 << 30, default[0])):
+        gm.set_prefill_weight_cache(budget)
+        assert f16_copies(gm) == (held, default[1])
+        gm.reset_kv_cache()
+        assert np.array_equal(gm.prefill(ids), want)
+    gm.set_prefill_weight_cache(0)
+    gm.set_prefill_pieces(3)
+    gm.reset_kv_cache()
+    assert f16_copies(gm) == (0, 0) and logit_err(gm.prefill(ids), want) < TOL
+    gm.close()
+
+
 def test_prefill_needs_matching_widths_and_groups(ctx):
     """Block formats take the prompt pass when the widths are multiples of the 64-wide K tile and
     q|k|v, gate|up each multiply with one kind of activation; otherwise run_kv steps token by token."""
