@@ -1986,11 +1986,12 @@ int HfModel::make_half_group(int l, int g, char *dst) {
     return rc;
 }
 
-// Whether `need` bytes of copies are within the budget and leave enough of the device
+// Whether `need` bytes of copies are within the budget and leave half of the device free: a model made without them has a
+// slower prompt pass, and one that does not find its memory beside them cannot be made at all.
 bool HfModel::half_fits(size_t need) const {
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = total_b = 0;
-    return need <= prefill_weight_cache_bytes_ && need + total_b / 8 <= free_b;
+    return need <= prefill_weight_cache_bytes_ && need + total_b / 2 <= free_b;
 }
 
 // The f16 products' matrices, which a smaller budget had made again for every chunk, kept once more if they fit.

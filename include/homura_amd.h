@@ -428,7 +428,7 @@ int hm_model_set_prefill_min(hm_model *m, int n_tokens);
 int hm_model_set_prefill_pieces(hm_model *m, int pieces);
 int hm_model_set_prefill_f16(hm_model *m, int on);
 /* HBM the prompt pass may keep for copies of the projections (default 32 GiB): f16 copies of bf16, Q8_0 and Q4_0 projections (2 bytes
- * a weight), made by hm_model_finalize; for block-quantised models also the dequantised ones (three bf16
+ * a weight), made by hm_model_finalize where half of the device stays free; for block-quantised models also the dequantised ones (three bf16
  * pieces = 6 bytes per weight). If all projections fit, and an eighth of the device
  * stays free, each is dequantised on first use and kept; otherwise, or with 0, every chunk
  * dequantises them again into one scratch matrix. f16 copies that do not fit are not used (bf16 numbers as above); a budget made smaller

@@ -366,6 +366,21 @@ def test_a_smaller_budget_gives_the_f16_copies_back(ctx, which):
     gm.close()
 
 
+def test_no_f16_copies_where_they_would_take_the_room_of_another_model(ctx):
+    """With more than half of the device taken, a model is made without the copies, and its prompt pass takes the bf16 pieces."""
+    cfg = synth_model.TINY
+    weights, ids = synth_model.synth_weights(cfg, 52), synth.token_ids(16, 66, cfg.vocab_size)
+    rows = []
+    for taken in (1 << 20, 150 << 30):  # of 288 GB
+        other = ctx.empty(taken // 4)
+        gm = synth_model.build_model(ctx, cfg, weights, 96)
+        assert (f16_copies(gm)[1] == 0) == (taken >> 30 > 0)
+        rows.append(gm.prefill(ids))
+        gm.close()
+        other.free()
+    assert logit_err(rows[1], rows[0]) < TOL
+
+
 def test_prefill_needs_matching_widths_and_groups(ctx):
     """Block formats take the prompt pass when the widths are multiples of the 64-wide K tile and
     q|k|v, gate|up each multiply with one kind of activation; otherwise run_kv steps token by token."""
