@@ -60,13 +60,18 @@ int hm_test_fill_lds(hm_ctx *ctx, uint32_t word);
  * weight format on a chip of `cus` CUs, and the most that the product of m <= rows rows writes (all its K slices). Host only. */
 int hm_test_prompt_product(int hm_dtype, int rows, int m, int k, int n, int cus, long long *floats_held, long long *floats_written);
 
-/* Test support and timing: one product of the prompt pass with the row kernel ahead of it. front 0: x [m][k] f32 through RMSNorm
- * (weights norm_w [k], eps 1e-6); front 1: x [m][2 k] as (gate, up) pairs through SiLU(gate) * up. w: bf16 rows [n][k], or the raw
- * blocks of Q8_0 / Q4_0. half 0: three bf16 pieces, 1: two f16 pieces (HM_ERR_STATE where the weights do not take that), 2: one bf16 piece. All
- * pointers are device memory. The result comes as *parts <= 8 slices out [parts][m][n] to be added, row r then times
- * row_factor[r]. With us: the product alone, mean of `rounds` launches over `copies` copies of the weights in turn. */
-int hm_test_prompt_rows(hm_ctx *ctx, int front, const float *x, const float *norm_w, int dtype, const void *w, int half, int m, int k,
-                        int n, float *out, float *row_factor, int *parts, int copies, int rounds, float *us);
+/* Test support: the tile and K slices (at most max_parts) of a product of gemm_tiles_mfma.hip on a chip of `cus` CUs; the few-rows kernel's
+ * tile of 32 or 64 rows by 32 or 64 columns where that takes it. kind 0: two f16 pieces with column factors, 1: with block scales, 2: one bf16 piece.
+ * k a multiple of 64. Host only. */
+int hm_test_product_tiles(int kind, int m, int k, int n, int cus, int max_parts, int *tile_m, int *tile_n, int *slices);
+
+/* Test support: one product of the prompt pass with the row kernel ahead of it. front 0: x [m][k] f32 through RMSNorm (weights norm_w
+ * [k], eps 1e-6); front 1: x [m][2 k] f32 as (gate, up) pairs through SiLU(gate) * up; front 2: x [m][k] bf16 rows as one piece. w: bf16
+ * rows [n][k], or the raw blocks of Q8_0 / Q4_0. half 0: three bf16 pieces, 1: two f16 pieces (HM_ERR_STATE where the weights do not take
+ * that). All pointers are device memory. The result comes as *parts <= 8 slices out [parts][m][n] to be added, row r then times
+ * row_factor[r]. */
+int hm_test_prompt_rows(hm_ctx *ctx, int front, const void *x, const float *norm_w, int dtype, const void *w, int half, int m, int k,
+                        int n, float *out, float *row_factor, int *parts);
 
 /* Test support: the bytes of f16 weight copies that a transformer's prompt pass holds, and how many of its groups of projections
  * (q|k|v, o, gate|up, down of every layer) multiply with them. */
