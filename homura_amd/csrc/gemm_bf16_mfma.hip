@@ -68,11 +68,11 @@ struct TileRegs {
 };
 
 // M, N: logical sizes; K: length of the k loop; lda: row stride of A; Kb: k extent of B (k wraps at Kb)
-// kt_per_split: K tiles per grid.y slice (a multiple of the register ring depth)
-// ldb, ldc: row strides of B ([N][K] layout) and C
+// kt_per_split: K tiles per grid.y slice (a multiple of the register ring depth; gemm_bf16_mfma_kernel)
+// ldb: row stride of B ([N][K] layout)
 struct GemmDims {
     int M, N, K, lda, Kb, kt_per_split;
-    int ldb, ldc;
+    int ldb;
     homura::GroupLists lists;  // grouped products: B is one [N][ldb] matrix per group
     homura::GatedAct act;      // ACT
     const float *weight;       // ACT: [entries]
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_bf16_mfma_kernel(const uint
     const int nk = min(g.kt_per_split, (K + TK - 1) / TK - kt_first);
     const int nkp = (nk + DEPTH - 1) / DEPTH * DEPTH;
     const int kbase = kt_first * TK;
-    C += (size_t)blockIdx.y * M * g.ldc;
+    C += (size_t)blockIdx.y * M * g.N;
     TileRegs t[DEPTH];
     // B's k offset of the next tile to request: runs along with the loop and wraps at Kb (ALIGNED only)
     int kb_run = kbase % g.Kb;
@@ -311,9 +311,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_bf16_mfma_kernel(const uint
                 const int col = n0 + wn * 64 + j * 32 + l32;
                 const float sum = acc[i][j][v] + xch[((i * 2 + j) * 16 + v) * 64];
                 if (interior)
-                    __builtin_nontemporal_store(sum, C + (size_t)row * g.ldc + col);
+                    __builtin_nontemporal_store(sum, C + (size_t)row * g.N + col);
                 else if (row < M && col < N)
-                    __builtin_nontemporal_store(sum, C + (size_t)row * g.ldc + col);
+                    __builtin_nontemporal_store(sum, C + (size_t)row * g.N + col);
             }
 }
 
@@ -399,9 +399,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_dma_kernel(const uint16_t *
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
 
-    const int kt_first = blockIdx.y * g.kt_per_split;
-    const int nk = min(g.kt_per_split, K / TK - kt_first);
-    if constexpr (!GR) C += (size_t)blockIdx.y * M * g.ldc;
+    const int nk = K / TK;
 
     // this thread's two rows of A and of B: instruction j of wavefront w fills rows 8 (2 w + j) .. + 7
     const uint16_t *a_src[2], *b_src[2];
@@ -423,7 +421,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_dma_kernel(const uint16_t *
     // k offset of the next tile to request (scalar; the loop is short enough for its bookkeeping to
     // show in the run time). A tile past the end re-reads the last one (nobody multiplies it), so every
     // iteration issues the same four loads and the wait counts below are exact.
-    int koff = kt_first * TK;
+    int koff = 0;
     auto request_one = [&](int buf, int o) {  // load o of the four of a tile
         char *base = dma_lds + buf * (2 * TILE_BYTES) + wave_dst + (o >> 1) * 1024;
         const int k = min(koff, K - TK);
@@ -588,7 +586,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_dma_kernel(const uint16_t *
                 if ((l32 & 3) == 0 && row < M && col + 3 < N) *reinterpret_cast<uint32_t *>(out + col / 2) = word;
             }
         } else {
-            float *c_row = C + (size_t)entry * g.ldc;
+            float *c_row = C + (size_t)entry * g.N;
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const int col = n0 + wn * 64 + j * 32 + l32;
@@ -609,9 +607,10 @@ int gemm_dma_launch(hm_ctx *ctx, const char *who, dim3 grid, const uint16_t *a, 
 
 // a_pieces > 1: A is a split matrix [M][a_pieces * K] and the k loop runs over all its pieces against the same B
 // (B's k index wraps at K), so C is the sum of the pieces' products.
-// ksplit: the K slices of a product (a [N][K] operand in whole stages: at most that many, gemm_tiles_mfma.hip decides)
+// ksplit: the K slices of a product (a [N][K] operand in whole stages: at most that many, and gemm_tiles_mfma.hip decides; slices of
+// other products are gemm_bf16_mfma_kernel's)
 int gemm_launch(hm_ctx *ctx, const char *who, const uint16_t *a, const uint16_t *b, float *c, int M, int K,
-                int N, bool b_nk, int ksplit = 1, int *ksplit_used = nullptr, int ldc = 0, int a_pieces = 1) {
+                int N, bool b_nk, int ksplit = 1, int *ksplit_used = nullptr, int a_pieces = 1) {
     HM_CHECK_CTX(ctx);
     HM_REQUIRE(ctx, a && b && c, "%s: NULL pointer", who);
     HM_REQUIRE(ctx, M > 0 && N > 0 && K > 0 && K % 32 == 0, "%s: need M, N > 0 and K %% 32 == 0 (M=%d K=%d N=%d)", who,
@@ -628,11 +627,9 @@ int gemm_launch(hm_ctx *ctx, const char *who, const uint16_t *a, const uint16_t 
     g.K = a_pieces * K;
     g.lda = a_pieces * K;
     g.ldb = K;
-    g.ldc = ldc > 0 ? ldc : N;
-    HM_REQUIRE(ctx, g.ldc >= N, "%s: ldc %d below N %d", who, g.ldc, N);
     // Tiles of other sizes, and slices, go elsewhere; one slice of 128 x 128 tiles stays here, where four tiles are on their way instead
     // of three: 707 rows 576 -> 4512 9.5 us (10.1 there), 700 rows 2048 -> 4500 19.8 (21.8), 512 rows 2048 -> 8192 20.9 (21.5)
-    if (b_nk && K % TK == 0 && a_pieces == 1 && g.ldc == N) {
+    if (b_nk && K % TK == 0 && a_pieces == 1) {
         if (!homura::gemm_tiles_square(M, K, N, ctx->num_cus, ksplit_used ? ksplit : 1))
             return homura::gemm_tiles_bf16(ctx, a, b, c, M, K, N, ksplit, ksplit_used);
         ksplit = 1;
@@ -642,7 +639,7 @@ int gemm_launch(hm_ctx *ctx, const char *who, const uint16_t *a, const uint16_t 
     g.kt_per_split = ((nk_total + ksplit - 1) / ksplit + GEMM_DEPTH - 1) / GEMM_DEPTH * GEMM_DEPTH;
     const int slices = (nk_total + g.kt_per_split - 1) / g.kt_per_split;
     if (ksplit_used) *ksplit_used = slices;
-    const dim3 grid((unsigned)tiles, (unsigned)slices);
+    const dim3 grid((unsigned)tiles, (unsigned)slices);  // (one slice wherever the loads go to LDS directly)
     const bool aligned = g.K % TK == 0 && g.Kb % TK == 0;
     if (b_nk && aligned) {
         const int rc = gemm_dma_launch<false>(ctx, who, grid, a, b, c, g);
@@ -668,8 +665,6 @@ int homura::gemm_grouped_dma(hm_ctx *ctx, const uint16_t *d_a, const uint16_t *d
     GemmDims g{};
     g.N = N;
     g.K = g.Kb = g.lda = g.ldb = K;
-    g.ldc = N;
-    g.kt_per_split = K / TK;
     g.lists = lists;
     int rc;
     if (act) {
@@ -710,7 +705,7 @@ int homura::gemm_split_split_nk(hm_ctx *ctx, const uint16_t *d_a_split, const ui
 int homura::gemm_split_kn(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, const uint16_t *d_b_kn, float *d_c, int M,
                           int K, int N) {
     HM_REQUIRE(ctx, pieces >= 1 && pieces <= 3, "gemm_split_kn: %d pieces (1..3)", pieces);
-    return gemm_launch(ctx, "gemm_split_kn", d_a_split, d_b_kn, d_c, M, K, N, false, 1, nullptr, 0, pieces);
+    return gemm_launch(ctx, "gemm_split_kn", d_a_split, d_b_kn, d_c, M, K, N, false, 1, nullptr, pieces);
 }
 
 extern "C" int hm_gemm_bf16(hm_ctx *ctx, const uint16_t *d_a_mk, const uint16_t *d_b_kn, float *d_c,
