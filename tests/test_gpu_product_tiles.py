@@ -143,6 +143,36 @@ def test_scales_follow_the_values(ctx, dtype):
     assert np.all(np.linalg.norm(got - want, axis=1) <= 1e-6 * np.linalg.norm(want, axis=1))
 
 
+def outliers(ratio, dtype, front):
+    """Rows with a few values `ratio` times the others', and weights that bring their products down to the others' size"""
+    rng = np.random.default_rng(12)
+    m, k, n = 150, 1024, 400
+    raw, w = weights(dtype, n, k, rng)
+    norm_w = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    x = rng.standard_normal((m, k * (1 + front))).astype(np.float32)
+    if front:
+        x[:, 2 * np.arange(5, k, 97) + 1] *= ratio
+        w = w.copy()
+        w[:, 5::97] /= ratio  # (a power of two)
+        if dtype == DTYPE_BF16:
+            raw, w = bf16(w)
+    else:
+        x[:, 5::97] *= ratio
+        norm_w[5::97] /= ratio
+    return x, norm_w, raw, w, n
+
+
+@pytest.mark.parametrize("front,dtype", [(0, DTYPE_BF16), (0, DTYPE_Q8_0), (1, DTYPE_BF16)])
+def test_rows_with_outliers(ctx, front, dtype):
+    """Values 2^13 times the others in a row, which two f16 pieces hold with every bit that three bf16 pieces do (the second piece ends
+    2^39 below the largest value's bound, 24 bits below a value 2^15 below it). The bound as above."""
+    x, norm_w, raw, w, n = outliers(2.0 ** 13, dtype, front)
+    want = rows_of(front, x, norm_w) @ w.T.astype(np.float64)
+    err = [np.linalg.norm(product(ctx, front, x, norm_w, dtype, raw, n, half) - want) / np.linalg.norm(want) for half in (1, 0)]
+    print(f"front {front} dtype {dtype}: {err[0]:.2e}, three bf16 pieces {err[1]:.2e}", flush=True)
+    assert err[0] <= 4e-7 and err[0] <= 1.25 * err[1]
+
+
 @pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_Q8_0])
 def test_rows_whose_squares_overflow(ctx, dtype):
     """A finite row whose sum of squares f32 cannot hold is divided by infinity: zeros, as the three bf16 pieces and the decode kernels
