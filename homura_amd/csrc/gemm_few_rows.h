@@ -30,8 +30,9 @@ inline bool few_rows_pays(int pieces, int M, int N, int cus) {
 int few_rows_slices(int M, int K, int N, int cus, int max_parts);
 
 // C[M][N] f32 (row stride ldc) = (sum of the pieces of A [M][pieces K])  x  B [N][K]^T, M <= FEW_ROWS, K % 32 == 0; with d_scales
-// (pieces = 3) B holds the integers of a block format and d_scales [K / 32][npad] the scale of every 32-wide block, npad >= N
+// (pieces = 3, or 2 with half) B holds the integers of a block format and d_scales [K / 32][npad] the scale of every 32-wide block, npad >= N
 // rounded up to 128. With parts the result may come as up to max_parts K slices, slice s at d_c + s * M * ldc.
+// half: f16 operands (gemm_half_nk).
 int gemm_few_rows(hm_ctx *ctx, const uint16_t *d_a_split, int pieces, const uint16_t *d_b_nk, const float *d_scales, int npad,
                   float *d_c, int M, int K, int N, int max_parts, int *parts, int ldc, const HalfProduct *half = nullptr);
 

@@ -1,15 +1,18 @@
 // The prompt pass's products on f16 matrix instructions: every f32 activation as two f16 pieces against weights that are f16
 // without loss, two matrix instructions where three bf16 pieces take three.
 //
-// x 2^e = p0 + p1, p0 = f16(x 2^e), p1 = f16(x 2^e - p0): 23 to 24 significant bits down to 2^-24, f16's last subnormal. The
-// exponents e keep p0 in range whatever the input: a bound on |x| is known where the weights are, and x 2^e stays below 2^15.
+// x 2^e = p0 + p1, p0 = f16(x 2^e), p1 = f16(x 2^e - p0). p1 ends at 2^-24, f16's last subnormal: 23 to 24 significant bits of a
+// scaled value of 2^-1 and more, which is 2^15 below the bound, and a bit less with every binade below that (three bf16 pieces hold all 24 at
+// any size). Rows with outliers of 2^13 times their other values, brought down by their weights, come out as with three bf16 pieces
+// (errors 0.9 of theirs); of 2^16 1.2 to 1.6 times, of 2^18 4 to 6 times as far off. The exponents e keep p0 in range whatever the finite
+// input: a bound on |x| is known where the weights are, and x 2^e stays below 2^15.
 //   a norm's output       |x_k| <= sqrt(dim) |w_k|                      one e per column, folded into the norm's weights
 //   attention's output    a mean of value rows, |v_j| <= sqrt(dim) |W_v[j] o w|_2 + |b_j| (Cauchy-Schwarz)   one e per value column
 //   SiLU(gate) up         no useful bound ahead                         one e per row, from the row's maximum
 // What is multiplied into a column of the activations is divided out of that column of the weights, so a product needs one
 // factor per output row of the weights, 2^-r, which also puts the row's largest weight at 2^14 .. 2^15. All factors are powers
 // of two. A matrix takes this way only if every one of its weights is then an f16 exactly (bf16 weights: 31 binades of a row,
-// Q8_0 / Q4_0 integers: 16 binades of a block's columns); otherwise it keeps the three bf16 pieces.
+// Q8_0 / Q4_0 integers: 24 binades of a block's columns); otherwise it keeps the three bf16 pieces.
 #pragma once
 
 #include <cstdint>

@@ -3,11 +3,11 @@
 //
 // The reference multiplies f32 activations by bf16 weights (make_mixed_matmul_region,
 // src/graph_builder/emit_linalg.rs:2224-2307). The MFMA takes 16-bit operands on both sides, so every f32 activation x is
-// carried as pieces: two f16 pieces where the weights are f16 without loss (half_weights.h), and otherwise bf16 pieces, p0 = bf16(x), p1 = bf16(x - p0), p2 = bf16(x - p0 - p1);
-// the products of the pieces are summed in the f32 accumulator. Two pieces keep 16 significant bits
-// of x, three keep all 24, which is what the path uses by default: K and V rows are rounded to bf16
-// when they enter the cache, and activations that are off in the 17th bit flip that rounding for
-// a few elements per row.
+// carried as pieces: two f16 pieces where the weights are f16 without loss (half_weights.h), and otherwise bf16 pieces,
+// p0 = bf16(x), p1 = bf16(x - p0), p2 = bf16(x - p0 - p1);
+// the products of the pieces are summed in the f32 accumulator. Two bf16 pieces keep 16 significant bits
+// of x, which is not the default: K and V rows are rounded to bf16 when they enter the cache, and activations that are off in the
+// 17th bit flip that rounding for a few elements per row.
 // A "split" matrix is [rows][pieces * dim] bf16: piece p in columns [p * dim, (p + 1) * dim).
 #pragma once
 

@@ -606,7 +606,8 @@ class HfModel(DecoderModel):
         self._check(self.lib.hm_model_set_prefill_f16(self.h, int(on)))
 
     def set_prefill_weight_cache(self, nbytes: int):
-        """Block-quantised models: HBM the prompt pass may keep for dequantised projections (0 = none)."""
+        """HBM the prompt pass may keep for f16 copies of the projections and, of block-quantised models, for the dequantised ones
+        (0 = none; hm_model_set_prefill_weight_cache)."""
         self._check(self.lib.hm_model_set_prefill_weight_cache(self.h, nbytes))
 
 

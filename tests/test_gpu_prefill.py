@@ -13,8 +13,8 @@ from homura_amd.runtime import DTYPE_BF16, DTYPE_Q8_0
 pytestmark = pytest.mark.gpu
 
 # Logit metric of this file: largest absolute difference over the largest |logit| of the reference,
-# bound 2e-3. The arithmetic itself agrees to a few 1e-6 of the logit scale (three bf16 pieces carry
-# every bit of the f32 activations). What is left are K/V elements that land on the other side of a
+# bound 2e-3. The arithmetic itself agrees to a few 1e-6 of the logit scale (two f16 pieces carry
+# 23 to 24 bits of the f32 activations, three bf16 pieces every bit). What is left are K/V elements that land on the other side of a
 # bf16 rounding boundary when they enter the cache, because the matrix cores sum in another order than
 # the oracle: such an element is off by one bf16 ulp (0.4%), and with the few cached rows of these
 # tests (softmax weights of 0.01-1 per row) one of them moves logits by up to ~4e-4 of their scale.
