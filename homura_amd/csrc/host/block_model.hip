@@ -1551,6 +1551,7 @@ int BlockModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         const Rope *rope = layer_rope_[li];
         rc = prefill_mixer((int)run, li, rope ? rope->cos.as<float>() : nullptr, rope ? rope->sin.as<float>() : nullptr, n, past, &y_parts);
         if (rc != HM_OK) return rc;
+        if (run + 1 == runs_.size() && !h_logits && !p.capture) break;  // the rows behind the last mixer have no reader
         pending = &l.norm1b;
         if (s.ff.width) {
             if ((rc = rows(cfg_.pre_norms ? l.norm2.ptr() : nullptr, np, nullptr)) != HM_OK) return rc;

@@ -299,6 +299,20 @@ def test_a_new_request_does_not_see_the_last_one(ctx):
     m.close()
 
 
+def test_a_prompt_without_logits_leaves_the_same_state(ctx):
+    """The feed-forward behind the last mixer has no reader then."""
+    cfg = bf.config([bf.attn(), bf.recurrence(), bf.scan(ff=50)])
+    m = bf.build(ctx, cfg, bf.weights(cfg), 128, DTYPE_BF16)
+    a, rows = tokens(cfg, 60), []
+    for want in (True, False):
+        m.reset_kv_cache()
+        m.prefill(a[:40], want_logits=want)
+        m.prefill(a[40:57], want_logits=want)
+        rows.append(np.concatenate([m.run_kv(a[i:i + 1]) for i in range(57, 60)]))
+    assert np.array_equal(rows[0], rows[1])
+    m.close()
+
+
 def test_cache_is_full_when_it_is(ctx):
     cfg = bf.config([bf.scan(), bf.attn()])
     m = bf.build(ctx, cfg, bf.weights(cfg), 20, DTYPE_F32)

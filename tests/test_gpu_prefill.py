@@ -155,6 +155,28 @@ def _quant_case(which):
     }[which]
 
 
+@pytest.mark.parametrize("which", ["bf16", "q8_0", "q4_k_m_mix"])
+def test_a_prompt_without_logits_leaves_the_same_cache(ctx, which):
+    """Without logits the pass ends with the last layer's cache rows: the steps behind it are those behind a pass with logits,
+    bit for bit, also where a second portion attends to the first."""
+    if which == "bf16":
+        cfg, mix, qkn = synth_model.TINY, None, True
+    else:
+        (cfg, mix), qkn = _quant_case(which), False
+    weights = synth_model.synth_weights(cfg, 1718, has_qk_norm=qkn, proj_dtypes=mix)
+    m = synth_model.build_model(ctx, cfg, weights, 128, has_qk_norm=qkn, proj_dtypes=mix)
+    ids = synth.token_ids(19, 75, cfg.vocab_size)
+    rows = []
+    for want in (True, False):
+        m.reset_kv_cache()
+        m.prefill(ids[:40], want_logits=want)
+        m.prefill(ids[40:71], want_logits=want)
+        assert m.kv_cache_len() == 71
+        rows.append(np.concatenate([m.run_kv(ids[i:i + 1]) for i in range(71, 75)]))
+    assert np.array_equal(rows[0], rows[1])
+    m.close()
+
+
 @pytest.mark.parametrize("which,past,n", [("q8_0", 0, 37), ("q4_0_wide_vocab", 30, 70), ("q4_k", 0, 50), ("q6_k", 17, 33),
                                           ("q4_k_m_mix", 40, 130), ("q8_0_and_k_quants_by_group", 0, 64)])
 def test_quantised_prefill_logits_and_following_decode(ctx, which, past, n):
