@@ -48,7 +48,7 @@ constexpr int CT = 256;     // communicating threads
 constexpr int SPIN_MAX = 1 << 20;
 constexpr int MAX_LAYERS = 64;
 
-template <int HIDDEN_, int H_, int KVH_, int HD_, int INTER_, int NWG_, int NR_ = 4, int XR_ = 0>
+template <int HIDDEN_, int H_, int KVH_, int HD_, int INTER_, int NWG_, int NR_ = 4, int XR_ = 0, bool ALL_ = false>
 struct Geo {
     static constexpr int HIDDEN = HIDDEN_, H = H_, KVH = KVH_, HD = HD_, INTER = INTER_, NWG = NWG_;
     static constexpr int G = H / KVH, QD = H * HD, KVD = KVH * HD, NQKV = QD + 2 * KVD;
@@ -69,7 +69,11 @@ struct Geo {
     static constexpr int NR = NR_;                             // row rounds a wavefront keeps in registers
     static constexpr int LPR = HD / 8, RPI = WAVE / LPR;       // lanes per cache row, rows per load
     static constexpr int XR = XR_;                             // further rounds, streamed inside the attention phase
-    static constexpr int MAX_KV = SPH * (NR + XR) * NCW * RPI;
+    // Short caches: every workgroup of a KV head attends over all of its cached rows (the registers hold them, the new row comes on
+    // top). Nothing is split, so nothing is folded: two of a layer's six exchanges fall away.
+    static constexpr bool ALL = ALL_;
+    static constexpr int MAX_KV = ALL ? NR * NCW * RPI + 1 : SPH * (NR + XR) * NCW * RPI;
+    static_assert(!ALL || XR == 0, "short caches are held in registers");
     static constexpr int FPW = QD / NWG;                       // folded attention outputs per workgroup
     static constexpr int PART = G * HD + 2 * G;                // one split's partial: o[G][HD], (m, l)[G]
     static constexpr int NJ = HIDDEN / CT;                     // hidden elements per communicating thread
@@ -788,9 +792,22 @@ struct SliceRows<FUSED_WF_K8, R, KS, KTOT> {
 template <class GE>
 struct Split {
     int kh, split, nsl, n0, cnt, cached;
-    bool owner;
+    bool attends;  // has rows to attend over
+    bool owner;    // among them the new one
+    bool appends;  // and writes it to the cache
     __device__ Split(int wg, int pos) {
         const int kv_len = pos + 1;
+        if constexpr (GE::ALL) {
+            kh = wg % GE::KVH;
+            split = wg / GE::KVH;
+            nsl = 1;
+            n0 = 0;
+            cnt = kv_len;
+            cached = pos;
+            attends = owner = true;
+            appends = split == 0;
+            return;
+        }
         const int chunk = (kv_len + GE::SPH - 1) / GE::SPH;
         nsl = (kv_len + chunk - 1) / chunk;
         kh = wg % GE::KVH;
@@ -801,6 +818,8 @@ struct Split {
         owner = split == nsl - 1;  // holds row `pos`, which is not in the cache yet
         cached = min(cnt, pos - n0);
         if (cached < 0) cached = 0;
+        attends = split < nsl;
+        appends = owner;
     }
 };
 
@@ -1009,7 +1028,7 @@ __device__ __forceinline__ void compute_role(const FusedDecodeArgs &a, Lds<GE> &
         //    merge the four. ──
         wg_barrier();
         load_wq(nx, 0, WQ_EARLY);
-        if (sp.split < sp.nsl) {
+        if (sp.attends) {
             float qv[G][8];
 #pragma unroll
             for (int g = 0; g < G; g++) lds_x8(sm.qs[g], dl * 8, qv[g]);
@@ -1474,7 +1493,7 @@ __device__ __forceinline__ void comm_role(const FusedDecodeArgs &a, Lds<GE> &sm,
         // ── into attention: this KV head's raw q rows (and k, v for the split that holds the new row),
         //    QK-norm + RoPE, cache append (reference src/hf/emitter.rs:629-649, src/runtime.rs:521-568) ──
         ps.where = 2u | (uint32_t)l << 4 | (uint32_t)wg << 12;
-        if (sp.split < sp.nsl) {
+        if (sp.attends) {
             for (int t = cwv; t < G + 2; t += 4) {
                 if (t >= G && !sp.owner) continue;
                 int unit[1] = {t * HD / 2 + lane};
@@ -1501,8 +1520,10 @@ __device__ __forceinline__ void comm_role(const FusedDecodeArgs &a, Lds<GE> &sm,
                     if (lane < HALF) {  // rounded to bf16 once; cache and this step use the same values
                         uint16_t *dst = cur.kcache + row_off;
                         const uint16_t r_lo = f32_to_bf16_rne_dev(lo), r_hi = f32_to_bf16_rne_dev(hi);
-                        dst[lane] = r_lo;
-                        dst[lane + HALF] = r_hi;
+                        if (sp.appends) {
+                            dst[lane] = r_lo;
+                            dst[lane + HALF] = r_hi;
+                        }
                         sm.knew[lane] = __uint_as_float((uint32_t)r_lo << 16);
                         sm.knew[lane + HALF] = __uint_as_float((uint32_t)r_hi << 16);
                     }
@@ -1510,7 +1531,7 @@ __device__ __forceinline__ void comm_role(const FusedDecodeArgs &a, Lds<GE> &sm,
                     uint16_t *dst = cur.vcache + row_off;
                     for (int i = lane; i < HD; i += WAVE) {
                         const uint16_t r = f32_to_bf16_rne_dev(sm.rowbuf[t][i]);
-                        dst[i] = r;
+                        if (sp.appends) dst[i] = r;
                         sm.vnew[i] = __uint_as_float((uint32_t)r << 16);
                     }
                 }
@@ -1521,136 +1542,162 @@ __device__ __forceinline__ void comm_role(const FusedDecodeArgs &a, Lds<GE> &sm,
         mark();
         wg_barrier();
         mark();
-        if (sp.split < sp.nsl) {
-            // merge the compute wavefronts' partials (one output per thread) and publish the split's
-            // (o, max, sum): o = sum_w exp(m_w - M) * (sum over w's row groups), in wavefront order. The
-            // threads of a head's first two outputs also publish the head's (max, sum): same weights.
+        if constexpr (GE::ALL) {
+            // merge the compute wavefronts' partials as below; the divided outputs are this workgroup's K slice of the O phase already
+            static_assert(GE::KSO == G * HD, "the O projection's slice is this KV head's outputs");
             for (int i = ct; i < G * HD; i += CT) {
                 const int g = i / HD, d = i % HD;
-                float mw[NCW], f[NCW], M = -INFINITY;
+                float mw[NCW], M = -INFINITY;
 #pragma unroll
                 for (int w = 0; w < NCW; w++) {
                     mw[w] = sm.wstat[w][g][0];
                     M = fmaxf(M, mw[w]);
                 }
-                float v = 0.f;
+                float v = 0.f, den = 0.f;
 #pragma unroll
                 for (int w = 0; w < NCW; w++) {
-                    f[w] = mw[w] == -INFINITY ? 0.f : __expf(mw[w] - M);
+                    const float f = mw[w] == -INFINITY ? 0.f : __expf(mw[w] - M);
                     float t = 0.f;
 #pragma unroll
                     for (int sb = 0; sb < GE::RPI; sb++) t += sm.part[w * GE::RPI + sb][g][d];
-                    v += f[w] * t;
+                    v += f * t;
+                    den += f * sm.wstat[w][g][1];
                 }
-                st_slot(lp, sp.split * GE::PART + i, v, tag, near_g);
-                if (d < 2) {
-                    float st = M;
-                    if (d == 1) {
-                        st = 0.f;
-#pragma unroll
-                        for (int w = 0; w < NCW; w++) st += f[w] * sm.wstat[w][g][1];
+                sm.attn[XLay<WF>::pos(i, GE::KSO)] = v * __builtin_amdgcn_rcpf(den);
+            }
+            mark();
+        } else {
+            if (sp.split < sp.nsl) {
+                // merge the compute wavefronts' partials (one output per thread) and publish the split's
+                // (o, max, sum): o = sum_w exp(m_w - M) * (sum over w's row groups), in wavefront order. The
+                // threads of a head's first two outputs also publish the head's (max, sum): same weights.
+                for (int i = ct; i < G * HD; i += CT) {
+                    const int g = i / HD, d = i % HD;
+                    float mw[NCW], f[NCW], M = -INFINITY;
+    #pragma unroll
+                    for (int w = 0; w < NCW; w++) {
+                        mw[w] = sm.wstat[w][g][0];
+                        M = fmaxf(M, mw[w]);
                     }
-                    st_slot(lp, sp.split * GE::PART + G * HD + 2 * g + d, st, tag, near_g);
+                    float v = 0.f;
+    #pragma unroll
+                    for (int w = 0; w < NCW; w++) {
+                        f[w] = mw[w] == -INFINITY ? 0.f : __expf(mw[w] - M);
+                        float t = 0.f;
+    #pragma unroll
+                        for (int sb = 0; sb < GE::RPI; sb++) t += sm.part[w * GE::RPI + sb][g][d];
+                        v += f[w] * t;
+                    }
+                    st_slot(lp, sp.split * GE::PART + i, v, tag, near_g);
+                    if (d < 2) {
+                        float st = M;
+                        if (d == 1) {
+                            st = 0.f;
+    #pragma unroll
+                            for (int w = 0; w < NCW; w++) st += f[w] * sm.wstat[w][g][1];
+                        }
+                        st_slot(lp, sp.split * GE::PART + G * HD + 2 * g + d, st, tag, near_g);
+                    }
                 }
             }
-        }
 
-        // ── fold the splits of this KV head for FPW of its outputs (one wavefront) ──
-        ps.where = 3u | (uint32_t)l << 4 | (uint32_t)wg << 12;
-        constexpr bool FOLD_HALVES = GE::SPH <= 32 && (GE::FPW / 2) % 2 == 0;
-        if (cwv == 0 && FOLD_HALVES) {
-            // lanes 0-31 fold the first half of the workgroup's outputs over the (at most 32) splits, lanes 32-63
-            // the second half: half the loads and half the sums a lane, and a sum ends inside 32 lanes
-            constexpr int HU = GE::FPW / 4;  // 16-byte units of outputs per lane
-            const int o0 = sp.split * GE::FPW;
-            const int t = o0 / HD, d0 = o0 % HD;
-            const int half = lane >> 5, sl = lane & 31;
-            const int pbase = sl * GE::PART;
-            int unit[HU + 1];
-            bool on[HU + 1];
-            u32x4 w[HU + 1];
-#pragma unroll
-            for (int u = 0; u < HU; u++) {
-                unit[u] = (pbase + t * HD + d0) / 2 + half * HU + u;
-                on[u] = sl < sp.nsl;
-            }
-            unit[HU] = (pbase + G * HD + 2 * t) / 2;
-            on[HU] = sl < sp.nsl;
-            poll_units<HU + 1>(ps, lp, unit, on, tag, w);
-            const float m_s = on[HU] ? __uint_as_float(w[HU].x) : -INFINITY;
-            const float l_s = on[HU] ? __uint_as_float(w[HU].z) : 0.f;
-            const float m = wave_max(m_s);  // both halves hold the same maxima
-            const float f = on[HU] ? __expf(m_s - m) : 0.f;
-            float red[2 * HU + 1];  // the sum of the splits' sums, then this half's weighted outputs
-            red[0] = f * l_s;
-#pragma unroll
-            for (int u = 0; u < HU; u++) {
-                red[1 + 2 * u] = f * __uint_as_float(w[u].x);
-                red[2 + 2 * u] = f * __uint_as_float(w[u].z);
-            }
-#pragma unroll
-            for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0xB1, 0xF>(red[i], 0.f);
-#pragma unroll
-            for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0x4E, 0xF>(red[i], 0.f);
-#pragma unroll
-            for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0x141, 0xF>(red[i], 0.f);
-#pragma unroll
-            for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0x140, 0xF>(red[i], 0.f);
-#pragma unroll
-            for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0x142, 0xA>(red[i], 0.f);  // lanes 31 and 63: the halves' totals
-            const int e = lane % (2 * HU);  // lane l < FPW publishes output l: half l / (2 HU), element l % (2 HU)
-            float num = 0.f, den = 0.f;
-#pragma unroll
-            for (int hh = 0; hh < 2; hh++) {
-                const float d0v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(red[0]), 31 + 32 * hh));
-#pragma unroll
-                for (int k = 0; k < 2 * HU; k++) {
-                    const float nv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(red[1 + k]), 31 + 32 * hh));
-                    if (lane / (2 * HU) == hh && e == k) {
-                        num = nv;
-                        den = d0v;
+            // ── fold the splits of this KV head for FPW of its outputs (one wavefront) ──
+            ps.where = 3u | (uint32_t)l << 4 | (uint32_t)wg << 12;
+            constexpr bool FOLD_HALVES = GE::SPH <= 32 && (GE::FPW / 2) % 2 == 0;
+            if (cwv == 0 && FOLD_HALVES) {
+                // lanes 0-31 fold the first half of the workgroup's outputs over the (at most 32) splits, lanes 32-63
+                // the second half: half the loads and half the sums a lane, and a sum ends inside 32 lanes
+                constexpr int HU = GE::FPW / 4;  // 16-byte units of outputs per lane
+                const int o0 = sp.split * GE::FPW;
+                const int t = o0 / HD, d0 = o0 % HD;
+                const int half = lane >> 5, sl = lane & 31;
+                const int pbase = sl * GE::PART;
+                int unit[HU + 1];
+                bool on[HU + 1];
+                u32x4 w[HU + 1];
+    #pragma unroll
+                for (int u = 0; u < HU; u++) {
+                    unit[u] = (pbase + t * HD + d0) / 2 + half * HU + u;
+                    on[u] = sl < sp.nsl;
+                }
+                unit[HU] = (pbase + G * HD + 2 * t) / 2;
+                on[HU] = sl < sp.nsl;
+                poll_units<HU + 1>(ps, lp, unit, on, tag, w);
+                const float m_s = on[HU] ? __uint_as_float(w[HU].x) : -INFINITY;
+                const float l_s = on[HU] ? __uint_as_float(w[HU].z) : 0.f;
+                const float m = wave_max(m_s);  // both halves hold the same maxima
+                const float f = on[HU] ? __expf(m_s - m) : 0.f;
+                float red[2 * HU + 1];  // the sum of the splits' sums, then this half's weighted outputs
+                red[0] = f * l_s;
+    #pragma unroll
+                for (int u = 0; u < HU; u++) {
+                    red[1 + 2 * u] = f * __uint_as_float(w[u].x);
+                    red[2 + 2 * u] = f * __uint_as_float(w[u].z);
+                }
+    #pragma unroll
+                for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0xB1, 0xF>(red[i], 0.f);
+    #pragma unroll
+                for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0x4E, 0xF>(red[i], 0.f);
+    #pragma unroll
+                for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0x141, 0xF>(red[i], 0.f);
+    #pragma unroll
+                for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0x140, 0xF>(red[i], 0.f);
+    #pragma unroll
+                for (int i = 0; i < 2 * HU + 1; i++) red[i] += dpp_move<0x142, 0xA>(red[i], 0.f);  // lanes 31 and 63: the halves' totals
+                const int e = lane % (2 * HU);  // lane l < FPW publishes output l: half l / (2 HU), element l % (2 HU)
+                float num = 0.f, den = 0.f;
+    #pragma unroll
+                for (int hh = 0; hh < 2; hh++) {
+                    const float d0v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(red[0]), 31 + 32 * hh));
+    #pragma unroll
+                    for (int k = 0; k < 2 * HU; k++) {
+                        const float nv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(red[1 + k]), 31 + 32 * hh));
+                        if (lane / (2 * HU) == hh && e == k) {
+                            num = nv;
+                            den = d0v;
+                        }
                     }
                 }
+                if (lane < GE::FPW) st_slot(la, o0 + lane, num * __builtin_amdgcn_rcpf(den), tag, near_g);
+            } else if (cwv == 0) {
+                constexpr int FU = GE::FPW / 2;
+                const int o0 = sp.split * GE::FPW;  // first output, counted inside the KV head's G * HD
+                const int t = o0 / HD, d0 = o0 % HD;
+                const int pbase = lane * GE::PART;
+                int unit[FU + 1];
+                bool on[FU + 1];
+                u32x4 w[FU + 1];
+    #pragma unroll
+                for (int u = 0; u < FU; u++) {
+                    unit[u] = (pbase + t * HD + d0) / 2 + u;
+                    on[u] = lane < sp.nsl;
+                }
+                unit[FU] = (pbase + G * HD + 2 * t) / 2;
+                on[FU] = lane < sp.nsl;
+                poll_units<FU + 1>(ps, lp, unit, on, tag, w);
+                const float m_s = on[FU] ? __uint_as_float(w[FU].x) : -INFINITY;
+                const float l_s = on[FU] ? __uint_as_float(w[FU].z) : 0.f;
+                const float m = wave_max(m_s);
+                const float f = on[FU] ? __expf(m_s - m) : 0.f;
+                float red[2 * FU + 1];  // the sum of the splits' sums, then the FPW weighted outputs
+                red[0] = f * l_s;
+    #pragma unroll
+                for (int u = 0; u < FU; u++) {
+                    red[1 + 2 * u] = f * __uint_as_float(w[u].x);
+                    red[2 + 2 * u] = f * __uint_as_float(w[u].z);
+                }
+                wave_sum_n<2 * FU + 1>(red);
+                float mine = 0.f;
+    #pragma unroll
+                for (int e = 0; e < GE::FPW; e++) mine = lane == e ? red[1 + e] : mine;
+                if (lane < GE::FPW) st_slot(la, o0 + lane, mine * __builtin_amdgcn_rcpf(red[0]), tag, near_g);
             }
-            if (lane < GE::FPW) st_slot(la, o0 + lane, num * __builtin_amdgcn_rcpf(den), tag, near_g);
-        } else if (cwv == 0) {
-            constexpr int FU = GE::FPW / 2;
-            const int o0 = sp.split * GE::FPW;  // first output, counted inside the KV head's G * HD
-            const int t = o0 / HD, d0 = o0 % HD;
-            const int pbase = lane * GE::PART;
-            int unit[FU + 1];
-            bool on[FU + 1];
-            u32x4 w[FU + 1];
-#pragma unroll
-            for (int u = 0; u < FU; u++) {
-                unit[u] = (pbase + t * HD + d0) / 2 + u;
-                on[u] = lane < sp.nsl;
-            }
-            unit[FU] = (pbase + G * HD + 2 * t) / 2;
-            on[FU] = lane < sp.nsl;
-            poll_units<FU + 1>(ps, lp, unit, on, tag, w);
-            const float m_s = on[FU] ? __uint_as_float(w[FU].x) : -INFINITY;
-            const float l_s = on[FU] ? __uint_as_float(w[FU].z) : 0.f;
-            const float m = wave_max(m_s);
-            const float f = on[FU] ? __expf(m_s - m) : 0.f;
-            float red[2 * FU + 1];  // the sum of the splits' sums, then the FPW weighted outputs
-            red[0] = f * l_s;
-#pragma unroll
-            for (int u = 0; u < FU; u++) {
-                red[1 + 2 * u] = f * __uint_as_float(w[u].x);
-                red[2 + 2 * u] = f * __uint_as_float(w[u].z);
-            }
-            wave_sum_n<2 * FU + 1>(red);
-            float mine = 0.f;
-#pragma unroll
-            for (int e = 0; e < GE::FPW; e++) mine = lane == e ? red[1 + e] : mine;
-            if (lane < GE::FPW) st_slot(la, o0 + lane, mine * __builtin_amdgcn_rcpf(red[0]), tag, near_g);
+            mark();
         }
-        mark();
 
         // ── into the O phase ──
         ps.where = 4u | (uint32_t)l << 4 | (uint32_t)wg << 12;
-        stage_group(la, GE::KSO / 2, tag, sm.attn);
+        if constexpr (!GE::ALL) stage_group(la, GE::KSO / 2, tag, sm.attn);
         wg_barrier();
         mark();
         wg_barrier();
@@ -1876,6 +1923,18 @@ using GeoQwen3_0p6bStream = Geo<1024, 16, 8, 128, 3072, 256, 8, 56>;
 using GeoSmallStream = Geo<512, 4, 2, 128, 1024, 64, 8, 56>;
 using GeoSmallQStream = Geo<1024, 8, 4, 128, 1024, 64, 8, 56>;
 
+// Short caches: 2, 3, 5 or 7 row rounds hold all of up to 32, 48, 80 or 112 cached rows. What a layer saves is the partials' exchange and the
+// folded heads'; what it pays are the rounds, about 6 us a token each (one pass over all of them). us a token at 14 / 41 / 72 / 105 cached
+// rows, the even cut's three rounds before: bf16 377 -> 331 / 335 / 349 / 364, Q8_0 360 -> 317 / 322 / 332 / 338, Q4_0 354 -> 309 / 313 / 325 /
+// 335, K-quants 413 -> 374 / 379 / 394 / 408. Six rounds (two passes) 357 where seven take 361, eight 370. Cut into runs of 32 to 64 rows whose
+// partials every workgroup folds for itself (one exchange less instead of two, up to 512 rows): 378 .. 390.
+template <int NR>
+using GeoQwen3_0p6bAll = Geo<1024, 16, 8, 128, 3072, 256, NR, 0, true>;
+template <int NR>
+using GeoSmallAll = Geo<512, 4, 2, 128, 1024, 64, NR, 0, true>;
+template <int NR>
+using GeoSmallQAll = Geo<1024, 8, 4, 128, 1024, 64, NR, 0, true>;
+
 template <class GE>
 bool shape_is(const FusedShape &s) {
     return s.hidden == GE::HIDDEN && s.heads == GE::H && s.kv_heads == GE::KVH && s.head_dim == GE::HD &&
@@ -1899,6 +1958,12 @@ Instance instance() {
 // live_rows = 0, the one that holds the most.
 const Instance *find_instance(const FusedShape &s, int live_rows = 1) {
     static const Instance table[] = {
+        instance<GeoQwen3_0p6bAll<2>, FUSED_WF_BF16>(), instance<GeoQwen3_0p6bAll<2>, FUSED_WF_Q8_0>(), instance<GeoQwen3_0p6bAll<2>, FUSED_WF_Q4_0>(), instance<GeoQwen3_0p6bAll<2>, FUSED_WF_K8>(),
+        instance<GeoQwen3_0p6bAll<3>, FUSED_WF_BF16>(), instance<GeoQwen3_0p6bAll<3>, FUSED_WF_Q8_0>(), instance<GeoQwen3_0p6bAll<3>, FUSED_WF_Q4_0>(), instance<GeoQwen3_0p6bAll<3>, FUSED_WF_K8>(),
+        instance<GeoQwen3_0p6bAll<5>, FUSED_WF_BF16>(), instance<GeoQwen3_0p6bAll<5>, FUSED_WF_Q8_0>(), instance<GeoQwen3_0p6bAll<5>, FUSED_WF_Q4_0>(), instance<GeoQwen3_0p6bAll<5>, FUSED_WF_K8>(),
+        instance<GeoQwen3_0p6bAll<7>, FUSED_WF_BF16>(), instance<GeoQwen3_0p6bAll<7>, FUSED_WF_Q8_0>(), instance<GeoQwen3_0p6bAll<7>, FUSED_WF_Q4_0>(), instance<GeoQwen3_0p6bAll<7>, FUSED_WF_K8>(),
+        instance<GeoSmallAll<2>, FUSED_WF_BF16>(), instance<GeoSmallQAll<2>, FUSED_WF_Q8_0>(), instance<GeoSmallQAll<2>, FUSED_WF_Q4_0>(), instance<GeoSmallQAll<2>, FUSED_WF_K8>(),
+        instance<GeoSmallAll<7>, FUSED_WF_BF16>(), instance<GeoSmallQAll<7>, FUSED_WF_Q8_0>(), instance<GeoSmallQAll<7>, FUSED_WF_Q4_0>(), instance<GeoSmallQAll<7>, FUSED_WF_K8>(),
         instance<GeoQwen3_0p6bShort, FUSED_WF_K8>(), instance<GeoSmallQShort, FUSED_WF_K8>(),
         instance<GeoQwen3_0p6b, FUSED_WF_K8>(), instance<GeoSmallQ, FUSED_WF_K8>(),
         instance<GeoQwen3_0p6bMid, FUSED_WF_K8>(), instance<GeoSmallQMid, FUSED_WF_K8>(),

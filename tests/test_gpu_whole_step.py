@@ -166,6 +166,43 @@ def test_quantised_whole_step_against_oracle_and_per_projection_path(ctx, name, 
     gm.close()
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "q8_0", "q4_0", "q4_k_m"])
+def test_short_caches_that_no_workgroup_splits(ctx, fmt):
+    """Up to 112 cached rows every workgroup attends over all of them, two to seven rounds of 16 rows in registers: no row at all, a
+    partly filled round, whole rounds, and the steps across the borders to the next instance and to the even cut. Logits against the
+    path of one launch per projection (the same products, attention summed in another order; new K and V elements may round to
+    the neighbouring bf16) and, bf16, against the oracle."""
+    from homura_amd.runtime import DTYPE_BF16, DTYPE_Q4_0, DTYPE_Q8_0
+    wdt = {"bf16": DTYPE_BF16, "q4_0": DTYPE_Q4_0}.get(fmt, DTYPE_Q8_0)
+    cfg = synth_model.SMALL_WS if fmt == "bf16" else synth_model.SMALL_WS_Q
+    mix = synth_model.q4_k_m_mix(cfg) if fmt == "q4_k_m" else None
+    weights = synth_model.synth_weights(cfg, 6161, wdt, has_qk_norm=True, proj_dtypes=mix)
+    gm = synth_model.build_model(ctx, cfg, weights, 256, wdt, has_qk_norm=True, proj_dtypes=mix)
+    om = mf.build_oracle_model(cfg, weights, 256, wdt, has_qk_norm=True, proj_dtypes=mix)
+    assert gm.whole_step_available() and gm.whole_step()
+    gm.set_prefill_min(0)
+    for rows in (0, 1, 15, 30, 48, 78, 110):
+        kv = synth_model.synth_kv(cfg, 700 + rows, max(rows, 1))
+        ids = synth.token_ids(701 + rows, 5, cfg.vocab_size)
+        out = []
+        for whole in (True, False):
+            gm.set_whole_step(whole)
+            gm.init_kv_cache(kv, rows)
+            say(f"short cache: {fmt}, {rows} rows, whole {whole}")
+            out.append(gm.run_kv(ids))
+            gm.whole_step_status()
+        gm.set_whole_step(True)
+        errs = [mf.rel_err(a, b) for a, b in zip(*out)]
+        # (Q8_K rounds an activation to eight bits: one that falls the other way moves the row by more)
+        assert (min(errs) < 1e-3 and max(errs) < 0.2) if fmt == "q4_k_m" else max(errs) < 1e-2, f"{rows} rows: {errs}"
+        if fmt == "bf16":
+            mf.oracle_init_kv(om, kv)
+            om.kv.reset(rows)
+            want = np.concatenate([om.run_kv(ids[i:i + 1]) for i in range(5)])
+            assert max(mf.rel_err(out[0][i], want[i]) for i in range(5)) < 1e-2, f"{rows} rows"
+    gm.close()
+
+
 def test_bias_and_no_qk_norm_variant(ctx):
     """Q/K/V biases ride in the Q|K|V phase; without QK-norm the rows go straight to RoPE."""
     cfg = dataclasses.replace(synth_model.SMALL_WS, attention_bias=True)
