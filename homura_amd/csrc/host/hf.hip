@@ -42,6 +42,10 @@ void precompute_rope_cos_sin(int head_dim, int max_seq_len, double theta, std::v
 
 namespace {
 
+// Live rows that the decode attention of a step with one launch per projection takes in one split, the most that a workgroup
+// of it holds in registers
+constexpr int ATTN_UNSPLIT = 128;
+
 // HOMURA_WHOLE_STEP_FAR=1 (read when the plan is built): the whole-step kernel takes every exchange through
 // memory, as it does when it does not find its workgroups dealt to the dies round-robin.
 int whole_step_far_only() {
@@ -522,10 +526,12 @@ int HfModel::finalize(int max_seq_len) {
     }
     // Before every step: the whole-step launch while the step's live rows (the cache and the new row) are
     // within what its attention phase holds, one launch per projection beyond (a longer conversation
-    // changes over once; a cache reset changes back). With one launch per projection the attention grid of the
-    // recorded step covers the live rows rounded up to a power of two (2048 at least) instead of the cache's
+    // changes over once; a cache reset changes back). With one launch per projection the attention grid
+    // covers the live rows rounded up to a power of two (2048 at least) instead of the cache's
     // capacity: a cache sized for 32768 rows with 1000 in it would otherwise start 30 workgroups that leave at
-    // once for every one that works, and fold its few partial results with the workgroup meant for hundreds.
+    // once for every one that works, and fold its few partial results with the workgroup meant for hundreds. Up to ATTN_UNSPLIT
+    // rows are one split, and the step has no fold: us a token at 40 / 115 rows, Qwen2.5-0.5B
+    // 676 / 705 -> 660 / 670, Qwen2.5-1.5B 1062 / 1086 -> 1057 / 1065, TinyLlama in Q4_0 712 / 728 -> 684 / 688.
     plan_->set_pre_run([this, fs]() {
         const int live = plan_->kv_cache_len() + 1;
         int rc = HM_OK;
@@ -540,13 +546,9 @@ int HfModel::finalize(int max_seq_len) {
             if (rc == HM_OK) rc = refresh_fused_table();
         }
         if (rc == HM_OK && !plan_->whole_step()) {
-            int span = 2048;
+            int span = live <= ATTN_UNSPLIT ? ATTN_UNSPLIT : 2048;
             while (span < live && span < max_seq_len_) span *= 2;
-            span = std::min(span, max_seq_len_);
-            if (span != plan_->attn_span()) {
-                plan_->set_attn_span(span);
-                rc = plan_->invalidate_graph();  // the recorded grids cover the old span
-            }
+            plan_->set_attn_span(std::min(span, max_seq_len_));
         }
         return rc;
     });
@@ -819,7 +821,7 @@ int HfModel::emit_transformer_plan() {
                 a.scale = (float)(1.0 / std::sqrt((double)hd));  // f64 -> f32 constant, emitter.rs:719
                 a.state = sc.plan->state();
                 a.span = sc.plan->attn_span();
-                a.fixed_chunk = att_chunk_fixed || a.span <= 2048 ? att_chunk : 128;
+                a.fixed_chunk = att_chunk_fixed || (a.span > ATTN_UNSPLIT && a.span <= 2048) ? att_chunk : 128;
                 a.phase = phase;
                 return a;
             };
@@ -1433,7 +1435,7 @@ int HfModel::emit_transformer_plan_quant() {
                 a.scale = (float)(1.0 / std::sqrt((double)hd));
                 a.state = sc.plan->state();
                 a.span = sc.plan->attn_span();
-                a.fixed_chunk = att_chunk_fixed || a.span <= 2048 ? att_chunk : 128;
+                a.fixed_chunk = att_chunk_fixed || (a.span > ATTN_UNSPLIT && a.span <= 2048) ? att_chunk : 128;
                 a.phase = phase;
                 return a;
             };

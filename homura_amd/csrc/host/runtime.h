@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <functional>
+#include <map>
 #include <memory>
 #include <string>
 #include <vector>
@@ -278,7 +279,7 @@ class ExecutionPlan {
     // Take the whole-step launch (when the plan has one) instead of the per-projection launches.
     int set_whole_step(bool on);
     bool whole_step() const { return whole_step_; }
-    // Forget the recorded step (its launches' arguments or kernels are about to change); the next run records anew.
+    // Forget the recorded steps (their launches' arguments or kernels are about to change); the next run records anew.
     int invalidate_graph();
     bool skips(const DeviceLaunch &l) const {
         return l.mode == (whole_step_ ? DeviceLaunch::Mode::PerKernel : DeviceLaunch::Mode::WholeStep);
@@ -286,8 +287,8 @@ class ExecutionPlan {
     // Called before a step is enqueued or captured, with the KV cache in place (device tables that
     // depend on the cache's addresses are refreshed here, outside any capture).
     void set_pre_run(std::function<int()> fn) { pre_run_ = std::move(fn); }
-    // Rows the decode attention's grid covers in a recorded step (0: the cache's capacity). Whoever sets it keeps
-    // the live rows within it and drops the recorded step when it changes.
+    // Rows the decode attention's grid covers (0: the cache's capacity). Whoever sets it keeps the live rows within it. A step
+    // is recorded once for every span it has run with (a few: spans are 128 and the powers of two from 2048 on).
     int attn_span() const { return attn_span_; }
     void set_attn_span(int rows) { attn_span_ = rows; }
 
@@ -343,8 +344,11 @@ class ExecutionPlan {
     bool whole_step_ = false;
     std::function<int()> pre_run_;
     int attn_span_ = 0;
-    hipGraph_t graph_ = nullptr;
-    hipGraphExec_t graph_exec_ = nullptr;
+    struct Recorded {
+        hipGraph_t graph;
+        hipGraphExec_t exec;
+    };
+    std::map<int, Recorded> graphs_;  // by attn_span_
 };
 
 }  // namespace homura

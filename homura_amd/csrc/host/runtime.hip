@@ -252,8 +252,10 @@ ExecutionPlan::~ExecutionPlan() {
         (void)hipEventDestroy(arm_done_);
     }
     if (arm_pinned_) (void)hipHostFree(arm_pinned_);
-    if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
-    if (graph_) (void)hipGraphDestroy(graph_);
+    for (auto &g : graphs_) {
+        (void)hipGraphExecDestroy(g.second.exec);
+        (void)hipGraphDestroy(g.second.graph);
+    }
 }
 
 void ExecutionPlan::alias_slot(size_t slot, size_t base_slot, size_t byte_offset) {
@@ -344,14 +346,7 @@ int ExecutionPlan::init_kv_cache(const float *const *h_kv, int seq_len, int max_
     if (!has_kv_info_) return hm_set_error(ctx_, HM_ERR_STATE, "init_kv_cache called but plan has no KV cache info");
     if (cache_ && cache_->max_len() != max_seq_len) {
         cache_.reset();
-        if (graph_exec_) {  // captured pointers are gone
-            (void)hipGraphExecDestroy(graph_exec_);
-            graph_exec_ = nullptr;
-        }
-        if (graph_) {
-            (void)hipGraphDestroy(graph_);
-            graph_ = nullptr;
-        }
+        if (const int rc = invalidate_graph(); rc != HM_OK) return rc;  // captured pointers are gone
     }
     int rc = ensure_kv_cache(max_seq_len);
     if (rc != HM_OK) return rc;
@@ -530,15 +525,13 @@ int ExecutionPlan::set_whole_step(bool on) {
 }
 
 int ExecutionPlan::invalidate_graph() {
-    if (graph_exec_) {
-        HM_HIP(ctx_, hipStreamSynchronize(ctx_->stream));
-        (void)hipGraphExecDestroy(graph_exec_);
-        graph_exec_ = nullptr;
+    if (graphs_.empty()) return HM_OK;
+    HM_HIP(ctx_, hipStreamSynchronize(ctx_->stream));
+    for (auto &g : graphs_) {
+        (void)hipGraphExecDestroy(g.second.exec);
+        (void)hipGraphDestroy(g.second.graph);
     }
-    if (graph_) {
-        (void)hipGraphDestroy(graph_);
-        graph_ = nullptr;
-    }
+    graphs_.clear();
     return HM_OK;
 }
 
@@ -553,11 +546,8 @@ int ExecutionPlan::run_kv(const std::vector<Buffer *> &inputs, std::vector<Buffe
     // A graph pays when a step is many launches. A step of one or two is quicker launched directly: the replay
     // of a one-node graph costs more on the GPU's queue than the kernel's own dispatch packet.
     if (use_graph_ && launches_per_step() > 2) {
-        if (!graph_exec_) {
-            if (graph_) {
-                (void)hipGraphDestroy(graph_);
-                graph_ = nullptr;
-            }
+        auto it = graphs_.find(attn_span_);
+        if (it == graphs_.end()) {
             HM_HIP(ctx_, hipStreamBeginCapture(ctx_->stream, hipStreamCaptureModeRelaxed));
             rc = run_steps(nullptr);
             hipGraph_t g = nullptr;
@@ -567,10 +557,12 @@ int ExecutionPlan::run_kv(const std::vector<Buffer *> &inputs, std::vector<Buffe
                 return rc;
             }
             HM_HIP(ctx_, e);
-            graph_ = g;
-            HM_HIP(ctx_, hipGraphInstantiate(&graph_exec_, graph_, nullptr, nullptr, 0));
+            Recorded r{g, nullptr};
+            if ((e = hipGraphInstantiate(&r.exec, g, nullptr, nullptr, 0)) != hipSuccess) (void)hipGraphDestroy(g);
+            HM_HIP(ctx_, e);
+            it = graphs_.emplace(attn_span_, r).first;
         }
-        HM_HIP(ctx_, hipGraphLaunch(graph_exec_, ctx_->stream));
+        HM_HIP(ctx_, hipGraphLaunch(it->second.exec, ctx_->stream));
     } else {
         rc = run_steps(nullptr);
         if (rc != HM_OK) return rc;

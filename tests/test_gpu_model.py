@@ -82,6 +82,28 @@ def test_tiny_graph_replay_matches_eager(ctx, tiny):
         gm.set_graph(False)
 
 
+@pytest.mark.parametrize("rows", [61, 126])
+def test_attention_of_one_split_and_across_its_border(ctx, tiny, rows):
+    """Up to 128 live rows the attention of a step with one launch per projection is one split without a fold (61: more than one of
+    the 64-row splits that longer caches take; 126: over the border and back to one split in a new request), eager and from the
+    graphs that are recorded for either span and kept."""
+    cfg, _w, gm, om = tiny
+    kv = synth_model.synth_kv(cfg, 40 + rows, rows)
+    ids = synth.token_ids(41 + rows, 6, cfg.vocab_size)
+    gm.set_prefill_min(0)
+    got = []
+    for graph in (False, True, True):
+        gm.set_graph(graph)
+        gm.init_kv_cache(kv, rows)
+        got.append(gm.run_kv(ids))
+    gm.set_graph(False)
+    gm.set_prefill_min(8)
+    mf.oracle_init_kv(om, kv)
+    want = np.concatenate([om.run_kv(ids[i:i + 1]) for i in range(6)])
+    assert max(mf.rel_err(got[0][i], want[i]) for i in range(6)) < 1e-2
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
 def test_kv_overflow_and_bad_input(ctx, tiny):
     cfg, weights, gm, _om = tiny
     kv = synth_model.synth_kv(cfg, 7, 158)
