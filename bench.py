@@ -428,7 +428,7 @@ def main() -> int:
         "dtype": "bf16 weights / f32 accumulate", "data": "synthetic",
         "config": {"workload": "Qwen3-0.6B-shape decode: 28 layers, hidden 1024, 16q/8kv heads x 128, "
                                "SwiGLU 3072, vocab 151936 tied head, KV cache 1024+ rows, batch 1, greedy",
-                   "kv_rows_start": pos0, "graph_replay": (not args.no_graph) and launches > 2,
+                   "kv_rows_start": pos0, "graph_replay": (not args.no_graph) and launches > 3,
                    "kernel_launches_per_step": launches},
         "roofline": roofline,
         "cpu_baseline": cpu_baseline,

@@ -273,7 +273,7 @@ class ExecutionPlan {
     // Arm the cursor: pos = cache length, step = 0, the given ids forced for the first steps.
     int arm(const int32_t *h_forced, int n_forced);
 
-    // Graph replay of the step (captured lazily on first use; arguments never change).
+    // Graph replay of the step (captured lazily on first use; arguments never change), on by default for steps of more than three launches.
     int enable_graph(bool on);
     bool graph_enabled() const { return use_graph_; }
     // Take the whole-step launch (when the plan has one) instead of the per-projection launches.
@@ -340,7 +340,7 @@ class ExecutionPlan {
     hipEvent_t arm_done_ = nullptr;
     int out_cap_ = 0;
     bool prepared_ = false;
-    bool use_graph_ = false;
+    bool use_graph_ = true;
     bool whole_step_ = false;
     std::function<int()> pre_run_;
     int attn_span_ = 0;
@@ -349,6 +349,7 @@ class ExecutionPlan {
         hipGraphExec_t exec;
     };
     std::map<int, Recorded> graphs_;  // by attn_span_
+    int recorded(const Recorded **out);
 };
 
 }  // namespace homura

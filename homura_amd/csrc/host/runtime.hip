@@ -535,6 +535,32 @@ int ExecutionPlan::invalidate_graph() {
     return HM_OK;
 }
 
+// The recorded step for the present span, recorded now if this is its first. Where it cannot be recorded the step has been enqueued
+// launch by launch instead, as all later ones will be, and *out is NULL.
+int ExecutionPlan::recorded(const Recorded **out) {
+    *out = nullptr;
+    auto it = graphs_.find(attn_span_);
+    if (it == graphs_.end()) {
+        Recorded r{nullptr, nullptr};
+        hipError_t e = hipStreamBeginCapture(ctx_->stream, hipStreamCaptureModeRelaxed);
+        if (e == hipSuccess) {
+            const int rc = run_steps(nullptr);
+            e = hipStreamEndCapture(ctx_->stream, &r.graph);
+            if (rc != HM_OK) e = hipErrorUnknown;
+            if (e == hipSuccess) e = hipGraphInstantiate(&r.exec, r.graph, nullptr, nullptr, 0);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            if (r.graph) (void)hipGraphDestroy(r.graph);
+            use_graph_ = false;
+            return run_steps(nullptr);
+        }
+        it = graphs_.emplace(attn_span_, r).first;
+    }
+    *out = &it->second;
+    return HM_OK;
+}
+
 int ExecutionPlan::run_kv(const std::vector<Buffer *> &inputs, std::vector<Buffer> &weights,
                           int max_seq_len) {
     if (!prepared_) return hm_set_error(ctx_, HM_ERR_STATE, "plan not prepared");
@@ -543,29 +569,16 @@ int ExecutionPlan::run_kv(const std::vector<Buffer *> &inputs, std::vector<Buffe
     if ((rc = cache_->note_appended(1)) != HM_OK) return rc;  // "KV cache full"
     if ((rc = bind(inputs, weights)) != HM_OK) return rc;
     if (pre_run_ && (rc = pre_run_()) != HM_OK) return rc;
-    // A graph pays when a step is many launches. A step of one or two is quicker launched directly: the replay
-    // of a one-node graph costs more on the GPU's queue than the kernel's own dispatch packet.
-    if (use_graph_ && launches_per_step() > 2) {
-        auto it = graphs_.find(attn_span_);
-        if (it == graphs_.end()) {
-            HM_HIP(ctx_, hipStreamBeginCapture(ctx_->stream, hipStreamCaptureModeRelaxed));
-            rc = run_steps(nullptr);
-            hipGraph_t g = nullptr;
-            hipError_t e = hipStreamEndCapture(ctx_->stream, &g);
-            if (rc != HM_OK) {
-                if (g) (void)hipGraphDestroy(g);
-                return rc;
-            }
-            HM_HIP(ctx_, e);
-            Recorded r{g, nullptr};
-            if ((e = hipGraphInstantiate(&r.exec, g, nullptr, nullptr, 0)) != hipSuccess) (void)hipGraphDestroy(g);
-            HM_HIP(ctx_, e);
-            it = graphs_.emplace(attn_span_, r).first;
-        }
-        HM_HIP(ctx_, hipGraphLaunch(it->second.exec, ctx_->stream));
-    } else {
-        rc = run_steps(nullptr);
-        if (rc != HM_OK) return rc;
+    // A graph pays when a step is many launches: the host enqueues them at about the rate they run at and never gets ahead of a
+    // single step (run_kv with its logits read, us: Qwen2.5-0.5B 820 -> 730, 1.5B 1200 -> 1126, Nokuvik 1024 wide 1540 -> 1340, Ludalix 1250 ->
+    // 1125), and a replayed launch starts sooner behind the last (Qwen2.5-1.5B, step after step, 1086 -> 1060). A step of up to three
+    // is quicker launched directly (whole-step launch of a Q4_K_M model, head and pick: 64 sampled tokens 30.10 ms replayed, 29.95 ms direct).
+    if (use_graph_ && launches_per_step() > 3) {
+        const Recorded *r = nullptr;
+        if ((rc = recorded(&r)) != HM_OK) return rc;
+        if (r) HM_HIP(ctx_, hipGraphLaunch(r->exec, ctx_->stream));
+    } else if ((rc = run_steps(nullptr)) != HM_OK) {
+        return rc;
     }
     // one advance after all layers appended (reference src/runtime.rs:1875-1880)
     cache_->advance_by(cache_->new_tokens());
