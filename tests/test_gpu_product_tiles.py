@@ -195,6 +195,26 @@ def test_rows_whose_squares_overflow(ctx, dtype):
         assert np.all(np.linalg.norm(got - want, axis=1) <= 1e-6 * np.linalg.norm(want, axis=1))
 
 
+# each instance of the row kernels: vectors and threads a row, the widths where they change, and a width past the vectors that are kept
+@pytest.mark.parametrize("front,m,k", [(0, 5, 1024), (0, 5, 1088), (0, 5, 2048), (0, 5, 2112), (1, 3, 1024), (1, 513, 1024), (1, 513, 2048),
+                                       (1, 513, 3072), (1, 513, 4096), (1, 513, 4160), (1, 513, 8192), (1, 513, 8256), (1, 512, 1088),
+                                       (1, 512, 4160), (1, 512, 8256), (1, 2, 16384)])
+def test_row_kernels_of_every_width(ctx, front, m, k):
+    """Gates from -100, where 1 + exp(-g) leaves f32's range, to 100. A row against float64, the bound as above with the factor of two
+    that a single row of 8 results may lie off the whole's norm."""
+    rng = np.random.default_rng(k + m)
+    norm_w = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    raw, w = weights(DTYPE_BF16, 8, k, rng)
+    x = rng.standard_normal((m, k * (1 + front))).astype(np.float32)
+    if front:
+        x[:, 0::2] = rng.uniform(-100, 100, (m, k))
+    with np.errstate(over="ignore"):
+        want = rows_of(front, x, norm_w) @ w.T.astype(np.float64)
+    got = product(ctx, front, x, norm_w, DTYPE_BF16, raw, 8)
+    assert np.linalg.norm(got - want) <= 4e-7 * np.linalg.norm(want)
+    assert np.all(np.linalg.norm(got - want, axis=1) <= 8e-7 * np.linalg.norm(want, axis=1))
+
+
 @pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_Q8_0])
 @pytest.mark.parametrize("k", [512, 2048])
 def test_gated_rows_of_every_finite_size(ctx, dtype, k):
