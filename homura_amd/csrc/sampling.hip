@@ -423,13 +423,24 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_token_kernel(SampleArgs
 }
 
 // ── Small top_k (<= 64) over a large vocabulary: two launches instead of one workgroup's eight passes ──
-// Front: a workgroup per 1024 tokens applies penalties and temperature, takes its maximum and the sum of
-// exponentials relative to it, and keeps the 64 of its tokens that come first by (logit descending, token
-// ascending), in token order: the vocabulary's top_k are among them. Back: one workgroup combines the maxima and sums (sum over the
-// vocabulary = sum_b sum_b * exp(max_b - max), equal to the single pass's up to rounding) and runs the shared
-// selection over the kept tokens; it selects by logit, which orders tokens like their exponentials except
-// where two different logits round to one exponential.
-constexpr int FRONT_KEEP = 64;
+// Front: a wavefront per group of 64 to 256 tokens applies penalties and temperature and writes the group's maximum,
+// the sum of its exponentials relative to it and its first four tokens by (logit descending, token ascending): one
+// trip to memory and ten reductions, no LDS. Back: one workgroup combines maxima and sums (sum over the vocabulary =
+// sum_g sum_g * exp(max_g - max), equal to the single pass's up to rounding). The K-th largest of the groups' first
+// keys is a floor for the K-th largest of the vocabulary (K tokens reach it), so the top K are among the kept tokens
+// that reach it, a hundred or so, unless all four of a group do: then the groups that reach the floor are read again.
+// It selects by logit, which orders tokens like their exponentials except where two different logits round to one
+// exponential.
+// What bounds the pair is latency: a launch, one trip to memory and the barriers between the steps of a single
+// workgroup, whose instructions come from memory too (the step before it has swept the instruction cache): loops
+// here are rolled, and what is rare lies behind a branch. 151936 tokens, top_k 50, behind a whole-step decode kernel:
+// front 4.7 us, back 5.6 (the 64 first of every 1024 tokens by a radix select in a workgroup each, and all of those
+// looked through by the back: 6.6 and 11.7; the listed groups always read again, instead of kept tokens: 4.6 and 10.4).
+constexpr int FRONT_THREADS = 256;
+constexpr int FRONT_MAX_K = WAVE;                 // largest top_k
+constexpr int FRONT_GROUP_BITS = 6;               // tokens of a group: the least power of two from 64 with at most 1024 groups
+constexpr int FRONT_UNITS = SAMPLE_THREADS / 4;   // the floor is taken over at most so many maxima
+constexpr int FRONT_LIST = 128;                   // groups that the back reads without picking K of them first
 
 // larger float <-> larger key (-inf the smallest key of all finite and infinite values)
 __device__ __forceinline__ unsigned order_key(float x) {
@@ -439,259 +450,292 @@ __device__ __forceinline__ unsigned order_key(float x) {
 __device__ __forceinline__ float key_value(unsigned k) {
     return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
-
-struct FrontOut {
-    unsigned *key;  // [blocks][FRONT_KEEP]
-    int *idx;       // [blocks][FRONT_KEEP]
-    float *stat;    // [blocks][2]: maximum, sum of exponentials relative to it
-};
-__host__ __device__ inline FrontOut front_out(float *work, int blocks) {
-    FrontOut f;
-    f.key = reinterpret_cast<unsigned *>(work);
-    f.idx = reinterpret_cast<int *>(work) + (size_t)blocks * FRONT_KEEP;
-    f.stat = work + (size_t)blocks * FRONT_KEEP * 2;
-    return f;
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ unsigned dpp_keys(unsigned k) {
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)k, CTRL, ROW_MASK, 0xF, false);
+}
+__device__ __forceinline__ unsigned wave_max_key(unsigned k) {  // (the steps of wave_max)
+    k = max(k, dpp_keys<0xB1, 0xF>(k));
+    k = max(k, dpp_keys<0x4E, 0xF>(k));
+    k = max(k, dpp_keys<0x141, 0xF>(k));
+    k = max(k, dpp_keys<0x140, 0xF>(k));
+    k = max(k, dpp_keys<0x142, 0xA>(k));
+    k = max(k, dpp_keys<0x143, 0xC>(k));
+    return (unsigned)__builtin_amdgcn_readlane((int)k, 63);
 }
 
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_front_kernel(SampleArgs a) {
-    __shared__ unsigned hist[4096];
-    __shared__ float red[SAMPLE_THREADS / WAVE], red_s[SAMPLE_THREADS / WAVE];
-    __shared__ int red_i[SAMPLE_THREADS / WAVE];
-    __shared__ unsigned sel_prefix, sel_need;
-    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
-    const int i = blockIdx.x * SAMPLE_THREADS + tid;
-    const bool on = i < a.vocab;
+constexpr int FRONT_KEEP = 4;
+struct FrontOut {
+    unsigned *key;  // [groups][FRONT_KEEP]
+    int *token;     // [groups][FRONT_KEEP]
+    float *most, *sum;
+};
+__host__ __device__ inline FrontOut front_out(float *work, int groups) {
+    const size_t n = (size_t)groups * FRONT_KEEP;
+    return FrontOut{reinterpret_cast<unsigned *>(work), reinterpret_cast<int *>(work) + n, work + 2 * n, work + 2 * n + groups};
+}
+
+__global__ __launch_bounds__(FRONT_THREADS) void sample_front_kernel(SampleArgs a, int groups, int group_bits) {
+    const int lane = threadIdx.x & (WAVE - 1), g = (int)((blockIdx.x * FRONT_THREADS + threadIdx.x) / WAVE);
+    if (g >= groups) return;
     const float inv_temp = 1.0f / a.cfg.temperature;
-    const float x = on ? penalised(a.logits[i], a.counts ? a.counts[i] : 0, a.cfg) * inv_temp : -INFINITY;
-    float m = wave_max(x);
-    if (lane == 0) red[wave] = m;
-    if (tid == 0) {
-        sel_prefix = 0;
-        sel_need = FRONT_KEEP;
+    const int first = g << group_bits, end = min(a.vocab, first + (1 << group_bits)), chunks = group_bits <= 8 ? 1 : 1 << (group_bits - 8);
+    auto load = [&](int j, float (&x)[4]) {
+        const int base = first + j * 256 + lane;
+        float l[4];
+        int c[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = min(base + u * WAVE, end - 1);
+            l[u] = a.logits[i];
+            c[u] = a.counts ? a.counts[i] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) x[u] = base + u * WAVE < end ? penalised(l[u], c[u], a.cfg) * inv_temp : -INFINITY;
+    };
+    float x[4], m = -INFINITY;
+    for (int j = 0; j < chunks; j++) {
+        load(j, x);
+#pragma unroll
+        for (int u = 0; u < 4; u++) m = fmaxf(m, x[u]);
     }
-    __syncthreads();
-    m = red[0];
-    for (int w = 1; w < SAMPLE_THREADS / WAVE; w++) m = fmaxf(m, red[w]);
-    const float e = (on && x > -INFINITY) ? expf(x - m) : 0.f;
-    const float ws = wave_sum(e);
-    if (lane == 0) red_s[wave] = ws;
-    // The 64 tokens that come first by (logit descending, token ascending), kept in token order: the key of the
-    // 64th by a radix select over the 1024 keys (12 + 10 + 10 bits, one element per thread), then everything
-    // above it and the lowest-numbered of the tokens equal to it. Tokens past the vocabulary carry the key of
-    // -inf and come last among equals.
-    const unsigned key = order_key(x);
-    for (int pass = 0; pass < 3; pass++) {
-        const int shift = pass == 0 ? 20 : pass == 1 ? 10 : 0;
-        const int bits = pass == 0 ? 12 : 10;
-        const int bpt = (1 << bits) / SAMPLE_THREADS;  // bins per thread: 4, 1, 1
-        for (int b = tid; b < (1 << bits); b += SAMPLE_THREADS) hist[b] = 0;
-        __syncthreads();
-        const unsigned prefix = sel_prefix, need = sel_need;
-        const unsigned mask = pass == 0 ? 0u : 0xFFFFFFFFu << (shift + bits);
-        if ((key & mask) == prefix) atomicAdd(&hist[(key >> shift) & ((1u << bits) - 1u)], 1u);
-        __syncthreads();
-        unsigned mine = 0;
-        for (int j = 0; j < bpt; j++) mine += hist[tid * bpt + j];
-        unsigned incl = mine;  // inclusive prefix sum over threads, low bins first
-        for (int off = 1; off < WAVE; off <<= 1) {
-            const unsigned up = __shfl_up(incl, off, WAVE);
-            if (lane >= off) incl += up;
-        }
-        if (lane == WAVE - 1) red_i[wave] = (int)incl;
-        __syncthreads();
-        unsigned before = 0, total = 0;
-        for (int w = 0; w < SAMPLE_THREADS / WAVE; w++) {
-            if (w < wave) before += (unsigned)red_i[w];
-            total += (unsigned)red_i[w];
-        }
-        const unsigned above = total - (before + incl);  // elements in higher bins
-        if (above < need && need <= above + mine) {      // exactly one thread
-            unsigned acc = above;
-            for (int j = bpt - 1; j >= 0; j--) {
-                const unsigned h = hist[tid * bpt + j];
-                if (acc + h >= need) {
-                    sel_prefix = prefix | ((unsigned)(tid * bpt + j) << shift);
-                    sel_need = need - acc;
-                    break;
+    m = wave_max(m);
+    float e = 0.f;
+    for (int j = 0; j < chunks; j++) {
+        if (chunks > 1) load(j, x);
+#pragma unroll
+        for (int u = 0; u < 4; u++) e += x[u] > -INFINITY ? expf(x[u] - m) : 0.f;
+    }
+    e = wave_sum(e);
+    // The group's tokens in order, each the first of those behind the one before it. (Lanes past the group's end hold
+    // the key of -inf and higher token numbers.)
+    unsigned last = 0xFFFFFFFFu, my_key = 0;
+    int last_token = -1, my_token = 0;
+#pragma unroll 1
+    for (int r = 0; r < FRONT_KEEP; r++) {
+        unsigned best = 0;
+        int token = 0x7FFFFFFF;
+        for (int j = 0; j < chunks; j++) {
+            if (chunks > 1) load(j, x);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const unsigned k = order_key(x[u]);
+                const int t = first + j * 256 + u * WAVE + lane;
+                if (((k < last) | ((k == last) & (t > last_token))) & (k > best)) {
+                    best = k;
+                    token = t;
                 }
-                acc += h;
             }
         }
-        __syncthreads();
+        last = wave_max_key(best);
+        last_token = (int)~wave_max_key(best == last ? ~(unsigned)token : 0u);
+        if (lane == r) {
+            my_key = last;
+            my_token = last_token;
+        }
     }
-    const unsigned T = sel_prefix, need_eq = sel_need;
-    // rank of this thread among the threads whose key equals T (thread order = token order)
-    const bool eq = key == T;
-    const unsigned long long em = __ballot(eq);
-    if (lane == 0) red_i[wave] = __popcll(em);
-    __syncthreads();
-    unsigned eq_rank = __popcll(em & ((1ull << lane) - 1ull));
-    for (int w = 0; w < wave; w++) eq_rank += (unsigned)red_i[w];
-    __syncthreads();
-    const bool keep = key > T || (eq && eq_rank < need_eq);
-    const unsigned long long km = __ballot(keep);
-    if (lane == 0) red_i[wave] = __popcll(km);
-    __syncthreads();
-    unsigned pos = __popcll(km & ((1ull << lane) - 1ull));
-    for (int w = 0; w < wave; w++) pos += (unsigned)red_i[w];
-    const FrontOut f = front_out(a.work, gridDim.x);
-    if (keep) {  // exactly FRONT_KEEP threads
-        f.key[(size_t)blockIdx.x * FRONT_KEEP + pos] = key;
-        f.idx[(size_t)blockIdx.x * FRONT_KEEP + pos] = on ? i : 0x7FFFFFFF;
+    const FrontOut f = front_out(a.work, groups);
+    if (lane < FRONT_KEEP) {
+        f.key[g * FRONT_KEEP + lane] = my_key;
+        f.token[g * FRONT_KEEP + lane] = my_token;
     }
-    if (tid == 0) {
-        float sum = 0.f;
-        for (int w = 0; w < SAMPLE_THREADS / WAVE; w++) sum += red_s[w];
-        f.stat[blockIdx.x * 2] = m;
-        f.stat[blockIdx.x * 2 + 1] = sum;
+    if (lane == 0) {
+        f.most[g] = m;
+        f.sum[g] = e;
     }
 }
 
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_back_kernel(SampleArgs a, int blocks) {
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_back_kernel(SampleArgs a, int groups, int group_bits) {
     __shared__ SelectShared sh;
+    __shared__ unsigned group_key[SAMPLE_THREADS], floor_key, listed, survived, more;
+    __shared__ alignas(16) unsigned unit_key[FRONT_UNITS];
+    __shared__ float red_sum[SAMPLE_THREADS / WAVE];
+    __shared__ int list[SAMPLE_THREADS];
+    // a survivor as one 64-bit number that orders like (logit descending, token ascending): key, then the
+    // token counted down from the largest
+    __shared__ unsigned long long fcomp[SAMPLE_MAX_K];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
-    const StepInfo st = load_step(a);
-    const FrontOut f = front_out(a.work, blocks);
-    // This kernel is one workgroup, and every dependent trip to memory costs it a couple of microseconds: the kept
-    // tokens (up to PRE per thread) are asked for before anything waits on the blocks' statistics.
-    constexpr int PRE = 16;
-    const int n_kept = blocks * FRONT_KEEP;
-    const bool preloaded = n_kept <= PRE * SAMPLE_THREADS;
-    unsigned pk[PRE];
-    int pi[PRE];
-    if (preloaded) {
-#pragma unroll
-        for (int u = 0; u < PRE; u++) {
-            const int j = tid + u * SAMPLE_THREADS;
-            pk[u] = j < n_kept ? f.key[j] : 0u;
-            pi[u] = j < n_kept ? f.idx[j] : 0;
-        }
+    const FrontOut f = front_out(a.work, groups);
+    const float gm = tid < groups ? f.most[tid] : -INFINITY, gs = tid < groups ? f.sum[tid] : 0.f;
+    u32x4 kept_key{0u, 0u, 0u, 0u}, kept_token{0u, 0u, 0u, 0u};
+    if (tid < groups) {
+        kept_key = *reinterpret_cast<const u32x4 *>(f.key + tid * FRONT_KEEP);
+        kept_token = *reinterpret_cast<const u32x4 *>(f.token + tid * FRONT_KEEP);
     }
-    float m = -INFINITY;
-    for (int b = tid; b < blocks; b += SAMPLE_THREADS) m = fmaxf(m, f.stat[b * 2]);
-    m = wave_max(m);
+    const unsigned key = kept_key[0];
+    const StepInfo st = load_step(a);
+    const float inv_temp = 1.0f / a.cfg.temperature;
+    const unsigned K = (unsigned)min(a.cfg.top_k, a.vocab);
+    // Up to 256 units, four threads each: the groups, or fours of them (64 at least: the vocabulary has 4096 tokens or more)
+    const bool fours = groups > FRONT_UNITS;
+    const int units = fours ? (groups + 3) / 4 : groups;
+    unsigned four = max(key, dpp_keys<0xB1, 0xF>(key));
+    four = max(four, dpp_keys<0x4E, 0xF>(four));
+    group_key[tid] = key;
+    if (fours ? (tid & 3) == 0 : tid < FRONT_UNITS) unit_key[fours ? tid / 4 : tid] = fours ? four : key;
+    if (tid == 0) {
+        floor_key = 0xFFFFFFFFu;
+        listed = survived = more = 0;
+    }
+    float m = wave_max(gm);
     if (lane == 0) sh.red_f[wave] = m;
     __syncthreads();
     m = sh.red_f[0];
+#pragma unroll
     for (int w = 1; w < SAMPLE_THREADS / WAVE; w++) m = fmaxf(m, sh.red_f[w]);
-    __syncthreads();
-    float sum = 0.f;
-    for (int b = tid; b < blocks; b += SAMPLE_THREADS) {
-        const float bm = f.stat[b * 2];
-        if (bm > -INFINITY) sum += f.stat[b * 2 + 1] * expf(bm - m);
+    float sum = wave_sum(gm > -INFINITY ? gs * expf(gm - m) : 0.f);
+    if (lane == 0) red_sum[wave] = sum;
+    // the K-th largest of the units' keys: the least of those with fewer than K above them; four threads count for one unit
+    if (tid / WAVE * (WAVE / 4) < units) {
+        const int unit = tid / 4, part = (units + 15) / 16 * 4, from = (tid & 3) * part;
+        const unsigned mine = unit_key[unit];
+        unsigned above = 0;
+#pragma unroll 2
+        for (int c = from; c < from + part; c += 4) {  // (units <= 256: the last part ends within unit_key, and keys past the units are 0)
+            const u32x4 o = *reinterpret_cast<const u32x4 *>(&unit_key[c]);
+#pragma unroll
+            for (int u = 0; u < 4; u++) above += o[u] > mine ? 1u : 0u;
+        }
+        above += dpp_keys<0xB1, 0xF>(above);
+        above += dpp_keys<0x4E, 0xF>(above);
+        if ((tid & 3) == 0 && unit < units && above < K) atomicMin(&floor_key, mine);
     }
-    sum = wave_sum(sum);
-    if (lane == 0) sh.red_f[wave] = sum;
     __syncthreads();
     sum = 0.f;
-    for (int w = 0; w < SAMPLE_THREADS / WAVE; w++) sum += sh.red_f[w];
-    __syncthreads();
-    auto weight = [&](unsigned key) {
-        const float x = key_value(key);
+#pragma unroll
+    for (int w = 0; w < SAMPLE_THREADS / WAVE; w++) sum += red_sum[w];
+    const unsigned floor = floor_key;
+    auto weight = [&](unsigned k) {
+        const float x = key_value(k);
         return x > -INFINITY ? expf(x - m) : 0.f;
     };
-    // The K-th largest of the blocks' maxima is a floor for the K-th largest logit of the vocabulary (K tokens reach
-    // it), so only kept tokens at or above it can be among the top K: usually a hundred or so of the blocks * 64.
-    // With at most 1024 of them the selection is done by rank: every survivor counts the survivors ahead of it in
-    // (logit descending, token ascending), the first K take their rank as their place, and after normalisation and
-    // min_p the same count over (probability descending, token ascending) gives the order the reference's
-    // sequential loops walk. A flat distribution (more survivors) takes the general selection over the full list.
-    // a survivor as one 64-bit number that orders like (logit descending, token ascending): key, then the
-    // token counted down from the largest
-    __shared__ unsigned bkey[SAMPLE_THREADS], tau, fcount;
-    __shared__ unsigned long long fcomp[SAMPLE_MAX_K];
-    const unsigned K = (unsigned)min(a.cfg.top_k, a.vocab);
-    if (preloaded && blocks <= SAMPLE_THREADS && (unsigned)blocks >= K && K >= 1 && K <= (unsigned)WAVE) {
-        bkey[tid] = tid < blocks ? order_key(f.stat[tid * 2]) : 0u;
-        if (tid == 0) fcount = 0;
-        __syncthreads();
-        if (tid < blocks) {
-            const unsigned mine = bkey[tid];
-            unsigned rank = 0;
-#pragma unroll 16
-            for (int c = 0; c < blocks; c++) {  // (unrolled: sixteen LDS reads in flight, not one)
-                const unsigned o = bkey[c];
-                rank += ((o > mine) | ((o == mine) & (c < tid))) ? 1u : 0u;
-            }
-            if (rank == K - 1) tau = mine;
+    auto survive = [&](unsigned k, int token) {
+        const unsigned at = atomicAdd(&survived, 1u);
+        if (at < (unsigned)SAMPLE_MAX_K) fcomp[at] = ((unsigned long long)k << 32) | (unsigned)(0x7FFFFFFF - token);
+    };
+    bool in = tid < groups && key >= floor;
+    if (in) {
+#pragma unroll 1
+        for (int u = 0; u < FRONT_KEEP && kept_key[0] >= floor; u++) {
+            survive(kept_key[0], (int)kept_token[0]);
+            kept_key = u32x4{kept_key[1], kept_key[2], kept_key[3], 0u};
+            kept_token = u32x4{kept_token[1], kept_token[2], kept_token[3], 0u};
+            if (u == FRONT_KEEP - 1) more = 1;
         }
+    }
+    __syncthreads();
+    if (more || survived > (unsigned)SAMPLE_MAX_K) {
+        // A group may have more than it kept, or the list takes no more: the tokens of the groups that reach the floor, read again. With more of
+        // those than the list takes (equal keys all over the vocabulary) the first K groups by (key descending, group
+        // ascending), which hold K tokens that come ahead of every other group's.
+        if (in) list[atomicAdd(&listed, 1u)] = tid;
         __syncthreads();
-        const unsigned floor_key = tau;
-#pragma unroll
-        for (int u = 0; u < PRE; u++) {
-            const int j = tid + u * SAMPLE_THREADS;
-            if (j < n_kept && pk[u] >= floor_key) {
-                const unsigned at = atomicAdd(&fcount, 1u);
-                if (at < (unsigned)SAMPLE_MAX_K) fcomp[at] = ((unsigned long long)pk[u] << 32) | (unsigned)(0x7FFFFFFF - pi[u]);
-            }
-        }
+        if (tid == 0) survived = 0;
+        int n_list = (int)listed;
         __syncthreads();
-        const int nf = (int)fcount;
-        if (nf <= SAMPLE_MAX_K) {
-            float (&cand_p)[SAMPLE_MAX_K] = sh.cand_p;
-            int (&cand_i)[SAMPLE_MAX_K] = sh.cand_i;
-            if (tid < nf) {
-                const unsigned long long mine = fcomp[tid];
-                const int mi = 0x7FFFFFFF - (int)(unsigned)(mine & 0xFFFFFFFFull);
-                unsigned rank = 0;
-#pragma unroll 16
-                for (int c = 0; c < nf; c++) rank += fcomp[c] > mine ? 1u : 0u;  // (straight-line: sixteen LDS reads in flight)
-                if (rank < K) {  // normalise, min_p (the maximum probability is exp(0) / sum)
-                    float p = weight((unsigned)(mine >> 32)) / sum;
-                    if (a.cfg.min_p > 0.0f && p < a.cfg.min_p * (1.0f / sum)) p = 0.0f;
-                    cand_p[rank] = p;
-                    cand_i[rank] = mi;
-                }
-            }
+        if (n_list > FRONT_LIST) {
+            unsigned ahead = 0;
+            for (int c = 0; c < groups; c++) ahead += (group_key[c] > key) | ((group_key[c] == key) & (c < tid)) ? 1u : 0u;
+            in = in && ahead < K;
+            if (in) list[ahead] = tid;
+            n_list = (int)min((unsigned)n_list, K);
             __syncthreads();
-            if (wave != 0) return;
-            // K <= 64 candidates, one per lane: place by (probability descending, token ascending), then the
-            // reference's sequential loops (src/generate.rs:771-800) over the lanes
-            const int nc = (int)K;
-            const float p0 = lane < nc ? cand_p[lane] : -1.0f;
-            const int i0 = lane < nc ? cand_i[lane] : 0x7FFFFFFF;
-            // (lanes past nc hold (-1, largest token): behind every candidate. Constant lane numbers: the
-            // loops below are straight-line code.)
-            int place = 0;
-#pragma unroll
-            for (int c = 0; c < WAVE; c++) {
-                const float pc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p0), c));
-                const int ic = __builtin_amdgcn_readlane(i0, c);
-                place += cand_before(pc, ic, p0, i0) ? 1 : 0;
-            }
-            // lane l wants the candidate whose place is l: scatter through LDS (wavefront 0 only; no other
-            // wavefront touches cand_p / cand_i any more)
-            cand_p[SAMPLE_MAX_K / 2 + place] = p0;  // (the candidates' places are 0 .. nc - 1; every other lane writes slot nc)
-            cand_i[SAMPLE_MAX_K / 2 + place] = i0;
-            __builtin_amdgcn_wave_barrier();  // (LDS operations of a wavefront execute in order)
-            const float p = lane < nc ? cand_p[SAMPLE_MAX_K / 2 + lane] : 0.0f;
-            const int ci = cand_i[SAMPLE_MAX_K / 2 + lane];
-            // The reference's three loops add the same probabilities in the same order from zero: cumulative until
-            // top_p is reached, the total of the kept candidates (= that cumulative sum), and the running sum
-            // the draw is compared with. One chain of additions gives all three; lane i keeps the sum after
-            // candidate i. (Lanes past nc add 0.)
-            float chain = 0.0f, upto = 0.0f;
-#pragma unroll
-            for (int i = 0; i < WAVE; i++) {
-                chain += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), i));
-                upto = lane == i ? chain : upto;
-            }
-            const unsigned long long live = nc >= WAVE ? ~0ull : ((1ull << nc) - 1ull);
-            const unsigned long long reached = __ballot(upto >= a.cfg.top_p) & live;
-            const int cutoff = reached ? __ffsll((long long)reached) : nc;  // index of the first + 1
-            const float total = cutoff > 0 ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(upto), cutoff - 1)) : 0.0f;
-            const float r = st.draw * total;
-            const unsigned long long kept = cutoff >= WAVE ? ~0ull : ((1ull << cutoff) - 1ull);
-            const unsigned long long hit = __ballot(upto >= r) & kept;
-            const int at = hit ? __ffsll((long long)hit) - 1 : cutoff - 1;
-            const int pick = at >= 0 ? __builtin_amdgcn_readlane(ci, at) : 0;
-            if (lane == 0) deliver_pick(a, st, pick);
+        }
+        auto token_at = [&](int j) { return (list[j >> group_bits] << group_bits) + (j & ((1 << group_bits) - 1)); };
+        auto logit_at = [&](int j) {
+            const int i = min(token_at(j), a.vocab - 1);
+            return LogitAndCount{a.logits[i], a.counts ? a.counts[i] : 0};
+        };
+        // (tokens past the vocabulary come last: the smallest key, the largest number)
+        auto key_of = [&](int j, LogitAndCount v) { return token_at(j) < a.vocab ? order_key(penalised(v.l, v.c, a.cfg) * inv_temp) : 0u; };
+        auto idx_at = [&](int j) { return token_at(j) < a.vocab ? token_at(j) : 0x7FFFFFFF; };
+        const int n = n_list << group_bits;
+        sweep(n, tid, logit_at, [&](int j, LogitAndCount v) {
+            const unsigned k = key_of(j, v);
+            if (k >= floor) survive(k, idx_at(j));
+        });
+        __syncthreads();
+        if (survived > (unsigned)SAMPLE_MAX_K) {  // a flat distribution: the general selection, which wants its items in token order
+            const unsigned long long mask = __ballot(in);
+            if (lane == 0) sh.red_i[wave] = __popcll(mask);
+            __syncthreads();
+            int at = __popcll(mask & ((1ull << lane) - 1ull));
+            for (int w = 0; w < wave; w++) at += sh.red_i[w];
+            if (in) list[at] = tid;
+            __syncthreads();
+            select_sort_draw(sh, a, st, n, a.vocab, sum, [&](int j) { return key_of(j, logit_at(j)); }, idx_at, weight);
             return;
         }
     }
-    // padding entries (tokens past the vocabulary) carry the key of -inf and the largest token number: they sort
-    // behind every real token and are never among the vocabulary's top_k
-    select_sort_draw(sh, a, st, n_kept, a.vocab, sum, [&](int j) { return f.key[j]; }, [&](int j) { return f.idx[j]; }, weight);
+    // Selection by rank: every survivor counts the survivors ahead of it, and the first K take their rank as their
+    // place.
+    const int nf = (int)survived;
+    float (&cand_p)[SAMPLE_MAX_K] = sh.cand_p;
+    int (&cand_i)[SAMPLE_MAX_K] = sh.cand_i;
+    {
+        const int bits = nf <= SAMPLE_THREADS / 8 ? 3 : 0, s = tid >> bits;  // eight threads count for one survivor, or one
+        const unsigned long long mine = fcomp[min(s, nf - 1)];
+        unsigned rank = 0;
+#pragma unroll 4
+        for (int c = tid & ((1 << bits) - 1); c < nf; c += 1 << bits) rank += fcomp[c] > mine ? 1u : 0u;
+        if (bits) {
+            rank += dpp_keys<0xB1, 0xF>(rank);
+            rank += dpp_keys<0x4E, 0xF>(rank);
+            rank += dpp_keys<0x141, 0xF>(rank);
+        }
+        if (s < nf && rank < K) {  // normalise, min_p (the maximum probability is exp(0) / sum)
+            float p = weight((unsigned)(mine >> 32)) / sum;
+            if (a.cfg.min_p > 0.0f && p < a.cfg.min_p * (1.0f / sum)) p = 0.0f;
+            cand_p[rank] = p;
+            cand_i[rank] = 0x7FFFFFFF - (int)(unsigned)(mine & 0xFFFFFFFFull);
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    // K <= 64 candidates, one per lane, in the order the reference's sequential loops walk (src/generate.rs:771-800):
+    // probability descending, token ascending. That is their order already, except where two logits have one
+    // probability (rounding, min_p).
+    const int nc = min((int)K, nf);
+    float p = lane < nc ? cand_p[lane] : 0.0f;
+    int ci = lane < nc ? cand_i[lane] : 0;
+    const float p_next = __shfl_down(p, 1, WAVE);
+    const int i_next = __shfl_down(ci, 1, WAVE);
+    if (__ballot(lane + 1 < nc && !cand_before(p, ci, p_next, i_next))) {
+        int place = 0;
+        for (int c = 0; c < nc; c++) {
+            const float pc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), c));
+            const int ic = __builtin_amdgcn_readlane(ci, c);
+            place += cand_before(pc, ic, p, ci) ? 1 : 0;
+        }
+        // lane l wants the candidate whose place is l: scatter through LDS, where every place holds a candidate before
+        // (wavefront 0 only; no other wavefront touches cand_p / cand_i any more, and a wavefront's LDS operations
+        // execute in order)
+        if (lane < nc) {
+            cand_p[place] = p;
+            cand_i[place] = ci;
+        }
+        __builtin_amdgcn_wave_barrier();
+        p = lane < nc ? cand_p[lane] : 0.0f;
+        ci = lane < nc ? cand_i[lane] : 0;
+    }
+    // The reference's three loops add the same probabilities in the same order from zero: cumulative until top_p is
+    // reached, the total of the kept candidates (= that cumulative sum), and the running sum the draw is compared
+    // with. One chain of additions gives all three, lane i ends with the sum after candidate i: every step adds to each
+    // lane's p the lane before's sum (0 ahead of lane 0), and the i-th step leaves lane i - 1's at its last value.
+    float upto = 0.0f;
+    for (int i = 0; i < nc; i += 8)
+#pragma unroll
+        for (int u = 0; u < 8; u++) upto = dpp_move<0x138, 0xF>(upto, 0.0f) + p;  // wave_shr:1
+    const unsigned long long live = nc >= WAVE ? ~0ull : ((1ull << nc) - 1ull);
+    const unsigned long long reached = __ballot(upto >= a.cfg.top_p) & live;
+    const int cutoff = reached ? __ffsll((long long)reached) : nc;  // index of the first + 1
+    const float total = cutoff > 0 ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(upto), cutoff - 1)) : 0.0f;
+    const float r = st.draw * total;
+    const unsigned long long kept = cutoff >= WAVE ? ~0ull : ((1ull << cutoff) - 1ull);
+    const unsigned long long hit = __ballot(upto >= r) & kept;
+    const int at = hit ? __ffsll((long long)hit) - 1 : cutoff - 1;
+    const int pick = at >= 0 ? __builtin_amdgcn_readlane(ci, at) : 0;
+    if (lane == 0) deliver_pick(a, st, pick);
 }
 
 __global__ void count_tokens_kernel(const uint32_t *__restrict__ ids, int n_ids, int *__restrict__ counts, int vocab) {
@@ -719,14 +763,16 @@ int sample_check_config(hm_ctx *ctx, const hm_sampling_config *cfg, bool device)
 }
 
 // One workgroup for everything, or the front / back pair when top_k is small and the vocabulary large (the pair
-// keeps its 130 words per 1024 tokens in `work`, which has a word per token).
+// keeps its three words per group of 64 tokens or more in `work`, which has a word per token).
 static int sample_enqueue(hm_ctx *ctx, const SampleArgs &a) {
-    const bool pair = a.cfg.temperature > 0.0f && a.cfg.top_k >= 1 && a.cfg.top_k <= FRONT_KEEP && a.vocab >= 4096;
+    const bool pair = a.cfg.temperature > 0.0f && a.cfg.top_k >= 1 && a.cfg.top_k <= FRONT_MAX_K && a.vocab >= 4096;
     if (pair) {
-        const int blocks = (a.vocab + SAMPLE_THREADS - 1) / SAMPLE_THREADS;
-        hipLaunchKernelGGL(sample_front_kernel, dim3(blocks), dim3(SAMPLE_THREADS), 0, ctx->stream, a);
+        int bits = FRONT_GROUP_BITS;
+        while (((a.vocab - 1) >> bits) + 1 > SAMPLE_THREADS) bits++;
+        const int groups = ((a.vocab - 1) >> bits) + 1, per_block = FRONT_THREADS / WAVE;
+        hipLaunchKernelGGL(sample_front_kernel, dim3((groups + per_block - 1) / per_block), dim3(FRONT_THREADS), 0, ctx->stream, a, groups, bits);
         HM_LAUNCH_CHECK(ctx);
-        hipLaunchKernelGGL(sample_back_kernel, dim3(1), dim3(SAMPLE_THREADS), 0, ctx->stream, a, blocks);
+        hipLaunchKernelGGL(sample_back_kernel, dim3(1), dim3(SAMPLE_THREADS), 0, ctx->stream, a, groups, bits);
     } else {
         hipLaunchKernelGGL(sample_token_kernel, dim3(1), dim3(SAMPLE_THREADS), 0, ctx->stream, a);
     }

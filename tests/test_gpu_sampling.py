@@ -103,6 +103,30 @@ def test_two_launch_sampler_with_ties_and_masked_logits(ctx, vocab, top_k):
     assert compared >= 16
 
 
+# groups of 64, 128, 256 and 512 tokens with the last one full and not, 64 to 1024 of them, one and 64 candidates
+@pytest.mark.parametrize("vocab,top_k", [(4096, 64), (4097, 1), (16384, 50), (16385, 50), (65536, 64), (65537, 40), (262144, 64), (262145, 50)])
+def test_two_launch_sampler_of_every_group_size(ctx, vocab, top_k):
+    """Penalties on a third of the tokens that lead, and leading tokens at the groups' and the vocabulary's edges."""
+    gen = np.random.default_rng(vocab + top_k)
+    cfg = Cfg(temperature=0.8, top_k=top_k, top_p=0.97, min_p=0.01, repetition_penalty=1.2, frequency_penalty=0.2, presence_penalty=0.1)
+    compared = 0
+    for trial in range(4):
+        logits = (gen.standard_normal(vocab) * 2.5).astype(np.float32)
+        edges = [0, 63, 64, 127, 128, 255, 256, 511, 512, vocab - 2, vocab - 1]
+        logits[edges] = logits.max() + gen.uniform(-2, 1, len(edges)).astype(np.float32)
+        generated = np.argsort(-logits)[:120:3].tolist() if trial else []
+        d = ctx.to_device(logits)
+        a, b = pyoracle.Rng(70 + trial), runtime.Rng(70 + trial)
+        for _ in range(6):
+            want, margins = pyoracle.sample_token(logits, cfg, generated, a, want_margins=True)
+            got = ctx.sample_token(d, vocab, lib_cfg(cfg), generated, b)
+            if not on_edge(margins, cfg):
+                assert got == want, (vocab, top_k, trial)
+                compared += 1
+        d.free()
+    assert compared >= 16
+
+
 def test_device_sampler_reference_cases_and_errors(ctx):
     # sample_token_greedy and min_p_filters_low_prob (src/generate.rs:891-900, :990-1008)
     d = ctx.to_device(np.array([0.0, 1.0, 0.5, 0.2], np.float32))
