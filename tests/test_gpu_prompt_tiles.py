@@ -219,6 +219,28 @@ def test_selective_scan_in_segments(ctx, n):
     m.close()
 
 
+# one chunk at its limit, two of uneven and of equal rows, five
+@pytest.mark.parametrize("n", [512, 513, 1024, 2050])
+def test_gated_recurrence_in_chunks(ctx, n):
+    """As above for rows that one workgroup does not hold: chunks of them against portions of 100, the tolerance as there. Widths on
+    both sides of a workgroup's 16 channels, filter histories that reach across the portions."""
+    cfg = {"architecture": "Nokuvik", "vocab": 96, "width": 64, "embedding": {"scale": 1.0}, "norm": {"eps": 1e-5}, "loop": None,
+           "layers": [{"type": "rglru", "mlp": None, "mixer": {"width": w, "conv": c, "blocks": b}} for w, c, b in ((60, 3, 3), (64, 4, 1), (144, 2, 9))]}
+    m = synth_model.build_block_model(ctx, cfg, 3, 4096, DTYPE_F32)
+    ids = synth.token_ids(n, n + 51, cfg["vocab"])
+    for past in (0, 50):
+        got = []
+        for step in (n, 100):
+            m.reset_kv_cache()
+            if past:
+                m.prefill(ids[:past], want_logits=False)
+            out = [m.prefill(ids[at:min(at + step, past + n)]) for at in range(past, past + n, step)]
+            got.append((np.concatenate(out).astype(np.float64), m.run_kv(ids[past + n:past + n + 1])[0].astype(np.float64)))
+        for a, b in zip(*got):
+            assert np.abs(a - b).max() <= 2e-4 * np.abs(b).max()
+    m.close()
+
+
 def test_long_k_quant_prompt_with_wide_rows(ctx):
     """Rows of 18 blocks need two K slices (a workgroup's tables hold 16), also where the tiles alone fill the chip."""
     cfg = synth_model.TransformerConfig(hidden_size=2048, intermediate_size=4608, num_attention_heads=16, num_hidden_layers=1, vocab_size=512,
