@@ -26,6 +26,21 @@ struct GemvConv {
     int gelu_from = 0;                   // rows from here on: out = gelu_tanh(W.x + bias) (0: none)
 };
 
+// Prologue of a matrix memory's output projection (matrix_memory.h): the row is what the memory's heads put out, every head over its
+// normaliser and its root mean square, weighted and gated. K == heads * vdim <= 4096, vdim 64, 128, 256 or 512, so that a head's columns
+// belong to one wavefront.
+struct GemvHeads {
+    const float *raw = nullptr;          // [heads][cols], the normaliser's product in column vdim
+    const float *gate = nullptr, *norm = nullptr;  // [heads * vdim]
+    const float *tops = nullptr;         // [2][heads]: the half behind position p is (p + 1) % 2
+    const DecodeState *state = nullptr;  // position of the token
+    int heads = 0, vdim = 0, cols = 0;
+    float eps = 0.f;
+};
+inline bool gemv_takes_heads(int heads, int vdim, int K) {
+    return heads > 0 && (vdim == 64 || vdim == 128 || vdim == 256 || vdim == 512) && heads * vdim == K && K <= 4096;
+}
+
 struct GemvArgs {
     const float *x = nullptr;                  // [M][K]
     const void *w = nullptr;                   // [N][K] bf16 (or f32 when w_f32)
@@ -45,6 +60,7 @@ struct GemvArgs {
     float *argmax_val = nullptr;               // [argmax_cap]
     int *argmax_idx = nullptr;                 // [argmax_cap]
     int argmax_cap = 0;
+    GemvHeads heads;                           // instead of x and the prologue above
     GemvConv conv;                             // GEMV_EPI_CONV
     homura::GatedAct act;                      // paired epilogue
 };

@@ -9,6 +9,7 @@
 //       last-arriver fold in fixed order).
 // These are HBM-bandwidth kernels: algorithmic traffic is K*N*2 bytes of weights per call.
 #include "gemv_bf16.h"
+#include "matrix_memory.h"
 
 // ─────────────────────────── [N][K] stream layout ───────────────────────────
 
@@ -425,7 +426,9 @@ bool try_oneshot(hm_ctx *ctx, const GemvArgs &a, int epi, int *rc) {
 // PRO: residual add and RMSNorm of the activation row (reference src/hf/emitter.rs:787,
 // src/graph_builder/emit_linalg.rs:7-26) on the pieces in registers - the wavefronts' chunks cover the row
 // exactly once, so their sums of squares add up to the row's. Nothing is staged in LDS. PRO = 2: the residual
-// is normalised on its own first (a layer with a norm behind its sublayer), with a second round of the same sums.
+// is normalised on its own first (a layer with a norm behind its sublayer), with a second round of the same sums. PRO = 3: the heads of
+// a matrix memory (GemvHeads), each inside a wavefront, so no barrier more. A launch of its own for them was bound by itself and its two
+// trips to memory (heads of 4 x 256: 2.6 us and 3.1 for the product, 3.9 together).
 __device__ __forceinline__ float gelu_tanh_dev(float z) {
     const float u = 0.79788456080286535588f * (z + 0.044715f * z * z * z);
     return 0.5f * z * (1.0f + tanhf(u));
@@ -442,18 +445,34 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_bf16_nk_splitk_kernel(GemvA
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 x0[NC], x1[NC], p0[PRO ? NC : 1], p1[PRO ? NC : 1], n0[PRO ? NC : 1], n1[PRO ? NC : 1];
     f32x4 q0[PRO == 2 ? NC : 1], q1[PRO == 2 ? NC : 1];
+    float den[PRO == 3 ? NC : 1], top[PRO == 3 ? NC : 1];
     u32x4 wv[NC][R];
 #pragma unroll
     for (int c = 0; c < NC; c++) {
         const int k = ((c * GEMV_WAVES + wave) * WAVE + lane) * 8;
         const bool ok = k < K;
+        if constexpr (PRO == 3) {
+            const GemvHeads &m = a.heads;
+            const int h = ok ? k / m.vdim : 0;
+            const float *raw = m.raw + (size_t)h * m.cols, *o = raw + (ok ? k - h * m.vdim : 0);
+            x0[c] = ok ? *reinterpret_cast<const f32x4 *>(o) : zero;
+            x1[c] = ok ? *reinterpret_cast<const f32x4 *>(o + 4) : zero;
+            p0[c] = ok ? *reinterpret_cast<const f32x4 *>(m.gate + k) : zero;
+            p1[c] = ok ? *reinterpret_cast<const f32x4 *>(m.gate + k + 4) : zero;
+            n0[c] = ok ? *reinterpret_cast<const f32x4 *>(m.norm + k) : zero;
+            n1[c] = ok ? *reinterpret_cast<const f32x4 *>(m.norm + k + 4) : zero;
+            den[c] = raw[m.vdim];
+            const float even = m.tops[h], odd = m.tops[m.heads + h];  // (both: the position is on its way too)
+            top[c] = (m.state->pos + 1) & 1 ? odd : even;
+            continue;
+        }
         x0[c] = ok ? *reinterpret_cast<const f32x4 *>(a.x + k) : zero;
         x1[c] = ok ? *reinterpret_cast<const f32x4 *>(a.x + k + 4) : zero;
         if constexpr (PRO == 2) {
             q0[c] = ok ? *reinterpret_cast<const f32x4 *>(a.post_norm_w + k) : zero;
             q1[c] = ok ? *reinterpret_cast<const f32x4 *>(a.post_norm_w + k + 4) : zero;
         }
-        if constexpr (PRO != 0) {
+        if constexpr (PRO == 1 || PRO == 2) {
             p0[c] = (ok && a.prologue_residual) ? *reinterpret_cast<const f32x4 *>(a.prologue_residual + k) : zero;
             p1[c] = (ok && a.prologue_residual) ? *reinterpret_cast<const f32x4 *>(a.prologue_residual + k + 4) : zero;
             n0[c] = (ok && a.norm_w) ? *reinterpret_cast<const f32x4 *>(a.norm_w + k) : zero;
@@ -471,7 +490,26 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_bf16_nk_splitk_kernel(GemvA
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above goes out before any arithmetic below
-    if constexpr (PRO != 0) {
+    if constexpr (PRO == 3) {
+        const int lanes = a.heads.vdim / 8;  // of a head
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            float ss = x0[c].x * x0[c].x + x0[c].y * x0[c].y + x0[c].z * x0[c].z + x0[c].w * x0[c].w;
+            ss += x1[c].x * x1[c].x + x1[c].y * x1[c].y + x1[c].z * x1[c].z + x1[c].w * x1[c].w;
+            ss += dpp_move<0xB1, 0xF>(ss, 0.f);   // quad_perm [1,0,3,2]
+            ss += dpp_move<0x4E, 0xF>(ss, 0.f);   // quad_perm [2,3,0,1]
+            ss += dpp_move<0x141, 0xF>(ss, 0.f);  // row_half_mirror
+            for (int off = 8; off < lanes; off <<= 1) ss += __shfl_xor(ss, off, WAVE);
+            float inv_den;
+            const float inv = homura::memory_head_scale(ss, a.heads.vdim, den[c], expf(-top[c]), a.heads.eps, inv_den);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                x0[c][j] = x0[c][j] * inv_den * inv * n0[c][j] / (1.0f + expf(-p0[c][j]));
+                x1[c][j] = x1[c][j] * inv_den * inv * n1[c][j] / (1.0f + expf(-p1[c][j]));
+            }
+        }
+    }
+    if constexpr (PRO == 1 || PRO == 2) {
         const float mean_over = (float)(a.norm_dim ? a.norm_dim : K);
         if constexpr (PRO == 2) {
             float sq = 0.f;
@@ -578,7 +616,10 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_bf16_nk_splitk_kernel(GemvA
 template <int R, int NC>
 int launch_splitk(hm_ctx *ctx, const GemvArgs &a, int epi, bool pro) {
     const int grid = (a.N + R - 1) / R;
-    if (pro) {
+    if (a.heads.raw) {
+        if constexpr (NC <= 2 && R <= 4)
+            hipLaunchKernelGGL((gemv_bf16_nk_splitk_kernel<R, NC, 3>), dim3(grid), dim3(GEMV_THREADS), 0, ctx->stream, a, epi);
+    } else if (pro) {
         if constexpr (NC <= 4 && R >= 4) {
             if (a.post_norm_w)
                 hipLaunchKernelGGL((gemv_bf16_nk_splitk_kernel<R, NC, 2>), dim3(grid), dim3(GEMV_THREADS), 0, ctx->stream, a, epi);
@@ -594,7 +635,7 @@ int launch_splitk(hm_ctx *ctx, const GemvArgs &a, int epi, bool pro) {
 
 // Post-norms, padded rows, activations beside SiLU and the convolution epilogue are in the cut-row kernel only.
 bool gemv_needs_splitk(const GemvArgs &a, int epi) {
-    return a.post_norm_w || a.norm_dim || epi == GEMV_EPI_CONV || (epi == GEMV_EPI_SILU_MUL_PAIRS && a.act.kind != homura::GatedAct::Silu);
+    return a.heads.raw || a.post_norm_w || a.norm_dim || epi == GEMV_EPI_CONV || (epi == GEMV_EPI_SILU_MUL_PAIRS && a.act.kind != homura::GatedAct::Silu);
 }
 
 // One activation row, bf16 weights, rows of 512 .. 16384 elements (with a prologue: up to 8192), fewer than
@@ -620,6 +661,7 @@ bool try_splitk(hm_ctx *ctx, const GemvArgs &a, int epi, int *rc) {
     // 16 rows gain nothing more (32 steps of Qwen2.5-1.5B, 1536 -> 17920: 40.8 ms with 4, 40.1 with 8, 40.7 with 16).
     int r;
     if (pro) r = a.N >= 8192 ? 8 : 4;
+    else if (a.heads.raw) r = 4;  // (12 bytes per k and the gates' exponentials: 1024 -> 1024 5.3 / 4.1 / 3.9 us with 1 / 2 / 4 rows)
     else r = (a.K >= 4096 && a.N >= 2048) ? 4 : ((a.N <= 1536 && bytes < ((size_t)17 << 19)) ? 1 : 2);
     if (epi == GEMV_EPI_SILU_MUL_PAIRS && r == 1) r = 2;
 #define HM_SPLITK(RR, CC) \
@@ -681,6 +723,11 @@ int gemv_bf16_nk_launch(hm_ctx *ctx, GemvArgs a, int M, int epi) {
     if (gemv_needs_splitk(a, epi)) {
         HM_REQUIRE(ctx, M == 1 && !a.w_f32 && epi != GEMV_EPI_ARGMAX && a.K <= ((a.norm_w || a.prologue_residual || a.resid_out) ? 8192 : 16384),
                    "gemv: post-norm, padded norm, other activations and convolution take one bf16 row of at most 8192 (without a prologue 16384) elements");
+        const GemvHeads &m = a.heads;
+        HM_REQUIRE(ctx, !m.raw || (gemv_takes_heads(m.heads, m.vdim, a.K) && m.cols > m.vdim && m.cols % 4 == 0 && m.gate && m.norm && m.tops && m.state &&
+                                   !a.norm_w && !a.prologue_residual && !a.resid_out && !a.post_norm_w &&
+                                   (((uintptr_t)m.raw | (uintptr_t)m.gate | (uintptr_t)m.norm) % 16) == 0),
+                   "gemv: a matrix memory's heads of 64, 128, 256 or 512 columns fill a row of at most 4096");
         HM_REQUIRE(ctx, !a.post_norm_w || a.prologue_residual, "gemv: a post-norm needs the row it normalises");
         if (epi == GEMV_EPI_CONV)
             HM_REQUIRE(ctx, a.conv.rows > 0 && a.conv.rows <= a.N && a.conv.taps > 0 && a.conv.w && a.conv.b && a.conv.ring && a.conv.state,

@@ -757,7 +757,7 @@ int BlockModel::emit_plan() {
     const Vec *pending = nullptr;   // y waits to be added behind this norm
     // One projection of the row in `in`; of the residual with what is pending, and through norm_w if there is one.
     auto gemv = [&](const std::string &name, const Linear &lin, size_t in, size_t out, const float *norm_w, int epi, const float *bias = nullptr,
-                    std::function<void(const StepContext &, GemvArgs &)> more = nullptr) {
+                    std::function<void(const StepContext &, GemvArgs &)> more = nullptr, size_t also = SIZE_MAX) {
         const size_t src = in;
         size_t next = in;
         const float *post = nullptr;
@@ -769,6 +769,7 @@ int BlockModel::emit_plan() {
         const bool to_act = epi == GEMV_EPI_SILU_MUL_PAIRS;
         std::vector<size_t> ins{src};
         std::vector<size_t> outs{out};
+        if (also != SIZE_MAX) ins.push_back(also);
         if (post) {
             ins.push_back(s_y);
             outs.push_back(next);
@@ -838,6 +839,8 @@ int BlockModel::emit_plan() {
             cur = s_xa;
         }
         const Linear *out_w = nullptr;
+        size_t out_in = s_act, out_also = SIZE_MAX;
+        std::function<void(const StepContext &, GemvArgs &)> out_args;
         if (s.mixer == MixerKind::LatentAttention) {
             const LatentAttentionSpec &a = s.attn;
             gemv("gemv[latent_down]", l.la_down, cur, s_d1, norm1, GEMV_EPI_NONE);
@@ -988,9 +991,26 @@ int BlockModel::emit_plan() {
             };
             step("Memory", "memory_step", 8.0 * shape.memory_floats() + 4.0 * d.mm_n, 0, {s_d1}, {s_d2},
                  [=](const StepContext &sc) -> int { return matrix_memory_step_launch(sc.ctx, args(sc)); });
-            step("Memory", "memory_out", 16.0 * shape.heads * shape.vdim, 0, {s_d1, s_d2}, {s_act},
-                 [=](const StepContext &sc) -> int { return matrix_memory_step_out_launch(sc.ctx, args(sc)); });
             out_w = &l.mm_o;
+            if (gemv_takes_heads(shape.heads, shape.vdim, l.mm_o.kp)) {
+                out_in = s_d2;
+                out_also = s_d1;
+                out_args = [=](const StepContext &sc, GemvArgs &g) {
+                    const MatrixMemoryStepArgs x = args(sc);
+                    g.heads.raw = x.raw;
+                    g.heads.gate = x.row + at.g;
+                    g.heads.norm = x.norm;
+                    g.heads.tops = x.state + shape.memory_floats();
+                    g.heads.state = x.cursor;
+                    g.heads.heads = shape.heads;
+                    g.heads.vdim = shape.vdim;
+                    g.heads.cols = shape.cols();
+                    g.heads.eps = x.eps;
+                };
+            } else {
+                step("Memory", "memory_out", 16.0 * shape.heads * shape.vdim, 0, {s_d1, s_d2}, {s_act},
+                     [=](const StepContext &sc) -> int { return matrix_memory_step_out_launch(sc.ctx, args(sc)); });
+            }
         } else {
             st.tap_rows = s.rec.taps;
             st.tap_width = d.width;
@@ -1024,7 +1044,7 @@ int BlockModel::emit_plan() {
             out_w = &l.lr_o;
         }
         specs.push_back(st);
-        gemv("gemv[mixer_out]", *out_w, s_act, s_y, nullptr, GEMV_EPI_NONE);
+        gemv("gemv[mixer_out]", *out_w, out_in, s_y, nullptr, GEMV_EPI_NONE, nullptr, out_args, out_also);
         pending = &l.norm1b;
         if (!s.ff.width) continue;
         const float *norm2 = cfg_.pre_norms ? l.norm2.ptr() : nullptr;

@@ -55,6 +55,12 @@ struct MatrixMemoryStepArgs {
 int matrix_memory_step_launch(hm_ctx *ctx, const MatrixMemoryStepArgs &a);
 int matrix_memory_step_out_launch(hm_ctx *ctx, const MatrixMemoryStepArgs &a);
 
+// Norm of one head's columns: ss their sum of squares, den the normaliser's product, floor_ e^-m.
+__device__ __forceinline__ float memory_head_scale(float ss, int vdim, float den, float floor_, float eps, float &inv_den) {
+    inv_den = 1.0f / (fmaxf(fabsf(den), floor_) + 1e-6f);
+    return 1.0f / sqrtf(ss * inv_den * inv_den / (float)vdim + eps);
+}
+
 // ── prompt pass, n rows at positions past .. past + n - 1 ──
 struct MatrixMemoryRowsArgs {
     MatrixMemoryShape s;

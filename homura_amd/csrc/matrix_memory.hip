@@ -92,12 +92,6 @@ __global__ __launch_bounds__(256) void matrix_memory_step_kernel(MatrixMemorySte
     if (tid == 0 && tile == 0) tops[((pos + 1) & 1) * s.heads + h] = top;
 }
 
-// norm and gates of one head: o(c) the raw columns, g(c) the output gate's logits
-__device__ __forceinline__ float head_scale(float ss, int vdim, float den, float floor_, float eps, float &inv_den) {
-    inv_den = 1.0f / (fmaxf(fabsf(den), floor_) + 1e-6f);
-    return 1.0f / sqrtf(ss * inv_den * inv_den / (float)vdim + eps);
-}
-
 __global__ __launch_bounds__(256) void matrix_memory_step_out_kernel(MatrixMemoryStepArgs a) {
     __shared__ float red[4];
     const MatrixMemoryShape &s = a.s;
@@ -123,7 +117,7 @@ __global__ __launch_bounds__(256) void matrix_memory_step_out_kernel(MatrixMemor
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
     float inv_den;
-    const float inv = head_scale((red[0] + red[1]) + (red[2] + red[3]), s.vdim, den, expf(-top), a.eps, inv_den);
+    const float inv = memory_head_scale((red[0] + red[1]) + (red[2] + red[3]), s.vdim, den, expf(-top), a.eps, inv_den);
 #pragma unroll
     for (int j = 0; j < KEEP; j++) {
         const int c = tid + j * 256;
@@ -713,7 +707,7 @@ __global__ __launch_bounds__(256) void matrix_memory_out_kernel(MatrixMemoryRows
             }
             ss += (x[j][0] * x[j][0] + x[j][1] * x[j][1]) + (x[j][2] * x[j][2] + x[j][3] * x[j][3]);
         }
-        const float inv = head_scale(wave_sum(ss), s.vdim, den, low, a.eps, inv_den);
+        const float inv = memory_head_scale(wave_sum(ss), s.vdim, den, low, a.eps, inv_den);
 #pragma unroll
         for (int j = 0; j < KEEP; j++) {
             const int c = (lane + 64 * j) * 4;
@@ -726,7 +720,7 @@ __global__ __launch_bounds__(256) void matrix_memory_out_kernel(MatrixMemoryRows
         return;
     }
     for (int c = lane; c < s.vdim; c += 64) ss += o[c] * o[c];
-    const float inv = head_scale(wave_sum(ss), s.vdim, den, low, a.eps, inv_den);
+    const float inv = memory_head_scale(wave_sum(ss), s.vdim, den, low, a.eps, inv_den);
     for (int c = lane; c < s.vdim; c += 64) {
         const float y = o[c] * inv_den * inv * a.norm[(size_t)h * s.vdim + c] / (1.0f + expf(-source_at(in, t, a.at.g + h * s.vdim + c)));
         split_store(out, a.out_cols, h * s.vdim + c, y, a.out_pieces);

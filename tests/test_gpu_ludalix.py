@@ -103,6 +103,13 @@ def test_one_mechanism(ctx, name, dtype):
     check(ctx, cfg, 45, dtype, seed=20, prefill_min=0)
 
 
+# heads that the output projection takes as they come: of 8 to 64 lanes, fewer than a wavefront's, a row of one and of two chunks, the
+# longest; and the next beyond each limit
+@pytest.mark.parametrize("heads,vdim", [(1, 64), (9, 64), (3, 128), (4, 256), (9, 256), (1, 512), (8, 512), (9, 512), (3, 32), (2, 96), (1, 1024)])
+def test_memory_heads_in_the_output_projection(ctx, heads, vdim):
+    check(ctx, lf.config([lf.memory(heads=heads, dim=24, vdim=vdim), lf.memory(heads=heads, dim=24, vdim=vdim)]), 24, "f32", prefill_min=0)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("width,ff,experts,top", [(64, 64, 3, 1), (128, 200, 6, 2), (320, 128, 2, 2), (192, 448, 40, 5)])
 def test_expert_products(ctx, width, ff, experts, top, dtype):
