@@ -363,21 +363,25 @@ __global__ __launch_bounds__(256) void selective_step_kernel(SelectiveStepArgs a
 // becomes); the state each segment starts from follows from the totals of those before it, and a second walk gives
 // the states.
 //
-// More rows than a workgroup holds are cut into chunks (grid.y) for two launches. ENDS: the totals of every chunk but
-// the last, left in g.prod and g.sum, with the state the first one starts from. Then every chunk folds the totals ahead
-// of it. (A launch a chunk fills half the chip with 2048 channels and waits for memory and for the chunk ahead each time:
-// 2048 rows of 2048 channels 41.3 us in four launches, 8.6 + 15.5 so.)
+// More rows than a workgroup holds are cut into chunks (grid.y) for two launches. ENDS: of every chunk but the last, all whole, the
+// pairs (p, q) that take the state it starts from to the one it ends with, s = p s + q for each in turn: the totals of all segments but
+// the last and the last one's rows. Then every chunk takes the first one's state through the pairs of those ahead of it. That is
+// how the state moves from chunk to chunk in launches one behind the other, add for add, so a prompt gives the same bits in one pass as in
+// portions of LR_MAX_ROWS. (A launch a chunk fills half the chip with 2048 channels and waits for memory and for the chunk ahead
+// each time: 2048 rows of 2048 channels 41.3 us in four launches, 8.7 + 15.6 so.)
 constexpr int LR_SEGS = 64, LR_LEN = 8, LR_MAX_ROWS = LR_SEGS * LR_LEN;
-constexpr int LR_CHUNKS = 64;  // of a pair of launches
+constexpr int LR_LINKS = (LR_SEGS - 1 + LR_LEN) * 16;  // pairs of a chunk's 16 channels
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 struct RecurrenceChunks {
-    int rows = 0;                                            // of a chunk; 0: there is only one
-    float *state = nullptr, *prod = nullptr, *sum = nullptr; // [width], [chunks][width], [chunks][width]
+    f32x2 *links = nullptr;  // [chunks - 1][ceil(width / 16)][segments, then rows][16]; NULL: there is one chunk
+    float *state = nullptr;  // [ceil(width / 16) * 16]
 };
 template <bool ENDS>
 __global__ __launch_bounds__(16 * LR_SEGS) void linear_recurrence_kernel(LinearRecurrenceArgs a, RecurrenceChunks g) {
-    __shared__ float s_p[LR_SEGS][16], s_q[LR_SEGS][16];
+    __shared__ float s_p[LR_SEGS][16], s_q[LR_SEGS][16], s_start[16];
+    __shared__ f32x2 s_link[ENDS ? 1 : LR_LINKS];
     const int ch = threadIdx.x & 15, seg = threadIdx.x >> 4, c0 = blockIdx.x * 16, c = c0 + ch;
-    const int t_first = blockIdx.y * g.rows, n = g.rows ? min(a.n, t_first + g.rows) : a.n;  // rows t_first .. n - 1
+    const int t_first = blockIdx.y * LR_MAX_ROWS, n = min(a.n, t_first + LR_MAX_ROWS);  // rows t_first .. n - 1
     const bool live = c < a.channels;
     const int cc = live ? c : 0;
     const int len = (n - t_first + LR_SEGS - 1) / LR_SEGS, t_begin = min(n, t_first + seg * len), rows = min(n, t_begin + len) - t_begin;
@@ -385,13 +389,19 @@ __global__ __launch_bounds__(16 * LR_SEGS) void linear_recurrence_kernel(LinearR
     const float *gr = a.gates + blk * 2 * a.block_pad + (cc - blk * a.block_width), *gi = gr + a.block_pad;
     const float rb = a.r_bias[cc], ib = a.i_bias[cc], decay = a.decay[cc];
     float av[LR_LEN], bv[LR_LEN], yv[LR_LEN];
-    float S;  // (a.state is read ahead of the barrier: one segment writes it at the end; the other chunks have their copy of it)
-    if (ENDS || !g.rows) {
-        S = a.past && live ? a.state[c] : 0.f;
-    } else {
-        S = g.state[cc];
-        for (int q = 0; q < (int)blockIdx.y; q++) S = fmaf(g.prod[(size_t)q * a.width + cc], S, g.sum[(size_t)q * a.width + cc]);
-    }
+    // (a.state is read ahead of the barrier: one segment writes it at the end; the workgroups of several chunks have their copy of it)
+    float S = !ENDS && g.links ? g.state[c] : a.past && live ? a.state[c] : 0.f;
+    // The first wavefront brings the pairs of the chunks ahead, one chunk's on the way here while another's are taken in turn. (The whole
+    // workgroup bringing them, two barriers a chunk: 18.3 us instead of 15.6, 2048 rows of 2048 channels.)
+    constexpr int NA = (LR_LINKS + WAVE - 1) / WAVE;
+    f32x2 ahead[NA];
+    auto at = [&](int j) { return min((int)threadIdx.x + j * WAVE, LR_LINKS - 1); };
+    auto ask = [&](int q) {
+        const f32x2 *from = g.links + ((size_t)q * gridDim.x + blockIdx.x) * LR_LINKS;
+#pragma unroll
+        for (int j = 0; j < NA; j++) ahead[j] = from[at(j)];
+    };
+    if (!ENDS && blockIdx.y && threadIdx.x < WAVE) ask(0);
     {
         float r_[LR_LEN], i_[LR_LEN], u_[LR_LEN];
 #pragma unroll
@@ -416,32 +426,33 @@ __global__ __launch_bounds__(16 * LR_SEGS) void linear_recurrence_kernel(LinearR
             P *= av[k];
             Q = fmaf(av[k], Q, bv[k]);
         }
-    s_p[seg][ch] = P;
-    s_q[seg][ch] = Q;
-    __syncthreads();
     if constexpr (ENDS) {
-        if (threadIdx.x >= WAVE) return;  // one wavefront, sixteen segments a lane; then lanes 0 .. 15 have the quarters joined
-        P = 1.f;
-        Q = 0.f;
-#pragma unroll 8
-        for (int k = 0; k < LR_SEGS / 4; k++) {
-            const float p = s_p[seg * (LR_SEGS / 4) + k][ch];
-            P *= p;
-            Q = fmaf(p, Q, s_q[seg * (LR_SEGS / 4) + k][ch]);
+        f32x2 *to = g.links + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * LR_LINKS + threadIdx.x;
+        if (seg < LR_SEGS - 1) {
+            *to = f32x2{P, Q};
+        } else {
+#pragma unroll
+            for (int k = 0; k < LR_LEN; k++) to[k * 16] = f32x2{av[k], bv[k]};
         }
-        for (int off = 16; off < WAVE; off <<= 1) {
-            const float p = __shfl_down(P, off, WAVE), q = __shfl_down(Q, off, WAVE);
-            Q = fmaf(p, Q, q);
-            P *= p;
-        }
-        if (threadIdx.x < 16 && live) {
-            const size_t at = (size_t)blockIdx.y * a.width + c;
-            g.prod[at] = P;
-            g.sum[at] = Q;
-            if (blockIdx.y == 0) g.state[c] = S;
-        }
+        if (blockIdx.y == 0 && seg == 0) g.state[c] = S;
         return;
     }
+    s_p[seg][ch] = P;
+    s_q[seg][ch] = Q;
+    if (blockIdx.y && threadIdx.x < WAVE) {
+        for (int q = 0; q < (int)blockIdx.y; q++) {
+#pragma unroll
+            for (int j = 0; j < NA; j++) s_link[at(j)] = ahead[j];
+            if (q + 1 < (int)blockIdx.y) ask(q + 1);
+            __builtin_amdgcn_wave_barrier();  // (LDS operations of a wavefront execute in order)
+#pragma unroll
+            for (int k = 0; k < LR_LINKS / 16; k++) S = fmaf(s_link[k * 16 + ch][0], S, s_link[k * 16 + ch][1]);
+            __builtin_amdgcn_wave_barrier();
+        }
+        if (seg == 0) s_start[ch] = S;
+    }
+    __syncthreads();
+    if (blockIdx.y) S = s_start[ch];
 #pragma unroll 8
     for (int s = 0; s < seg; s++) S = fmaf(s_p[s][ch], S, s_q[s][ch]);
     if (live) {
@@ -603,14 +614,14 @@ int linear_recurrence_launch(hm_ctx *ctx, const LinearRecurrenceArgs &a) {
                         a.block_width > 0 && a.block_pad >= a.block_width && a.channels % a.block_width == 0 && a.pieces >= 1 && a.pieces <= 3 &&
                         !bad_source(a.conv_in, a.width), "linear_recurrence: bad shape");
     const size_t gate_ld = (size_t)(a.channels / a.block_width) * 2 * a.block_pad;
+    const int groups = (a.width + 15) / 16;
     const dim3 block(16 * LR_SEGS);
-    dim3 grid((a.width + 15) / 16);
-    // (the kernels' part of the workspace)
-    const int most = (int)std::min<size_t>(LR_CHUNKS, ((size_t)16 << 20) / sizeof(float) / 2 / a.width);
-    const int at_once = LR_MAX_ROWS * std::max(most - 1, 1);
-    for (int at = 0; at < a.n; at += at_once) {
+    // chunks of a pair of launches: as many as the kernels' part of the workspace holds the pairs of (2048 channels: 14 and the last)
+    const size_t part = (size_t)16 << 20, state_bytes = (size_t)groups * 16 * sizeof(float), chunk_bytes = (size_t)groups * LR_LINKS * sizeof(f32x2);
+    const int most = part > state_bytes ? (int)std::min<size_t>((part - state_bytes) / chunk_bytes, 63) + 1 : 1;
+    for (int at = 0; at < a.n; at += most * LR_MAX_ROWS) {
         LinearRecurrenceArgs b = a;
-        b.n = std::min(a.n - at, at_once);
+        b.n = std::min(a.n - at, most * LR_MAX_ROWS);
         b.past = a.past + at;
         b.u = a.u + (size_t)at * a.width;
         b.y = a.y + (size_t)at * a.width;
@@ -619,15 +630,12 @@ int linear_recurrence_launch(hm_ctx *ctx, const LinearRecurrenceArgs &a) {
         b.conv_in.p = a.conv_in.p + (size_t)at * a.conv_in.ld;
         RecurrenceChunks g;
         const int chunks = (b.n + LR_MAX_ROWS - 1) / LR_MAX_ROWS;
-        grid.y = chunks;
         if (chunks > 1) {
-            g.rows = (b.n + chunks - 1) / chunks;
             g.state = static_cast<float *>(ctx->workspace);
-            g.prod = g.state + a.width;
-            g.sum = g.prod + (size_t)chunks * a.width;
-            hipLaunchKernelGGL(linear_recurrence_kernel<true>, dim3(grid.x, chunks - 1), block, 0, ctx->stream, b, g);
+            g.links = reinterpret_cast<f32x2 *>(g.state + (size_t)groups * 16);
+            hipLaunchKernelGGL(linear_recurrence_kernel<true>, dim3(groups, chunks - 1), block, 0, ctx->stream, b, g);
         }
-        hipLaunchKernelGGL(linear_recurrence_kernel<false>, grid, block, 0, ctx->stream, b, g);
+        hipLaunchKernelGGL(linear_recurrence_kernel<false>, dim3(groups, chunks), block, 0, ctx->stream, b, g);
         HM_LAUNCH_CHECK(ctx);
     }
     return HM_OK;

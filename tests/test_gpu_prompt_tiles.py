@@ -241,6 +241,25 @@ def test_gated_recurrence_in_chunks(ctx, n):
     m.close()
 
 
+# whole chunks of 512 rows, with a last one of 88 and of 300 rows; of 8192 channels a pair of launches takes four chunks
+@pytest.mark.parametrize("n,shapes", [(n, ((60, 3, 3), (64, 4, 1), (144, 2, 9))) for n in (1024, 1112, 2348, 4096)] + [(2348, ((8192, 4, 128),))])
+def test_gated_recurrence_in_one_pass_as_in_portions(ctx, n, shapes):
+    """A prompt of several chunks in one pass against portions of a chunk each, whose states go through memory: the same bits, for the
+    products of these widths add up alike whatever the rows (one slice, 32-bit sums in order)."""
+    cfg = {"architecture": "Nokuvik", "vocab": 96, "width": 64, "embedding": {"scale": 1.0}, "norm": {"eps": 1e-5}, "loop": None,
+           "layers": [{"type": "rglru", "mlp": None, "mixer": {"width": w, "conv": c, "blocks": b}} for w, c, b in shapes]}
+    m = synth_model.build_block_model(ctx, cfg, 3, 8192, DTYPE_F32)
+    ids = synth.token_ids(n + 1, n + 1, cfg["vocab"])
+    got = []
+    for step in (n, 512):
+        m.reset_kv_cache()
+        rows = [m.prefill(ids[at:min(at + step, n)]) for at in range(0, n, step)]
+        got.append((np.concatenate(rows), m.run_kv(ids[n:n + 1])))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    m.close()
+
+
 def test_long_k_quant_prompt_with_wide_rows(ctx):
     """Rows of 18 blocks need two K slices (a workgroup's tables hold 16), also where the tiles alone fill the chip."""
     cfg = synth_model.TransformerConfig(hidden_size=2048, intermediate_size=4608, num_attention_heads=16, num_hidden_layers=1, vocab_size=512,
