@@ -110,6 +110,12 @@ def test_memory_heads_in_the_output_projection(ctx, heads, vdim):
     check(ctx, lf.config([lf.memory(heads=heads, dim=24, vdim=vdim), lf.memory(heads=heads, dim=24, vdim=vdim)]), 24, "f32", prefill_min=0)
 
 
+# rows that end inside a wavefront, at one, and at a workgroup's last
+@pytest.mark.parametrize("heads,vdim", [(3, 64), (4, 256), (3, 512), (4, 512)])
+def test_memory_heads_without_an_eps(ctx, heads, vdim):
+    check(ctx, lf.config([lf.memory(heads=heads, dim=24, vdim=vdim)], eps=0.0), 12, "f32", prefill_min=0)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("width,ff,experts,top", [(64, 64, 3, 1), (128, 200, 6, 2), (320, 128, 2, 2), (192, 448, 40, 5)])
 def test_expert_products(ctx, width, ff, experts, top, dtype):
