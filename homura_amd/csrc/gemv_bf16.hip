@@ -501,13 +501,13 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_bf16_nk_splitk_kernel(GemvA
             ss += dpp_move<0x141, 0xF>(ss, 0.f);  // row_half_mirror
             for (int off = 8; off < lanes; off <<= 1) ss += __shfl_xor(ss, off, WAVE);
             float inv_den;
-            const float inv = homura::memory_head_scale(ss, a.heads.vdim, den[c], expf(-top[c]), a.heads.eps, inv_den);
+            float inv = homura::memory_head_scale(ss, a.heads.vdim, den[c], expf(-top[c]), a.heads.eps, inv_den);
             // (a lane past the row's end has no head: its sum of squares is 0, and without an eps its scale no number)
-            const bool ok = ((c * GEMV_WAVES + wave) * WAVE + lane) * 8 < K;
+            if (((c * GEMV_WAVES + wave) * WAVE + lane) * 8 >= K) inv = 0.f;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                x0[c][j] = ok ? x0[c][j] * inv_den * inv * n0[c][j] / (1.0f + expf(-p0[c][j])) : 0.f;
-                x1[c][j] = ok ? x1[c][j] * inv_den * inv * n1[c][j] / (1.0f + expf(-p1[c][j])) : 0.f;
+                x0[c][j] = x0[c][j] * inv_den * inv * n0[c][j] / (1.0f + expf(-p0[c][j]));
+                x1[c][j] = x1[c][j] * inv_den * inv * n1[c][j] / (1.0f + expf(-p1[c][j]));
             }
         }
     }
