@@ -187,6 +187,8 @@ SIGNATURES = {
     "hm_model_reset_kv_cache": (_I, [_P]),
     "hm_model_kv_cache_len": (_I, [_P]),
     "hm_model_set_graph": (_I, [_P, _I]),
+    "hm_model_recorded_steps": (_I, [_P]),
+    "hm_model_inject_recording_failures": (_I, [_P, _I]),
     "hm_model_set_whole_step": (_I, [_P, _I]),
     "hm_model_whole_step": (_I, [_P]),
     "hm_model_whole_step_available": (_I, [_P]),

@@ -193,6 +193,18 @@ int hm_model_set_graph(hm_model *m, int on) {
     return m->impl->plan()->enable_graph(on != 0);
 }
 
+int hm_model_recorded_steps(hm_model *m) {
+    if (!m) return HM_ERR_INVALID;
+    return m->impl->plan() ? m->impl->plan()->recorded_steps() : 0;
+}
+
+int hm_model_inject_recording_failures(hm_model *m, int n) {
+    if (!m || n < 0) return HM_ERR_INVALID;
+    if (!m->impl->plan()) return hm_set_error(m->ctx, HM_ERR_STATE, "model not finalized");
+    m->impl->plan()->inject_record_failures(n);
+    return HM_OK;
+}
+
 int hm_model_set_whole_step(hm_model *m, int on) {
     if (!m) return HM_ERR_INVALID;
     HfModel *hf = m->hf("hm_model_set_whole_step");

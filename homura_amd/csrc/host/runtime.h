@@ -274,8 +274,11 @@ class ExecutionPlan {
     int arm(const int32_t *h_forced, int n_forced);
 
     // Graph replay of the step (captured lazily on first use; arguments never change), on by default for steps of more than three launches.
+    // Where the default cannot be recorded the steps are launched one by one, and hm_last_error says why; they are tried again once asked
+    // for, or once what is recorded changes (invalidate_graph). Asked for by enable_graph(true), the failure is run_kv's.
     int enable_graph(bool on);
-    bool graph_enabled() const { return use_graph_; }
+    int recorded_steps() const { return (int)graphs_.size(); }
+    void inject_record_failures(int n) { inject_record_failures_ = n; }  // test support: the next n recordings fail
     // Take the whole-step launch (when the plan has one) instead of the per-projection launches.
     int set_whole_step(bool on);
     bool whole_step() const { return whole_step_; }
@@ -340,7 +343,8 @@ class ExecutionPlan {
     hipEvent_t arm_done_ = nullptr;
     int out_cap_ = 0;
     bool prepared_ = false;
-    bool use_graph_ = true;
+    bool use_graph_ = true, graph_asked_ = false, record_failed_ = false;
+    int inject_record_failures_ = 0;
     bool whole_step_ = false;
     std::function<int()> pre_run_;
     int attn_span_ = 0;

@@ -514,7 +514,8 @@ int ExecutionPlan::time_kernels(const std::vector<Buffer *> &inputs, std::vector
 }
 
 int ExecutionPlan::enable_graph(bool on) {
-    use_graph_ = on;
+    use_graph_ = graph_asked_ = on;
+    record_failed_ = false;
     return HM_OK;
 }
 
@@ -525,6 +526,7 @@ int ExecutionPlan::set_whole_step(bool on) {
 }
 
 int ExecutionPlan::invalidate_graph() {
+    record_failed_ = false;
     if (graphs_.empty()) return HM_OK;
     HM_HIP(ctx_, hipStreamSynchronize(ctx_->stream));
     for (auto &g : graphs_) {
@@ -535,25 +537,26 @@ int ExecutionPlan::invalidate_graph() {
     return HM_OK;
 }
 
-// The recorded step for the present span, recorded now if this is its first. Where it cannot be recorded the step has been enqueued
-// launch by launch instead, as all later ones will be, and *out is NULL.
+// The recorded step for the present span, recorded now if this is its first.
 int ExecutionPlan::recorded(const Recorded **out) {
-    *out = nullptr;
     auto it = graphs_.find(attn_span_);
     if (it == graphs_.end()) {
+        if (inject_record_failures_ > 0) {
+            inject_record_failures_--;
+            return hm_set_error(ctx_, HM_ERR_HIP, "recording the decode step failed: test support asked for it");
+        }
         Recorded r{nullptr, nullptr};
+        int rc = HM_OK;
         hipError_t e = hipStreamBeginCapture(ctx_->stream, hipStreamCaptureModeRelaxed);
         if (e == hipSuccess) {
-            const int rc = run_steps(nullptr);
+            rc = run_steps(nullptr);
             e = hipStreamEndCapture(ctx_->stream, &r.graph);
-            if (rc != HM_OK) e = hipErrorUnknown;
-            if (e == hipSuccess) e = hipGraphInstantiate(&r.exec, r.graph, nullptr, nullptr, 0);
+            if (e == hipSuccess && rc == HM_OK) e = hipGraphInstantiate(&r.exec, r.graph, nullptr, nullptr, 0);
         }
-        if (e != hipSuccess) {
+        if (rc != HM_OK || e != hipSuccess) {
             (void)hipGetLastError();
             if (r.graph) (void)hipGraphDestroy(r.graph);
-            use_graph_ = false;
-            return run_steps(nullptr);
+            return rc != HM_OK ? rc : hm_set_error(ctx_, HM_ERR_HIP, "recording the decode step failed: %s", hipGetErrorString(e));
         }
         it = graphs_.emplace(attn_span_, r).first;
     }
@@ -573,13 +576,19 @@ int ExecutionPlan::run_kv(const std::vector<Buffer *> &inputs, std::vector<Buffe
     // single step (run_kv with its logits read, us: Qwen2.5-0.5B 820 -> 730, 1.5B 1200 -> 1126, Nokuvik 1024 wide 1540 -> 1340, Ludalix 1250 ->
     // 1125), and a replayed launch starts sooner behind the last (Qwen2.5-1.5B, step after step, 1086 -> 1060). A step of up to three
     // is quicker launched directly (whole-step launch of a Q4_K_M model, head and pick: 64 sampled tokens 30.10 ms replayed, 29.95 ms direct).
-    if (use_graph_ && launches_per_step() > 3) {
-        const Recorded *r = nullptr;
-        if ((rc = recorded(&r)) != HM_OK) return rc;
-        if (r) HM_HIP(ctx_, hipGraphLaunch(r->exec, ctx_->stream));
-    } else if ((rc = run_steps(nullptr)) != HM_OK) {
-        return rc;
+    // Recording and instantiating cost the first step of a span 0.3 to 0.9 ms once (135 to 289 launches; a new model's first step takes 1.0
+    // to 3.9 ms launched directly, so much is loaded then), which 4 to 25 us a step step after step, 10 to 100 with each one's logits read, earn
+    // back in 15 to 150 steps.
+    const Recorded *r = nullptr;
+    hipStreamCaptureStatus outer = hipStreamCaptureStatusNone;  // somebody else's recording takes the launches themselves
+    if (use_graph_ && !record_failed_ && launches_per_step() > 3 && hipStreamIsCapturing(ctx_->stream, &outer) == hipSuccess && outer == hipStreamCaptureStatusNone) {
+        if ((rc = recorded(&r)) != HM_OK) {
+            if (graph_asked_) return rc;
+            record_failed_ = true;
+        }
     }
+    if (r) HM_HIP(ctx_, hipGraphLaunch(r->exec, ctx_->stream));
+    else if ((rc = run_steps(nullptr)) != HM_OK) return rc;
     // one advance after all layers appended (reference src/runtime.rs:1875-1880)
     cache_->advance_by(cache_->new_tokens());
     return HM_OK;

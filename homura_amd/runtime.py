@@ -404,8 +404,16 @@ class DecoderModel:
         self._check(self.lib.hm_model_finalize(self.h, max_seq_len))
 
     def set_graph(self, on: bool):
-        """Replay each decode step from a captured HIP graph instead of launching kernel by kernel."""
+        """Replay each decode step from a captured HIP graph (the default) or launch kernel by kernel. Asked for here, a recording
+        that fails raises from the step; by default the kernels are launched one by one then."""
         self._check(self.lib.hm_model_set_graph(self.h, int(on)))
+
+    def recorded_steps(self) -> int:
+        return self._check(self.lib.hm_model_recorded_steps(self.h))
+
+    def inject_recording_failures(self, n: int):
+        """Test support: the next n recordings fail."""
+        self._check(self.lib.hm_model_inject_recording_failures(self.h, n))
 
     def reset_kv_cache(self):
         self._check(self.lib.hm_model_reset_kv_cache(self.h))

@@ -371,8 +371,14 @@ int hm_model_kv_cache_len(hm_model *m);    /* src/runtime.rs:1948-1950 */
 
 /* Replay every decode step from a captured HIP graph (on != 0, the default) or launch kernel by kernel. A step of
  * up to three launches (the whole-step kernel) is launched directly either way: that is quicker than replaying
- * so small a graph. No counterpart in the reference (its plan is a host loop over dlsym'ed functions). */
+ * so small a graph. Recording costs the first step 0.3 to 0.9 ms, and again the first one that passes 128, 2048, 4096 ... cached rows;
+ * what is recorded is kept. Where a recording fails, a model that this call was made for with on != 0 returns the error from the step; one
+ * left at the default launches kernel by kernel from then on, with the cause in hm_last_error, until this call or hm_model_set_whole_step
+ * has it try again. No counterpart in the reference (its plan is a host loop over dlsym'ed functions). */
 int hm_model_set_graph(hm_model *m, int on);
+int hm_model_recorded_steps(hm_model *m); /* how many are kept now */
+/* Test support, no counterpart in the reference: the next n recordings fail. */
+int hm_model_inject_recording_failures(hm_model *m, int n);
 
 /* One launch for a whole decode step's embedding row and decoder layers (on != 0) instead of one
  * launch per projection; the reference dispatches 1 + 3 * layers + 1 kernels per step

@@ -82,6 +82,55 @@ def test_tiny_graph_replay_matches_eager(ctx, tiny):
         gm.set_graph(False)
 
 
+@pytest.mark.parametrize("graph", [None, False, True])
+def test_steps_recorded_or_launched_one_by_one_against_the_oracle(ctx, graph):
+    """A model left at its default, told not to record and told to: a plan of more than three launches is recorded at its first step
+    unless told otherwise."""
+    cfg = synth_model.TINY
+    weights = synth_model.synth_weights(cfg, 4243)
+    gm = synth_model.build_model(ctx, cfg, weights, 96)
+    om = mf.build_oracle_model(cfg, weights, 96)
+    assert gm.launches_per_step() > 3
+    if graph is not None:
+        gm.set_graph(graph)
+    gm.set_prefill_min(0)
+    kv = synth_model.synth_kv(cfg, 27, 33)
+    gm.init_kv_cache(kv, 33)
+    mf.oracle_init_kv(om, kv)
+    ids = synth.token_ids(28, 5, cfg.vocab_size)
+    got = gm.run_kv(ids)
+    assert gm.recorded_steps() == (0 if graph is False else 1)
+    want = np.concatenate([om.run_kv(ids[i:i + 1]) for i in range(5)])
+    assert max(mf.rel_err(got[i], want[i]) for i in range(5)) < 1e-2
+    assert np.array_equal(gm.generate_greedy(ids[:2], 12), om.generate_greedy(ids[:2], 12)[0])
+    gm.close()
+
+
+def test_a_step_that_cannot_be_recorded(ctx):
+    """By default the launches go out one by one then, now and later, with the same bits and the cause to be read; a model told to record
+    raises instead, with the cache where it was, and has recorded its step once it can."""
+    cfg = synth_model.TINY
+    gm = synth_model.build_model(ctx, cfg, synth_model.synth_weights(cfg, 4244), 96)
+    gm.set_prefill_min(0)
+    ids = synth.token_ids(29, 6, cfg.vocab_size)
+
+    def run():
+        gm.reset_kv_cache()
+        return gm.run_kv(ids)
+
+    gm.inject_recording_failures(1)
+    first = run()
+    assert b"recording the decode step failed" in ctx.lib.hm_last_error(ctx.h)
+    assert np.array_equal(run(), first) and gm.recorded_steps() == 0
+    gm.set_graph(True)
+    gm.inject_recording_failures(1)
+    with pytest.raises(HomuraError, match="recording the decode step failed"):
+        run()
+    assert gm.kv_cache_len() == 0 and gm.recorded_steps() == 0
+    assert np.array_equal(run(), first) and gm.recorded_steps() == 1
+    gm.close()
+
+
 @pytest.mark.parametrize("rows", [61, 126])
 def test_attention_of_one_split_and_across_its_border(ctx, tiny, rows):
     """Up to 128 live rows the attention of a step with one launch per projection is one split without a fold (61: more than one of
