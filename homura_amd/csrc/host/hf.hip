@@ -46,6 +46,12 @@ namespace {
 // of it holds in registers
 constexpr int ATTN_UNSPLIT = 128;
 
+// Live rows from which that attention's grid has splits to fold: its span is min(ATTN_UNSPLIT, max_len) rows up to ATTN_UNSPLIT of them,
+// in chunks of `chunk`, and more than one chunk beyond.
+int fold_from_rows(int chunk, int max_len) {
+    return std::min(ATTN_UNSPLIT, max_len) > chunk ? 0 : ATTN_UNSPLIT + 1;
+}
+
 // HOMURA_WHOLE_STEP_FAR=1 (read when the plan is built): the whole-step kernel takes every exchange through
 // memory, as it does when it does not find its workgroups dealt to the dies round-robin.
 int whole_step_far_only() {
@@ -661,6 +667,7 @@ int HfModel::emit_transformer_plan() {
         att_chunk = std::min(128, std::max(32, std::atoi(e) / 32 * 32));
         att_chunk_fixed = true;
     }
+    const int fold_from = fold_from_rows(att_chunk_fixed ? att_chunk : ATTN_UNSPLIT, max_seq_len_);
 
     std::shared_ptr<PlanScratch> scr = scratch_;
     std::vector<CompiledKernel> kernels;
@@ -833,7 +840,8 @@ int HfModel::emit_transformer_plan() {
             DeviceLaunch a1b;
             a1b.name = "gqa_attn_fold";
             a1b.bytes_fixed = qd * 4.0;
-            a1b.bytes_per_kv_row = (double)(qd + 2 * H) * 4.0 / att_chunk;  // partials: one set per chunk
+            a1b.bytes_per_kv_row = (double)(qd + 2 * H) * 4.0 / att_chunk;  // partials: one set per chunk (beyond 2048 rows of 128: half of this)
+            a1b.from_rows = fold_from;
             a1b.fn = [=](const StepContext &sc) -> int {
                 return gqa_decode_attn_launch(sc.ctx, attn_args(sc, AttnArgs::FOLD_ONLY));
             };
@@ -1080,6 +1088,7 @@ int HfModel::emit_transformer_plan_quant() {
         att_chunk = std::min(128, std::max(32, std::atoi(e) / 32 * 32));
         att_chunk_fixed = true;
     }
+    const int fold_from = fold_from_rows(att_chunk_fixed ? att_chunk : ATTN_UNSPLIT, max_seq_len_);
 
     std::shared_ptr<PlanScratch> scr = scratch_;
     std::vector<CompiledKernel> kernels;
@@ -1446,7 +1455,8 @@ int HfModel::emit_transformer_plan_quant() {
             DeviceLaunch lf;
             lf.name = "gqa_attn_fold";
             lf.bytes_fixed = qd * 4.0;
-            lf.bytes_per_kv_row = (double)(qd + 2 * H) * 4.0 / att_chunk;
+            lf.bytes_per_kv_row = (double)(qd + 2 * H) * 4.0 / att_chunk;  // (beyond 2048 rows half of this)
+            lf.from_rows = fold_from;
             lf.fn = [=](const StepContext &sc) -> int {
                 return gqa_decode_attn_launch(sc.ctx, attn_args(sc, AttnArgs::FOLD_ONLY));
             };

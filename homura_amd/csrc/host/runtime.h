@@ -206,6 +206,7 @@ struct DeviceLaunch {
     // whole step. Entries of the way that is switched off are skipped.
     enum class Mode { Always, PerKernel, WholeStep };
     Mode mode = Mode::Always;
+    int from_rows = 0;                // enqueues nothing in steps of fewer live rows than this (the cache and the new row)
     std::function<int(const StepContext &)> fn;
 };
 struct CompiledKernel {
@@ -285,7 +286,7 @@ class ExecutionPlan {
     // Forget the recorded steps (their launches' arguments or kernels are about to change); the next run records anew.
     int invalidate_graph();
     bool skips(const DeviceLaunch &l) const {
-        return l.mode == (whole_step_ ? DeviceLaunch::Mode::PerKernel : DeviceLaunch::Mode::WholeStep);
+        return l.mode == (whole_step_ ? DeviceLaunch::Mode::PerKernel : DeviceLaunch::Mode::WholeStep) || kv_cache_len() + 1 < l.from_rows;
     }
     // Called before a step is enqueued or captured, with the KV cache in place (device tables that
     // depend on the cache's addresses are refreshed here, outside any capture).

@@ -153,6 +153,22 @@ def test_attention_of_one_split_and_across_its_border(ctx, tiny, rows):
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "q8_0"])
+def test_launches_of_a_step_with_one_split(ctx, fmt):
+    """A step of up to 128 live rows has no fold: it is neither counted nor timed."""
+    cfg, wdt = (synth_model.TINY, DTYPE_BF16) if fmt == "bf16" else (synth_model.TINY_LLAMA, 2)
+    qkn = fmt == "bf16"
+    gm = synth_model.build_model(ctx, cfg, synth_model.synth_weights(cfg, 53, wdt, has_qk_norm=qkn), 160, wdt, has_qk_norm=qkn)
+    count = {}
+    for rows in (127, 128):
+        gm.init_kv_cache(synth_model.synth_kv(cfg, 54, rows), rows)
+        count[rows] = gm.launches_per_step()
+        folds = [r for r in gm.profile_step(5) if r["label"] == "gqa_attn_fold"]
+        assert [r["launches"] for r in folds] == ([cfg.num_hidden_layers] if rows == 128 else [])
+    assert count[128] == count[127] + cfg.num_hidden_layers
+    gm.close()
+
+
 def test_kv_overflow_and_bad_input(ctx, tiny):
     cfg, weights, gm, _om = tiny
     kv = synth_model.synth_kv(cfg, 7, 158)
