@@ -56,7 +56,8 @@ def test_listed_shape_against_oracle(ctx, shape, fmt):
         else:
             assert errs.max() < 1e-2, what
 
-    # decode: five steps from a 70-row cache
+    # decode: five steps from a 70-row cache, launched one by one
+    gm.set_graph(False)
     gm.set_prefill_min(0)
     gm.init_kv_cache(kv, 70)
     mf.oracle_init_kv(om, kv)
@@ -87,7 +88,7 @@ def test_listed_shape_against_oracle(ctx, shape, fmt):
                                        ("smollm2-1.7b", "bf16"), ("qwen2.5-1.5b", "q8_0"), ("tinyllama-1.1b", "q4_0")])
 def test_listed_shape_on_longer_caches(ctx, shape, fmt):
     """One launch per projection on caches of thousands of rows: the attention grid of the recorded step covers
-    the live rows rounded up to a power of two (2048 at least) and is recorded anew when they outgrow it; beyond
+    the live rows rounded up to a power of two (2048 at least), and a step is recorded for each such span; beyond
     2048 rows a split takes 128 rows instead of 64 and the fold of the splits' partial results is shared out
     over groups of threads. Decode steps across both borders (2048, 4096 live rows), eager and replayed from a
     graph, against the oracle."""

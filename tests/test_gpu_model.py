@@ -69,6 +69,7 @@ def test_tiny_graph_replay_matches_eager(ctx, tiny):
     cfg, weights, gm, _om = tiny
     kv = synth_model.synth_kv(cfg, 17, 30)
     ids = synth.token_ids(18, 4, cfg.vocab_size)
+    gm.set_graph(False)
     gm.init_kv_cache(kv, 30)
     eager_tokens = gm.generate_greedy(ids, 24)
     eager_logits = gm.run_kv(ids[:1])
@@ -251,6 +252,7 @@ def test_quantised_plan_against_oracle(ctx, wdt, name):
     gm = synth_model.build_model(ctx, cfg, weights, 96, wdt, has_qk_norm=False)
     om = mf.build_oracle_model(cfg, weights, 96, wdt, has_qk_norm=False)
     kv = synth_model.synth_kv(cfg, 3, 37)
+    gm.set_graph(False)
     gm.init_kv_cache(kv, 37)
     mf.oracle_init_kv(om, kv)
     ids = synth.token_ids(4, 6, cfg.vocab_size)
@@ -372,6 +374,7 @@ def test_qkv_bias_model_against_oracle(ctx, wdt, name):
     om = mf.build_oracle_model(cfg, weights, 96, wdt, has_qk_norm=False)
     assert [s[0] for s in gm.weight_slots()] == [n for n, _ in weights]
     kv = synth_model.synth_kv(cfg, 8, 21)
+    gm.set_graph(False)
     gm.init_kv_cache(kv, 21)
     mf.oracle_init_kv(om, kv)
     ids = synth.token_ids(6, 5, cfg.vocab_size)
@@ -404,6 +407,7 @@ def test_kquant_plan_against_oracle(ctx, which):
     om = mf.build_oracle_model(cfg, weights, 96, has_qk_norm=False, proj_dtypes=mix)
     assert [s[0] for s in gm.weight_slots()] == [n for n, _ in weights]
     kv = synth_model.synth_kv(cfg, 3, 29)
+    gm.set_graph(False)
     gm.init_kv_cache(kv, 29)
     mf.oracle_init_kv(om, kv)
     ids = synth.token_ids(4, 5, cfg.vocab_size)

@@ -167,14 +167,18 @@ def test_quantised_whole_step_against_oracle_and_per_projection_path(ctx, name, 
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "q8_0", "q4_0", "q4_k_m"])
-def test_short_caches_that_no_workgroup_splits(ctx, fmt):
-    """Up to 112 cached rows every workgroup attends over all of them, two to seven rounds of 16 rows in registers: no row at all, a
-    partly filled round, whole rounds, and the steps across the borders to the next instance and to the even cut. Logits against the
-    path of one launch per projection (the same products, attention summed in another order; new K and V elements may round to
-    the neighbouring bf16) and, bf16, against the oracle."""
+@pytest.mark.parametrize("shape", ["small", "qwen3-0.6b"])
+def test_short_caches_that_no_workgroup_splits(ctx, shape, fmt):
+    """Up to 112 cached rows every workgroup attends over all of them, rounds of 16 rows in registers: no row at all, a partly filled
+    round, whole rounds, and the steps across the borders to the next instance and to the even cut. The 0.6B shape has instances
+    of two, three, five and seven rounds, the small ones of two and seven. Logits against the path of one launch per projection (the same
+    products, attention summed in another order; new K and V elements may round to the neighbouring bf16) and, bf16,
+    against the oracle."""
     from homura_amd.runtime import DTYPE_BF16, DTYPE_Q4_0, DTYPE_Q8_0
     wdt = {"bf16": DTYPE_BF16, "q4_0": DTYPE_Q4_0}.get(fmt, DTYPE_Q8_0)
     cfg = synth_model.SMALL_WS if fmt == "bf16" else synth_model.SMALL_WS_Q
+    if shape != "small":
+        cfg = dataclasses.replace(synth_model.QWEN3_0P6B, num_hidden_layers=2, vocab_size=1000, tie_word_embeddings=fmt == "bf16")
     mix = synth_model.q4_k_m_mix(cfg) if fmt == "q4_k_m" else None
     weights = synth_model.synth_weights(cfg, 6161, wdt, has_qk_norm=True, proj_dtypes=mix)
     gm = synth_model.build_model(ctx, cfg, weights, 256, wdt, has_qk_norm=True, proj_dtypes=mix)
@@ -193,13 +197,20 @@ def test_short_caches_that_no_workgroup_splits(ctx, fmt):
             gm.whole_step_status()
         gm.set_whole_step(True)
         errs = [mf.rel_err(a, b) for a, b in zip(*out)]
-        # (Q8_K rounds an activation to eight bits: one that falls the other way moves the row by more)
-        assert (min(errs) < 1e-3 and max(errs) < 0.2) if fmt == "q4_k_m" else max(errs) < 1e-2, f"{rows} rows: {errs}"
+        # Of the logits' scale: a K or V element that rounds the other way has moved it by up to 1e-4, against the oracle and at a softmax
+        # weight near 1 by 4e-4; an activation that Q8_K's eight bits round the other way, one step in ten or so, by up to 6e-3 (1 to 4 % in
+        # the smallest models).
+        off = np.array([np.abs(a - b).max() / np.abs(b).max() for a, b in zip(*out)])
+        assert (np.sum(off < 1e-3) >= 3 and off.max() < 5e-2) if fmt == "q4_k_m" else off.max() < 1e-3, f"{rows} rows: {off}"
+        if shape == "small":
+            assert (min(errs) < 1e-3 and max(errs) < 0.2) if fmt == "q4_k_m" else max(errs) < 1e-2, f"{rows} rows: {errs}"
         if fmt == "bf16":
             mf.oracle_init_kv(om, kv)
             om.kv.reset(rows)
             want = np.concatenate([om.run_kv(ids[i:i + 1]) for i in range(5)])
-            assert max(mf.rel_err(out[0][i], want[i]) for i in range(5)) < 1e-2, f"{rows} rows"
+            assert max(np.abs(out[0][i] - want[i]).max() / np.abs(want[i]).max() for i in range(5)) < 2e-3, f"{rows} rows"
+            if shape == "small":
+                assert max(mf.rel_err(out[0][i], want[i]) for i in range(5)) < 1e-2, f"{rows} rows"
     gm.close()
 
 
