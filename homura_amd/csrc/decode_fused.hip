@@ -1033,9 +1033,9 @@ __device__ __forceinline__ void compute_role(const FusedDecodeArgs &a, Lds<GE> &
 #pragma unroll
             for (int g = 0; g < G; g++) lds_x8(sm.qs[g], dl * 8, qv[g]);
             const bool with_new = sp.owner && cw == 0;  // the new row rides with wavefront 0 of the last split
-            // The rounds held in registers are taken PR at a time, at most four (the float forms of more would not
-            // fit beside the weight slices, and a spilled register is reloaded through the same in-order memory
-            // pipeline the weight requests wait in): one pass up to four rounds, two of three or of four beyond;
+            // The rounds held in registers are taken PR at a time, as many as have their float forms fit beside the weight
+            // slices (a spilled register is reloaded through the same in-order memory pipeline the weight requests wait
+            // in): one pass up to five rounds and of seven (245 registers for bf16), two of three or of four for six and eight;
             // passes after the first rescale what the earlier ones left. A pass costs its reductions and
             // exponentials whatever its width: eight rounds as four passes of two took 0.519 ms a token at 4000 rows,
             // as two of four 0.507. Streamed sets (below) stay two rounds wide, the ring holds three of them. The

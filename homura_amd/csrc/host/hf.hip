@@ -2426,8 +2426,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         qa.eps = eps;
         if ((rc = qkv_post_launch(ctx_, qa)) != HM_OK) return rc;
         // Without logits nobody reads the hidden state behind the last layer: its cache rows are all that a chunk leaves. (512 tokens
-        // of the Qwen3-0.6B shape and the step behind them 3.41 -> 3.33 ms, 6001 and 16 steps 37.5 -> 36.7; what a test captures
-        // wants the rest as well.)
+        // of the Qwen3-0.6B shape and the step behind them 3.41 -> 3.33 ms; what a test captures wants the rest as well.)
         if (l + 1 == c.num_hidden_layers && !h_logits && !p.capture) break;
         // attention kernel (reference src/hf/emitter.rs:683-758): causal attention, then the O projection
         PrefillAttnArgs aa;

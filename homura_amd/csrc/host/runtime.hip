@@ -574,11 +574,11 @@ int ExecutionPlan::run_kv(const std::vector<Buffer *> &inputs, std::vector<Buffe
     if (pre_run_ && (rc = pre_run_()) != HM_OK) return rc;
     // A graph pays when a step is many launches: the host enqueues them at about the rate they run at and never gets ahead of a
     // single step (run_kv with its logits read, us: Qwen2.5-0.5B 820 -> 730, 1.5B 1200 -> 1126, Nokuvik 1024 wide 1540 -> 1340, Ludalix 1250 ->
-    // 1125), and a replayed launch starts sooner behind the last (Qwen2.5-1.5B, step after step, 1086 -> 1060). A step of up to three
+    // 1125; on a machine whose host is quicker 715 -> 705, 1160 -> 1088, 1307 -> 1305, 1155 -> 1076), and a replayed launch starts sooner behind the last (Qwen2.5-1.5B, step after step, 1086 -> 1060). A step of up to three
     // is quicker launched directly (whole-step launch of a Q4_K_M model, head and pick: 64 sampled tokens 30.10 ms replayed, 29.95 ms direct).
-    // Recording and instantiating cost the first step of a span 0.3 to 0.9 ms once (135 to 289 launches; a new model's first step takes 1.0
-    // to 3.9 ms launched directly, so much is loaded then), which 4 to 25 us a step step after step, 10 to 100 with each one's logits read, earn
-    // back in 15 to 150 steps.
+    // Recording and instantiating cost the first step of a span 0.1 to 1.4 ms once, 0.3 to 0.9 mostly (135 to 289 launches; a new model's
+    // first step takes 1.0 to 3.9 ms launched directly, so much is loaded then). The transformers and Ludalix earn that back in some 10 to 50
+    // steps, Nokuvik with a quick host in a few hundred.
     const Recorded *r = nullptr;
     hipStreamCaptureStatus outer = hipStreamCaptureStatusNone;  // somebody else's recording takes the launches themselves
     if (use_graph_ && !record_failed_ && launches_per_step() > 3 && hipStreamIsCapturing(ctx_->stream, &outer) == hipSuccess && outer == hipStreamCaptureStatusNone) {

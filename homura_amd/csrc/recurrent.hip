@@ -170,8 +170,8 @@ __device__ __forceinline__ void store_taps(const RowSource &in, const TapRing &r
 // ENDS: every segment but the last from a zero state (the first one from the chunk's) to its end, states only; left in
 // g.ends, with the segment's sum of steps: the segment multiplies a state by e^(A sum). Then every segment folds the ends
 // ahead of it into the state it starts from and is scanned in full. 2048 tokens, 2048 channels of 16 states: 91 us in one
-// segment, 30 + 18 in eight. (16 states: 128 registers at most, so that the four workgroups a CU gets of eight segments are all
-// resident; with the 129 that the compiler takes by itself a fourth of them came after the rest: 33 + 19.)
+// segment, 32 to 33 + 19.4 in eight. (16 states: 128 registers at most, so that the four workgroups a CU gets of eight segments are
+// all resident; with the 129 that the compiler takes by itself 33.3 to 34.1 + 19.2.)
 struct ScanSegments {
     int rows = 0;                    // of a segment, a multiple of the tile; 0: the chunk is one segment
     float *ends = nullptr;           // [segments][inner][state_pad]: slot 0 the chunk's first state, slot g + 1 the end of segment g

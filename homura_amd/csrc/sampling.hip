@@ -423,12 +423,14 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_token_kernel(SampleArgs
 }
 
 // ── Small top_k (<= 64) over a large vocabulary: two launches instead of one workgroup's eight passes ──
-// Front: a wavefront per group of 64 to 256 tokens applies penalties and temperature and writes the group's maximum,
-// the sum of its exponentials relative to it and its first four tokens by (logit descending, token ascending): one
-// trip to memory and ten reductions, no LDS. Back: one workgroup combines maxima and sums (sum over the vocabulary =
+// Front: a wavefront per group of 64 tokens or more (the least power of two with at most 1024 groups) applies penalties
+// and temperature and writes the group's maximum, the sum of its exponentials relative to it and its first four tokens by
+// (logit descending, token ascending): one trip to memory and ten reductions, no LDS. (Groups of more than 256 tokens, which
+// vocabularies beyond 262144 have, do not stay in registers and are read again for each of these.) Back: one workgroup combines maxima and sums (sum over the vocabulary =
 // sum_g sum_g * exp(max_g - max), equal to the single pass's up to rounding). The K-th largest of the groups' first
 // keys is a floor for the K-th largest of the vocabulary (K tokens reach it), so the top K are among the kept tokens
-// that reach it, a hundred or so, unless all four of a group do: then the groups that reach the floor are read again.
+// that reach it, a hundred or so, unless all four of a group do: then the groups that reach the floor are read again, up to
+// 128 of them, and the first K by (key descending, group ascending) of more.
 // It selects by logit, which orders tokens like their exponentials except where two different logits round to one
 // exponential.
 // What bounds the pair is latency: a launch, one trip to memory and the barriers between the steps of a single
@@ -763,7 +765,8 @@ int sample_check_config(hm_ctx *ctx, const hm_sampling_config *cfg, bool device)
 }
 
 // One workgroup for everything, or the front / back pair when top_k is small and the vocabulary large (the pair
-// keeps its three words per group of 64 tokens or more in `work`, which has a word per token).
+// keeps ten words per group in `work`, which has a word per token: a group has 64 tokens or more, but for the last one).
+static_assert((2 * FRONT_KEEP + 2) * 2 <= 1 << FRONT_GROUP_BITS, "front_out fits a word per token, the last group's too");
 static int sample_enqueue(hm_ctx *ctx, const SampleArgs &a) {
     const bool pair = a.cfg.temperature > 0.0f && a.cfg.top_k >= 1 && a.cfg.top_k <= FRONT_MAX_K && a.vocab >= 4096;
     if (pair) {

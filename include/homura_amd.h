@@ -371,7 +371,7 @@ int hm_model_kv_cache_len(hm_model *m);    /* src/runtime.rs:1948-1950 */
 
 /* Replay every decode step from a captured HIP graph (on != 0, the default) or launch kernel by kernel. A step of
  * up to three launches (the whole-step kernel) is launched directly either way: that is quicker than replaying
- * so small a graph. Recording costs the first step 0.3 to 0.9 ms, and again the first one that passes 128, 2048, 4096 ... cached rows;
+ * so small a graph. Recording costs the first step 0.1 to 1.4 ms, and again the first one that passes 128, 2048, 4096 ... cached rows;
  * what is recorded is kept. Where a recording fails, a model that this call was made for with on != 0 returns the error from the step; one
  * left at the default launches kernel by kernel from then on, with the cause in hm_last_error, until this call or hm_model_set_whole_step
  * has it try again. No counterpart in the reference (its plan is a host loop over dlsym'ed functions). */
@@ -385,7 +385,7 @@ int hm_model_inject_recording_failures(hm_model *m, int n);
  * (src/hf/emitter.rs:1016-1021). Served for bf16, all-Q8_0, all-Q4_0 and Q4_K / Q6_K (in any mix per
  * projection) models whose shape has a kernel instance (hm_model_whole_step_available); on by default then, and for bf16 models the same launch runs the
  * LM head and the greedy pick. The cache may be of any length: a step takes the instance of the kernel that
- * holds its live rows (1536, 2048, 3072, 4096 or 32768 of them; the smaller the faster; the last streams the rows beyond
+ * holds its live rows (33, 49, 81, 113, 1536, 2048, 3072, 4096 or 32768 of them; the smaller the faster; the last streams the rows beyond
  * 4096 inside its attention phase), beyond 32768 the per-projection path, chosen step by step. Results agree with the per-projection
  * path to f32 summation order.
  *
