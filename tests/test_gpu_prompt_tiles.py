@@ -117,11 +117,12 @@ def test_prompt_rows_ahead_of_an_infinite_value(ctx, monkeypatch, groups, H, kvh
 
 
 @pytest.mark.parametrize("M,K,N", [(1, 32, 8), (7, 96, 200), (24, 1024, 6144), (31, 160, 4097), (32, 896, 33), (33, 32, 64), (37, 4864, 896),
-                                   (64, 1056, 1001), (64, 1536, 17920), (64, 2080, 6150), (24, 96, 17920), (31, 96, 31501)])
+                                   (64, 1056, 1001), (64, 1536, 17920), (64, 2080, 6150), (24, 96, 17920), (31, 96, 31501),
+                                   (8, 2080, 200), (9, 1056, 97), (16, 544, 6150), (17, 1056, 1001), (25, 2080, 97), (48, 1056, 6150), (49, 544, 200)])
 @pytest.mark.parametrize("form", ["f32", "bf16", "q8_0", "q4_0"])
 def test_products_of_few_rows(ctx, oracle, form, M, K, N):
     """Row tiles of 32 and 64, one and two tiles of B, half a group of 64 k at the end, columns that end inside a vector, one
-    round of workgroups and two, the last one full or not.
+    round of workgroups and two, the last one full or not, rows on both sides of where a load of A more is made.
     Bound as above; the block formats' scales are one rounding more a block."""
     if form != "f32" and form != "bf16" and K % 64:
         K = (K + 63) // 64 * 64
