@@ -429,8 +429,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_token_kernel(SampleArgs
 // vocabularies beyond 262144 have, do not stay in registers and are read again for each of these.) Back: one workgroup combines maxima and sums (sum over the vocabulary =
 // sum_g sum_g * exp(max_g - max), equal to the single pass's up to rounding). The K-th largest of the groups' first
 // keys is a floor for the K-th largest of the vocabulary (K tokens reach it), so the top K are among the kept tokens
-// that reach it, a hundred or so, unless all four of a group do: then the groups that reach the floor are read again, up to
-// 128 of them, and the first K by (key descending, group ascending) of more.
+// that reach it, a hundred or so, unless all four of a group do: then such groups are read again.
 // It selects by logit, which orders tokens like their exponentials except where two different logits round to one
 // exponential.
 // What bounds the pair is latency: a launch, one trip to memory and the barriers between the steps of a single
@@ -438,11 +437,13 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_token_kernel(SampleArgs
 // here are rolled, and what is rare lies behind a branch. 151936 tokens, top_k 50, behind a whole-step decode kernel:
 // front 4.7 us, back 5.6 (the 64 first of every 1024 tokens by a radix select in a workgroup each, and all of those
 // looked through by the back: 6.6 and 11.7; the listed groups always read again, instead of kept tokens: 4.6 and 10.4).
+// Rows that are no model's, 151936 tokens, top_k 50, a call from the host, us (a peaked row takes 29.5): all but ten tokens masked 29, equal
+// logits 37, the first 30 % well above the rest 43. With every group that reaches the floor, or the first 50 of them, read again and
+// no floor above zero probabilities: 107, 111 and 85; with the 64 first of every 1024 tokens: 73, 78 and 55.
 constexpr int FRONT_THREADS = 256;
 constexpr int FRONT_MAX_K = WAVE;                 // largest top_k
 constexpr int FRONT_GROUP_BITS = 6;               // tokens of a group: the least power of two from 64 with at most 1024 groups
 constexpr int FRONT_UNITS = SAMPLE_THREADS / 4;   // the floor is taken over at most so many maxima
-constexpr int FRONT_LIST = 128;                   // groups that the back reads without picking K of them first
 
 // larger float <-> larger key (-inf the smallest key of all finite and infinite values)
 __device__ __forceinline__ unsigned order_key(float x) {
@@ -549,7 +550,7 @@ __global__ __launch_bounds__(FRONT_THREADS) void sample_front_kernel(SampleArgs 
 
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_back_kernel(SampleArgs a, int groups, int group_bits) {
     __shared__ SelectShared sh;
-    __shared__ unsigned group_key[SAMPLE_THREADS], floor_key, listed, survived, more;
+    __shared__ unsigned floor_key, listed, survived[2], more;
     __shared__ alignas(16) unsigned unit_key[FRONT_UNITS];
     __shared__ float red_sum[SAMPLE_THREADS / WAVE];
     __shared__ int list[SAMPLE_THREADS];
@@ -573,11 +574,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_back_kernel(SampleArgs 
     const int units = fours ? (groups + 3) / 4 : groups;
     unsigned four = max(key, dpp_keys<0xB1, 0xF>(key));
     four = max(four, dpp_keys<0x4E, 0xF>(four));
-    group_key[tid] = key;
     if (fours ? (tid & 3) == 0 : tid < FRONT_UNITS) unit_key[fours ? tid / 4 : tid] = fours ? four : key;
     if (tid == 0) {
         floor_key = 0xFFFFFFFFu;
-        listed = survived = more = 0;
+        listed = survived[0] = survived[1] = more = 0;
     }
     float m = wave_max(gm);
     if (lane == 0) sh.red_f[wave] = m;
@@ -606,43 +606,102 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_back_kernel(SampleArgs 
     sum = 0.f;
 #pragma unroll
     for (int w = 0; w < SAMPLE_THREADS / WAVE; w++) sum += red_sum[w];
-    const unsigned floor = floor_key;
+    // What lies 104 below the maximum has the probability 0, of which nothing below depends: a vocabulary masked down to fewer than K
+    // tokens keeps those. (fmaxf leaves no NaN in m; behind an infinite m the floor stays.)
+    unsigned floor = m < INFINITY ? max(floor_key, order_key(m - 104.0f)) : floor_key;
     auto weight = [&](unsigned k) {
         const float x = key_value(k);
         return x > -INFINITY ? expf(x - m) : 0.f;
     };
+    int round = 0;  // 1: with groups read again
     auto survive = [&](unsigned k, int token) {
-        const unsigned at = atomicAdd(&survived, 1u);
+        const unsigned at = atomicAdd(&survived[round], 1u);
         if (at < (unsigned)SAMPLE_MAX_K) fcomp[at] = ((unsigned long long)k << 32) | (unsigned)(0x7FFFFFFF - token);
     };
     bool in = tid < groups && key >= floor;
-    if (in) {
+    auto keep = [&](unsigned k0, unsigned k1, unsigned k2, unsigned k3, unsigned i0, unsigned i1, unsigned i2, unsigned i3) {
 #pragma unroll 1
-        for (int u = 0; u < FRONT_KEEP && kept_key[0] >= floor; u++) {
-            survive(kept_key[0], (int)kept_token[0]);
-            kept_key = u32x4{kept_key[1], kept_key[2], kept_key[3], 0u};
-            kept_token = u32x4{kept_token[1], kept_token[2], kept_token[3], 0u};
-            if (u == FRONT_KEEP - 1) more = 1;
+        for (int u = 0; u < FRONT_KEEP && k0 >= floor; u++) {
+            survive(k0, (int)i0);
+            k0 = k1, k1 = k2, k2 = k3, k3 = 0u;
+            i0 = i1, i1 = i2, i2 = i3, i3 = 0u;
         }
+    };
+    if (in) {
+        keep(kept_key[0], kept_key[1], kept_key[2], kept_key[3], kept_token[0], kept_token[1], kept_token[2], kept_token[3]);
+        if (kept_key[3] >= floor) more = 1;
     }
+    // survivors ahead of `mine`, one of n, for which 1 << bits threads count
+    auto survivors_ahead = [&](unsigned long long mine, int n, int bits) {
+        unsigned rank = 0;
+#pragma unroll 4
+        for (int c = tid & ((1 << bits) - 1); c < n; c += 1 << bits) rank += fcomp[c] > mine ? 1u : 0u;
+        if (bits > 0) rank += dpp_keys<0xB1, 0xF>(rank);
+        if (bits > 1) rank += dpp_keys<0x4E, 0xF>(rank);
+        if (bits > 2) rank += dpp_keys<0x141, 0xF>(rank);
+        return rank;
+    };
+    auto threads_for = [](int n) { return n <= SAMPLE_THREADS / 8 ? 3 : n <= SAMPLE_THREADS / 4 ? 2 : n <= SAMPLE_THREADS / 2 ? 1 : 0; };
     __syncthreads();
-    if (more || survived > (unsigned)SAMPLE_MAX_K) {
-        // A group may have more than it kept, or the list takes no more: the tokens of the groups that reach the floor, read again. With more of
-        // those than the list takes (equal keys all over the vocabulary) the first K groups by (key descending, group
-        // ascending), which hold K tokens that come ahead of every other group's.
-        if (in) list[atomicAdd(&listed, 1u)] = tid;
-        __syncthreads();
-        if (tid == 0) survived = 0;
-        int n_list = (int)listed;
-        __syncthreads();
-        if (n_list > FRONT_LIST) {
-            unsigned ahead = 0;
-            for (int c = 0; c < groups; c++) ahead += (group_key[c] > key) | ((group_key[c] == key) & (c < tid)) ? 1u : 0u;
-            in = in && ahead < K;
-            if (in) list[ahead] = tid;
-            n_list = (int)min((unsigned)n_list, K);
+    if (more || survived[0] > (unsigned)SAMPLE_MAX_K) {
+        // A group may have more than it kept, or the list takes no more: only groups all of whose kept tokens reach the floor are read again.
+        // Of more than SAMPLE_THREADS / 8 survivors the K-th is a better floor to begin with (fewer have 32 such groups at most, which is one
+        // trip to memory). Of the groups that end at the floor itself (equal keys all over the vocabulary) the first in token order are
+        // taken that, with one token of each group above the floor, surely hold K tokens ahead of all others': as many of a group as it kept,
+        // then, of these groups, as many as it has.
+        const int had = (int)survived[0];
+        round = 1;
+        if (had > SAMPLE_THREADS / 8 && had <= SAMPLE_THREADS / 2) {
+            const int bits = threads_for(had);
+            const unsigned long long mine = fcomp[min(tid >> bits, had - 1)];
+            if (survivors_ahead(mine, had, bits) == K - 1) floor_key = (unsigned)(mine >> 32);
             __syncthreads();
+            floor = max(floor, floor_key);
+        } else if (had > SAMPLE_THREADS / 2 && had <= SAMPLE_MAX_K) {  // (counting as above is had compares a thread: 1000 of them 25 us, this 11)
+            const unsigned mine = tid < had ? (unsigned)(fcomp[tid] >> 32) : 0u;
+            const int bits = 32 - __clz((int)(floor ^ order_key(m)));  // below the ones that all keys from the floor to the maximum share
+            unsigned kth = bits < 32 ? floor >> bits << bits : 0u;
+            for (int bit = bits - 1; bit >= 0; bit--)
+                if (__syncthreads_count(mine >= (kth | 1u << bit)) >= (int)K) kth |= 1u << bit;
+            floor = max(floor, kth);
         }
+        in = in && key >= floor;
+        bool full = in && kept_key[3] >= floor, at_floor = in && key == floor;
+        if (full) list[atomicAdd(&listed, 1u)] = tid;
+        auto first_groups = [&](unsigned has) {  // drops groups at the floor
+            const unsigned mine = at_floor ? has : in ? 1u << 20 : 0u;
+            unsigned before = mine;
+            for (int off = 1; off < WAVE; off <<= 1) {
+                const unsigned up = __shfl_up(before, off, WAVE);
+                if (lane >= off) before += up;
+            }
+            if (lane == WAVE - 1) sh.red_i[wave] = (int)before;
+            __syncthreads();
+            before -= mine;
+            unsigned above = 0;
+            for (int w = 0; w < SAMPLE_THREADS / WAVE; w++) {
+                if (w < wave) before += (unsigned)sh.red_i[w];
+                above += (unsigned)sh.red_i[w] >> 20;
+            }
+            at_floor = at_floor && above + (before & 0xFFFFFu) < K;
+            in = in && (at_floor || key > floor);
+            full = full && in;
+            __syncthreads();
+        };
+        auto enlist = [&](bool mine) {  // lists groups in order; how many
+            const unsigned long long mask = __ballot(mine);
+            if (lane == 0) sh.red_i[wave] = __popcll(mask);
+            __syncthreads();
+            int at = __popcll(mask & ((1ull << lane) - 1ull)), all = 0;
+            for (int w = 0; w < SAMPLE_THREADS / WAVE; w++) {
+                if (w < wave) at += sh.red_i[w];
+                all += sh.red_i[w];
+            }
+            if (mine) list[at] = tid;
+            fcomp[tid] = 0;
+            __syncthreads();
+            return all;
+        };
         auto token_at = [&](int j) { return (list[j >> group_bits] << group_bits) + (j & ((1 << group_bits) - 1)); };
         auto logit_at = [&](int j) {
             const int i = min(token_at(j), a.vocab - 1);
@@ -651,40 +710,41 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_back_kernel(SampleArgs 
         // (tokens past the vocabulary come last: the smallest key, the largest number)
         auto key_of = [&](int j, LogitAndCount v) { return token_at(j) < a.vocab ? order_key(penalised(v.l, v.c, a.cfg) * inv_temp) : 0u; };
         auto idx_at = [&](int j) { return token_at(j) < a.vocab ? token_at(j) : 0x7FFFFFFF; };
-        const int n = n_list << group_bits;
-        sweep(n, tid, logit_at, [&](int j, LogitAndCount v) {
+        const int n_floor = __syncthreads_count(at_floor);
+        int n_list = (int)listed;
+        if (n_floor > 1) {
+            const unsigned reach = 1u + (kept_key[1] >= floor) + (kept_key[2] >= floor) + (kept_key[3] >= floor);
+            first_groups(reach);
+            n_list = enlist(full);
+            sweep(n_list << group_bits, tid, logit_at, [&](int j, LogitAndCount v) {  // (a wavefront's tokens are of one group)
+                const unsigned long long has = __ballot(key_of(j, v) >= floor);
+                if (lane == 0) atomicAdd(&fcomp[list[j >> group_bits]], (unsigned long long)__popcll(has));
+            });
+            __syncthreads();
+            first_groups(full ? (unsigned)min(fcomp[tid], (unsigned long long)K) : reach);
+            n_list = enlist(full);
+        }
+        if (in && !full) keep(kept_key[0], kept_key[1], kept_key[2], kept_key[3], kept_token[0], kept_token[1], kept_token[2], kept_token[3]);
+        sweep(n_list << group_bits, tid, logit_at, [&](int j, LogitAndCount v) {
             const unsigned k = key_of(j, v);
             if (k >= floor) survive(k, idx_at(j));
         });
         __syncthreads();
-        if (survived > (unsigned)SAMPLE_MAX_K) {  // a flat distribution: the general selection, which wants its items in token order
-            const unsigned long long mask = __ballot(in);
-            if (lane == 0) sh.red_i[wave] = __popcll(mask);
-            __syncthreads();
-            int at = __popcll(mask & ((1ull << lane) - 1ull));
-            for (int w = 0; w < wave; w++) at += sh.red_i[w];
-            if (in) list[at] = tid;
-            __syncthreads();
+        if (survived[1] > (unsigned)SAMPLE_MAX_K) {  // a flat distribution: the general selection, which wants its items in token order
+            const int n = enlist(in) << group_bits;
             select_sort_draw(sh, a, st, n, a.vocab, sum, [&](int j) { return key_of(j, logit_at(j)); }, idx_at, weight);
             return;
         }
     }
     // Selection by rank: every survivor counts the survivors ahead of it, and the first K take their rank as their
     // place.
-    const int nf = (int)survived;
+    const int nf = (int)survived[round];
     float (&cand_p)[SAMPLE_MAX_K] = sh.cand_p;
     int (&cand_i)[SAMPLE_MAX_K] = sh.cand_i;
     {
-        const int bits = nf <= SAMPLE_THREADS / 8 ? 3 : 0, s = tid >> bits;  // eight threads count for one survivor, or one
+        const int bits = threads_for(nf), s = tid >> bits;
         const unsigned long long mine = fcomp[min(s, nf - 1)];
-        unsigned rank = 0;
-#pragma unroll 4
-        for (int c = tid & ((1 << bits) - 1); c < nf; c += 1 << bits) rank += fcomp[c] > mine ? 1u : 0u;
-        if (bits) {
-            rank += dpp_keys<0xB1, 0xF>(rank);
-            rank += dpp_keys<0x4E, 0xF>(rank);
-            rank += dpp_keys<0x141, 0xF>(rank);
-        }
+        const unsigned rank = survivors_ahead(mine, nf, bits);
         if (s < nf && rank < K) {  // normalise, min_p (the maximum probability is exp(0) / sum)
             float p = weight((unsigned)(mine >> 32)) / sum;
             if (a.cfg.min_p > 0.0f && p < a.cfg.min_p * (1.0f / sum)) p = 0.0f;

@@ -127,6 +127,34 @@ def test_two_launch_sampler_of_every_group_size(ctx, vocab, top_k):
     assert compared >= 16
 
 
+@pytest.mark.parametrize("top_k", [1, 50, 64])
+@pytest.mark.parametrize("vocab", [4096, 16385, 65537, 262145])
+def test_two_launch_sampler_of_masked_and_flat_rows(ctx, vocab, top_k):
+    """Rows that a mask leaves fewer than top_k tokens of (-inf, and finite values whose probability is 0), one of which shares its
+    group with a dozen others; equal logits everywhere; a few tokens, some in one group, above a plateau that ends at the floor."""
+    gen = np.random.default_rng(vocab + top_k)
+    cfg = Cfg(temperature=0.7, top_k=top_k, top_p=0.9, repetition_penalty=1.1)
+    some = np.concatenate([gen.integers(0, vocab, 9), np.arange(70, 83)])
+    rows = {"-inf": np.full(vocab, -np.inf, np.float32), "-1e9": np.full(vocab, -1e9, np.float32), "equal": np.full(vocab, 0.5, np.float32),
+            "plateau": np.where(gen.random(vocab) < 0.3, 1.0, 0.0).astype(np.float32)}
+    for name in ("-inf", "-1e9"):
+        rows[name][some] = gen.standard_normal(len(some)) * 2
+    rows["plateau"][some] = 1.5 + 0.01 * np.arange(len(some))
+    rows["plateau"][vocab - 1] = 1.0
+    compared = 0
+    for name, logits in rows.items():
+        d = ctx.to_device(logits)
+        a, b = pyoracle.Rng(80), runtime.Rng(80)
+        for _ in range(8):
+            want, margins = pyoracle.sample_token(logits, cfg, [5, 70, 71], a, want_margins=True)
+            got = ctx.sample_token(d, vocab, lib_cfg(cfg), [5, 70, 71], b)
+            if not on_edge(margins, cfg):
+                assert got == want, (vocab, top_k, name)
+                compared += 1
+        d.free()
+    assert compared >= 24
+
+
 def test_device_sampler_reference_cases_and_errors(ctx):
     # sample_token_greedy and min_p_filters_low_prob (src/generate.rs:891-900, :990-1008)
     d = ctx.to_device(np.array([0.0, 1.0, 0.5, 0.2], np.float32))
