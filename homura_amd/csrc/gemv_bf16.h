@@ -27,7 +27,7 @@ struct GemvConv {
 };
 
 // Prologue of a matrix memory's output projection (matrix_memory.h): the row is what the memory's heads put out, every head over its
-// normaliser and its root mean square, weighted and gated. K == heads * vdim <= 4096, vdim 64, 128, 256 or 512, so that a head's columns
+// normaliser and its root mean square, weighted and gated. K == heads * vdim, vdim 64, 128, 256 or 512, so that a head's columns
 // belong to one wavefront.
 struct GemvHeads {
     const float *raw = nullptr;          // [heads][cols], the normaliser's product in column vdim
@@ -37,8 +37,11 @@ struct GemvHeads {
     int heads = 0, vdim = 0, cols = 0;
     float eps = 0.f;
 };
-inline bool gemv_takes_heads(int heads, int vdim, int K) {
-    return heads > 0 && (vdim == 64 || vdim == 128 || vdim == 256 || vdim == 512) && heads * vdim == K && K <= 4096;
+// Every workgroup of four outputs does the heads' arithmetic for itself, so long rows and many outputs want them from a launch of their own: us a
+// layer that launch costs more (less), 1024 -> 1024 0.85, 2048 -> 2048 0.55, 2048 -> 4096 0.33, 1024 -> 4096 0.2, 256 -> 4096 0.55; 512 -> 6144
+// (0.2), 256 -> 8192 (1.8), 2560 -> 2560 (0.8), 4096 -> 2048 (0.1), 4096 -> 4096 (1.2), 4096 -> 8192 (3.1).
+inline bool gemv_takes_heads(int heads, int vdim, int N, int K) {
+    return heads > 0 && (vdim == 64 || vdim == 128 || vdim == 256 || vdim == 512) && heads * vdim == K && K <= 2048 && N <= 4096;
 }
 
 struct GemvArgs {

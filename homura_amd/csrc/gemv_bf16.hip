@@ -619,7 +619,7 @@ template <int R, int NC>
 int launch_splitk(hm_ctx *ctx, const GemvArgs &a, int epi, bool pro) {
     const int grid = (a.N + R - 1) / R;
     if (a.heads.raw) {
-        if constexpr (NC <= 2 && R <= 4)
+        if constexpr (NC == 1 && R == 4)
             hipLaunchKernelGGL((gemv_bf16_nk_splitk_kernel<R, NC, 3>), dim3(grid), dim3(GEMV_THREADS), 0, ctx->stream, a, epi);
     } else if (pro) {
         if constexpr (NC <= 4 && R >= 4) {
@@ -726,10 +726,10 @@ int gemv_bf16_nk_launch(hm_ctx *ctx, GemvArgs a, int M, int epi) {
         HM_REQUIRE(ctx, M == 1 && !a.w_f32 && epi != GEMV_EPI_ARGMAX && a.K <= ((a.norm_w || a.prologue_residual || a.resid_out) ? 8192 : 16384),
                    "gemv: post-norm, padded norm, other activations and convolution take one bf16 row of at most 8192 (without a prologue 16384) elements");
         const GemvHeads &m = a.heads;
-        HM_REQUIRE(ctx, !m.raw || (gemv_takes_heads(m.heads, m.vdim, a.K) && m.cols > m.vdim && m.cols % 4 == 0 && m.gate && m.norm && m.tops && m.state &&
+        HM_REQUIRE(ctx, !m.raw || (gemv_takes_heads(m.heads, m.vdim, a.N, a.K) && m.cols > m.vdim && m.cols % 4 == 0 && m.gate && m.norm && m.tops && m.state &&
                                    !a.norm_w && !a.prologue_residual && !a.resid_out && !a.post_norm_w &&
                                    (((uintptr_t)m.raw | (uintptr_t)m.gate | (uintptr_t)m.norm) % 16) == 0),
-                   "gemv: a matrix memory's heads of 64, 128, 256 or 512 columns fill a row of at most 4096");
+                   "gemv: a matrix memory's heads of 64, 128, 256 or 512 columns fill a row of at most 2048, for 4096 outputs or fewer");
         HM_REQUIRE(ctx, !a.post_norm_w || a.prologue_residual, "gemv: a post-norm needs the row it normalises");
         if (epi == GEMV_EPI_CONV)
             HM_REQUIRE(ctx, a.conv.rows > 0 && a.conv.rows <= a.N && a.conv.taps > 0 && a.conv.w && a.conv.b && a.conv.ring && a.conv.state,

@@ -992,7 +992,7 @@ int BlockModel::emit_plan() {
             step("Memory", "memory_step", 8.0 * shape.memory_floats() + 4.0 * d.mm_n, 0, {s_d1}, {s_d2},
                  [=](const StepContext &sc) -> int { return matrix_memory_step_launch(sc.ctx, args(sc)); });
             out_w = &l.mm_o;
-            if (gemv_takes_heads(shape.heads, shape.vdim, l.mm_o.kp)) {
+            if (gemv_takes_heads(shape.heads, shape.vdim, l.mm_o.np, l.mm_o.kp)) {
                 out_in = s_d2;
                 out_also = s_d1;
                 out_args = [=](const StepContext &sc, GemvArgs &g) {

@@ -103,11 +103,17 @@ def test_one_mechanism(ctx, name, dtype):
     check(ctx, cfg, 45, dtype, seed=20, prefill_min=0)
 
 
-# heads that the output projection takes as they come: of 8 to 64 lanes, fewer than a wavefront's, a row of one and of two chunks, the
-# longest; and the next beyond each limit
-@pytest.mark.parametrize("heads,vdim", [(1, 64), (9, 64), (3, 128), (4, 256), (9, 256), (1, 512), (8, 512), (9, 512), (3, 32), (2, 96), (1, 1024)])
+# heads that the output projection takes as they come: of 8 to 64 lanes, fewer than a wavefront's, the longest row; and the next beyond
+# each limit
+@pytest.mark.parametrize("heads,vdim", [(1, 64), (9, 64), (3, 128), (4, 256), (8, 256), (9, 256), (1, 512), (4, 512), (5, 512), (8, 512), (9, 512),
+                                        (3, 32), (2, 96), (1, 1024)])
 def test_memory_heads_in_the_output_projection(ctx, heads, vdim):
     check(ctx, lf.config([lf.memory(heads=heads, dim=24, vdim=vdim), lf.memory(heads=heads, dim=24, vdim=vdim)]), 24, "f32", prefill_min=0)
+
+
+@pytest.mark.parametrize("width", [4096, 4160])  # the most outputs that take the heads as they come, and the next
+def test_memory_heads_of_a_wide_model(ctx, width):
+    check(ctx, lf.config([lf.memory(heads=3, dim=24, vdim=64)], width=width), 8, "f32", prefill_min=0)
 
 
 # rows that end inside a wavefront, at one, and at a workgroup's last
