@@ -607,8 +607,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_back_kernel(SampleArgs 
 #pragma unroll
     for (int w = 0; w < SAMPLE_THREADS / WAVE; w++) sum += red_sum[w];
     // What lies 104 below the maximum has the probability 0, of which nothing below depends: a vocabulary masked down to fewer than K
-    // tokens keeps those. (fmaxf leaves no NaN in m; behind an infinite m the floor stays.)
-    unsigned floor = m < INFINITY ? max(floor_key, order_key(m - 104.0f)) : floor_key;
+    // tokens keeps those. (fmaxf leaves no NaN in m; behind an infinite m, or a min_p that leaves no token a probability, the floor stays.)
+    unsigned floor = m < INFINITY && a.cfg.min_p <= 1.0f ? max(floor_key, order_key(m - 104.0f)) : floor_key;
     auto weight = [&](unsigned k) {
         const float x = key_value(k);
         return x > -INFINITY ? expf(x - m) : 0.f;

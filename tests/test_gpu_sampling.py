@@ -151,6 +151,9 @@ def test_two_launch_sampler_of_masked_and_flat_rows(ctx, vocab, top_k):
             if not on_edge(margins, cfg):
                 assert got == want, (vocab, top_k, name)
                 compared += 1
+        if name == "-inf" and top_k > len(some):  # a min_p that leaves no probability: the first token, masked or not
+            none = Cfg(temperature=0.7, top_k=top_k, top_p=0.9, min_p=1.5, repetition_penalty=1.0)
+            assert ctx.sample_token(d, vocab, lib_cfg(none), [], b) == pyoracle.sample_token(logits, none, [], a) == 0
         d.free()
     assert compared >= 24
 
