@@ -63,13 +63,19 @@ int gemm_pieces_scaled_nk(hm_ctx *ctx, const uint16_t *d_a_split, const uint16_t
 // The same products with f16 operands (half_weights.h): two f16 pieces per activation, B [N][K] f16, column n of the result times
 // unscale[n]; block-scaled integers (d_scales) carry their factors in the scales, unscale is NULL then, and npad >= half_scale_cols(N). K % 64 == 0.
 // (gemm_half_wide: its widest tiles, gemm_pieces_mfma.hip; stages of 32 k)
+// gated (gate_scale with it): neighbouring columns are (gate, up) pairs, and silu(gate) up times gate_scale [N / 2] leaves as two f16
+// pieces, gated [M][2 (N / 2)], instead of d_c: one slice, N % 2 == 0. gemm_half_gated_pays: whether that is the quicker way, or slices and
+// silu_mul_half_launch behind them.
 struct HalfProduct {
     const float *unscale;
+    const float *gate_scale = nullptr;
+    uint16_t *gated = nullptr;
 };
+bool gemm_half_gated_pays(bool scaled, int M, int K, int N, int cus, int max_parts);
 int gemm_half_nk(hm_ctx *ctx, const uint16_t *d_a_half, const uint16_t *d_b_half, const HalfProduct &half, const float *d_scales,
                  int npad, float *d_c, int M, int K, int N, int max_parts = 1, int *parts = nullptr);
 inline int half_scale_cols(int N) { return (N + 191) / 192 * 192 > (N + 127) / 128 * 128 ? (N + 191) / 192 * 192 : (N + 127) / 128 * 128; }
-int gemm_half_wide(hm_ctx *ctx, const uint16_t *d_a_half, const uint16_t *d_b_half, const float *d_unscale, float *d_c, int M, int K, int N,
+int gemm_half_wide(hm_ctx *ctx, const uint16_t *d_a_half, const uint16_t *d_b_half, const HalfProduct &half, float *d_c, int M, int K, int N,
                    int slices, int stages_per_split);
 // One bf16 piece by the same kernel (its operands checked by the caller: 16-byte aligned, K % 64 == 0)
 // gemm_tiles_square: its choice is one slice of 128 x 128 tiles, which gemm_dma_kernel (gemm_bf16_mfma.hip) multiplies faster

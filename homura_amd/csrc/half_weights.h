@@ -8,7 +8,10 @@
 // input: a bound on |x| is known where the weights are, and x 2^e stays below 2^15.
 //   a norm's output       |x_k| <= sqrt(dim) |w_k|                      one e per column, folded into the norm's weights
 //   attention's output    a mean of value rows, |v_j| <= sqrt(dim) |W_v[j] o w|_2 + |b_j| (Cauchy-Schwarz)   one e per value column
-//   SiLU(gate) up         no useful bound ahead                         one e per row, from the row's maximum
+//   SiLU(gate) up         |g_j u_j| <= dim |W_g[j] o w|_2 |W_u[j] o w|_2   one e per column, so that the gate|up product can write the
+//                         rows itself. Rows of normal values lie 2^10 to 2^11 below that (2^-28 of themselves is lost, f32's own rounding
+//                         2^-24). A row whose gates all lie far below zero is
+//                         off by no more than that. Where a column's factor would cost the down weights bits: one e per row, from its maximum
 // What is multiplied into a column of the activations is divided out of that column of the weights, so a product needs one
 // factor per output row of the weights, 2^-r, which also puts the row's largest weight at 2^14 .. 2^15. All factors are powers
 // of two. A matrix takes this way only if every one of its weights is then an f16 exactly (bf16 weights: 31 binades of a row,
@@ -28,6 +31,11 @@ int half_norm_scales(hm_ctx *ctx, const float *d_w, int dim, float *d_w_scaled, 
 // (or NULL). d_scale [N] = 2^e, and d_exps [H * hd]: the exponents by column of the attention's output, row n = (KV head, dim).
 int half_value_scales(hm_ctx *ctx, int hm_dtype, const void *d_wv, const float *d_norm_w, const float *d_bias, int N, int K, int H,
                       int hd, float *d_scale, int *d_exps, int *d_flag);
+
+// The gated rows' exponents: rows_bound [2 inter] = sqrt(dim) |W[n] o w|_2 of the gate (even) and up (odd) rows, row n of the matrix in
+// place n * mult + off; then scale [inter] = 2^e and the exponents e by column.
+int half_row_bounds(hm_ctx *ctx, int hm_dtype, const void *d_w, const float *d_norm_w, int N, int K, float *d_bounds, int mult, int off);
+int half_gated_scales(hm_ctx *ctx, const float *d_bounds, int inter, float *d_scale, int *d_exps, int *d_flag);
 
 // bf16 rows [N][K] -> f16(w 2^(r - e)) and unscale[n] = 2^-r. d_exps [K] or NULL (all 0).
 int half_rows(hm_ctx *ctx, const uint16_t *d_w, const int *d_exps, int N, int K, uint16_t *d_out, float *d_unscale, int *d_flag);

@@ -1979,9 +1979,10 @@ int HfModel::make_half_group(int l, int g, char *dst) {
     static const char *const name[7] = {"self_attn.q_proj.weight", "self_attn.k_proj.weight", "self_attn.v_proj.weight",
                                         "self_attn.o_proj.weight", "mlp.gate_proj.weight", "mlp.up_proj.weight", "mlp.down_proj.weight"};
     const HalfGroup hg = half_group(g);
-    const int *e = half_exps_.as<int>() + (size_t)l * (2 * hidden + qd);
-    const int *col[4] = {e, e + 2 * hidden, e + hidden, nullptr};
-    int *flag = half_flags_.as<int>() + l * 4 + g;
+    const int *e = half_exps_.as<int>() + (size_t)l * (2 * hidden + qd + inter);
+    const bool gated = (bool)half_[l].gated;
+    const int *col[4] = {e, e + 2 * hidden, e + hidden, gated ? e + 2 * hidden + qd : nullptr};
+    int *flag = half_flags_.as<int>() + l * 5 + (g == 3 && gated ? 4 : g);
     uint16_t *w = reinterpret_cast<uint16_t *>(dst);
     float *factors = reinterpret_cast<float *>(dst + hg.factors);
     if (weight_dtype_ == DType::BF16) {
@@ -2037,7 +2038,7 @@ int HfModel::keep_half_weights() {
 int HfModel::build_half_weights() {
     drop_half_weights();
     const TransformerConfig &c = cfg_;
-    const int L = c.num_hidden_layers, hidden = c.hidden_size, hd = c.head_dim(), qd = c.q_dim(), kvd = c.kv_dim();
+    const int L = c.num_hidden_layers, hidden = c.hidden_size, inter = c.intermediate_size, hd = c.head_dim(), qd = c.q_dim(), kvd = c.kv_dim();
     if (!prefill_available() || prefill_weight_cache_bytes_ == 0) return HM_OK;
     const bool bf16 = weight_dtype_ == DType::BF16;
     size_t need = 0;
@@ -2045,20 +2046,22 @@ int HfModel::build_half_weights() {
         for (int g = 0; g < 4; g++) need += half_takes(l, g) ? half_group(g).bytes : 0;
     if (need == 0 || !half_fits(need)) return HM_OK;
 
-    half_exps_ = Buffer::alloc(ctx_, {(int64_t)L * (2 * hidden + qd)}, DType::F32);
-    half_flags_ = Buffer::alloc(ctx_, {(int64_t)L * 4}, DType::F32);
-    if (!half_exps_ || !half_flags_) {
+    half_exps_ = Buffer::alloc(ctx_, {(int64_t)L * (2 * hidden + qd + inter)}, DType::F32);
+    half_flags_ = Buffer::alloc(ctx_, {(int64_t)L * 5}, DType::F32);  // of the groups, and of the down matrix with column factors
+    const Buffer bounds = Buffer::alloc(ctx_, {2 * (int64_t)inter}, DType::F32);
+    if (!half_exps_ || !half_flags_ || !bounds) {
         (void)hipGetLastError();
         drop_half_weights();
         return HM_OK;
     }
-    HM_HIP(ctx_, hipMemsetAsync(half_flags_.ptr(), 0, (size_t)L * 16, ctx_->stream));
+    HM_HIP(ctx_, hipMemsetAsync(half_flags_.ptr(), 0, (size_t)L * 20, ctx_->stream));
     half_.resize((size_t)L);
     int rc = HM_OK;
     for (int l = 0; l < L && rc == HM_OK; l++) {
         HalfLayer &h = half_[l];
         const std::string pre = "model.layers." + std::to_string(l) + ".";
-        int *e1 = half_exps_.as<int>() + (size_t)l * (2 * hidden + qd), *e2 = e1 + hidden, *eo = e2 + hidden, *flag = half_flags_.as<int>() + l * 4;
+        int *e1 = half_exps_.as<int>() + (size_t)l * (2 * hidden + qd + inter), *e2 = e1 + hidden, *eo = e2 + hidden, *eg = eo + qd;
+        int *flag = half_flags_.as<int>() + l * 5;
         const float *w1 = weight_f32(pre + "input_layernorm.weight"), *w2 = weight_f32(pre + "post_attention_layernorm.weight");
         h.norms = Buffer::alloc(ctx_, {2 * (int64_t)hidden}, DType::F32);
         h.values = Buffer::alloc(ctx_, {kvd}, DType::F32);
@@ -2075,15 +2078,42 @@ int HfModel::build_half_weights() {
                                         : weight_bufs_[slot_by_name_.at(pre + "self_attn.v_proj.weight")].ptr(),
                                    w1, lp.qkv_bias ? lp.qkv_bias.as<float>() + qd + kvd : nullptr, kvd, hidden, c.num_attention_heads, hd,
                                    h.values.as<float>(), eo, flag + 1);
+        if (rc == HM_OK && half_takes(l, 2) && half_takes(l, 3)) {
+            h.gated = Buffer::alloc(ctx_, {inter}, DType::F32);
+            if (!h.gated) {
+                rc = HM_ERR_OOM;
+                break;
+            }
+            if (bf16)
+                rc = half_row_bounds(ctx_, HM_DTYPE_BF16, lp.gate_up.ptr(), w2, 2 * inter, hidden, bounds.as<float>(), 1, 0);
+            else
+                for (int j = 4; j <= 5 && rc == HM_OK; j++)
+                    rc = half_row_bounds(ctx_, (int)proj_dtype(l, j),
+                                         weight_bufs_[slot_by_name_.at(pre + (j == 4 ? "mlp.gate_proj.weight" : "mlp.up_proj.weight"))].ptr(), w2, inter,
+                                         hidden, bounds.as<float>(), 2, j - 4);
+            if (rc == HM_OK) rc = half_gated_scales(ctx_, bounds.as<float>(), inter, h.gated.as<float>(), eg, flag + 4);
+        }
         for (int g = 0; g < 4 && rc == HM_OK; g++) {
             if (!half_takes(l, g)) continue;
             h.w[g] = Buffer::alloc(ctx_, {(int64_t)(half_group(g).bytes + 3) / 4}, DType::F32);
             rc = h.w[g] ? make_half_group(l, g, h.w[g].as<char>()) : HM_ERR_OOM;
         }
     }
-    std::vector<int> bad((size_t)L * 4, 1);
-    if (rc == HM_OK) rc = hm_download(ctx_, bad.data(), half_flags_.ptr(), (size_t)L * 16);
-    const int synced = hm_sync(ctx_);
+    std::vector<int> bad((size_t)L * 5, 1);
+    if (rc == HM_OK) rc = hm_download(ctx_, bad.data(), half_flags_.ptr(), (size_t)L * 20);
+    int synced = hm_sync(ctx_);
+    bool again = false;
+    for (int l = 0; l < L && rc == HM_OK && synced == HM_OK; l++) {  // down matrices that column factors would round
+        if (!half_[l].gated || !bad[(size_t)l * 5 + 4]) continue;
+        half_[l].gated = Buffer();
+        again = true;
+        rc = make_half_group(l, 3, half_[l].w[3].as<char>());
+    }
+    if (again) {
+        if (rc == HM_OK) rc = hm_download(ctx_, bad.data(), half_flags_.ptr(), (size_t)L * 20);
+        const int settled = hm_sync(ctx_);
+        if (synced == HM_OK) synced = settled;
+    }
     if (rc == HM_ERR_OOM) {
         (void)hipGetLastError();
         drop_half_weights();
@@ -2092,7 +2122,7 @@ int HfModel::build_half_weights() {
     if (rc != HM_OK) return rc;
     for (int l = 0; l < L; l++)
         for (int g = 0; g < 4; g++) {
-            half_[l].ok[g] = (bool)half_[l].w[g] && !bad[(size_t)l * 4 + g];
+            half_[l].ok[g] = (bool)half_[l].w[g] && !bad[(size_t)l * 5 + g];
             if (!half_[l].ok[g]) half_[l].w[g] = Buffer();
         }
     return synced;
@@ -2325,7 +2355,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     const Buffer *i8 = nullptr;  // the planes of the group about to be multiplied, if it takes that path
     int8_t *q8 = p.q8 ? p.q8.as<int8_t>() : nullptr;
     float *q8s = p.q8s ? p.q8s.as<float>() : nullptr;
-    auto project = [&](int l, int first, int count, const Buffer &packed, int K, float *out) -> int {
+    auto project = [&](int l, int first, int count, const Buffer &packed, int K, float *out, const uint16_t *rows, uint16_t *gated) -> int {
         int N = 0;
         for (int j = first; j < first + count; j++) N += proj_n[j];
         if (const int g = first == 0 ? 0 : first == 3 ? 1 : first == 4 ? 2 : 3; half(l, g)) {
@@ -2334,8 +2364,13 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
             if (!kept)
                 if (const int made = make_half_group(l, g, w); made != HM_OK) return made;
             const float *f = reinterpret_cast<const float *>(w + half_matrix_bytes(N, K));
-            return gemm_half_nk(ctx_, split, reinterpret_cast<const uint16_t *>(w), HalfProduct{quant ? nullptr : f}, quant ? f : nullptr,
-                                quant ? half_scale_cols(N) : 0, out, n, K, N, MP, &parts);
+            HalfProduct hp{quant ? nullptr : f};
+            if (gated) {
+                hp.gate_scale = half_[l].gated.as<float>();
+                hp.gated = gated;
+            }
+            return gemm_half_nk(ctx_, rows, reinterpret_cast<const uint16_t *>(w), hp, quant ? f : nullptr, quant ? half_scale_cols(N) : 0, out, n, K,
+                                N, MP, &parts);
         }
         if (!quant) return gemm_split_nk(ctx_, split, np, packed.as<uint16_t>(), out, n, K, N, MP, &parts);
         if (i8) {
@@ -2402,7 +2437,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         rc = rmsnorm_split_launch(ctx_, x, res, res_parts, h0 ? half_[l].norms.as<float>() : weight_f32(pre + "input_layernorm.weight"), split,
                                   h0 ? 2 : np, res ? h : nullptr, n, hidden, eps, q8k(l, 0), q8k(l, 0) ? capture_at(l, 0) : nullptr,
                                   i8 ? q8 : nullptr, i8 ? q8s : nullptr, h0, res_scale);
-        if (rc == HM_OK) rc = project(l, 0, 3, lp.qkv, hidden, qkv);
+        if (rc == HM_OK) rc = project(l, 0, 3, lp.qkv, hidden, qkv, split, nullptr);
         if (rc != HM_OK) return rc;
         QkvPostArgs qa;
         qa.qkv = qkv;
@@ -2456,24 +2491,31 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         if (o_q8k && !i8 && (rc = split_rows_launch(ctx_, gate_up, split, np, (size_t)n, qd, true)) != HM_OK) return rc;
         if (o_q8k && capture_at(l, 1))
             HM_HIP(ctx_, hipMemcpyAsync(capture_at(l, 1), gate_up, (size_t)n * qd * 4, hipMemcpyDeviceToDevice, ctx_->stream));
-        if ((rc = project(l, 3, 1, lp.o, qd, proj_out)) != HM_OK) return rc;
+        if ((rc = project(l, 3, 1, lp.o, qd, proj_out, split, nullptr)) != HM_OK) return rc;
         // MLP kernel (reference src/hf/emitter.rs:767-822); h holds the layer's input by now
         i8 = i8_planes(l, 2, 4, 2, hidden);
         rc = rmsnorm_split_launch(ctx_, h, proj_out, parts,
                                   h2 ? half_[l].norms.as<float>() + hidden : weight_f32(pre + "post_attention_layernorm.weight"), split,
                                   h2 ? 2 : np, resid, n, hidden, eps, q8k(l, 4), q8k(l, 4) ? capture_at(l, 2) : nullptr,
                                   i8 ? q8 : nullptr, i8 ? q8s : nullptr, h2);
-        if (rc == HM_OK) rc = project(l, 4, 2, lp.gate_up, hidden, gate_up);
+        // The gate|up product's workgroups write the gated rows themselves where they have whole sums (into the scratch of the f32
+        // rows: `split` is what they read)
+        const bool by_column = h3 && half_[l].gated;
+        uint16_t *gated = nullptr;
+        if (h2 && by_column && gemm_half_gated_pays(quant, n, hidden, 2 * inter, ctx_->num_cus, MP)) gated = reinterpret_cast<uint16_t *>(gate_up);
+        if (rc == HM_OK) rc = project(l, 4, 2, lp.gate_up, hidden, gate_up, split, gated);
         i8 = i8_planes(l, 3, 6, 1, inter);
-        if (rc == HM_OK && h3) rc = silu_mul_half_launch(ctx_, gate_up, parts, split, p.row_unscale.as<float>(), n, inter);
-        else if (rc == HM_OK) rc = silu_mul_split_launch(ctx_, gate_up, parts, split, np, n, inter, q8k(l, 6), q8k(l, 6) ? capture_at(l, 3) : nullptr,
+        if (rc == HM_OK && !gated && h3)
+            rc = silu_mul_half_launch(ctx_, gate_up, parts, split, by_column ? nullptr : p.row_unscale.as<float>(), n, inter,
+                                      by_column ? half_[l].gated.as<float>() : nullptr);
+        else if (rc == HM_OK && !gated) rc = silu_mul_split_launch(ctx_, gate_up, parts, split, np, n, inter, q8k(l, 6), q8k(l, 6) ? capture_at(l, 3) : nullptr,
                                                     i8 ? q8 : nullptr, i8 ? q8s : nullptr);
-        if (rc == HM_OK) rc = project(l, 6, 1, lp.down, inter, proj_out);
+        if (rc == HM_OK) rc = project(l, 6, 1, lp.down, inter, proj_out, gated ? gated : split, nullptr);
         i8 = nullptr;
         if (rc != HM_OK) return rc;
         x = resid;
         res = proj_out;
-        res_scale = h3 ? p.row_unscale.as<float>() : nullptr;
+        res_scale = h3 && !by_column ? p.row_unscale.as<float>() : nullptr;
         res_parts = parts;
     }
     if (h_logits) {  // LM head (reference src/hf/emitter.rs:828-862) for every row

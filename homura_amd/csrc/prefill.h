@@ -58,9 +58,11 @@ int silu_mul_split_launch(hm_ctx *ctx, const float *d_gu, int parts, uint16_t *d
                           float *d_q8_scale = nullptr);
 
 // The same rows as two f16 pieces, each row times a power of two that puts its largest value at 2^14 .. 2^15; row_unscale [rows]
-// receives the inverse. inter <= SILU_HALF_MAX.
+// receives the inverse. With d_col_scale [inter] every column times its factor instead (half_gated_scales), and no row factors
+// (d_row_unscale NULL). inter <= SILU_HALF_MAX.
 constexpr int SILU_HALF_MAX = 16384;
-int silu_mul_half_launch(hm_ctx *ctx, const float *d_gu, int parts, uint16_t *d_out_half, float *d_row_unscale, int rows, int inter);
+int silu_mul_half_launch(hm_ctx *ctx, const float *d_gu, int parts, uint16_t *d_out_half, float *d_row_unscale, int rows, int inter,
+                         const float *d_col_scale = nullptr);
 
 // The tail of the reference's QKV kernel for S rows at positions past .. past + S - 1
 // (src/hf/emitter.rs:604-649): bias add, per-head QK-norm, RoPE on q and k in place, and the

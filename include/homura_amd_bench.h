@@ -73,6 +73,12 @@ int hm_test_product_tiles(int kind, int m, int k, int n, int cus, int max_parts,
 int hm_test_prompt_rows(hm_ctx *ctx, int front, const void *x, const float *norm_w, int dtype, const void *w, int half, int m, int k,
                         int n, float *out, float *row_factor, int *parts);
 
+/* Test support: the gate|up product of the prompt pass and its gated rows with column factors: x [m][k] f32 through RMSNorm (norm_w [k], eps
+ * 1e-6), w [2 inter][k] bf16 rows or Q8_0 / Q4_0 blocks as (gate, up) pairs of rows. fused 1: the product's workgroups write the rows, 0: its
+ * slices go through the row kernel. out [m][2][inter] f16 pieces of silu(gate) up times scale [inter]. *pays: what the prompt pass would take. */
+int hm_test_gated_rows(hm_ctx *ctx, const void *x, const float *norm_w, int dtype, const void *w, int fused, int m, int k, int inter,
+                       uint16_t *out, float *scale, int *pays);
+
 /* Test support: the bytes of f16 weight copies that a transformer's prompt pass holds, and how many of its groups of projections
  * (q|k|v, o, gate|up, down of every layer) multiply with them. */
 int hm_test_prefill_f16_copies(hm_model *m, size_t *bytes, int *groups);

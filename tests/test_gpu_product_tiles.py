@@ -305,3 +305,63 @@ def test_one_bf16_piece_against_float64(ctx, m, k, n):
     for buf in (da, db, out):
         buf.free()
     assert np.linalg.norm(got - want) <= 4e-7 * np.linalg.norm(want)
+
+
+# the few-rows kernel's tiles, each tile of 64 rows, 128 x 128 and 128 x 256, rows and columns off their size, an odd number of pairs
+@pytest.mark.parametrize("m,k,inter", [(1, 64, 4), (31, 192, 50), (24, 192, 3074), (64, 320, 37), (37, 896, 2434), (65, 64, 21), (70, 320, 1100),
+                                       (181, 1024, 3072), (400, 128, 3074), (513, 192, 1540), (700, 128, 2052), (640, 1024, 3073), (1905, 128, 2052),
+                                       (2048, 1024, 3072)])
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_Q8_0, DTYPE_Q4_0])
+def test_gated_rows_from_the_product(ctx, dtype, m, k, inter):
+    """silu(gate) up as the gate|up product's workgroups write it, in two f16 pieces with a factor per column, and out of the row kernel.
+    Bound: gate and up as above (a sum over k moves by at most 4e-7 of the norms' product, silu's slope is below 1.1), f32's rounding of the
+    value and the second piece's last place."""
+    print(f"dtype {dtype} {m} x {k} x {inter}", flush=True)
+    rng = np.random.default_rng(m * 7 + k + inter)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    norm_w = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    raw, w = weights(dtype, 2 * inter, k, rng)
+    rows, w = rows_of(0, x, norm_w), w.astype(np.float64)
+    gu = rows @ w.T
+    g, u = gu[:, 0::2], gu[:, 1::2]
+    size = np.linalg.norm(rows, axis=1)[:, None] * np.linalg.norm(w, axis=1)
+    off = 2e-6 / np.sqrt(k) * np.maximum(1, np.sqrt(k) / 5) * size  # single values: five times what the whole is off
+    silu = g / (1 + np.exp(-g))
+    dx, dn, dw = ctx.to_device(x), ctx.to_device(norm_w), ctx.to_device(raw)
+    guard = 256
+    for fused in ([1, 0] if inter % 4 == 0 else [1]):
+        out, scale, pays = ctx.to_device(np.full(m * 2 * inter + guard, 0x7B7B, np.uint16)), ctx.empty(inter), C.c_int(0)
+        ctx._check(ctx.lib.hm_test_gated_rows(ctx.h, dx.ptr, dn.ptr, dtype, dw.ptr, fused, m, k, inter, out.ptr, scale.ptr, C.byref(pays)))
+        got, f = out.download(np.uint16, (m * 2 * inter + guard,)), scale.download(np.float32, (inter,)).astype(np.float64)
+        assert np.all(got[m * 2 * inter:] == 0x7B7B), "wrote past the end"
+        p = got[:m * 2 * inter].view(np.float16).reshape(m, 2, inter).astype(np.float64)
+        bound = 1.1 * off[:, 0::2] * np.abs(u) + np.abs(silu) * off[:, 1::2] + off[:, 0::2] * off[:, 1::2] + 2.0 ** -21 * np.abs(silu * u) + 2.0 ** -24 / f
+        assert np.all(np.abs(p.sum(1) / f - silu * u) <= bound)
+        assert np.linalg.norm(p.sum(1) / f - silu * u) <= 1e-6 * np.linalg.norm(silu * u)
+        for b in (out, scale):
+            b.free()
+    for b in (dx, dn, dw):
+        b.free()
+
+
+def test_down_weights_that_column_factors_would_round(ctx):
+    """A gate and an up row 2^6 times the others move their column of the down weights 2^12 up, and a weight 2^-27 of its row's largest then
+    out of f16: that layer's gated rows keep a factor of their own, and the pass agrees with the steps that take one token at a time."""
+    cfg = synth_model.TINY
+    w = synth_model.synth_weights(cfg, 43)
+    for name, values in w:
+        if name.endswith(("layers.0.mlp.gate_proj.weight", "layers.0.mlp.up_proj.weight")):  # [in][out]
+            values[:, 0] = bf16((values[:, 0].astype(np.uint32) << 16).view(np.float32) * 64)[0]
+        if name.endswith("layers.0.mlp.down_proj.weight"):
+            values[0, 0], values[5, 0] = bf16(np.float32([0.05, 0.05 * 2.0 ** -27]))[0]
+    gm = synth_model.build_model(ctx, cfg, w, 128)
+    nbytes, groups = C.c_size_t(), C.c_int()
+    gm._check(gm.lib.hm_test_prefill_f16_copies(gm.h, C.byref(nbytes), C.byref(groups)))
+    assert groups.value == 4 * cfg.num_hidden_layers
+    ids = synth.token_ids(9, 70, cfg.vocab_size)
+    at_once = gm.prefill(ids)[-1]
+    gm.reset_kv_cache()
+    for t in ids:
+        last = gm.run_kv([int(t)])
+    assert np.linalg.norm(at_once - np.asarray(last).reshape(-1)) <= 2e-3 * np.linalg.norm(last)
+    gm.close()
