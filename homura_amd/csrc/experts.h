@@ -50,7 +50,17 @@ struct ExpertsStepArgs {
     int *choice = nullptr;              // [top]
     float *hidden = nullptr;            // [top][ff]
     float *y = nullptr;                 // [width]
+    // The router and the residual ahead of it in the same launch (experts_step_routes): the row is x, or x + RMSNorm(add) * add_w with
+    // add, and goes to row_out; `logits` stays unread.
+    const uint16_t *router = nullptr;   // [experts][K]
+    const float *add = nullptr, *add_w = nullptr;  // [K]
+    int norm_dim = 0;                   // elements the norm's mean runs over
+    float eps = 0.f;
+    float *row_out = nullptr;           // [K]
 };
+// Every workgroup then multiplies the whole router itself, so it must be small: 128 KB. Steps of six mixtures among eight layers, us in two
+// launches and in one: 32 experts of 1024 225.7 / 213.6, 64 226.3 / 220.9, 32 of 2048 340.1 / 333.5, 64 (256 KB) 340.4 / 351.9.
+inline bool experts_step_routes(int experts, int K) { return experts <= 64 && K <= 2048 && experts * K <= 1 << 16; }
 int experts_step_up_launch(hm_ctx *ctx, const ExpertsStepArgs &a);
 int experts_step_down_launch(hm_ctx *ctx, const ExpertsStepArgs &a);
 

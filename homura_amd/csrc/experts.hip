@@ -28,9 +28,12 @@ __device__ __forceinline__ void choose_top(float (&z)[PER], int E, int top, F em
                 at = lane + 64 * j;
             }
         const float m = wave_max(at == 0x7fffffff ? -INFINITY : best);
-        int idx = best == m ? at : 0x7fffffff;
+        int idx = 0x7fffffff;
 #pragma unroll
-        for (int d = 1; d < 64; d *= 2) idx = min(idx, __shfl_xor(idx, d));
+        for (int j = PER - 1; j >= 0; j--) {
+            const unsigned long long lanes = __ballot(best == m && at == lane + 64 * j);
+            if (lanes) idx = __builtin_ctzll(lanes) + 64 * j;
+        }
         if ((idx & 63) == lane) gone |= 1u << (idx >> 6);
         emit(place, idx, m);
     }
@@ -192,6 +195,97 @@ __global__ __launch_bounds__(256) void experts_step_up_kernel(ExpertsStepArgs a)
     if (blockIdx.x == 0 && tid == 0) a.choice[blockIdx.y] = e;
 }
 
+// The same with the router and the residual ahead of it: a workgroup a CU forms the row, its wavefronts multiply the router's rows (asked for
+// ahead of everything, they do not depend on the row), all of them make the choice from the logits in LDS, and every wavefront takes whole
+// (gate, up) pairs of rows. In a launch of its own the router was bound by that launch and its trips to memory (32 experts of 1024: 3.9 us
+// and 6.8 for the rows behind it; 8.6 together). What bounds it: the row, the logits, the choice and the chosen rows are four dependent trips.
+constexpr int ROUTE_WAVES = 12;
+template <int EPW, int NC>
+__global__ __launch_bounds__(ROUTE_WAVES * 64) void experts_step_route_up_kernel(ExpertsStepArgs a) {
+    __shared__ __attribute__((aligned(16))) float xs[NC * 512];
+    __shared__ float red[ROUTE_WAVES], logit[64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = tid * 4;
+    const bool mine = i < a.K;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v = zero, r = zero, rw = zero;
+    if (mine) {
+        v = *reinterpret_cast<const f32x4 *>(a.x + i);
+        if (a.add) {
+            r = *reinterpret_cast<const f32x4 *>(a.add + i);
+            rw = *reinterpret_cast<const f32x4 *>(a.add_w + i);
+        }
+    }
+    u32x4 wr[EPW][NC];
+#pragma unroll
+    for (int e = 0; e < EPW; e++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int k = (c * 64 + lane) * 8;
+            wr[e][c] = k < a.K ? *reinterpret_cast<const u32x4 *>(a.router + (size_t)min(wave + e * ROUTE_WAVES, a.experts - 1) * a.K + k)
+                               : u32x4{0u, 0u, 0u, 0u};
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    if (a.add) {
+        const float ss = wave_sum((r.x * r.x + r.y * r.y) + (r.z * r.z + r.w * r.w));
+        if (lane == 0) red[wave] = ss;
+        __syncthreads();
+        float tot = 0.f;
+#pragma unroll
+        for (int w = 0; w < ROUTE_WAVES; w++) tot += red[w];
+        v = v + (r * (1.0f / sqrtf(tot / (float)a.norm_dim + a.eps))) * rw;
+    }
+    if (i < NC * 512) *reinterpret_cast<f32x4 *>(xs + i) = v;  // (zero past K)
+    if (blockIdx.x == 0 && mine && a.row_out) *reinterpret_cast<f32x4 *>(a.row_out + i) = v;
+    __syncthreads();
+    f32x4 x[NC][2];
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) x[c][h] = *reinterpret_cast<const f32x4 *>(xs + (c * 64 + lane) * 8 + 4 * h);
+#pragma unroll
+    for (int e = 0; e < EPW; e++) {
+        float z = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; c++) z = dot8(wr[e][c], x[c][0], x[c][1], z);
+        z = wave_sum(z);
+        if (lane == 0 && wave + e * ROUTE_WAVES < a.experts) logit[wave + e * ROUTE_WAVES] = z;
+    }
+    __syncthreads();
+    float z[1] = {lane < a.experts ? logit[lane] : 0.f};
+    int chosen = 0;  // lane p: place p's expert and logit
+    float chosen_z = 0.f;
+    choose_top<1>(z, a.experts, a.top, [&](int place, int idx, float m) {
+        if (lane == place) {
+            chosen = idx;
+            chosen_z = m;
+        }
+    });
+    if (blockIdx.x == 0 && tid < a.top) a.choice[tid] = chosen;
+    const int pairs = a.top * a.ff;
+    for (int p = blockIdx.x * ROUTE_WAVES + wave; p < pairs; p += gridDim.x * ROUTE_WAVES) {
+        const int place = p / a.ff, e = __builtin_amdgcn_readlane(chosen, place);
+        const uint16_t *w = a.gate_up + ((size_t)e * a.ff + (p - place * a.ff)) * 2 * a.K;
+        u32x4 wv[2][NC];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                const int k = (c * 64 + lane) * 8;
+                wv[h][c] = k < a.K ? ld128_stream(w + (size_t)h * a.K + k) : u32x4{0u, 0u, 0u, 0u};
+            }
+        float g = 0.f, u = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            g = dot8(wv[0][c], x[c][0], x[c][1], g);
+            u = dot8(wv[1][c], x[c][0], x[c][1], u);
+        }
+        g = wave_sum(g);
+        u = wave_sum(u);
+        const float weight = score(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(chosen_z), place)));
+        if (lane == 0) a.hidden[p] = gated_act(a.act, weight * g, weight * u);
+    }
+}
+
 // Workgroup: R output rows; the hidden rows of all places are one long row, cut across the four wavefronts in pieces of
 // eight elements, which never straddle two places.
 template <int R, int NC>
@@ -270,8 +364,19 @@ int sum_places_launch(hm_ctx *ctx, float *d_y, int places, size_t n) {
 }
 
 int experts_step_up_launch(hm_ctx *ctx, const ExpertsStepArgs &a) {
-    HM_REQUIRE(ctx, !bad_choice(a.experts, a.top) && a.x && a.logits && a.gate_up && a.choice && a.hidden, "experts_step_up: bad arguments");
+    HM_REQUIRE(ctx, !bad_choice(a.experts, a.top) && a.x && (a.logits || a.router) && a.gate_up && a.choice && a.hidden, "experts_step_up: bad arguments");
     HM_REQUIRE(ctx, a.K > 0 && a.K % 32 == 0 && a.ff > 0 && a.ff % 32 == 0 && al16(a.x) && al16(a.gate_up), "experts_step_up: bad shape");
+    if (a.router) {
+        HM_REQUIRE(ctx, experts_step_routes(a.experts, a.K) && al16(a.router) && al16(a.add) && al16(a.add_w) && al16(a.row_out) &&
+                            (!a.add || (a.add_w && a.norm_dim > 0)), "experts_step_up: no router of %d experts of %d in the same launch", a.experts, a.K);
+        const int wgs = (int)std::min<long long>(ctx->num_cus, ((long long)a.top * a.ff + ROUTE_WAVES - 1) / ROUTE_WAVES);
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(wgs), dim3(ROUTE_WAVES * 64), 0, ctx->stream, a); };
+        const bool few = a.experts <= 3 * ROUTE_WAVES;
+        if (a.K <= 1024) few ? go(experts_step_route_up_kernel<3, 2>) : go(experts_step_route_up_kernel<6, 2>);
+        else few ? go(experts_step_route_up_kernel<3, 4>) : go(experts_step_route_up_kernel<6, 4>);
+        HM_LAUNCH_CHECK(ctx);
+        return HM_OK;
+    }
     constexpr int R = 4;
     const dim3 g((2 * a.ff + R - 1) / R, a.top), b(256);
     if (a.experts <= 64) hipLaunchKernelGGL((experts_step_up_kernel<R, 1>), g, b, 0, ctx->stream, a);

@@ -1054,14 +1054,25 @@ int BlockModel::emit_plan() {
                  [=](const StepContext &, GemvArgs &g) { g.act = gated; });
             gemv("gemv[down]", l.down, s_act, s_y, nullptr, GEMV_EPI_NONE);
         } else {
-            gemv("gemv[router]", l.router, cur, s_d2, nullptr, GEMV_EPI_NONE);
-            const size_t x_slot = cur;
             const int experts = s.ff.experts, top = s.ff.top, ff = d.ff;
+            const bool routes = experts_step_routes(experts, wp);
+            if (!routes) gemv("gemv[router]", l.router, cur, s_d2, nullptr, GEMV_EPI_NONE);
+            const size_t x_slot = cur, x_next = cur == s_xa ? s_xb : s_xa;
+            const Linear *router = routes ? &l.router : nullptr;
+            const Vec *post = routes ? pending : nullptr;
             std::shared_ptr<StepScratch> scr = step_;
             auto args = [=](const StepContext &sc) {
                 ExpertsStepArgs x;
                 x.x = sc.pool[x_slot]->as<float>();
-                x.logits = sc.pool[s_d2]->as<float>();
+                if (router) x.router = router->ptr();
+                else x.logits = sc.pool[s_d2]->as<float>();
+                if (post) {
+                    x.add = sc.pool[s_y]->as<float>();
+                    x.add_w = post->ptr();
+                    x.norm_dim = W;
+                    x.eps = eps;
+                    x.row_out = sc.pool[x_next]->as<float>();
+                }
                 x.gate_up = lw->gate_up.ptr();
                 x.down = lw->down.ptr();
                 x.experts = experts;
@@ -1075,10 +1086,14 @@ int BlockModel::emit_plan() {
                 x.y = sc.pool[s_y]->as<float>();
                 return x;
             };
-            step("Experts", "experts_up", top * (4.0 * ff * wp + 4.0 * ff) + 4.0 * (wp + experts), 0, {x_slot, s_d2}, {s_act},
+            step("Experts", routes ? "router+experts_up" : "experts_up",
+                 top * (4.0 * ff * wp + 4.0 * ff) + 4.0 * (wp + experts) + (routes ? 2.0 * experts * wp : 0) + (post ? 12.0 * wp : 0), 0,
+                 post ? std::vector<size_t>{x_slot, s_y} : routes ? std::vector<size_t>{x_slot} : std::vector<size_t>{x_slot, s_d2},
+                 post ? std::vector<size_t>{s_act, x_next} : std::vector<size_t>{s_act},
                  [=](const StepContext &sc) -> int { return experts_step_up_launch(sc.ctx, args(sc)); });
             step("Experts", "experts_down", top * (2.0 * ff * wp + 4.0 * ff) + 4.0 * wp, 0, {s_act}, {s_y},
                  [=](const StepContext &sc) -> int { return experts_step_down_launch(sc.ctx, args(sc)); });
+            if (post) cur = x_next;
         }
         pending = &l.norm2b;
     }

@@ -131,6 +131,16 @@ def test_expert_products(ctx, width, ff, experts, top, dtype):
     check(ctx, cfg, 30, dtype, seed=40, cuts=range(12, 30))
 
 
+# the router in the experts' launch: up to 36 and 64 of them, rows of up to 1024 and 2048, the largest router and one past it, rows that end
+# inside a wavefront's load, as many places as experts, more pairs of rows than the launch has wavefronts
+@pytest.mark.parametrize("width,experts,top,ff", [(1024, 36, 4, 40), (1056, 37, 3, 33), (1024, 64, 64, 32), (1056, 62, 2, 64), (1056, 63, 2, 64), (2048, 32, 2, 64), (2080, 9, 2, 40),
+                                                  (200, 65, 5, 64), (300, 8, 4, 900)])
+def test_router_in_the_experts_launch(ctx, width, experts, top, ff):
+    cfg = lf.config([lf.memory(heads=1, dim=4, vdim=12, mlp=lf.moe(experts=experts, top=top, ff=ff)), lf.attn(mlp=lf.moe(experts=experts, top=top, ff=ff))],
+                    width=width)
+    check(ctx, cfg, 12, "f32", prefill_min=0)
+
+
 @pytest.mark.parametrize("gates", [(-6.0, 3.0), (5.0, -4.0), (-6.0, -6.0), (6.0, 6.0)])
 def test_extreme_gates(ctx, gates):
     """Input gates far below the running maximum's start and above it, memories that are forgotten at once or never."""
