@@ -36,3 +36,7 @@ struct AttnArgs {
 int gqa_attn_fixed_scratch_setup(hm_ctx *ctx);
 
 int gqa_decode_attn_launch(hm_ctx *ctx, const AttnArgs &a);
+
+// Whether the decode plan's attention over a grid of `span` rows in chunks of `chunk` has a fold of its own behind it (more than one split, and
+// not folded by the last of their workgroups)
+bool gqa_decode_attn_folds(const hm_ctx *ctx, int H, int kvh, int hd, int span, int chunk);

@@ -5,11 +5,12 @@
 // its KV head (the reference's `h floordiv g` map, src/graph_builder/emit_linalg.rs:123-127),
 // so each K/V row is read from HBM once. Rows are streamed with 16-byte loads: HD/8 lanes
 // cover a row, 64/(HD/8) rows per wavefront instruction. Scores live in LDS; softmax is f32.
-// Partial (o, max, sum) triples go to the workspace and a second, tiny kernel folds them per
-// (batch, kv head) in split order, so the result does not depend on timing.
+// Partial (o, max, sum) triples go to the workspace and are folded per (batch, kv head) in an order that does not depend on timing: by
+// the last workgroup of a head's splits where those sit on one die (die_fold.h), else by a second, tiny kernel.
 // Algorithmic HBM traffic: 2 * kv_len * HD * 2 bytes per (batch, kv head).
 #include "attention.h"
 #include "bf16_pieces.h"
+#include "die_fold.h"
 
 namespace {
 
@@ -50,12 +51,79 @@ __device__ __forceinline__ float row_group_sum(float v) {
     return v;
 }
 
+// Splits folded by the last of their workgroups (die_fold.h): `splits` of the grid per group of heads, 0: in a launch of its own
+struct DieFold {
+    int splits, groups;
+    unsigned int *arrived;
+};
+
+// The whole workgroup: heads <= 8 heads whose nsplit <= DIE_SPLITS_MAX partial results (o [HD]; max and sum) lie `all` heads apart, one head
+// behind the other, to out [heads * HD]. Thread (head, split) makes that split's weight. Threads take four outputs each, and where that
+// leaves some over, every second or fourth split of them; the sums of those meet in LDS.
+// (Few instructions count: they are cold, one workgroup of a group runs them once.)
+template <int HD>
+__device__ __forceinline__ void fold_here(const float *po, const float *pml, float *__restrict__ out, int heads, int nsplit, int all) {
+    constexpr int AHEAD = 8;  // splits asked for at a time
+    static_assert(homura::DIE_SPLITS_MAX == 32 && ATT_THREADS == 8 * 32 && 8 * HD / 4 <= ATT_THREADS, "a split a lane of half a wavefront");
+    __shared__ float s_w[8][32];
+    __shared__ f32x4 s_o[ATT_THREADS];
+    const int tid = threadIdx.x, h = tid >> 5, sp = tid & 31, vecs = heads * (HD / 4);
+    const int lg = vecs > 128 ? 8 : vecs > 64 ? 7 : 6;  // threads of a share of the splits, as a power of two
+    const int shares = ATT_THREADS >> lg, first = tid >> lg, v = tid & ((1 << lg) - 1), oh = min(v * 4 / HD, heads - 1);
+    const uint32_t stride = (uint32_t)all * HD, last = (uint32_t)(nsplit - 1) * stride;
+    const float *mine = po + min(v, vecs - 1) * 4;
+    uint32_t at = (uint32_t)first * stride;
+    f32x4 O = {0.f, 0.f, 0.f, 0.f};
+    const bool live = h < heads && sp < nsplit;
+    const float *ml = pml + ((live ? sp : 0) * all + (live ? h : 0)) * 2;
+    const float m = live ? homura::from_die(ml) : -INFINITY, l = homura::from_die(ml + 1);
+    for (int u0 = 0; u0 * shares < nsplit; u0 += AHEAD) {
+        f32x4 o[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) o[u] = homura::from_die4(mine + min(at + (uint32_t)(u * shares) * stride, last));
+        if (u0 == 0) {
+            float M = m;
+            M = fmaxf(M, dpp_move<0xB1, 0xF>(M, 0.f));
+            M = fmaxf(M, dpp_move<0x4E, 0xF>(M, 0.f));
+            M = fmaxf(M, dpp_move<0x141, 0xF>(M, 0.f));
+            M = fmaxf(M, dpp_move<0x140, 0xF>(M, 0.f));
+            M = fmaxf(M, __shfl_xor(M, 16, WAVE));
+            const float w = live ? expf(m - M) : 0.f;
+            float L = live ? w * l : 0.f;
+            L += dpp_move<0xB1, 0xF>(L, 0.f);
+            L += dpp_move<0x4E, 0xF>(L, 0.f);
+            L += dpp_move<0x141, 0xF>(L, 0.f);
+            L += dpp_move<0x140, 0xF>(L, 0.f);
+            L += __shfl_xor(L, 16, WAVE);
+            s_w[h][sp] = w / L;
+            __syncthreads();
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            const int split = first + (u0 + u) * shares;
+            if (split < nsplit) {  // (past the last split: not its sum again, 0 times infinity is NaN)
+                const float wu = s_w[oh][split];
+#pragma unroll
+                for (int k = 0; k < 4; k++) O[k] = fmaf(wu, o[u][k], O[k]);
+            }
+        }
+        at += (uint32_t)(AHEAD * shares) * stride;
+    }
+    if (shares > 1) {
+        s_o[tid] = O;
+        __syncthreads();
+        if (first) return;
+        for (int g = 1; g < shares; g++) O += s_o[(g << lg) + tid];
+    }
+    if (v < vecs) *reinterpret_cast<f32x4 *>(out + v * 4) = O;
+}
+
 template <int HD, int G>
 __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
     const float *__restrict__ q, uint16_t *__restrict__ kcache, uint16_t *__restrict__ vcache,
-    float *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml, int kvh,
+    float *__restrict__ out, float *part_o, float *part_ml, int kvh,
     int max_len, int kv_len_arg, int chunk, float scale, const DecodeState *__restrict__ state,
-    int lds_front, AttnFuse fuse, int g_total) {
+    int lds_front, AttnFuse fuse, int g_total, DieFold die) {
     constexpr int LPR = HD / 8;      // lanes per row
     constexpr int RPI = WAVE / LPR;  // rows per wavefront instruction
     extern __shared__ float sm[];
@@ -70,7 +138,14 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
     // A workgroup serves G of the g_total query heads that share a KV head (all of them when g_total <= G):
     // blockIdx.y = kv head * groups + group. Heads past g_total in the last group multiply zeros and write nothing.
     const int ngroups = (g_total + G - 1) / G;
-    const int split = blockIdx.x, kvhd = blockIdx.y / ngroups, hg = blockIdx.y % ngroups, b = blockIdx.z;
+    int split = blockIdx.x, group = 0, yb = blockIdx.y, b = blockIdx.z;
+    if (die.splits) {
+        homura::die_place(blockIdx.x, die.splits, group, split);
+        if (group >= die.groups) return;
+        yb = group % (kvh * ngroups);
+        b = group / (kvh * ngroups);
+    }
+    const int kvhd = yb / ngroups, hg = yb % ngroups;
     const int g0 = hg * G, g_here = min(G, g_total - g0);
     const int H = kvh * g_total;
     const int n0 = split * chunk;
@@ -292,6 +367,9 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
         pml[tid * 2] = s_m[tid];
         pml[tid * 2 + 1] = s_l[tid];
     }
+    if (!die.splits || !homura::last_on_die(die.arrived, group, nsplit)) return;
+    fold_here<HD>(part_o + (pair * nsplit * g_total + g0) * HD, part_ml + (pair * nsplit * g_total + g0) * 2,
+                  out + ((size_t)b * H + kvhd * g_total + g0) * HD, g_here, nsplit, g_total);
 }
 
 // Long caches (more rows per workgroup than fit in registers at once): the workgroup walks its rows in
@@ -317,8 +395,8 @@ constexpr float LAZY = 8.0f;
 template <int HD, int G>
 __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_stream_kernel(
     const float *__restrict__ q, const uint16_t *__restrict__ kcache,
-    const uint16_t *__restrict__ vcache, float *__restrict__ out, float *__restrict__ part_o,
-    float *__restrict__ part_ml, int kvh, int max_len, int kv_len, int chunk, float scale) {
+    const uint16_t *__restrict__ vcache, float *__restrict__ out, float *part_o,
+    float *part_ml, int kvh, int max_len, int kv_len, int chunk, float scale, DieFold die) {
     constexpr int KS = HD / 32;  // k steps of the score MFMA
     constexpr int DS = HD / 8;   // 8-dim slices of a row
     static_assert(IT_ROWS == 32 * ATT_WAVES, "32 rows per wavefront and step");
@@ -330,7 +408,14 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_stream_kernel(
 
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
     const int l16 = lane & 15, kg = lane >> 4;
-    const int split = blockIdx.x, nsplit = gridDim.x, kvhd = blockIdx.y, b = blockIdx.z;
+    int split = blockIdx.x, nsplit = gridDim.x, group = 0, kvhd = blockIdx.y, b = blockIdx.z;
+    if (die.splits) {
+        homura::die_place(blockIdx.x, die.splits, group, split);
+        if (group >= die.groups) return;
+        nsplit = die.splits;
+        kvhd = group % kvh;
+        b = group / kvh;
+    }
     const int H = kvh * G;
     const int n0 = split * chunk;
     const size_t head_base = ((size_t)b * kvh + kvhd) * max_len * HD;
@@ -524,9 +609,11 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_stream_kernel(
         pml[tid * 2] = s_m[tid];
         pml[tid * 2 + 1] = s_l[tid];
     }
+    if (!die.splits || !homura::last_on_die(die.arrived, group, nsplit)) return;
+    fold_here<HD>(part_o + pair * nsplit * G * HD, part_ml + pair * nsplit * G * 2, out + ((size_t)b * H + kvhd * G) * HD, G, nsplit, G);
 }
 
-// Second half of the split attention: one workgroup per (batch, query head) folds that head's partial
+// Second half of the split attention where its splits are on several dies: one workgroup per (batch, query head) folds that head's partial
 // (o, max, sum) triples. A separate launch instead of a "last workgroup to arrive" fold: the kernel boundary
 // orders the partial writes, so no device-scope fence (a full L2 write-back + invalidate on this chip) is needed.
 constexpr int FOLD_BATCH = 32;      // splits fetched per batch, all loads of a batch in flight together
@@ -688,9 +775,16 @@ __global__ void kv_append_kernel(uint16_t *__restrict__ kc, uint16_t *__restrict
 // at most four, else two (the kernel's length grows with the heads it serves, and with two KV heads a 1024-row
 // cache gives only 32 workgroups of all heads; groups of three or four measured slower than two at G = 6 .. 8,
 // single heads slower again).
+constexpr int heads_a_workgroup(int g) { return g <= 4 ? g : 2; }
+DieFold die_fold(hm_ctx *ctx, long long groups, int nsplit, int chunk, int hd) {
+    if (!homura::die_fold_pays(ctx, groups, nsplit, 4.0 * groups * nsplit * chunk * hd)) return DieFold{0, 0, nullptr};
+    return DieFold{nsplit, (int)groups, ctx->counters};
+}
+
 template <int HD, int G>
 int launch_attn(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
-    constexpr int GB = G <= 4 ? G : 2, NG = (G + GB - 1) / GB;
+    constexpr int GB = heads_a_workgroup(G), NG = (G + GB - 1) / GB;
+    const DieFold die = die_fold(ctx, (long long)a.B * a.kvh * NG, nsplit, chunk, HD);
     // scores [GB][chunk] + partials of every row-subgroup of every wavefront [4 * RPI][GB][HD]
     const size_t front = (size_t)GB * chunk;
     const size_t lds = (front + (size_t)ATT_WAVES * (WAVE / (HD / 8)) * GB * HD) * sizeof(float);
@@ -706,14 +800,14 @@ int launch_attn(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
             lds_limit_raised = true;
         }
         HM_REQUIRE(ctx, lds <= 96 * 1024, "gqa_decode_attn: LDS need %zu too large", lds);
-        hipLaunchKernelGGL((gqa_decode_attn_kernel<HD, GB>), dim3(nsplit, a.kvh * NG, a.B), dim3(ATT_THREADS),
-                           lds, ctx->stream, a.q, const_cast<uint16_t *>(a.kcache),
+        hipLaunchKernelGGL((gqa_decode_attn_kernel<HD, GB>), die.splits ? dim3(homura::die_grid(die.groups, nsplit)) : dim3(nsplit, a.kvh * NG, a.B),
+                           dim3(ATT_THREADS), lds, ctx->stream, a.q, const_cast<uint16_t *>(a.kcache),
                            const_cast<uint16_t *>(a.vcache), a.out, part_o, part_ml, a.kvh, a.max_len,
-                           a.kv_len, chunk, a.scale, a.state, (int)front, f, G);
+                           a.kv_len, chunk, a.scale, a.state, (int)front, f, G, die);
         HM_LAUNCH_CHECK(ctx);
     }
     // nsplit is the grid's split count: 1 means no call can ever need a fold
-    if (nsplit > 1 && a.phase != AttnArgs::SPLIT_ONLY) {
+    if (nsplit > 1 && !die.splits && a.phase != AttnArgs::SPLIT_ONLY) {
         const int rc = launch_fold<HD, G>(ctx, a, part_o, part_ml, nsplit, chunk, a.state);
         if (rc != HM_OK) return rc;
     }
@@ -727,11 +821,12 @@ int launch_attn_stream(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
     float *part_o = a.partials ? a.partials : (float *)ctx->workspace;
     float *part_ml = part_o + pairs * nsplit * G * HD;
     HM_REQUIRE(ctx, chunk % IT_ROWS == 0, "gqa_decode_attn: chunk %d must be a multiple of %d", chunk, IT_ROWS);
-    hipLaunchKernelGGL((gqa_decode_attn_stream_kernel<HD, G>), dim3(nsplit, a.kvh, a.B),
+    const DieFold die = die_fold(ctx, (long long)pairs, nsplit, chunk, HD);
+    hipLaunchKernelGGL((gqa_decode_attn_stream_kernel<HD, G>), die.splits ? dim3(homura::die_grid(die.groups, nsplit)) : dim3(nsplit, a.kvh, a.B),
                        dim3(ATT_THREADS), 0, ctx->stream, a.q, a.kcache, a.vcache, a.out, part_o,
-                       part_ml, a.kvh, a.max_len, a.kv_len, chunk, a.scale);
+                       part_ml, a.kvh, a.max_len, a.kv_len, chunk, a.scale, die);
     HM_LAUNCH_CHECK(ctx);
-    if (nsplit > 1) {
+    if (nsplit > 1 && !die.splits) {
         const int rc = launch_fold<HD, G>(ctx, a, part_o, part_ml, nsplit, chunk, (const DecodeState *)nullptr);
         if (rc != HM_OK) return rc;
     }
@@ -781,6 +876,12 @@ int gqa_attn_fixed_scratch_setup(hm_ctx *ctx) {
     HM_REQUIRE(ctx, p != nullptr, "gqa_decode_attn: the fixed partials array has no device address");
     ctx->attn_fixed_scratch = p;
     return HM_OK;
+}
+
+bool gqa_decode_attn_folds(const hm_ctx *ctx, int H, int kvh, int hd, int span, int chunk) {
+    const int g = H / kvh, gb = heads_a_workgroup(g), nsplit = (span + chunk - 1) / chunk;
+    const long long groups = (long long)kvh * ((g + gb - 1) / gb);
+    return nsplit > 1 && !homura::die_fold_pays(ctx, groups, nsplit, 4.0 * groups * nsplit * chunk * hd);
 }
 
 int gqa_decode_attn_launch(hm_ctx *ctx, const AttnArgs &a) {

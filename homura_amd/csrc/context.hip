@@ -23,6 +23,28 @@ int hm_set_error(hm_ctx *ctx, int code, const char *fmt, ...) {
     return code;
 }
 
+__global__ void note_die_kernel(unsigned int *die) {
+    if (threadIdx.x == 0) die[blockIdx.x] = __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 0xF;
+}
+
+// Grids of a few sizes, so that they begin on different dies: every workgroup where the one eight ids before it was.
+// HOMURA_FOLD_LAUNCH=1: not looked at, folds are launches of their own (for comparisons).
+static bool find_dies_round_robin(hm_ctx *ctx) {
+    const char *e = std::getenv("HOMURA_FOLD_LAUNCH");
+    if (e && std::atoi(e) != 0) return false;
+    unsigned int die[1024];
+    unsigned int *d_die = static_cast<unsigned int *>(ctx->workspace);
+    for (int n : {1024, 259, 1021}) {
+        hipLaunchKernelGGL(note_die_kernel, dim3(n), dim3(64), 0, ctx->stream, d_die);
+        if (hipGetLastError() != hipSuccess || hipMemcpyAsync(die, d_die, (size_t)n * 4, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+            hipStreamSynchronize(ctx->stream) != hipSuccess)
+            return false;
+        for (int i = 8; i < n; i++)
+            if (die[i] != die[i - 8]) return false;
+    }
+    return true;
+}
+
 extern "C" {
 
 const char *hm_version(void) { return "homura_amd 0.1 (gfx950)"; }
@@ -58,7 +80,7 @@ hm_ctx *hm_init(int device) {
         return nullptr;
     }
     ctx->workspace_bytes = (size_t)64 << 20;
-    ctx->num_counters = 4096;
+    ctx->num_counters = 1 << 16;
     if (hipMalloc(&ctx->workspace, ctx->workspace_bytes) != hipSuccess ||
         hipMalloc((void **)&ctx->counters, ctx->num_counters * sizeof(unsigned int)) !=
             hipSuccess) {
@@ -68,6 +90,7 @@ hm_ctx *hm_init(int device) {
     }
     (void)hipMemsetAsync(ctx->counters, 0, ctx->num_counters * sizeof(unsigned int), ctx->stream);
     (void)hipStreamSynchronize(ctx->stream);
+    ctx->dies_round_robin = find_dies_round_robin(ctx);
     if (gqa_attn_fixed_scratch_setup(ctx) != HM_OK) {
         hm_set_error(nullptr, HM_ERR_HIP, "%s", ctx->last_error.c_str());
         hm_destroy(ctx);

@@ -18,9 +18,11 @@ struct hm_ctx {
     // Workspace for kernels that need partial results (split-K / split-KV); allocated once.
     void *workspace = nullptr;
     size_t workspace_bytes = 0;
-    // 4-byte counters used by "last workgroup finishes" reductions; always left at zero.
+    // 4-byte counters used by "last workgroup finishes" reductions (die_fold.h); always left at zero.
     unsigned int *counters = nullptr;
     size_t num_counters = 0;
+    // Workgroups whose ids are equal modulo eight run on one accelerator die (found by running some when the context is made).
+    bool dies_round_robin = false;
     // Device address, on this context's device, of the fixed array behind hm_gqa_decode_attn_noalloc.
     void *attn_fixed_scratch = nullptr;
     std::string last_error;

@@ -46,10 +46,21 @@ namespace {
 // of it holds in registers
 constexpr int ATTN_UNSPLIT = 128;
 
-// Live rows from which that attention's grid has splits to fold: its span is min(ATTN_UNSPLIT, max_len) rows up to ATTN_UNSPLIT of them,
-// in chunks of `chunk`, and more than one chunk beyond.
-int fold_from_rows(int chunk, int max_len) {
-    return std::min(ATTN_UNSPLIT, max_len) > chunk ? 0 : ATTN_UNSPLIT + 1;
+// Rows that attention's grid covers for `live` of them, and the rows of a split (`fixed` of them if not 0)
+int attn_span_for(int live, int max_len) {
+    int span = live <= ATTN_UNSPLIT ? ATTN_UNSPLIT : 2048;
+    while (span < live && span < max_len) span *= 2;
+    return std::min(span, max_len);
+}
+int attn_chunk_for(int span, int fixed) { return fixed ? fixed : span > ATTN_UNSPLIT && span <= 2048 ? 64 : 128; }
+
+// Live rows from which that attention has a fold in a launch of its own
+int fold_from_rows(const hm_ctx *ctx, int H, int kvh, int hd, int fixed, int max_len) {
+    for (int from = 0, span = 0; span < max_len; from = span + 1) {
+        span = attn_span_for(from, max_len);
+        if (gqa_decode_attn_folds(ctx, H, kvh, hd, span, attn_chunk_for(span, fixed))) return from;
+    }
+    return max_len + 1;
 }
 
 // HOMURA_WHOLE_STEP_FAR=1 (read when the plan is built): the whole-step kernel takes every exchange through
@@ -552,9 +563,7 @@ int HfModel::finalize(int max_seq_len) {
             if (rc == HM_OK) rc = refresh_fused_table();
         }
         if (rc == HM_OK && !plan_->whole_step()) {
-            int span = live <= ATTN_UNSPLIT ? ATTN_UNSPLIT : 2048;
-            while (span < live && span < max_seq_len_) span *= 2;
-            plan_->set_attn_span(std::min(span, max_seq_len_));
+            plan_->set_attn_span(attn_span_for(live, max_seq_len_));
         }
         return rc;
     });
@@ -661,13 +670,12 @@ int HfModel::emit_transformer_plan() {
     // attention split: rows per workgroup (kept in registers); HOMURA_ATT_CHUNK overrides
     // rows per attention split: 64 while the grid covers 2048 rows, 128 beyond (measured on 2 and 32 KV heads:
     // 1 % slower at 1024 rows, 13 % faster at 30000); HOMURA_ATT_CHUNK fixes it
-    int att_chunk = 64;
-    bool att_chunk_fixed = false;
+    int att_chunk = 64, att_chunk_fixed = 0;
     if (const char *e = std::getenv("HOMURA_ATT_CHUNK")) {
         att_chunk = std::min(128, std::max(32, std::atoi(e) / 32 * 32));
-        att_chunk_fixed = true;
+        att_chunk_fixed = att_chunk;
     }
-    const int fold_from = fold_from_rows(att_chunk_fixed ? att_chunk : ATTN_UNSPLIT, max_seq_len_);
+    const int fold_from = fold_from_rows(ctx_, (int)H, (int)kvh, (int)hd, att_chunk_fixed, max_seq_len_);
 
     std::shared_ptr<PlanScratch> scr = scratch_;
     std::vector<CompiledKernel> kernels;
@@ -828,7 +836,7 @@ int HfModel::emit_transformer_plan() {
                 a.scale = (float)(1.0 / std::sqrt((double)hd));  // f64 -> f32 constant, emitter.rs:719
                 a.state = sc.plan->state();
                 a.span = sc.plan->attn_span();
-                a.fixed_chunk = att_chunk_fixed || (a.span > ATTN_UNSPLIT && a.span <= 2048) ? att_chunk : 128;
+                a.fixed_chunk = attn_chunk_for(a.span, att_chunk_fixed);
                 a.phase = phase;
                 return a;
             };
@@ -1082,13 +1090,12 @@ int HfModel::emit_transformer_plan_quant() {
 
     // rows per attention split: 64 while the grid covers 2048 rows, 128 beyond (measured on 2 and 32 KV heads:
     // 1 % slower at 1024 rows, 13 % faster at 30000); HOMURA_ATT_CHUNK fixes it
-    int att_chunk = 64;
-    bool att_chunk_fixed = false;
+    int att_chunk = 64, att_chunk_fixed = 0;
     if (const char *e = std::getenv("HOMURA_ATT_CHUNK")) {
         att_chunk = std::min(128, std::max(32, std::atoi(e) / 32 * 32));
-        att_chunk_fixed = true;
+        att_chunk_fixed = att_chunk;
     }
-    const int fold_from = fold_from_rows(att_chunk_fixed ? att_chunk : ATTN_UNSPLIT, max_seq_len_);
+    const int fold_from = fold_from_rows(ctx_, (int)H, (int)kvh, (int)hd, att_chunk_fixed, max_seq_len_);
 
     std::shared_ptr<PlanScratch> scr = scratch_;
     std::vector<CompiledKernel> kernels;
@@ -1444,7 +1451,7 @@ int HfModel::emit_transformer_plan_quant() {
                 a.scale = (float)(1.0 / std::sqrt((double)hd));
                 a.state = sc.plan->state();
                 a.span = sc.plan->attn_span();
-                a.fixed_chunk = att_chunk_fixed || (a.span > ATTN_UNSPLIT && a.span <= 2048) ? att_chunk : 128;
+                a.fixed_chunk = attn_chunk_for(a.span, att_chunk_fixed);
                 a.phase = phase;
                 return a;
             };

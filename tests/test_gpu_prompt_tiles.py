@@ -1,4 +1,5 @@
 """Tiles of the prompt pass's matrix products at the sizes where their choice turns (GPU)."""
+import ctypes as C
 import dataclasses
 
 import numpy as np
@@ -335,3 +336,46 @@ def test_fold_keeps_an_infinite_value(ctx, H, kvh, hd, kv_len):
     assert np.all(got[:, 5] == np.inf) and np.all(np.isfinite(np.delete(got, 5, 1)))
     for buf in (dq, dk, dv, do):
         buf.free()
+
+
+# Groups of splits that sit on one die each: one to eight heads of a workgroup (four, two or one share of the splits a thread), two to
+# thirty-two splits, four groups and as many as the dies hold, both kernels; and the same through a fold in a launch of its own
+@pytest.mark.parametrize("B,H,kvh,hd,kv_len", [(4, 1, 1, 64, 65), (1, 32, 32, 64, 500), (4, 4, 1, 128, 600), (8, 3, 1, 128, 2047), (1, 16, 8, 128, 1000),
+                                               (8, 12, 2, 128, 4096), (8, 14, 2, 64, 5000), (4, 64, 8, 128, 4001), (16, 5, 1, 64, 4096),
+                                               (6, 14, 2, 64, 777)])
+def test_splits_folded_on_their_die(ctx, monkeypatch, B, H, kvh, hd, kv_len):
+    """Eager twice and replayed three times (the arrivals are counted anew every time), with other work between. A softmax over f32 sums:
+    2^-20 of the largest value holds a few thousand additions, and the long caches' two-piece operands 2^-17 of their terms."""
+    rng = np.random.default_rng(kv_len + H)
+    q = rng.standard_normal((B, H, hd)).astype(np.float32)
+    k, v = (synth.f32_to_bf16_rne(rng.standard_normal((B, kvh, kv_len, hd)).astype(np.float32)) for _ in range(2))
+    k64, v64 = (np.repeat(synth.bf16_to_f32(x).astype(np.float64), H // kvh, 1) for x in (k, v))
+    s = np.einsum("bhnd,bhd->bhn", k64, q.astype(np.float64)) * hd ** -0.5
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = np.einsum("bhn,bhnd->bhd", p / p.sum(-1, keepdims=True), v64)
+    monkeypatch.setenv("HOMURA_FOLD_LAUNCH", "1")
+    apart = type(ctx)(0)
+    got = []
+    for c in (ctx, apart):
+        dq, dk, dv, do, other = c.to_device(q), c.to_device(k), c.to_device(v), c.empty(B * H * hd), c.empty(256 * hd)
+        call = lambda out: c.gqa_decode_attn(dq, dk, dv, out, B, H, kvh, hd, kv_len, kv_len, hd ** -0.5)
+        for _ in range(2):
+            call(do)
+        got.append(do.download(np.float32, (B, H, hd)))
+        graph = C.c_void_p()
+        c._check(c.lib.hm_graph_begin(c.h))
+        call(do)
+        c.gqa_decode_attn(dq, dk, dv, other, 1, H // kvh, 1, hd, kv_len, min(kv_len, 300), hd ** -0.5)
+        c._check(c.lib.hm_graph_end(c.h, C.byref(graph)))
+        for _ in range(3):
+            c._check(c.lib.hm_fill_zero(c.h, do.ptr, B * H * hd * 4))
+            c._check(c.lib.hm_graph_launch(c.h, graph, 1))
+            assert np.array_equal(do.download(np.float32, (B, H, hd)), got[-1])
+            c.gqa_decode_attn(dq, dk, dv, other, 1, H // kvh, 1, hd, kv_len, kv_len, hd ** -0.5)
+        c._check(c.lib.hm_graph_destroy(c.h, graph))
+        for buf in (dq, dk, dv, do, other):
+            buf.free()
+    apart.close()
+    for out in got:
+        assert np.abs(out - want).max() <= 2.0 ** -17 * np.abs(v64).max()
+    assert np.abs(got[0] - got[1]).max() <= 2.0 ** -21 * np.abs(v64).max()
