@@ -66,11 +66,16 @@ int gemm_pieces_scaled_nk(hm_ctx *ctx, const uint16_t *d_a_split, const uint16_t
 // gated (gate_scale with it): neighbouring columns are (gate, up) pairs, and silu(gate) up times gate_scale [N / 2] leaves as two f16
 // pieces, gated [M][2 (N / 2)], instead of d_c: one slice, N % 2 == 0. gemm_half_gated_pays: whether that is the quicker way, or slices and
 // silu_mul_half_launch behind them.
+// tail (with head_dim 64 or 128): the product is a q|k|v projection of M = tail->S rows, and its workgroups hand their head rows on as
+// qkv_post_launch does: q [M][N] at tail->qkv, k and v in the caches, nothing to d_c. One slice. gemm_half_tail_pays as above.
+struct QkvPostArgs;
 struct HalfProduct {
     const float *unscale;
     const float *gate_scale = nullptr;
     uint16_t *gated = nullptr;
+    const QkvPostArgs *tail = nullptr;
 };
+bool gemm_half_tail_pays(bool scaled, int head_dim, int M, int K, int N, int cus, int max_parts);
 bool gemm_half_gated_pays(bool scaled, int M, int K, int N, int cus, int max_parts);
 int gemm_half_nk(hm_ctx *ctx, const uint16_t *d_a_half, const uint16_t *d_b_half, const HalfProduct &half, const float *d_scales,
                  int npad, float *d_c, int M, int K, int N, int max_parts = 1, int *parts = nullptr);
@@ -81,6 +86,10 @@ int gemm_half_wide(hm_ctx *ctx, const uint16_t *d_a_half, const uint16_t *d_b_ha
 // gemm_tiles_square: its choice is one slice of 128 x 128 tiles, which gemm_dma_kernel (gemm_bf16_mfma.hip) multiplies faster
 bool gemm_tiles_square(int M, int K, int N, int cus, int max_parts);
 int gemm_tiles_bf16(hm_ctx *ctx, const uint16_t *d_a, const uint16_t *d_b_nk, float *d_c, int M, int K, int N, int max_parts, int *parts);
+// The gate|up product of one bf16 piece with its activation: act(gate, up) of neighbouring columns as bf16, d_out [M][N / 2]; K % 64 == 0.
+// gemm_gated_pays: whether that is the quicker way (not where the few-rows kernel multiplies).
+int gemm_gated_nk(hm_ctx *ctx, const uint16_t *d_a, const uint16_t *d_b_nk, uint16_t *d_out, int M, int K, int N, const GatedAct &act);
+bool gemm_gated_pays(int M, int K, int N, int cus, int max_parts);
 int gemm_half_slices(bool scaled, int M, int K, int N, int cus, int max_parts);
 // The K slices that a product of activation pieces with b_pieces (1 or 3) pieces of B, or with a block-scaled B, comes in
 int gemm_pieces_slices(int b_pieces, bool scaled, int M, int K, int N, int cus, int max_parts);

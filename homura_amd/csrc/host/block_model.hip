@@ -1484,6 +1484,10 @@ int BlockModel::prefill_feed_forward(int layer, int n, int *y_parts) {
     g.width = ff;
     g.out_split = sb;
     if (!s.experts) {
+        if (np == 1 && gemm_gated_pays(n, wp, 2 * ff, ctx_->num_cus, MP)) {
+            if ((rc = gemm_gated_nk(ctx_, sa, l.gate_up.ptr(), sb, n, wp, 2 * ff, s.act)) != HM_OK) return rc;
+            return gemm_split_nk(ctx_, sb, np, l.down.ptr(), y, n, ff, wp, MP, y_parts);
+        }
         if ((rc = gemm_split_nk(ctx_, sa, np, l.gate_up.ptr(), d1, n, wp, 2 * ff, MP, &parts)) != HM_OK) return rc;
         if (s.act.kind == GatedAct::Silu) {
             rc = silu_mul_split_launch(ctx_, d1, parts, sb, np, n, ff);

@@ -2362,7 +2362,8 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     const Buffer *i8 = nullptr;  // the planes of the group about to be multiplied, if it takes that path
     int8_t *q8 = p.q8 ? p.q8.as<int8_t>() : nullptr;
     float *q8s = p.q8s ? p.q8s.as<float>() : nullptr;
-    auto project = [&](int l, int first, int count, const Buffer &packed, int K, float *out, const uint16_t *rows, uint16_t *gated) -> int {
+    auto project = [&](int l, int first, int count, const Buffer &packed, int K, float *out, const uint16_t *rows, uint16_t *gated,
+                       const QkvPostArgs *tail = nullptr) -> int {
         int N = 0;
         for (int j = first; j < first + count; j++) N += proj_n[j];
         if (const int g = first == 0 ? 0 : first == 3 ? 1 : first == 4 ? 2 : 3; half(l, g)) {
@@ -2376,6 +2377,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
                 hp.gate_scale = half_[l].gated.as<float>();
                 hp.gated = gated;
             }
+            hp.tail = tail;
             return gemm_half_nk(ctx_, rows, reinterpret_cast<const uint16_t *>(w), hp, quant ? f : nullptr, quant ? half_scale_cols(N) : 0, out, n, K,
                                 N, MP, &parts);
         }
@@ -2444,12 +2446,8 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         rc = rmsnorm_split_launch(ctx_, x, res, res_parts, h0 ? half_[l].norms.as<float>() : weight_f32(pre + "input_layernorm.weight"), split,
                                   h0 ? 2 : np, res ? h : nullptr, n, hidden, eps, q8k(l, 0), q8k(l, 0) ? capture_at(l, 0) : nullptr,
                                   i8 ? q8 : nullptr, i8 ? q8s : nullptr, h0, res_scale);
-        if (rc == HM_OK) rc = project(l, 0, 3, lp.qkv, hidden, qkv, split, nullptr);
-        if (rc != HM_OK) return rc;
         QkvPostArgs qa;
         qa.qkv = qkv;
-        qa.parts = parts;
-        qa.part_stride = (size_t)n * nqkv;
         qa.bias = lp.qkv_bias ? lp.qkv_bias.as<float>() : nullptr;
         if (has_qk_norm_) {
             qa.qw = weight_f32(pre + "self_attn.q_norm.weight");
@@ -2466,7 +2464,12 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         qa.max_len = kv->max_len();
         qa.past = past;
         qa.eps = eps;
-        if ((rc = qkv_post_launch(ctx_, qa)) != HM_OK) return rc;
+        const bool tail = h0 && gemm_half_tail_pays(quant, hd, n, hidden, nqkv, ctx_->num_cus, MP);  // the product's workgroups do the rest
+        if (rc == HM_OK) rc = project(l, 0, 3, lp.qkv, hidden, qkv, split, nullptr, tail ? &qa : nullptr);
+        qa.parts = parts;
+        qa.part_stride = (size_t)n * nqkv;
+        if (rc == HM_OK && !tail) rc = qkv_post_launch(ctx_, qa);
+        if (rc != HM_OK) return rc;
         // Without logits nobody reads the hidden state behind the last layer: its cache rows are all that a chunk leaves. (512 tokens
         // of the Qwen3-0.6B shape and the step behind them 3.41 -> 3.33 ms; what a test captures wants the rest as well.)
         if (l + 1 == c.num_hidden_layers && !h_logits && !p.capture) break;

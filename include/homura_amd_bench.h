@@ -79,6 +79,18 @@ int hm_test_prompt_rows(hm_ctx *ctx, int front, const void *x, const float *norm
 int hm_test_gated_rows(hm_ctx *ctx, const void *x, const float *norm_w, int dtype, const void *w, int fused, int m, int k, int inter,
                        uint16_t *out, float *scale, int *pays);
 
+/* Test support: the q|k|v projection of the prompt pass in f16 pieces and its tail: x [S][k] f32 through RMSNorm (norm_w [k], eps), w
+ * [(H + 2 kvh) hd][k] bf16 rows or Q8_0 / Q4_0 blocks; bias, and qw with kw, may be NULL. fused 1: the product's workgroups do the tail, 0: its slices go
+ * through the row kernel. q [S][(H + 2 kvh) hd] (its q columns), caches [kvh][max_len][hd] rows past .. *pays: what the prompt pass would take. */
+int hm_test_qkv_product(hm_ctx *ctx, const void *x, const float *norm_w, int dtype, const void *w, int fused, int S, int k, int H, int kvh, int hd,
+                        const float *bias, const float *qw, const float *kw, const float *cos, const float *sin, float *q, uint16_t *kcache,
+                        uint16_t *vcache, int max_len, int past, float eps, int *pays);
+
+/* Test support: a gate|up product of one bf16 piece with its activation, a [m][k], b [n][k] as (gate, up) pairs of rows, out [m][n / 2] bf16; kind 0
+ * silu(g) u, 1 the clamped sigmoid gate. *pays: whether the prompt pass of a list-of-layers model would take it. */
+int hm_test_gated_product(hm_ctx *ctx, const uint16_t *a, const uint16_t *b, uint16_t *out, int m, int k, int n, int kind, float limit, float slope,
+                          int *pays);
+
 /* Test support: the bytes of f16 weight copies that a transformer's prompt pass holds, and how many of its groups of projections
  * (q|k|v, o, gate|up, down of every layer) multiply with them. */
 int hm_test_prefill_f16_copies(hm_model *m, size_t *bytes, int *groups);

@@ -365,3 +365,84 @@ def test_down_weights_that_column_factors_would_round(ctx):
         last = gm.run_kv([int(t)])
     assert np.linalg.norm(at_once - np.asarray(last).reshape(-1)) <= 2e-3 * np.linalg.norm(last)
     gm.close()
+
+
+# every tile of one bf16 piece in one slice, rows and pairs of columns off its size
+@pytest.mark.parametrize("tile,m,k,n", [((64, 64), 65, 192, 74), ((64, 128), 513, 1024, 3078), ((64, 192), 700, 128, 4106), ((128, 128), 1000, 1024, 3082),
+                                        ((128, 192), 1300, 192, 3402), ((128, 256), 1905, 1024, 4106), ((128, 192), 2047, 1024, 6144)])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_gated_product_of_one_bf16_piece(ctx, kind, tile, m, k, n):
+    """gate and up as above (4e-7 of the norms' product, single values five times that), either activation's slope below 2, and bf16's rounding."""
+    from homura_amd import _ffi
+    tm, tn, sl = C.c_int(), C.c_int(), C.c_int()
+    assert _ffi.load().hm_test_product_tiles(2, m, k, n, 256, 1, C.byref(tm), C.byref(tn), C.byref(sl)) == 0
+    assert (tm.value, tn.value, sl.value) == (*tile, 1)
+    rng = np.random.default_rng(m + k + n)
+    a, av = bf16(rng.standard_normal((m, k)).astype(np.float32))
+    b, bv = bf16(rng.standard_normal((n, k)).astype(np.float32) * k ** -0.5)
+    guard, limit, slope, pays = 256, 1.2, 1.702, C.c_int()
+    da, db, out = ctx.to_device(a), ctx.to_device(b), ctx.to_device(np.full(m * n // 2 + guard, 0x7B7B, np.uint16))
+    ctx._check(ctx.lib.hm_test_gated_product(ctx.h, da.ptr, db.ptr, out.ptr, m, k, n, kind, limit, slope, C.byref(pays)))
+    got = out.download(np.uint16, (m * n // 2 + guard,))
+    for buf in (da, db, out):
+        buf.free()
+    assert np.all(got[m * n // 2:] == 0x7B7B), "wrote past the end"
+    got = (got[:m * n // 2].astype(np.uint32) << 16).view(np.float32).reshape(m, n // 2).astype(np.float64)
+    gu = av.astype(np.float64) @ bv.T.astype(np.float64)
+    g, u = gu[:, 0::2], gu[:, 1::2]
+    off = 2e-6 * np.linalg.norm(av, axis=1)[:, None] * np.linalg.norm(bv, axis=1).max()
+    if kind:
+        g, u = np.minimum(g, limit), np.clip(u, -limit, limit) + 1
+    s = g / (1 + np.exp(-(slope if kind else 1) * g))
+    assert np.all(np.abs(got - s * u) <= 2.0 ** -8 * np.abs(s * u) + 2 * off * (np.abs(u) + np.abs(s) + off))
+
+
+# the tiles that hold whole heads (64 x 64, 64 x 128, 64 x 192, 128 x 128, 128 x 256), ragged rows, heads that end inside a tile, rows already cached
+@pytest.mark.parametrize("S,k,H,kvh,hd,past", [(65, 64, 2, 1, 64, 0), (70, 896, 14, 2, 64, 3), (200, 320, 14, 2, 64, 0), (333, 1024, 32, 4, 64, 5),
+                                               (700, 128, 32, 4, 64, 0), (130, 192, 3, 1, 128, 1), (511, 1024, 16, 8, 128, 0), (999, 192, 16, 8, 128, 7),
+                                               (1905, 128, 16, 8, 128, 0), (1905, 128, 32, 16, 64, 2), (2049, 128, 32, 16, 64, 0)])
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_Q8_0])
+def test_qkv_tail_from_the_product(ctx, dtype, S, k, H, kvh, hd, past):
+    """Against float64 (the bound as above, on what the norm and the rotation make of it), and against the row kernel's: a rounding of the
+    projection at most, so k and v are the same bf16 or its neighbour. Rows of the caches outside the chunk stay what they were."""
+    print(f"dtype {dtype} {S} x {k}, {H} + 2 x {kvh} heads of {hd}", flush=True)
+    rng = np.random.default_rng(S + k + H)
+    n, max_len = (H + 2 * kvh) * hd, past + S + 3
+    normed, biased = k != 896, k == 896
+    x = rng.standard_normal((S, k)).astype(np.float32)
+    norm_w = (1 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    raw, w = weights(dtype, n, k, rng)
+    bias = rng.standard_normal(n).astype(np.float32) if biased else np.zeros(n, np.float32)
+    qw, kw = (1 + 0.1 * rng.standard_normal((2, hd))).astype(np.float32)
+    cos, sin = rng.standard_normal((2, max_len, hd)).astype(np.float32)
+    rows = (rows_of(0, x, norm_w) @ w.T.astype(np.float64) + bias).reshape(S, H + 2 * kvh, hd)
+    turned = rows[:, :H + kvh]
+    if normed:
+        scale = np.where(np.arange(H + kvh)[:, None] < H, qw, kw)
+        turned = turned / np.sqrt((turned ** 2).mean(-1, keepdims=True) + EPS) * scale
+    c, s = (t[past:past + S, None].astype(np.float64) for t in (cos, sin))
+    swapped = np.concatenate([-turned[..., hd // 2:], turned[..., :hd // 2]], -1)
+    want = np.concatenate([turned * c + swapped * s, rows[:, H + kvh:]], 1)
+    dev = [ctx.to_device(v) for v in (x, norm_w, raw, bias, qw, kw, cos, sin)]
+    got = []
+    for fused in (1, 0):
+        q, pays = ctx.to_device(np.full(S * n + 64, -77.0, np.float32)), C.c_int()
+        kc, vc = (ctx.to_device(np.full(kvh * max_len * hd, 0x7B7B, np.uint16)) for _ in range(2))
+        ctx._check(ctx.lib.hm_test_qkv_product(ctx.h, dev[0].ptr, dev[1].ptr, dtype, dev[2].ptr, fused, S, k, H, kvh, hd, dev[3].ptr if biased else None,
+                                               *((dev[4].ptr, dev[5].ptr) if normed else (None, None)), dev[6].ptr, dev[7].ptr, q.ptr, kc.ptr, vc.ptr,
+                                               max_len, past, EPS, C.byref(pays)))
+        flat = q.download(np.float32, (S * n + 64,))
+        assert np.all(flat[S * n:] == -77.0)
+        cache = [b.download(np.uint16, (kvh, max_len, hd)) for b in (kc, vc)]
+        for b in cache:
+            assert np.all(b[:, :past] == 0x7B7B) and np.all(b[:, past + S:] == 0x7B7B)
+        kv = [(b[:, past:past + S].astype(np.uint32) << 16).view(np.float32).transpose(1, 0, 2).astype(np.float64) for b in cache]
+        got.append([flat[:S * n].reshape(S, -1, hd)[:, :H].astype(np.float64), *kv])
+        for b in (q, kc, vc):
+            b.free()
+    for b in dev:
+        b.free()
+    for mine, his, ref in zip(got[0], got[1], (want[:, :H], want[:, H:H + kvh], want[:, H + kvh:])):
+        assert np.linalg.norm(mine - ref) <= (8e-7 if mine.shape[1] == H and mine is got[0][0] else 2.0 ** -8) * np.linalg.norm(ref)
+        assert np.all(np.abs(mine - his) <= 2.0 ** -7 * np.abs(his) + 4e-6 * np.sqrt((ref ** 2).mean()))
+    assert np.linalg.norm(got[0][0] - got[1][0]) <= 8e-7 * np.linalg.norm(got[1][0])
