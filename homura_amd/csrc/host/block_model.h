@@ -161,7 +161,7 @@ class BlockModel : public DecoderModel {
     int upload_matrix(const Target &t, const uint16_t *h_nk);
     int upload_vector(const Target &t, const float *h);
     int step_inputs(std::vector<Buffer *> &inputs) override;
-    int prefill_chunk(const int32_t *h_ids, int n, float *h_logits) override;
+    int prefill_chunk(const int32_t *d_ids, int n, float *h_logits) override;
     const char *prefill_needs() const override;
     int mark_position() override;
     int rewind_to_mark(int mark_len, const std::vector<int32_t> &kept) override;
@@ -201,7 +201,7 @@ class BlockModel : public DecoderModel {
     struct PrefillScratch {
         static constexpr int MAX_PARTS = 8;
         int rows = 0;
-        Buffer ids, x, x0, y, d1, d2, d3, f1, f2, f3, split_a, split_b, lat, kvf, kws, vws, logits;
+        Buffer x, x0, y, d1, d2, d3, f1, f2, f3, split_a, split_b, lat, kvf, kws, vws, logits;
         Buffer mm_q, mm_k, mm_values, mm_ahead, mm_gates, mm_log_w, mm_weights, mm_decay;                 // matrix memory
         Buffer choice, choice_weight, expert_list, expert_count;           // mixture of experts
         Buffer captured;

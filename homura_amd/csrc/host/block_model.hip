@@ -1191,7 +1191,7 @@ int BlockModel::prepare_prefill() {
         b = Buffer::alloc(ctx_, {(n + 1) / 2 * 2}, t);
         return b && hm_fill_zero(ctx_, b.ptr(), b.bytes()) == HM_OK;
     };
-    const bool ok = make(p.ids, rows, DType::F32) && make(p.x, rows * wp_, DType::F32) && make(p.x0, rows * wp_, DType::F32) &&
+    const bool ok = make(p.x, rows * wp_, DType::F32) && make(p.x0, rows * wp_, DType::F32) &&
                     make(p.y, std::max(sliced(wp_), rows * top * wp_), DType::F32) && make(p.d1, sliced(d1), DType::F32) && make(p.d2, sliced(d2), DType::F32) &&
                     make(p.d3, sliced(d3), DType::F32) && make(p.f1, rows * f1, DType::F32) && make(p.f2, rows * f2, DType::F32) && make(p.f3, rows * f3, DType::F32) &&
                     make(p.split_a, rows * 3 * split, DType::BF16) && make(p.split_b, rows * 3 * split, DType::BF16) && make(p.lat, lat, DType::BF16) &&
@@ -1531,7 +1531,7 @@ int BlockModel::prefill_feed_forward(int layer, int n, int *y_parts) {
     return rc;
 }
 
-int BlockModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
+int BlockModel::prefill_chunk(const int32_t *d_ids, int n, float *h_logits) {
     int rc = prepare_prefill();
     if (rc != HM_OK) return rc;
     PrefillScratch &p = pf_;
@@ -1540,8 +1540,7 @@ int BlockModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     const size_t row_floats = (size_t)n * wp;
     float *x = p.x.as<float>(), *x0 = p.x0.as<float>(), *y = p.y.as<float>(), *d1 = p.d1.as<float>();
     uint16_t *sa = p.split_a.as<uint16_t>();
-    if ((rc = hm_upload(ctx_, p.ids.ptr(), h_ids, (size_t)n * 4)) != HM_OK) return rc;
-    if ((rc = embed_scaled_launch(ctx_, p.ids.as<int32_t>(), embed_.ptr(), x, n, cfg_.vocab, wp, (float)cfg_.embed_scale, waves(), past)) != HM_OK) return rc;
+    if ((rc = embed_scaled_launch(ctx_, d_ids, embed_.ptr(), x, n, cfg_.vocab, wp, (float)cfg_.embed_scale, waves(), past)) != HM_OK) return rc;
     if (cfg_.loop_times && (rc = hm_copy(ctx_, x0, x, row_floats * 4)) != HM_OK) return rc;
     // x [+ norm_b(y)] -> x, and through norm_w (or as it is, with x0 behind it) into split_a
     const Vec *pending = nullptr;

@@ -80,12 +80,13 @@ class DecoderModel {
 
   protected:
     DecoderModel() = default;
-    // One chunk of the prompt pass (n <= prefill_chunk_rows() ids, host pointer): appends n rows to the cache.
-    virtual int prefill_chunk(const int32_t *h_ids, int n, float *h_logits) = 0;
+    // One chunk of the prompt pass (n <= prefill_chunk_rows() ids, in memory that the device reads): appends n rows to the cache.
+    virtual int prefill_chunk(const int32_t *d_ids, int n, float *h_logits) = 0;
     virtual const char *prefill_needs() const = 0;  // for the error message when the pass is not available
     virtual int step_inputs(std::vector<Buffer *> &inputs) = 0;
-    // End of a call: stream synchronisation and whatever the steps left to be looked at.
-    virtual int finish_sync() { return hm_sync(ctx_); }
+    // End of a call: stream synchronisation and whatever the steps left to be looked at. With words, first that many 4-byte words from d_src
+    // to pinned h_dst.
+    virtual int finish_sync(void *h_dst = nullptr, const void *d_src = nullptr, size_t words = 0);
     // Runs the body of a call; a model whose steps can fail recoverably runs it again.
     virtual int guarded(const std::function<int()> &body) { return body(); }
     // 64 bytes of device status words to fetch with the logits row of a step (NULL: nothing to look at), and
@@ -98,6 +99,18 @@ class DecoderModel {
     virtual int mark_position() { return HM_OK; }
     virtual int rewind_to_mark(int mark_len, const std::vector<int32_t> &kept);
     int check_ids(const int64_t *ids, int n, std::vector<int32_t> &out);
+
+    // Pinned host memory that kernels read and write: of run_kv, a logits row and the status words, which arrive with one
+    // synchronisation; a prompt's ids; a generation's draws and tokens. Every call synchronises before it returns, or before it uses a
+    // block again.
+    struct Pinned {
+        void *p = nullptr;
+        size_t bytes = 0;
+        template <class T>
+        T *as() const { return static_cast<T *>(p); }
+    };
+    int pinned_for(Pinned &b, size_t bytes);
+    Pinned stage_, prompt_ids_, draws_, tokens_;
 
     hm_ctx *ctx_ = nullptr;
     bool finalized_ = false;
@@ -122,9 +135,8 @@ class DecoderModel {
     int generate_once(const int64_t *h_prompt, int n_prompt, int max_new, const hm_sampling_config &cfg, uint64_t seed,
                       int eos_token, int32_t *h_tokens, int *n_out);
     int bench_decode_once(int64_t first_id, int n_steps, float *ms_out, int32_t *h_tokens);
-    // pinned host staging of run_kv: a logits row and the status words arrive with one synchronisation
-    void *h_stage_ = nullptr;
-    size_t h_stage_bytes_ = 0;
+    // The prompt pass without the synchronisation at its end, for calls that go on
+    int prefill_enqueue(const int64_t *h_ids, int n_ids, float *h_logits);
     struct SamplerScratch { Buffer work, counts, token, list, draws; int list_cap = 0, draws_cap = 0; } sampler_;
 };
 

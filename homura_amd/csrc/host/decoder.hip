@@ -4,11 +4,36 @@
 #include <algorithm>
 #include <cstring>
 
+#include "../light_ops.h"
+
 namespace homura {
 
 DecoderModel::~DecoderModel() {
     if (ctx_) hm_sync(ctx_);
-    if (h_stage_) (void)hipHostFree(h_stage_);
+    for (Pinned *b : {&stage_, &prompt_ids_, &draws_, &tokens_})
+        if (b->p) (void)hipHostFree(b->p);
+}
+
+// At least `bytes` of pinned memory. A larger block takes the place of one that the stream may still be reading.
+int DecoderModel::pinned_for(Pinned &b, size_t bytes) {
+    if (b.bytes >= bytes) return HM_OK;
+    if (b.p) {
+        const int rc = hm_sync(ctx_);
+        (void)hipHostFree(b.p);
+        b = Pinned{};
+        if (rc != HM_OK) return rc;
+    }
+    size_t size = 4096;
+    while (size < bytes) size *= 2;
+    HM_HIP(ctx_, hipHostMalloc(&b.p, size, hipHostMallocDefault));
+    b.bytes = size;
+    return HM_OK;
+}
+
+int DecoderModel::finish_sync(void *h_dst, const void *d_src, size_t words) {
+    const int rc = words ? move_words_launch(ctx_, h_dst, d_src, words) : HM_OK;
+    const int synced = hm_sync(ctx_);
+    return rc == HM_OK ? synced : rc;
 }
 
 int DecoderModel::check_ids(const int64_t *ids, int n, std::vector<int32_t> &out) {
@@ -46,20 +71,14 @@ int DecoderModel::run_kv_once(const int64_t *h_ids, int n_ids, float *h_logits) 
     // src/hf/model.rs:340-371). The row and the whole-step status words are copied into pinned host memory
     // behind the step, so a token costs one stream synchronisation.
     const size_t row_bytes = (size_t)vocab_size() * 4;
-    if (h_logits && h_stage_bytes_ < row_bytes + 64) {
-        if (h_stage_) (void)hipHostFree(h_stage_);
-        h_stage_ = nullptr;
-        h_stage_bytes_ = 0;
-        HM_HIP(ctx_, hipHostMalloc(&h_stage_, row_bytes + 64, hipHostMallocDefault));
-        h_stage_bytes_ = row_bytes + 64;
-    }
+    if (h_logits && (rc = pinned_for(stage_, row_bytes + 64)) != HM_OK) return rc;
     for (int i = 0; i < n_ids; i++) {
         if ((rc = plan_->run_kv(inputs, weight_bufs_, max_seq_len_)) != HM_OK) return rc;
         if (!h_logits) continue;
-        char *stage = static_cast<char *>(h_stage_);
-        HM_HIP(ctx_, hipMemcpyAsync(stage, plan_->slot(logits_slot)->ptr(), row_bytes, hipMemcpyDeviceToHost, ctx_->stream));
+        char *stage = stage_.as<char>();
         const void *status = pending_status_words();
-        if (status) HM_HIP(ctx_, hipMemcpyAsync(stage + row_bytes, status, 64, hipMemcpyDeviceToHost, ctx_->stream));
+        rc = move_words_launch(ctx_, stage, plan_->slot(logits_slot)->ptr(), row_bytes / 4, status ? stage + row_bytes : nullptr, status);
+        if (rc != HM_OK) return rc;
         HM_HIP(ctx_, hipStreamSynchronize(ctx_->stream));
         std::memcpy(h_logits + (size_t)i * vocab_size(), stage, row_bytes);
         if (status && (rc = check_status_words(reinterpret_cast<const uint32_t *>(stage + row_bytes))) != HM_OK) return rc;
@@ -68,6 +87,11 @@ int DecoderModel::run_kv_once(const int64_t *h_ids, int n_ids, float *h_logits) 
 }
 
 int DecoderModel::prefill(const int64_t *h_ids, int n_ids, float *h_logits) {
+    const int rc = prefill_enqueue(h_ids, n_ids, h_logits);
+    return rc == HM_OK ? hm_sync(ctx_) : rc;
+}
+
+int DecoderModel::prefill_enqueue(const int64_t *h_ids, int n_ids, float *h_logits) {
     if (!finalized_) return hm_set_error(ctx_, HM_ERR_STATE, "model not finalized");
     if (!prefill_available())
         return hm_set_error(ctx_, HM_ERR_INVALID, "prefill: needs %s", prefill_needs());
@@ -77,12 +101,15 @@ int DecoderModel::prefill(const int64_t *h_ids, int n_ids, float *h_logits) {
     std::vector<int32_t> ids;
     int rc = check_ids(h_ids, n_ids, ids);
     if (rc != HM_OK) return rc;
+    if ((rc = hm_sync(ctx_)) != HM_OK) return rc;  // (nothing to wait for, unless a call failed behind its prompt)
+    if ((rc = pinned_for(prompt_ids_, (size_t)n_ids * 4)) != HM_OK) return rc;
+    std::memcpy(prompt_ids_.p, ids.data(), (size_t)n_ids * 4);
     for (int at = 0; at < n_ids; at += chunk_rows_) {
         const int n = std::min(chunk_rows_, n_ids - at);
-        rc = prefill_chunk(ids.data() + at, n, h_logits ? h_logits + (size_t)at * vocab_size() : nullptr);
+        rc = prefill_chunk(prompt_ids_.as<int32_t>() + at, n, h_logits ? h_logits + (size_t)at * vocab_size() : nullptr);
         if (rc != HM_OK) return rc;
     }
-    return hm_sync(ctx_);
+    return HM_OK;
 }
 
 int DecoderModel::kv_cache_len() const { return plan_ ? plan_->kv_cache_len() : 0; }
@@ -116,7 +143,7 @@ int DecoderModel::generate_greedy_once(const int64_t *h_prompt, int n_prompt, in
     if (prefill_min_ > 0 && n_prompt - 1 >= prefill_min_ && prefill_available()) {
         // reference HfGenerationContext::prefill (src/hf/model.rs:321-336): the prompt in one pass; its
         // last token goes through the decode step, whose pick is generated token 0
-        int rc = prefill(h_prompt, n_prompt - 1, nullptr);
+        int rc = prefill_enqueue(h_prompt, n_prompt - 1, nullptr);
         if (rc != HM_OK) return rc;
         h_prompt += n_prompt - 1;
         n_prompt = 1;
@@ -133,8 +160,10 @@ int DecoderModel::generate_greedy_once(const int64_t *h_prompt, int n_prompt, in
     for (int i = 0; i < steps; i++)
         if ((rc = plan_->run_kv(inputs, weight_bufs_, max_seq_len_)) != HM_OK) return rc;
     // the pick after prompt token n_prompt-1 is generated token 0
-    rc = hm_download(ctx_, h_tokens, plan_->out_tokens() + (n_prompt - 1), (size_t)n_new * 4);
-    return rc == HM_OK ? finish_sync() : rc;
+    if ((rc = pinned_for(tokens_, (size_t)n_new * 4)) != HM_OK) return rc;
+    rc = finish_sync(tokens_.p, plan_->out_tokens() + (n_prompt - 1), n_new);
+    if (rc == HM_OK) std::memcpy(h_tokens, tokens_.p, (size_t)n_new * 4);
+    return rc;
 }
 
 // sampling.hip
@@ -181,12 +210,14 @@ int DecoderModel::generate_once(const int64_t *h_prompt, int n_prompt, int max_n
         s.list_cap = max_new;
     }
     const bool penalties = cfg.repetition_penalty != 1.0f || cfg.frequency_penalty != 0.0f || cfg.presence_penalty != 0.0f;
-    if ((rc = zero_ints_launch(ctx_, s.counts.as<int>(), (size_t)vocab)) != HM_OK) return rc;
     // prompt: everything but its last token only has to reach the cache
     // (reference HfGenerationContext::prefill, src/hf/model.rs:321-336)
     if (n_prompt > 1) {
-        if ((rc = run_kv_once(h_prompt, n_prompt - 1, nullptr)) != HM_OK) return rc;
+        const bool at_once = prefill_min_ > 0 && n_prompt - 1 >= prefill_min_ && prefill_available();
+        rc = at_once ? prefill_enqueue(h_prompt, n_prompt - 1, nullptr) : run_kv_once(h_prompt, n_prompt - 1, nullptr);
+        if (rc != HM_OK) return rc;
     }
+    if ((rc = zero_ints_launch(ctx_, s.counts.as<int>(), (size_t)vocab)) != HM_OK) return rc;
     uint64_t rng = hm_rng_seed(seed);
     std::vector<Buffer *> inputs;
     step_inputs(inputs);
@@ -202,27 +233,27 @@ int DecoderModel::generate_once(const int64_t *h_prompt, int n_prompt, int max_n
         // step that produced it (the reference stops there: src/generate.rs:231-246).
         const bool own_pick = greedy && !penalties;
         if (!greedy) {
-            std::vector<float> draws((size_t)max_new);
-            for (auto &d : draws) d = hm_rng_next_f32(&rng);
+            if ((rc = pinned_for(draws_, (size_t)max_new * 4)) != HM_OK) return rc;
+            for (int i = 0; i < max_new; i++) draws_.as<float>()[i] = hm_rng_next_f32(&rng);
             if (s.draws_cap < max_new) {
                 s.draws = Buffer::alloc(ctx_, {max_new}, DType::F32);
                 if (!s.draws) return HM_ERR_OOM;
                 s.draws_cap = max_new;
             }
-            if ((rc = hm_upload(ctx_, s.draws.ptr(), draws.data(), draws.size() * 4)) != HM_OK) return rc;
+            if ((rc = move_words_launch(ctx_, s.draws.ptr(), draws_.p, max_new)) != HM_OK) return rc;
         }
-        const int chunk_cap = std::min(plan_->out_capacity(), 16);
-        std::vector<int32_t> got((size_t)chunk_cap);
+        // (no end-of-sequence token: nothing to be looked at in between)
+        const int chunk_cap = std::min(plan_->out_capacity(), eos_token >= 0 ? 16 : 256);
+        if ((rc = pinned_for(tokens_, (size_t)chunk_cap * 4)) != HM_OK) return rc;
+        const int32_t *got = tokens_.as<int32_t>();
         int done = 0;
         while (done < max_new) {
             const int len0 = kv_cache_len();
             const int n = std::min({chunk_cap, max_new - done, max_seq_len_ - len0});
             if (n <= 0) break;  // context limit (src/generate.rs:188-194)
             if (eos_token >= 0 && (rc = mark_position()) != HM_OK) return rc;
-            if ((rc = plan_->arm(&current, 1)) != HM_OK) return rc;
             int32_t *d_stop = s.token.as<int32_t>() + 1;
-            const int32_t minus_one = -1;
-            if (!own_pick && (rc = hm_upload(ctx_, d_stop, &minus_one, 4)) != HM_OK) return rc;
+            if ((rc = plan_->arm(&current, 1, own_pick ? nullptr : d_stop)) != HM_OK) return rc;
             for (int i = 0; i < n; i++) {
                 if ((rc = plan_->run_kv(inputs, weight_bufs_, max_seq_len_)) != HM_OK) return rc;
                 if (own_pick) continue;
@@ -232,7 +263,9 @@ int DecoderModel::generate_once(const int64_t *h_prompt, int n_prompt, int max_n
                                         d_stop, s.token.as<int32_t>());
                 if (rc != HM_OK) return rc;
             }
-            rc = hm_download(ctx_, got.data(), own_pick ? plan_->out_tokens() : s.list.as<int32_t>() + done, (size_t)n * 4);
+            const int32_t *d_got = own_pick ? plan_->out_tokens() : s.list.as<int32_t>() + done;
+            if (done + n == max_new) rc = finish_sync(tokens_.p, d_got, n);
+            else if ((rc = move_words_launch(ctx_, tokens_.p, d_got, n)) == HM_OK) rc = hm_sync(ctx_);
             if (rc != HM_OK) return rc;
             int taken = n;
             for (int i = 0; i < n; i++)
@@ -244,7 +277,7 @@ int DecoderModel::generate_once(const int64_t *h_prompt, int n_prompt, int max_n
             if (taken < n) {
                 // what the steps behind the stop left in the cache is dropped
                 std::vector<int32_t> kept{current};
-                kept.insert(kept.end(), got.begin(), got.begin() + taken);
+                kept.insert(kept.end(), got, got + taken);
                 if ((rc = rewind_to_mark(len0, kept)) != HM_OK) return rc;
                 break;
             }

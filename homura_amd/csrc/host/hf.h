@@ -114,12 +114,12 @@ class HfModel : public DecoderModel {
     int emit_transformer_plan_quant();  // reference src/hf/emitter_quant.rs:1142-1503
     int step_inputs(std::vector<Buffer *> &inputs) override;
     int refresh_fused_table();
-    int finish_sync() override;
+    int finish_sync(void *h_dst = nullptr, const void *d_src = nullptr, size_t words = 0) override;
     int recover_whole_step();
     int guarded(const std::function<int()> &body) override;  // runs it again after a recovered whole-step timeout
     const void *pending_status_words() override;
     int check_status_words(const uint32_t *h_ctl) override;
-    int prefill_chunk(const int32_t *h_ids, int n, float *h_logits) override;
+    int prefill_chunk(const int32_t *d_ids, int n, float *h_logits) override;
     const char *prefill_needs() const override;
     const float *weight_f32(const std::string &name) const;
 
@@ -166,7 +166,7 @@ class HfModel : public DecoderModel {
     // prefill pass: activations of one chunk of rows
     struct PrefillScratch {
         int rows = 0;
-        Buffer ids, h, resid, split, qkv, proj_out, gate_up, logits, row_unscale;
+        Buffer h, resid, split, qkv, proj_out, gate_up, logits, row_unscale;
         Buffer wsplit;  // block formats: the matrices of one group of projections as three bf16 pieces per weight
         std::vector<Buffer> wcache;  // [layer * 4 + group] resident copies of the same (q|k|v, o, gate|up, down)
         // K-quant groups on the integer matrix cores: the chunk's Q8_K rows (int8 values, one f32 scale per
@@ -211,6 +211,7 @@ class HfModel : public DecoderModel {
     void drop_half_weights();
     int build_half_weights();
     int refresh_half_weights();
+    Pinned status_;             // of the whole-step launches, at the end of a call
     bool half_wanted_ = true;   // set_prefill_f16
     bool half_waits_ = false;   // not built for want of prompt passes (set_prefill_min(0)): the next one builds them
     size_t prefill_weight_cache_bytes_ = (size_t)32 << 30;

@@ -6,6 +6,7 @@
 #include <cstdlib>
 
 #include "../attention.h"
+#include "../light_ops.h"
 #include "../decode_fused.h"
 #include "../kquant_planes8.h"
 #include "../gemm_kquant_i8.h"
@@ -254,6 +255,7 @@ int HfModel::build_k8_planes() {
 
 HfModel::~HfModel() {
     if (ctx_) hm_sync(ctx_);
+    if (status_.p) (void)hipHostFree(status_.p);
 }
 
 int HfModel::set_weight_impl(int slot, const void *h_data, size_t bytes, bool nk_layout) {
@@ -1768,13 +1770,14 @@ int HfModel::whole_step_trace(unsigned long long *h_out, int cap, int *n_out) {
 constexpr int HM_RETRY_STEPS = -1000;
 
 // Stream sync plus, when steps went through the whole-step launch since the last look, its status words.
-int HfModel::finish_sync() {
-    int rc = hm_sync(ctx_);
-    if (rc != HM_OK || !fused_available_ || !fused_dirty_) return rc;
+int HfModel::finish_sync(void *h_dst, const void *d_src, size_t words) {
+    if (!fused_available_ || !fused_dirty_) return DecoderModel::finish_sync(h_dst, d_src, words);
+    int rc = pinned_for(status_, 64);
+    if (rc == HM_OK) rc = move_words_launch(ctx_, h_dst, d_src, words, status_.p, scratch_->fused_ctl.ptr());
+    const int synced = hm_sync(ctx_);
+    if (rc != HM_OK || synced != HM_OK) return rc != HM_OK ? rc : synced;
     fused_dirty_ = false;
-    uint32_t h[16] = {0};
-    rc = hm_download(ctx_, h, scratch_->fused_ctl.ptr(), sizeof(h));
-    return rc == HM_OK ? check_fused_words(h) : rc;
+    return check_fused_words(status_.as<uint32_t>());
 }
 
 // What a host copy of the whole-step control words says: HM_OK, HM_RETRY_STEPS after the recovery from a wait
@@ -2154,7 +2157,7 @@ int prompt_product_slices(DType dtype, int M, int K, int N, int cus) {
     return std::max(pieces, kquant ? (K % 256 ? 1 : kq_i8_slices(M, K, N, cus, MP)) : gemm_pieces_slices(1, true, M, K, N, cus, MP));
 }
 
-int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
+int HfModel::prefill_chunk(const int32_t *d_ids, int n, float *h_logits) {
     constexpr int HEAD_ROWS = 512;  // rows whose logits are held at a time
     const TransformerConfig &c = cfg_;
     const int hidden = c.hidden_size, inter = c.intermediate_size, vocab = c.vocab_size;
@@ -2193,7 +2196,6 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
             grown.wcache = std::move(p.wcache);
             p = std::move(grown);
         }
-        p.ids = Buffer::alloc(ctx_, {rows}, DType::F32);  // int32 ids
         p.h = Buffer::alloc(ctx_, {rows, hidden}, DType::F32);
         p.resid = Buffer::alloc(ctx_, {rows, hidden}, DType::F32);
         p.split = Buffer::alloc(ctx_, {rows, 3 * widest}, DType::BF16);
@@ -2201,7 +2203,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         p.proj_out = Buffer::alloc(ctx_, {std::max(sliced(3, qd, hidden), sliced(6, inter, hidden))}, DType::F32);
         p.gate_up = Buffer::alloc(ctx_, {std::max<int64_t>(sliced(4, hidden, 2 * (int64_t)inter), (int64_t)rows * qd)}, DType::F32);
         p.row_unscale = Buffer::alloc(ctx_, {rows}, DType::F32);
-        if (!p.ids || !p.h || !p.resid || !p.split || !p.qkv || !p.proj_out || !p.gate_up || !p.row_unscale) return HM_ERR_OOM;
+        if (!p.h || !p.resid || !p.split || !p.qkv || !p.proj_out || !p.gate_up || !p.row_unscale) return HM_ERR_OOM;
         if (quant && widest % 256 == 0) {  // Q8_K rows for K-quant groups (a float holds four of the int8 values)
             p.q8 = Buffer::alloc(ctx_, {rows, widest / 4}, DType::F32);
             p.q8s = Buffer::alloc(ctx_, {rows, widest / 256}, DType::F32);
@@ -2220,8 +2222,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
     }
     KvCache *kv = plan_->kv_cache();
     const int past = kv->current_len();
-    int rc = hm_upload(ctx_, p.ids.ptr(), h_ids, (size_t)n * 4);
-    if (rc != HM_OK) return rc;
+    int rc = HM_OK;
     float *h = p.h.as<float>(), *resid = p.resid.as<float>(), *qkv = p.qkv.as<float>();
     float *proj_out = p.proj_out.as<float>(), *gate_up = p.gate_up.as<float>();
     uint16_t *split = p.split.as<uint16_t>();
@@ -2419,7 +2420,7 @@ int HfModel::prefill_chunk(const int32_t *h_ids, int n, float *h_logits) {
         }
         return gemm_split_split_nk(ctx_, split, wsplit, out, n, K, N, MP, &parts);
     };
-    rc = embed_launch(ctx_, nullptr, p.ids.as<int32_t>(), weight_f32("model.embed_tokens.weight"), h, n, vocab, hidden);
+    rc = embed_launch(ctx_, nullptr, d_ids, weight_f32("model.embed_tokens.weight"), h, n, vocab, hidden);
     if (rc != HM_OK) return rc;
     // where (layer, group)'s rows of this chunk go in the capture buffer, or nullptr
     auto capture_at = [&](int l, int group) -> float * {

@@ -272,7 +272,7 @@ class ExecutionPlan {
     int32_t *out_tokens() const { return out_tokens_.as<int32_t>(); }
     int out_capacity() const { return out_cap_; }
     // Arm the cursor: pos = cache length, step = 0, the given ids forced for the first steps.
-    int arm(const int32_t *h_forced, int n_forced);
+    int arm(const int32_t *h_forced, int n_forced, int *d_stop = nullptr);
 
     // Graph replay of the step (captured lazily on first use; arguments never change), on by default for steps of more than three launches.
     // Where the default cannot be recorded the steps are launched one by one, and hm_last_error says why; they are tried again once asked
@@ -338,8 +338,8 @@ class ExecutionPlan {
     std::vector<Buffer> kv_views_;  // per-step views of the cache bound to present_kv slots
     std::vector<Buffer *> pool_;
     Buffer state_, forced_, out_tokens_;
-    // arm(): the cursor and the forced ids go out from pinned host memory with asynchronous copies (no stream
-    // synchronisation per call); the event tells when that memory may be written again
+    // arm() of more forced ids than go along as launch arguments: cursor and ids leave pinned host memory with asynchronous copies (no stream
+    // synchronisation; the event says when the memory is free again)
     void *arm_pinned_ = nullptr;
     hipEvent_t arm_done_ = nullptr;
     int out_cap_ = 0;

@@ -4,6 +4,8 @@
 #include <algorithm>
 #include <map>
 
+#include "../light_ops.h"
+
 namespace homura {
 
 // ── dtype maths (reference src/dtype.rs:8-92) ────────────────────────────────
@@ -362,10 +364,12 @@ void ExecutionPlan::reset_kv_cache() {
     if (cache_) cache_->reset(0);
 }
 
-int ExecutionPlan::arm(const int32_t *h_forced, int n_forced) {
+int ExecutionPlan::arm(const int32_t *h_forced, int n_forced, int *d_stop) {
     if (!prepared_) return hm_set_error(ctx_, HM_ERR_STATE, "plan not prepared");
     if (n_forced > out_cap_) return hm_set_error(ctx_, HM_ERR_INVALID, "%d forced ids exceed the plan's capacity %d", n_forced, out_cap_);
     const DecodeState st{kv_cache_len(), 0, 0, n_forced};
+    if (n_forced <= ARM_IDS) return arm_launch(ctx_, state(), st, forced_.as<int32_t>(), h_forced, d_stop);
+    if (d_stop) return hm_set_error(ctx_, HM_ERR_INVALID, "arm: a stop word goes with up to %d forced ids", ARM_IDS);
     if (!arm_pinned_) {
         HM_HIP(ctx_, hipHostMalloc(&arm_pinned_, sizeof(DecodeState) + (size_t)out_cap_ * 4, hipHostMallocDefault));
         HM_HIP(ctx_, hipEventCreateWithFlags(&arm_done_, hipEventDisableTiming));

@@ -33,6 +33,14 @@ int argmax_candidates_launch(hm_ctx *ctx, const float *d_vals, const int *d_idxs
 // embedding of this step's input id (forced id while step < n_forced, else the last pick)
 int embed_step_launch(hm_ctx *ctx, const DecodeState *state, const int32_t *d_forced,
                       const float *d_table, float *d_out, int vocab, int hidden);
+// What a call leaves for the device and takes from it, by kernels instead of copies: a copy waits some 25 us on either side of itself
+// (a prompt's ids, cursor, forced id, logits row and status words were five of them).
+// The cursor, up to ARM_IDS forced ids and, if stop is not NULL, -1 to it, all as launch arguments.
+constexpr int ARM_IDS = 16;
+int arm_launch(hm_ctx *ctx, DecodeState *d_state, const DecodeState &st, int32_t *d_forced, const int32_t *h_ids, int *d_stop);
+// words 4-byte words between device memory and pinned host memory (either way), and 16 more from d_status to h_status if that is not
+// NULL. The host's side is free, or filled, once the stream has been synchronised with.
+int move_words_launch(hm_ctx *ctx, void *dst, const void *src, size_t words, void *h_status = nullptr, const void *d_status = nullptr);
 // fold the LM-head argmax candidates, record the pick, advance the cursor
 int finish_step_launch(hm_ctx *ctx, DecodeState *state, const float *d_vals, const int *d_idxs,
                        int n, int32_t *d_out_tokens, int out_cap);

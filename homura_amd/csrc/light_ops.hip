@@ -3,6 +3,9 @@
 // weight streams; they exist as separate entry points because the reference's quantised plan
 // runs them as separate kernels (src/hf/emitter_quant.rs:713-1134).
 #include "light_ops.h"
+
+#include <algorithm>
+
 #include "../../include/homura_amd_bench.h"
 
 namespace {
@@ -355,6 +358,52 @@ int embed_launch(hm_ctx *ctx, const int64_t *d_ids64, const int32_t *d_ids32, co
     HM_REQUIRE(ctx, n_ids > 0 && vocab > 0 && hidden > 0, "embed: bad shape");
     hipLaunchKernelGGL(embed_kernel, dim3(n_ids), dim3(256), 0, ctx->stream, d_ids64, d_ids32,
                        d_table, d_out, hidden, vocab);
+    HM_LAUNCH_CHECK(ctx);
+    return HM_OK;
+}
+
+struct ArmIds {
+    int32_t id[ARM_IDS];
+};
+__global__ void arm_kernel(DecodeState *state, DecodeState st, int32_t *forced, ArmIds ids, int *stop) {
+    if (threadIdx.x != 0) return;
+    *state = st;
+    if (stop) *stop = -1;
+#pragma unroll
+    for (int i = 0; i < ARM_IDS; i++)
+        if (i < st.n_forced) forced[i] = ids.id[i];
+}
+
+int arm_launch(hm_ctx *ctx, DecodeState *d_state, const DecodeState &st, int32_t *d_forced, const int32_t *h_ids, int *d_stop) {
+    HM_REQUIRE(ctx, d_state && st.n_forced >= 0 && st.n_forced <= ARM_IDS && (st.n_forced == 0 || (d_forced && h_ids)), "arm: bad arguments");
+    ArmIds ids{};
+    for (int i = 0; i < st.n_forced; i++) ids.id[i] = h_ids[i];
+    hipLaunchKernelGGL(arm_kernel, dim3(1), dim3(64), 0, ctx->stream, d_state, st, d_forced, ids, d_stop);
+    HM_LAUNCH_CHECK(ctx);
+    return HM_OK;
+}
+
+// Sixteen bytes a thread where both sides and the length allow it (608 KB to the host: 12 us, what its link takes).
+template <class V>
+__global__ __launch_bounds__(256) void move_words_kernel(V *__restrict__ dst, const V *__restrict__ src, size_t n, uint32_t *__restrict__ h_status,
+                                                         const uint32_t *__restrict__ d_status) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+    if (h_status && i < 16) h_status[i] = d_status[i];
+}
+
+int move_words_launch(hm_ctx *ctx, void *dst, const void *src, size_t words, void *h_status, const void *d_status) {
+    HM_REQUIRE(ctx, (words == 0 || (dst && src)) && ((uintptr_t)dst % 4) == 0 && ((uintptr_t)src % 4) == 0 && (h_status == nullptr) == (d_status == nullptr) &&
+                        ((uintptr_t)h_status % 4) == 0 && ((uintptr_t)d_status % 4) == 0, "move_words: bad arguments");
+    const bool vec = words % 4 == 0 && (((uintptr_t)dst | (uintptr_t)src) % 16) == 0;
+    const size_t n = vec ? words / 4 : words, wgs = std::max<size_t>(1, (n + 255) / 256);
+    HM_REQUIRE(ctx, wgs <= 0x7fffffff, "move_words: %zu words", words);
+    auto go = [&](auto kernel, auto *d, const auto *s) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, ctx->stream, d, s, n, static_cast<uint32_t *>(h_status),
+                           static_cast<const uint32_t *>(d_status));
+    };
+    if (vec) go(move_words_kernel<u32x4>, static_cast<u32x4 *>(dst), static_cast<const u32x4 *>(src));
+    else go(move_words_kernel<uint32_t>, static_cast<uint32_t *>(dst), static_cast<const uint32_t *>(src));
     HM_LAUNCH_CHECK(ctx);
     return HM_OK;
 }

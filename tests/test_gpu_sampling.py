@@ -295,3 +295,28 @@ def test_chat_turn_feeds_only_the_new_tokens(ctx):
     say(f"chat turn: {len(whole) - in_cache} new ids on {in_cache} cached, max logit difference "
         f"{np.abs(step - fresh).max():.2e} (scale {np.abs(fresh).max():.2f})")
     gm.close()
+
+
+@pytest.mark.parametrize("prompt,cfg", [(20, runtime.SamplingConfig()), (3, runtime.SamplingConfig()), (20, runtime.SamplingConfig(temperature=0.0, repetition_penalty=1.0)),
+                                        (40, runtime.SamplingConfig(temperature=0.0, repetition_penalty=1.3))])
+def test_portions_of_a_generation_do_not_show(ctx, prompt, cfg):
+    """Without an end token 256 steps go out at a time, with one 16: 300 tokens are the same, as is what the next request finds."""
+    mcfg = synth_model.TINY
+    gm = synth_model.build_model(ctx, mcfg, synth_model.synth_weights(mcfg, 61), 400)
+    ids = synth.token_ids(3, prompt, mcfg.vocab_size)
+    got = gm.generate(ids, 300, cfg, seed=9)
+    after = gm.run_kv(got[-1:])
+    absent = int(np.setdiff1d(np.arange(mcfg.vocab_size), got)[0])
+    gm.reset_kv_cache()
+    assert len(got) == 300 and np.array_equal(gm.generate(ids, 300, cfg, seed=9, eos_token_id=absent), got)
+    assert np.array_equal(gm.run_kv(got[-1:]), after)
+    gm.set_prefill_min(0)  # the prompt token by token, its ids as launch arguments and (more than 16) through memory
+    gm.reset_kv_cache()
+    gm.run_kv(ids[:-1], want_logits=False)
+    last = gm.run_kv(ids[-1:])
+    gm.set_prefill_min(8)
+    gm.reset_kv_cache()
+    gm.run_kv(ids[:-1], want_logits=False)
+    again = gm.run_kv(ids[-1:])
+    assert np.abs(last - again).max() <= 2e-3 * np.abs(again).max()  # (cache rows that round to bf16 the other way)
+    gm.close()
