@@ -1296,9 +1296,12 @@ int BlockModel::prefill_mixer(int run, int layer, const float *cos_tab, const fl
         c.out_split = sb;
         c.pieces = np;
         c.channels = c.block_width = c.block_pad = d.inner;
-        c.side = p.f3.as<float>();
-        c.side_cols = d.inner;
-        c.side_act = ConvRowsArgs::Silu;
+        const bool whole = in.parts == 1;  // sums of K slices are taken once, by the convolution
+        if (!whole) {
+            c.side = p.f3.as<float>();
+            c.side_cols = d.inner;
+            c.side_act = ConvRowsArgs::Silu;
+        }
         c.n = n;
         c.past = past;
         if ((rc = conv_rows_launch(ctx_, c)) != HM_OK) return rc;
@@ -1316,7 +1319,9 @@ int BlockModel::prefill_mixer(int run, int layer, const float *cos_tab, const fl
         x.bc_ld = pw;
         x.a_log2 = l.a_log2.ptr();
         x.d = l.d.ptr();
-        x.z = c.side;
+        x.z = whole ? in.p + d.inner : c.side;
+        x.z_ld = whole ? in.ld : d.inner;
+        x.z_raw = whole;
         x.state = cache->state(run);
         x.out_split = sa;
         x.pieces = np;
@@ -1343,9 +1348,12 @@ int BlockModel::prefill_mixer(int run, int layer, const float *cos_tab, const fl
     c.channels = s.rec.width;
     c.block_width = d.block;
     c.block_pad = d.block_pad;
-    c.side = p.f3.as<float>();
-    c.side_cols = d.width;
-    c.side_act = ConvRowsArgs::Gelu;
+    const bool whole = in.parts == 1;
+    if (!whole) {
+        c.side = p.f3.as<float>();
+        c.side_cols = d.width;
+        c.side_act = ConvRowsArgs::Gelu;
+    }
     c.n = n;
     c.past = past;
     if ((rc = conv_rows_launch(ctx_, c)) != HM_OK) return rc;
@@ -1359,7 +1367,10 @@ int BlockModel::prefill_mixer(int run, int layer, const float *cos_tab, const fl
     x.r_bias = l.r_b.ptr();
     x.i_bias = l.i_b.ptr();
     x.decay = l.decay.ptr();
-    x.y = c.side;
+    x.y = whole ? in.p + d.width : c.side;
+    x.y_bias = xin.bias + d.width;
+    x.y_ld = whole ? in.ld : d.width;
+    x.y_raw = whole;
     x.state = cache->state(run);
     x.out_split = sa;
     x.pieces = np;

@@ -47,7 +47,9 @@ struct SelectiveScanArgs {
     int bc_ld = 0;
     const float *a_log2 = nullptr;     // [inner][state_pad]: A * log2(e), 0 behind the true states
     const float *d = nullptr;          // [inner]
-    const float *z = nullptr;          // [n][inner]: silu of the gate rows
+    const float *z = nullptr;          // [n][z_ld]: silu of the gate rows, or (z_raw) the rows themselves
+    int z_ld = 0;
+    bool z_raw = false;
     float *state = nullptr;            // [inner][state_pad]
     uint16_t *out_split = nullptr;     // [n][pieces * inner]
     int pieces = 3;
@@ -74,7 +76,10 @@ struct LinearRecurrenceArgs {
     const float *u = nullptr;          // [n][width]
     const float *gates = nullptr;      // [n][blocks * 2 * block_pad]: block b's r columns, then its i columns
     const float *r_bias = nullptr, *i_bias = nullptr, *decay = nullptr;  // [width]
-    const float *y = nullptr;          // [n][width]: gelu_tanh of the other branch
+    const float *y = nullptr;          // [n][y_ld]: gelu_tanh of the other branch, or (y_raw) the branch itself ahead of y_bias [width]
+    const float *y_bias = nullptr;
+    int y_ld = 0;
+    bool y_raw = false;
     float *state = nullptr;            // [width]
     uint16_t *out_split = nullptr;     // [n][pieces * width]
     int pieces = 3;

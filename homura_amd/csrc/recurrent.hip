@@ -172,6 +172,8 @@ __device__ __forceinline__ void store_taps(const RowSource &in, const TapRing &r
 // ahead of it into the state it starts from and is scanned in full. 2048 tokens, 2048 channels of 16 states: 91 us in one
 // segment, 32 to 33 + 19.4 in eight. (16 states: 128 registers at most, so that the four workgroups a CU gets of eight segments are
 // all resident; with the 129 that the compiler takes by itself 33.3 to 34.1 + 19.2.)
+// z_raw: the gate rows come as the projection left them and take their SiLU here, 4 a thread and tile beside 64 exponentials; on their way
+// through the convolution they were read and written once more (2047 rows, 2048 channels: convolution 18.5 -> 11, scan 32.3 -> 34.9).
 struct ScanSegments {
     int rows = 0;                    // of a segment, a multiple of the tile; 0: the chunk is one segment
     float *ends = nullptr;           // [segments][inner][state_pad]: slot 0 the chunk's first state, slot g + 1 the end of segment g
@@ -185,6 +187,7 @@ __global__ __launch_bounds__(256, SPL == 1 ? 4 : 1) void selective_scan_kernel(S
     constexpr int E = SCAN_T * 16 / 256, EB = SCAN_T * SP / 256;
     __shared__ __attribute__((aligned(16))) float s_dt[16][SCAN_LD], s_dx[16][SCAN_LD], s_y[16][SCAN_LD];
     __shared__ __attribute__((aligned(16))) float s_b[SP][SCAN_LD], s_c[SP][SCAN_LD];
+    __shared__ float s_z[ENDS ? 1 : E][256];  // each thread's own: they wait here for the tile's results, not in registers
     const int tid = threadIdx.x, ch = tid >> 4, l = tid & 15, c0 = blockIdx.x * 16;
     const int seg = blockIdx.y, t_first = seg * g.rows, n = g.rows ? min(a.n, t_first + g.rows) : a.n;  // tokens t_first .. n - 1
     const size_t states = (size_t)a.inner * SP;
@@ -206,6 +209,7 @@ __global__ __launch_bounds__(256, SPL == 1 ? 4 : 1) void selective_scan_kernel(S
     const int ec = c0 + l, er = tid >> 4;  // this thread's channel and first row in loads and stores
     const bool odd = l & 1, upper = l & 2;
     const float d_c = a.d[ec], dt_bias = a.dt_bias[ec];
+    const float *zc = a.z + ec;
     float r_dt[E], r_x[E], r_z[E], r_b[EB], r_c[EB];
     auto load_tile = [&](int t0) {
 #pragma unroll
@@ -213,7 +217,7 @@ __global__ __launch_bounds__(256, SPL == 1 ? 4 : 1) void selective_scan_kernel(S
             const size_t at = (size_t)min(t0 + er + e * 16, n - 1) * a.inner + ec;
             r_dt[e] = a.dt[at];
             r_x[e] = a.x[at];
-            if (!ENDS) r_z[e] = a.z[at];
+            if (!ENDS) r_z[e] = zc[(size_t)min(t0 + er + e * 16, n - 1) * a.z_ld];
         }
 #pragma unroll
         for (int e = 0; e < EB; e++) {
@@ -225,13 +229,13 @@ __global__ __launch_bounds__(256, SPL == 1 ? 4 : 1) void selective_scan_kernel(S
     };
     load_tile(t_first);
     for (int t0 = t_first; t0 < n; t0 += SCAN_T) {
-        float x[E], z[E];
+        float x[E];
 #pragma unroll
         for (int e = 0; e < E; e++) {
             float dt = softplus_dev(r_dt[e] + dt_bias);
             if (t0 + er + e * 16 >= n) dt = 0.f;
             x[e] = r_x[e];
-            if (!ENDS) z[e] = r_z[e];
+            if (!ENDS) s_z[e][tid] = r_z[e];
             dt_sum += dt;
             s_dt[l][er + e * 16] = dt;
             s_dx[l][er + e * 16] = dt * x[e];
@@ -292,8 +296,10 @@ __global__ __launch_bounds__(256, SPL == 1 ? 4 : 1) void selective_scan_kernel(S
 #pragma unroll
         for (int e = 0; e < E; e++) {
             const int r = er + e * 16;
+            float z = s_z[e][tid];
+            if (a.z_raw) z = z * sigmoid_dev(z);
             if (t0 + r < n)
-                split_store(a.out_split + (size_t)(t0 + r) * a.pieces * a.inner, a.inner, ec, fmaf(d_c, x[e], s_y[l][r]) * z[e], a.pieces);
+                split_store(a.out_split + (size_t)(t0 + r) * a.pieces * a.inner, a.inner, ec, fmaf(d_c, x[e], s_y[l][r]) * z, a.pieces);
         }
         // (the next tile's staging writes none of what is read here: s_y is written behind its barrier)
     }
@@ -410,13 +416,18 @@ __global__ __launch_bounds__(16 * LR_SEGS) void linear_recurrence_kernel(LinearR
             r_[k] = gr[t * gate_ld];
             i_[k] = gi[t * gate_ld];
             u_[k] = a.u[t * a.width + cc];
-            if (!ENDS) yv[k] = a.y[t * a.width + cc];
+            if (!ENDS) yv[k] = a.y[t * a.y_ld + cc];
         }
 #pragma unroll
         for (int k = 0; k < LR_LEN; k++) {
             const float la = decay * sigmoid_dev(r_[k] + rb);
             av[k] = exp_dev(la);
             bv[k] = input_gain(2.0f * la, av[k] * av[k]) * (sigmoid_dev(i_[k] + ib) * u_[k]);
+        }
+        if (!ENDS && a.y_raw) {
+            const float yb = a.y_bias[cc];
+#pragma unroll
+            for (int k = 0; k < LR_LEN; k++) yv[k] = gelu_tanh_row(yv[k] + yb);
         }
     }
     float P = 1.f, Q = 0.f;
@@ -554,7 +565,7 @@ int conv_rows_launch(hm_ctx *ctx, const ConvRowsArgs &a) {
 int selective_scan_launch(hm_ctx *ctx, const SelectiveScanArgs &a) {
     HM_REQUIRE(ctx, a.x && a.dt && a.dt_bias && a.z && a.b && a.c && a.a_log2 && a.d && a.state && a.out_split && a.ring.ring && a.n > 0 && a.past >= 0, "selective_scan: bad arguments");
     HM_REQUIRE(ctx, a.inner > 0 && a.inner % 16 == 0 && a.ring.width == a.inner && a.bc_ld >= a.state_pad && a.pieces >= 1 && a.pieces <= 3 &&
-                        !bad_source(a.conv_in, a.inner), "selective_scan: bad shape");
+                        a.z_ld >= a.inner && !bad_source(a.conv_in, a.inner), "selective_scan: bad shape");
     // Segments of 128 tokens at least while the workgroups leave the chip short of four a CU (the 2048 tokens of a prompt of a
     // model with 30 such layers of 2048 channels: 13.11 ms in one segment, 12.66 / 12.05 / 11.58 / 11.56 in 2 / 4 / 8 / 16)
     const int tile = a.state_pad <= 32 ? 64 : 32, wgs = a.inner / 16;
@@ -612,7 +623,7 @@ int linear_recurrence_launch(hm_ctx *ctx, const LinearRecurrenceArgs &a) {
     HM_REQUIRE(ctx, a.u && a.gates && a.y && a.r_bias && a.i_bias && a.decay && a.state && a.out_split && a.ring.ring, "linear_recurrence: NULL pointer");
     HM_REQUIRE(ctx, a.n > 0 && a.past >= 0 && a.channels > 0 && a.channels <= a.width && a.ring.width == a.width &&
                         a.block_width > 0 && a.block_pad >= a.block_width && a.channels % a.block_width == 0 && a.pieces >= 1 && a.pieces <= 3 &&
-                        !bad_source(a.conv_in, a.width), "linear_recurrence: bad shape");
+                        a.y_ld >= a.width && (!a.y_raw || a.y_bias) && !bad_source(a.conv_in, a.width), "linear_recurrence: bad shape");
     const size_t gate_ld = (size_t)(a.channels / a.block_width) * 2 * a.block_pad;
     const int groups = (a.width + 15) / 16;
     const dim3 block(16 * LR_SEGS);
@@ -624,7 +635,7 @@ int linear_recurrence_launch(hm_ctx *ctx, const LinearRecurrenceArgs &a) {
         b.n = std::min(a.n - at, most * LR_MAX_ROWS);
         b.past = a.past + at;
         b.u = a.u + (size_t)at * a.width;
-        b.y = a.y + (size_t)at * a.width;
+        b.y = a.y + (size_t)at * a.y_ld;
         b.gates = a.gates + at * gate_ld;
         b.out_split = a.out_split + (size_t)at * a.pieces * a.width;
         b.conv_in.p = a.conv_in.p + (size_t)at * a.conv_in.ld;

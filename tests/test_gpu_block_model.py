@@ -459,3 +459,12 @@ def test_files_that_do_not_fit_are_named(ctx, tmp_path):
     with pytest.raises(HomuraError, match="missing weight"):
         m.finalize(32)
     m.close()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("n", [70, 300])
+def test_gate_rows_from_slices_and_whole(ctx, n, dtype):
+    """The gates of the scan and the recurrence straight from their projection, and from the convolution where it came in K slices (1100 wide)."""
+    for width in (1100, 96):
+        cfg = bf.config([bf.scan(inner=64, state=16), bf.scan(inner=130, state=33), bf.recurrence(), bf.recurrence(width=66, blocks=2)], width=width)
+        check(ctx, cfg, n, dtype, cuts=(n // 3,))
