@@ -90,6 +90,15 @@ int gemm_tiles_bf16(hm_ctx *ctx, const uint16_t *d_a, const uint16_t *d_b_nk, fl
 // gemm_gated_pays: whether that is the quicker way (not where the few-rows kernel multiplies).
 int gemm_gated_nk(hm_ctx *ctx, const uint16_t *d_a, const uint16_t *d_b_nk, uint16_t *d_out, int M, int K, int N, const GatedAct &act);
 bool gemm_gated_pays(int M, int K, int N, int cus, int max_parts);
+// The product of one bf16 piece that expands latents into the keys and values of all heads: columns [head * dim ..) go as bf16 to the rows
+// of k [heads][cap][kw], columns [v_at + head * vdim ..) to those of v [heads][cap][vw]; columns that are no head's go nowhere, and what a row has
+// behind dim and vdim stays as it was. gemm_heads_fits: not where the few-rows kernel multiplies.
+struct HeadRows {
+    int heads = 0, dim = 0, vdim = 0, v_at = 0, kw = 0, vw = 0, cap = 0;
+    uint16_t *k = nullptr, *v = nullptr;
+};
+int gemm_heads_nk(hm_ctx *ctx, const uint16_t *d_a, const uint16_t *d_b_nk, int M, int K, int N, const HeadRows &h);
+bool gemm_heads_fits(int M, int K, int N, int cus);
 int gemm_half_slices(bool scaled, int M, int K, int N, int cus, int max_parts);
 // The K slices that a product of activation pieces with b_pieces (1 or 3) pieces of B, or with a block-scaled B, comes in
 int gemm_pieces_slices(int b_pieces, bool scaled, int M, int K, int N, int cus, int max_parts);

@@ -1249,17 +1249,35 @@ int BlockModel::prefill_mixer(int run, int layer, const float *cos_tab, const fl
         r.past = past;
         if ((rc = latent_rows_launch(ctx_, r)) != HM_OK) return rc;
         if ((rc = gemm(l.la_uq, sb, np, d2, &second)) != HM_OK) return rc;
-        if ((rc = latent_q_rows_launch(ctx_, sh, second, cos_tab, sin_tab, f1, d.head_k, n, past)) != HM_OK) return rc;
+        const bool in_place = latent_q_turns_in_place(sh, second, d.head_k);
+        rc = in_place ? latent_q_turn_launch(ctx_, sh, second, d2, cos_tab, sin_tab, n, past)
+                      : latent_q_rows_launch(ctx_, sh, second, cos_tab, sin_tab, f1, d.head_k, n, past);
+        if (rc != HM_OK) return rc;
         // keys and values of every visible row
         const int first = sh.window ? std::max(0, past - (sh.window - 1)) : 0, rows = past + n - first;
-        if ((rc = latent_gather_launch(ctx_, sh, ring, p.lat.as<uint16_t>(), first, rows)) != HM_OK) return rc;
-        if ((rc = gemm_split_nk(ctx_, p.lat.as<uint16_t>(), sh.pieces, l.la_ukv.ptr(), p.kvf.as<float>(), rows, sh.rank_pad, d.ukv_n)) != HM_OK) return rc;
-        const RowSource kv{p.kvf.as<float>(), d.ukv_n, 1, 0, nullptr};
-        rc = latent_kv_rows_launch(ctx_, sh, kv, d.v_at, ring, p.kws.as<uint16_t>(), p.vws.as<uint16_t>(), d.head_k, d.head_v, rows, first, rows);
+        HeadRows hr;
+        hr.heads = a.heads;
+        hr.dim = a.dim;
+        hr.vdim = a.vdim;
+        hr.v_at = d.v_at;
+        hr.kw = d.head_k;
+        hr.vw = d.head_v;
+        hr.cap = rows;
+        hr.k = p.kws.as<uint16_t>();
+        hr.v = p.vws.as<uint16_t>();
+        const bool direct = latent_heads_whole(sh, d.head_k, d.head_v) && gemm_heads_fits(rows, sh.rank_pad, d.ukv_n, ctx_->num_cus);
+        if ((rc = latent_gather_launch(ctx_, sh, ring, p.lat.as<uint16_t>(), first, rows, direct ? &hr : nullptr)) != HM_OK) return rc;
+        if (direct) {
+            rc = gemm_heads_nk(ctx_, p.lat.as<uint16_t>(), l.la_ukv.ptr(), rows, sh.rank_pad, d.ukv_n, hr);
+        } else {
+            if ((rc = gemm_split_nk(ctx_, p.lat.as<uint16_t>(), sh.pieces, l.la_ukv.ptr(), p.kvf.as<float>(), rows, sh.rank_pad, d.ukv_n)) != HM_OK) return rc;
+            const RowSource kv{p.kvf.as<float>(), d.ukv_n, 1, 0, nullptr};
+            rc = latent_kv_rows_launch(ctx_, sh, kv, d.v_at, ring, hr.k, hr.v, d.head_k, d.head_v, rows, first, rows);
+        }
         if (rc != HM_OK) return rc;
         PrefillAttnArgs at;
-        at.q = f1;
-        at.ldq = a.heads * d.head_k;
+        at.q = in_place ? d2 : f1;
+        at.ldq = in_place ? second.ld : a.heads * d.head_k;
         at.kcache = p.kws.as<uint16_t>();
         at.vcache = p.vws.as<uint16_t>();
         at.out_split = sa;

@@ -11,6 +11,7 @@
 #pragma once
 #include <cstdint>
 
+#include "gemm_bf16_mfma.h"
 #include "hm_common.h"
 #include "row_source.h"
 
@@ -68,8 +69,13 @@ int latent_rows_launch(hm_ctx *ctx, const LatentRowsArgs &a);
 // q rows [n][heads * width] f32 with rotation, zero behind dim + rot_dim, from the raw projection
 int latent_q_rows_launch(hm_ctx *ctx, const LatentShape &s, const RowSource &q, const float *cos_tab, const float *sin_tab,
                          float *d_out, int width, int n, int past);
-// latents of positions first .. first + rows - 1 as a split matrix [rows][pieces * rank_pad]
-int latent_gather_launch(hm_ctx *ctx, const LatentShape &s, const uint16_t *ring, uint16_t *d_out, int first, int rows);
+// The same in place, for attention over rows as wide as the projection leaves them
+bool latent_q_turns_in_place(const LatentShape &s, const RowSource &q, int width);
+int latent_q_turn_launch(hm_ctx *ctx, const LatentShape &s, const RowSource &q, float *d_q, const float *cos_tab, const float *sin_tab, int n, int past);
+// latents of positions first .. first + rows - 1 as a split matrix [rows][pieces * rank_pad]; with heads (latent_heads_whole) also what
+// gemm_heads_nk leaves out of the keys and values: the rotated keys and zeros
+bool latent_heads_whole(const LatentShape &s, int kw, int vw);
+int latent_gather_launch(hm_ctx *ctx, const LatentShape &s, const uint16_t *ring, uint16_t *d_out, int first, int rows, const HeadRows *heads = nullptr);
 // keys [heads][cap][kw] and values [heads][cap][vw] as planes of s.pieces pieces (heads * cap * kw / vw elements
 // apart) from the expanded rows [rows][heads * dim | heads * vdim] f32 (the values start at column v_at) and the rotated keys
 int latent_kv_rows_launch(hm_ctx *ctx, const LatentShape &s, const RowSource &kv, int v_at, const uint16_t *ring, uint16_t *d_k,

@@ -547,6 +547,64 @@ __global__ __launch_bounds__(256) void latent_rows_kernel(LatentRowsArgs a) {
         split_store(row, a.q_rank_pad, i, i < a.q_rank ? (source_at(a.down, t, i) * inv) * a.q_norm[i] : 0.f, a.q_pieces);
 }
 
+// The same rows, one wavefront each: a row's vectors (VEC a lane) are asked for at once and stay in registers between the sum of squares and
+// the write-out, and nothing waits at a barrier. (The workgroup a row above reads every value twice, one after the other: 2047 rows of 768 and
+// 512 + 64 values 15.7 us, 6.2 here. Rows of more than 2048 values, 1024 in K slices, or of no whole vectors stay there.)
+template <int VEC, int PARTS>
+__global__ __launch_bounds__(256) void latent_rows_wave_kernel(LatentRowsArgs a) {
+    const LatentShape &s = a.s;
+    const int lane = threadIdx.x & 63, job = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (job >= 2 * a.n) return;
+    const bool cache = job >= a.n;
+    const int t = cache ? job - a.n : job, pos = a.past + t;
+    const int rank = cache ? s.rank : a.q_rank, pad = cache ? s.rank_pad : a.q_rank_pad;
+    const float *norm = cache ? a.kv_norm : a.q_norm;
+    const size_t at = (size_t)t * a.down.ld + (cache ? a.q_rank_pad : 0);
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v[VEC], w[VEC], key = zero, other = zero, c = zero, sn = zero;
+    const int i0 = lane * 4, half = s.rot_dims / 2;  // the rotated key: rot_pad <= 256
+#pragma unroll
+    for (int j = 0; j < VEC; j++) {
+        const int i = i0 + j * 256, k = min(i, rank - 4);
+        v[j] = sum_parts_upto<PARTS, f32x4>(a.down.p, at + k, a.down.parts, a.down.stride);
+        w[j] = *reinterpret_cast<const f32x4 *>(norm + k);
+        if (i >= rank) v[j] = zero;
+    }
+    if (cache && i0 < s.rot_dim) {
+        key = sum_parts_upto<PARTS, f32x4>(a.down.p, at + rank + i0, a.down.parts, a.down.stride);
+        if (i0 < s.rot_dims) {
+            other = sum_parts_upto<PARTS, f32x4>(a.down.p, at + rank + (i0 < half ? i0 + half : i0 - half), a.down.parts, a.down.stride);
+            c = *reinterpret_cast<const f32x4 *>(a.cos_tab + (size_t)pos * s.rot_dims + i0);
+            sn = *reinterpret_cast<const f32x4 *>(a.sin_tab + (size_t)pos * s.rot_dims + i0);
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < VEC; j++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) ss += v[j][k] * v[j][k];
+    const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)rank + a.eps);
+    uint16_t *row = cache ? a.ring + (size_t)(pos % s.ring_rows) * s.row_elems() : a.q_split + (size_t)t * a.q_pieces * pad;
+    const int width = cache ? s.row_width() : pad, pieces = cache ? s.pieces : a.q_pieces;
+#pragma unroll
+    for (int j = 0; j < VEC; j++) {
+        const int i = i0 + j * 256;
+        if (i >= pad) break;
+        f32x4 y;
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] = i < rank ? (v[j][k] * inv) * w[j][k] : 0.f;
+        split_store4(row, width, i, y, pieces);
+    }
+    if (cache && i0 < s.rot_pad) {
+        f32x4 y = key;
+        if (i0 < s.rot_dims) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) y[k] = i0 < half ? key[k] * c[k] - other[k] * sn[k] : key[k] * c[k] + other[k] * sn[k];
+        }
+        split_store4(row, width, s.rank_pad + i0, y, pieces);
+    }
+}
+
 // V elements of a query row a thread; V = 4 wants every part of a row to be whole vectors
 template <int V>
 __global__ __launch_bounds__(256) void latent_q_rows_kernel(LatentShape s, RowSource q, const float *__restrict__ cos_tab,
@@ -583,11 +641,49 @@ __global__ __launch_bounds__(256) void latent_q_rows_kernel(LatentShape s, RowSo
     }
 }
 
-// 16 bytes a thread
-__global__ __launch_bounds__(256) void latent_gather_kernel(LatentShape s, const uint16_t *__restrict__ ring, uint16_t *__restrict__ out,
-                                                            int first, size_t total) {
+// The rotation of the queries where they lie: rows of heads * (dim + rot_dim) as the attention reads them, so that only the pairs that turn
+// are touched, four of each half a thread (2047 rows of 16 heads, 64 of 192 values turned: 13.8 us copied, 5.7 here).
+__global__ __launch_bounds__(256) void latent_q_turn_kernel(LatentShape s, float *__restrict__ q, int ld, const float *__restrict__ cos_tab,
+                                                            const float *__restrict__ sin_tab, int past, size_t total) {
     const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= total) return;
+    const int half = s.rot_dims / 2, r = (int)(e % (half / 4)) * 4, h = (int)(e / (half / 4) % s.heads), t = (int)(e / (half / 4) / s.heads);
+    float *lo = q + (size_t)t * ld + h * (s.dim + s.rot_dim) + s.dim + r, *hi = lo + half;
+    const size_t tab = (size_t)(past + t) * s.rot_dims + r;
+    const f32x4 x = *reinterpret_cast<const f32x4 *>(lo), o = *reinterpret_cast<const f32x4 *>(hi);
+    const f32x4 c0 = *reinterpret_cast<const f32x4 *>(cos_tab + tab), s0 = *reinterpret_cast<const f32x4 *>(sin_tab + tab);
+    const f32x4 c1 = *reinterpret_cast<const f32x4 *>(cos_tab + tab + half), s1 = *reinterpret_cast<const f32x4 *>(sin_tab + tab + half);
+    f32x4 a, b;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        a[k] = x[k] * c0[k] - o[k] * s0[k];
+        b[k] = o[k] * c1[k] + x[k] * s1[k];
+    }
+    *reinterpret_cast<f32x4 *>(lo) = a;
+    *reinterpret_cast<f32x4 *>(hi) = b;
+}
+
+// 16 bytes a thread. Behind the `total` pieces of the split matrix (HeadTails): what the rows of k and v have behind the columns that the
+// product writes, of every head: the rotated key that they share, and zeros.
+struct HeadTails {
+    uint16_t *k = nullptr, *v = nullptr;
+    int kw = 0, vw = 0, cap = 0;
+    size_t pieces = 0;  // of eight elements
+};
+__global__ __launch_bounds__(256) void latent_gather_kernel(LatentShape s, const uint16_t *__restrict__ ring, uint16_t *__restrict__ out,
+                                                            int first, size_t total, HeadTails ht) {
+    size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= total) {
+        e -= total;
+        if (e >= ht.pieces) return;
+        const int kt = (ht.kw - s.dim) / 8, per = kt + (ht.vw - s.vdim) / 8, i = (int)(e % per);
+        const int h = (int)(e / per % s.heads), r = (int)(e / per / s.heads);
+        u32x4 x = {0u, 0u, 0u, 0u};
+        if (i < s.rot_dim / 8) x = ld128(ring + (size_t)((first + r) % s.ring_rows) * s.row_elems() + s.rank_pad + i * 8);
+        uint16_t *to = i < kt ? ht.k + ((size_t)h * ht.cap + r) * ht.kw + s.dim + i * 8 : ht.v + ((size_t)h * ht.cap + r) * ht.vw + s.vdim + (i - kt) * 8;
+        *reinterpret_cast<u32x4 *>(to) = x;
+        return;
+    }
     const int per_row = s.pieces * s.rank_pad / 8, c = (int)(e % per_row) * 8;
     const size_t r = e / per_row;
     const int p = c / s.rank_pad, i = c % s.rank_pad;
@@ -732,7 +828,36 @@ int latent_rows_launch(hm_ctx *ctx, const LatentRowsArgs &a) {
                "latent_rows: bad arguments");
     HM_REQUIRE(ctx, a.q_rank > 0 && a.q_rank_pad >= a.q_rank && a.q_pieces >= 1 && a.q_pieces <= 3 && a.down.ld >= a.q_rank_pad + a.s.rank + a.s.rot_dim &&
                         a.down.parts >= 1 && a.down.parts <= MAX_SUM_PARTS, "latent_rows: bad shape");
-    hipLaunchKernelGGL(latent_rows_kernel, dim3(a.n, 2), dim3(256), 0, ctx->stream, a);
+    // a wavefront a row where a row is whole vectors and fits its registers
+    const int pad = std::max(a.q_rank_pad, a.s.rank_pad);
+    auto aligned = [](const void *p, size_t n) { return (uintptr_t)p % n == 0; };
+    if (pad <= (a.down.parts == 1 ? 2048 : 1024) && a.s.rot_pad <= 256 && a.q_rank % 4 == 0 && a.q_rank_pad % 4 == 0 && a.s.rank % 4 == 0 && a.s.rot_dim % 4 == 0 && a.s.rot_dims % 8 == 0 &&
+        a.s.rot_dims <= a.s.rot_dim && a.down.ld % 4 == 0 && a.down.stride % 4 == 0 && !a.down.bias && aligned(a.down.p, 16) && aligned(a.q_norm, 16) &&
+        aligned(a.kv_norm, 16) && aligned(a.cos_tab, 16) && aligned(a.sin_tab, 16) && aligned(a.q_split, 8) && aligned(a.ring, 8)) {
+        const dim3 g((2 * a.n + 3) / 4), b(256);
+        if (pad <= 512 && a.down.parts == 1) hipLaunchKernelGGL((latent_rows_wave_kernel<2, 1>), g, b, 0, ctx->stream, a);
+        else if (pad <= 1024 && a.down.parts == 1) hipLaunchKernelGGL((latent_rows_wave_kernel<4, 1>), g, b, 0, ctx->stream, a);
+        else if (a.down.parts == 1) hipLaunchKernelGGL((latent_rows_wave_kernel<8, 1>), g, b, 0, ctx->stream, a);
+        else if (pad <= 512) hipLaunchKernelGGL((latent_rows_wave_kernel<2, MAX_SUM_PARTS>), g, b, 0, ctx->stream, a);
+        else hipLaunchKernelGGL((latent_rows_wave_kernel<4, MAX_SUM_PARTS>), g, b, 0, ctx->stream, a);
+    } else {
+        hipLaunchKernelGGL(latent_rows_kernel, dim3(a.n, 2), dim3(256), 0, ctx->stream, a);
+    }
+    HM_LAUNCH_CHECK(ctx);
+    return HM_OK;
+}
+
+bool latent_q_turns_in_place(const LatentShape &s, const RowSource &q, int width) {
+    return q.parts == 1 && !q.bias && width == s.dim + s.rot_dim && s.dim % 4 == 0 && s.rot_dim % 4 == 0 && s.rot_dims % 8 == 0 && s.rot_dims <= s.rot_dim &&
+           q.ld >= s.heads * width && q.ld % 4 == 0 && ((uintptr_t)q.p % 16) == 0;
+}
+
+int latent_q_turn_launch(hm_ctx *ctx, const LatentShape &s, const RowSource &q, float *d_q, const float *cos_tab, const float *sin_tab, int n, int past) {
+    HM_REQUIRE(ctx, d_q && d_q == q.p && cos_tab && sin_tab && n > 0 && past >= 0 && latent_q_turns_in_place(s, q, s.dim + s.rot_dim) &&
+                        ((uintptr_t)cos_tab % 16) == 0 && ((uintptr_t)sin_tab % 16) == 0, "latent_q_turn: bad arguments");
+    const size_t total = (size_t)n * s.heads * (s.rot_dims / 8);
+    if (total == 0) return HM_OK;
+    hipLaunchKernelGGL(latent_q_turn_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, s, d_q, q.ld, cos_tab, sin_tab, past, total);
     HM_LAUNCH_CHECK(ctx);
     return HM_OK;
 }
@@ -754,12 +879,22 @@ int latent_q_rows_launch(hm_ctx *ctx, const LatentShape &s, const RowSource &q, 
     return HM_OK;
 }
 
-int latent_gather_launch(hm_ctx *ctx, const LatentShape &s, const uint16_t *ring, uint16_t *d_out, int first, int rows) {
+int latent_gather_launch(hm_ctx *ctx, const LatentShape &s, const uint16_t *ring, uint16_t *d_out, int first, int rows, const HeadRows *heads) {
     HM_REQUIRE(ctx, ring && d_out && first >= 0 && rows > 0 && rows <= s.ring_rows && ((uintptr_t)d_out % 16) == 0, "latent_gather: bad arguments");
     const size_t total = (size_t)rows * s.pieces * s.rank_pad / 8;
-    hipLaunchKernelGGL(latent_gather_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, s, ring, d_out, first, total);
+    HeadTails t;
+    if (heads) {
+        HM_REQUIRE(ctx, latent_heads_whole(s, heads->kw, heads->vw) && heads->k && heads->v && heads->cap >= rows && ((uintptr_t)heads->k % 16) == 0 &&
+                            ((uintptr_t)heads->v % 16) == 0, "latent_gather: bad heads");
+        t = HeadTails{heads->k, heads->v, heads->kw, heads->vw, heads->cap, (size_t)rows * s.heads * ((heads->kw - s.dim + heads->vw - s.vdim) / 8)};
+    }
+    hipLaunchKernelGGL(latent_gather_kernel, dim3((unsigned)((total + t.pieces + 255) / 256)), dim3(256), 0, ctx->stream, s, ring, d_out, first, total, t);
     HM_LAUNCH_CHECK(ctx);
     return HM_OK;
+}
+
+bool latent_heads_whole(const LatentShape &s, int kw, int vw) {
+    return s.pieces == 1 && s.dim % 8 == 0 && s.rot_dim % 8 == 0 && s.vdim % 8 == 0 && kw % 8 == 0 && vw % 8 == 0 && kw >= s.dim + s.rot_dim && vw >= s.vdim;
 }
 
 int latent_kv_rows_launch(hm_ctx *ctx, const LatentShape &s, const RowSource &kv, int v_at, const uint16_t *ring, uint16_t *d_k,

@@ -461,6 +461,26 @@ def test_files_that_do_not_fit_are_named(ctx, tmp_path):
     m.close()
 
 
+# q latents of two, four and eight vectors a lane, cache rows of both, parts of rows that are no whole vectors (the workgroup a row);
+# queries that turn where they lie (192 = 128 + 64 wide), with a part that does not turn, and wider rows than the projection's;
+# keys and values written by their product, with columns behind them (head rows of 64 / 128), a head's end inside a tile, and 24 rows of few
+LATENTS = {
+    "turned_in_place": dict(heads=5, dim=128, rot_dim=64, rot_dims=64, vdim=128, q_rank=96, kv_rank=64),
+    "half_turned": dict(heads=3, dim=128, rot_dim=64, rot_dims=24, vdim=120, q_rank=1000, kv_rank=192),
+    "wider_rows": dict(heads=7, dim=24, rot_dim=8, rot_dims=8, vdim=40, q_rank=260, kv_rank=600),
+    "wide_latents": dict(heads=2, dim=64, rot_dim=64, rot_dims=48, vdim=64, q_rank=1030, kv_rank=1024),
+    "widest_latents": dict(heads=2, dim=64, rot_dim=64, rot_dims=64, vdim=64, q_rank=1540, kv_rank=128),
+    "odd_parts": dict(heads=3, dim=26, rot_dim=6, rot_dims=6, vdim=30, q_rank=70, kv_rank=64),
+}
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("name", list(LATENTS))
+def test_latent_rows_of_a_prompt(ctx, name, dtype):
+    cfg = bf.config([bf.attn(window=150, **LATENTS[name])])
+    check(ctx, cfg, 333, dtype, cuts=(24, 190))
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("n", [70, 300])
 def test_gate_rows_from_slices_and_whole(ctx, n, dtype):
