@@ -9,6 +9,8 @@
 //       last-arriver fold in fixed order).
 // These are HBM-bandwidth kernels: algorithmic traffic is K*N*2 bytes of weights per call.
 #include "gemv_bf16.h"
+
+#include <algorithm>
 #include "matrix_memory.h"
 
 // ─────────────────────────── [N][K] stream layout ───────────────────────────
@@ -434,6 +436,26 @@ __device__ __forceinline__ float gelu_tanh_dev(float z) {
     return 0.5f * z * (1.0f + tanhf(u));
 }
 
+// what becomes of a row's sum outside the paired epilogue
+__device__ __forceinline__ void finish_row(const GemvArgs &a, int epi, int row, float v) {
+    if (a.bias) v = v + a.bias[row];
+    if (epi == GEMV_EPI_CONV) {
+        const GemvConv &cv = a.conv;
+        if (row < cv.rows) {
+            const int pos = cv.state->pos;
+            float u = cv.b[row] + cv.w[(size_t)(cv.taps - 1) * cv.rows + row] * v;
+            for (int j = 1; j < cv.taps && j <= pos; j++)
+                u = fmaf(cv.w[(size_t)(cv.taps - 1 - j) * cv.rows + row], cv.ring[(size_t)((pos - j) % cv.taps) * cv.rows + row], u);
+            cv.ring[(size_t)(pos % cv.taps) * cv.rows + row] = v;
+            v = cv.silu ? u / (1.0f + expf(-u)) : u;
+        } else if (cv.gelu_from && row >= cv.gelu_from) {
+            v = gelu_tanh_dev(v);
+        }
+    }
+    if (epi == GEMV_EPI_RESIDUAL) v = a.epilogue_residual[row] + v;
+    a.out[row] = v;
+}
+
 template <int R, int NC, int PRO>
 __global__ __launch_bounds__(GEMV_THREADS) void gemv_bf16_nk_splitk_kernel(GemvArgs a, int epi) {
     __shared__ float part[GEMV_WAVES][R];
@@ -594,24 +616,135 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_bf16_nk_splitk_kernel(GemvA
             a.out[(row0 + 2 * t) / 2] = homura::gated_act(a.act, gte, up);
         }
     } else if (t < R && row0 + t < N) {
-        float v = row_sum(t);
-        const int row = row0 + t;
-        if (a.bias) v = v + a.bias[row];
-        if (epi == GEMV_EPI_CONV) {
-            const GemvConv &cv = a.conv;
-            if (row < cv.rows) {
-                const int pos = cv.state->pos;
-                float u = cv.b[row] + cv.w[(size_t)(cv.taps - 1) * cv.rows + row] * v;
-                for (int j = 1; j < cv.taps && j <= pos; j++)
-                    u = fmaf(cv.w[(size_t)(cv.taps - 1 - j) * cv.rows + row], cv.ring[(size_t)((pos - j) % cv.taps) * cv.rows + row], u);
-                cv.ring[(size_t)(pos % cv.taps) * cv.rows + row] = v;
-                v = cv.silu ? u / (1.0f + expf(-u)) : u;
-            } else if (cv.gelu_from && row >= cv.gelu_from) {
-                v = gelu_tanh_dev(v);
-            }
+        finish_row(a, epi, row0 + t, row_sum(t));
+    }
+}
+
+// Products behind a prologue, rows of up to 2048. Of the kernel above four wavefronts take a row whatever it fills, and every workgroup brings and
+// norms the activation row for its few rows of weights (at 1024 -> 4096 twice their bytes). Here the W wavefronts that a row takes keep their pieces
+// of the normed row in registers and stay: a workgroup takes G sets of R rows, then the next G R that are its, asked for ahead of the sums
+// of those at hand. The sums are those of the kernel above, bit for bit.
+// us a decode step, that kernel (eight rows a workgroup from 8192 outputs on, four below) / here: Qwen2.5-1.5B 1354 / 1266, Qwen2.5-0.5B 854 / 773,
+// TinyLlama 960 / 927, Nokuvik 1024 wide 1631 / 1475, Ludalix 1024 wide 1268 / 1203. What is in flight is enough with eight wavefronts a CU; more
+// rows, sets or workgroups wait behind one another's prologues.
+template <int W, int G, int R, int PRO>
+__global__ __launch_bounds__(WAVE * W * G) void gemv_bf16_nk_rolling_kernel(GemvArgs a, int epi) {
+    __shared__ float part[2][W * G][R];
+    __shared__ float red[W * G];
+    const int K = a.K, N = a.N;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wave = threadIdx.x / WAVE, sub = wave / W, first = sub * W;
+    const int k = ((wave - first) * WAVE + lane) * 8, kc = k < K ? k : 0;
+    const bool ok = k < K;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const int step = gridDim.x * G * R;
+    int row0 = (blockIdx.x * G + sub) * R;
+    f32x4 x0, x1, p0 = zero, p1 = zero, n0, n1, q0, q1;
+    auto ask = [&](const float *p, f32x4 &u, f32x4 &v) {
+        u = *reinterpret_cast<const f32x4 *>(p + kc);
+        v = *reinterpret_cast<const f32x4 *>(p + kc + 4);
+    };
+    ask(a.x, x0, x1);
+    if constexpr (PRO == 2) ask(a.post_norm_w, q0, q1);
+    if (a.prologue_residual) ask(a.prologue_residual, p0, p1);
+    if (a.norm_w) ask(a.norm_w, n0, n1);
+    u32x4 wv[2][R];
+    auto request = [&](int set, int row) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int at = row + r < N ? row + r : N - 1;  // clamp: stays inside the matrix
+            wv[set][r] = ld128_stream(static_cast<const uint16_t *>(a.w) + (size_t)at * K + kc);
         }
-        if (epi == GEMV_EPI_RESIDUAL) v = a.epilogue_residual[row] + v;
-        a.out[row] = v;
+    };
+    request(0, row0);
+    __builtin_amdgcn_sched_barrier(0);  // every request above goes out before any arithmetic below
+    auto mean_square = [&](const f32x4 &u, const f32x4 &v) {
+        float ss = u.x * u.x + u.y * u.y + u.z * u.z + u.w * u.w;
+        ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+        ss = wave_sum(ok ? ss : 0.f);
+        if (lane == 0) red[wave] = ss;
+        __syncthreads();
+        float tot = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; w++) tot += red[first + w];
+        return tot / (float)(a.norm_dim ? a.norm_dim : K);
+    };
+    if constexpr (PRO == 2) {
+        const float inv = 1.0f / sqrtf(mean_square(p0, p1) + a.eps);
+        p0 = (p0 * inv) * q0;
+        p1 = (p1 * inv) * q1;
+        __syncthreads();  // red is used again below
+    }
+    if (a.prologue_residual) {
+        x0 = x0 + p0;
+        x1 = x1 + p1;
+    }
+    if (blockIdx.x == 0 && sub == 0 && a.resid_out && ok) {
+        *reinterpret_cast<f32x4 *>(a.resid_out + k) = x0;
+        *reinterpret_cast<f32x4 *>(a.resid_out + k + 4) = x1;
+    }
+    if (a.norm_w) {
+        const float inv = 1.0f / sqrtf(mean_square(x0, x1) + a.eps);
+        x0 = (x0 * inv) * n0;
+        x1 = (x1 * inv) * n1;
+    }
+    float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+    for (int j = 0; j < 8; j++) xv[j] = ok ? xv[j] : 0.f;
+    // (the sets of rows of a workgroup end together: its last sub-group's rows may lie past N)
+    const int groups = (N + G * R - 1) / (G * R);
+    auto finish = [&](int set, int row) {
+        float acc[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r] = wave_sum(dot8(wv[set][r], xv, 0.f));
+        if (lane == 0) {
+#pragma unroll
+            for (int r = 0; r < R; r++) part[set][wave][r] = acc[r];
+        }
+        __syncthreads();
+        const int t = threadIdx.x, base = row - sub * R;
+        auto row_sum = [&](int i) {  // row i of the G R
+            const float *p = &part[set][i / R * W][i % R];
+            float v = p[0];
+#pragma unroll
+            for (int w = 1; w < W; w++) v += p[w * R];
+            return v;
+        };
+        if (epi == GEMV_EPI_SILU_MUL_PAIRS) {
+            if (t < G * R / 2 && base + 2 * t < N) a.out[(base + 2 * t) / 2] = homura::gated_act(a.act, row_sum(2 * t), row_sum(2 * t + 1));
+        } else if (t < G * R && base + t < N) {
+            finish_row(a, epi, base + t, row_sum(t));
+        }
+    };
+    for (int g = blockIdx.x; g < groups; g += 2 * gridDim.x, row0 += 2 * step) {
+        if (g + (int)gridDim.x < groups) request(1, row0 + step);
+        finish(0, row0);
+        if (g + (int)gridDim.x >= groups) break;
+        if (g + 2 * (int)gridDim.x < groups) request(0, row0 + 2 * step);
+        finish(1, row0 + step);
+    }
+}
+
+constexpr int ROLL_R = 4, ROLL_K = 4 * WAVE * 8;
+
+template <int W, int G>
+int launch_rolling(hm_ctx *ctx, const GemvArgs &a, int epi) {
+    const int groups = (a.N + G * ROLL_R - 1) / (G * ROLL_R), grid = std::min(groups, 4 / G * ctx->num_cus);
+    if (a.post_norm_w) hipLaunchKernelGGL((gemv_bf16_nk_rolling_kernel<W, G, ROLL_R, 2>), dim3(grid), dim3(WAVE * W * G), 0, ctx->stream, a, epi);
+    else hipLaunchKernelGGL((gemv_bf16_nk_rolling_kernel<W, G, ROLL_R, 1>), dim3(grid), dim3(WAVE * W * G), 0, ctx->stream, a, epi);
+    HM_LAUNCH_CHECK(ctx);
+    return HM_OK;
+}
+
+// K <= ROLL_K. One set of rows a workgroup and four workgroups a CU, or two and two: two halve what is read of the activations, and lose where
+// a row takes four wavefronts, or three and there are few rows. us a step with one / two, 1536 -> 17920 1275 / 1266, 896 -> 9728 786 / 773,
+// 2048 -> 11264 934 / 937, 1024 -> 3104 to 6144 (Nokuvik) 1487 / 1475, 1536 -> 2048 1275 / 1280, 2048 -> 2560 929 / 946.
+int launch_rolling_any(hm_ctx *ctx, const GemvArgs &a, int epi) {
+    switch ((a.K + 511) / 512) {
+    case 1: return launch_rolling<1, 2>(ctx, a, epi);
+    case 2: return launch_rolling<2, 2>(ctx, a, epi);
+    case 3: return a.N >= 8192 ? launch_rolling<3, 2>(ctx, a, epi) : launch_rolling<3, 1>(ctx, a, epi);
+    default: return launch_rolling<4, 1>(ctx, a, epi);
     }
 }
 
@@ -622,7 +755,7 @@ int launch_splitk(hm_ctx *ctx, const GemvArgs &a, int epi, bool pro) {
         if constexpr (NC == 1 && R == 4)
             hipLaunchKernelGGL((gemv_bf16_nk_splitk_kernel<R, NC, 3>), dim3(grid), dim3(GEMV_THREADS), 0, ctx->stream, a, epi);
     } else if (pro) {
-        if constexpr (NC <= 4 && R >= 4) {
+        if constexpr (NC > 1 && NC <= 4 && R >= 4) {  // (shorter rows: gemv_bf16_nk_rolling_kernel)
             if (a.post_norm_w)
                 hipLaunchKernelGGL((gemv_bf16_nk_splitk_kernel<R, NC, 2>), dim3(grid), dim3(GEMV_THREADS), 0, ctx->stream, a, epi);
             else
@@ -654,13 +787,15 @@ bool try_splitk(hm_ctx *ctx, const GemvArgs &a, int epi, int *rc) {
     const int per_wg = WAVE * 8 * GEMV_WAVES;  // k covered by one chunk of each wavefront
     const int nc = (a.K + per_wg - 1) / per_wg;
     if (nc > (pro ? 4 : 8) || ((a.K < 512 || a.N >= 65536) && !only_here)) return false;
+    if (pro && a.K <= ROLL_K) {
+        *rc = launch_rolling_any(ctx, a, epi);
+        return true;
+    }
     // Rows a workgroup, the best of 1 .. 16 measured over 25 shapes. Every workgroup reads the activation
     // pieces itself (4 bytes per k, 12 with residual and norm weights, against 2 R of weights), so a prologue
     // wants more rows; few short rows want one.
     const size_t bytes = (size_t)2 * a.K * a.N;
-    // With a prologue, us with 4 / 8 rows over 24 gate|up shapes of K 512 .. 3072: 512 -> 12288 8.2 / 7.0, 512 -> 24576 12.9 / 10.7,
-    // 1024 -> 8192 6.8 / 6.9, 1024 -> 12288 9.3 / 8.4, 2048 -> 8192 9.2 / 8.6, 3072 -> 8192 13.0 / 11.4, 3072 -> 24576 32.4 / 27.4;
-    // 16 rows gain nothing more (32 steps of Qwen2.5-1.5B, 1536 -> 17920: 40.8 ms with 4, 40.1 with 8, 40.7 with 16).
+    // With a prologue, us with 4 / 8 rows: 3072 -> 8192 13.0 / 11.4, 3072 -> 24576 32.4 / 27.4.
     int r;
     if (pro) r = a.N >= 8192 ? 8 : 4;
     else if (a.heads.raw) r = 4;  // (12 bytes per k and the gates' exponentials: 1024 -> 1024 5.3 / 4.1 / 3.9 us with 1 / 2 / 4 rows)
@@ -671,7 +806,7 @@ bool try_splitk(hm_ctx *ctx, const GemvArgs &a, int epi, int *rc) {
     HM_SPLITK(1, 1) HM_SPLITK(1, 2) HM_SPLITK(1, 3) HM_SPLITK(1, 4) HM_SPLITK(1, 5) HM_SPLITK(1, 6) HM_SPLITK(1, 7) HM_SPLITK(1, 8)
     HM_SPLITK(2, 1) HM_SPLITK(2, 2) HM_SPLITK(2, 3) HM_SPLITK(2, 4) HM_SPLITK(2, 5) HM_SPLITK(2, 6) HM_SPLITK(2, 7) HM_SPLITK(2, 8)
     HM_SPLITK(4, 1) HM_SPLITK(4, 2) HM_SPLITK(4, 3) HM_SPLITK(4, 4) HM_SPLITK(4, 5) HM_SPLITK(4, 6) HM_SPLITK(4, 7) HM_SPLITK(4, 8)
-    HM_SPLITK(8, 1) HM_SPLITK(8, 2) HM_SPLITK(8, 3) HM_SPLITK(8, 4)
+    HM_SPLITK(8, 2) HM_SPLITK(8, 3) HM_SPLITK(8, 4)
 #undef HM_SPLITK
     return false;
 }

@@ -488,3 +488,11 @@ def test_gate_rows_from_slices_and_whole(ctx, n, dtype):
     for width in (1100, 96):
         cfg = bf.config([bf.scan(inner=64, state=16), bf.scan(inner=130, state=33), bf.recurrence(), bf.recurrence(width=66, blocks=2)], width=width)
         check(ctx, cfg, n, dtype, cuts=(n // 3,))
+
+
+# one to four wavefronts a row, the last of them part of the way; one round of rows, several with a last one of few rows; the paired, the
+# plain and the convolution epilogue behind one norm and two
+@pytest.mark.parametrize("width,ff", [(72, 4107), (520, 33), (1000, 4200), (1024, 8300), (1100, 37), (1536, 4500), (1800, 8200), (2048, 37)])
+def test_decode_products_behind_a_norm(ctx, width, ff):
+    cfg = bf.config([bf.scan(inner=64, state=16, ff=ff), bf.recurrence(width=66, blocks=2, ff=ff), bf.attn(heads=3)], width=width)
+    check(ctx, cfg, 9, "bf16", prefill_min=0)
