@@ -9,6 +9,9 @@
 // the last workgroup of a head's splits where those sit on one die (die_fold.h), else by a second, tiny kernel.
 // Algorithmic HBM traffic: 2 * kv_len * HD * 2 bytes per (batch, kv head).
 #include "attention.h"
+
+#include <type_traits>
+
 #include "bf16_pieces.h"
 #include "die_fold.h"
 
@@ -23,8 +26,6 @@ __device__ __forceinline__ void unpack8(const u32x4 w, float *f) {
     f[4] = bf16_lo(w.z); f[5] = bf16_hi(w.z);
     f[6] = bf16_lo(w.w); f[7] = bf16_hi(w.w);
 }
-
-constexpr int NRG_MAX = 8;  // row groups per wavefront held in registers (K and V each)
 
 // Optional prologue fused into the attention kernel (decode plan, batch 1): the raw q|k|v row
 // produced by the QKV projection goes through the per-head QK-norm and RoPE of the reference's
@@ -118,7 +119,8 @@ __device__ __forceinline__ void fold_here(const float *po, const float *pml, flo
     if (v < vecs) *reinterpret_cast<f32x4 *>(out + v * 4) = O;
 }
 
-template <int HD, int G>
+// NRG: row groups of the chunk that a wavefront holds in registers (K and V each).
+template <int HD, int G, int NRG>
 __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
     const float *__restrict__ q, uint16_t *__restrict__ kcache, uint16_t *__restrict__ vcache,
     float *__restrict__ out, float *part_o, float *part_ml, int kvh,
@@ -152,23 +154,24 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
     const size_t head_base = ((size_t)b * kvh + kvhd) * max_len * HD;
     const uint16_t *kbase = kcache + head_base + (size_t)n0 * HD + dl * 8;
     const uint16_t *vbase = vcache + head_base + (size_t)n0 * HD + dl * 8;
-    const int nrg = chunk / (ATT_WAVES * RPI);  // row groups per wavefront (<= NRG_MAX)
 
-    // The live length first (one scalar load): splits past it leave without touching memory.
-    const int kv_len = state ? state->pos + 1 : kv_len_arg;
-    const int nsplit = (kv_len + chunk - 1) / chunk;  // live splits; the grid may be larger
-    if (split >= nsplit) return;
-    const int cnt = min(kv_len, n0 + chunk) - n0;
-
-    // ── every live K and V row of the chunk is requested before anything waits ──
-    u32x4 kreg[NRG_MAX], vreg[NRG_MAX];
+    // ── every K and V row of the chunk is requested before anything waits, the live length among it: rows past it are dropped below, and
+    //    splits past it leave. (Addresses held inside the cache rather than loads behind conditions: the compiler waited for the first of those
+    //    ahead of the others, a second trip to memory, and the length was a third. 0.8 to 0.9 us a call: 4 sequences x 14 heads on 2 x 64, 700 rows
+    //    19.3 -> 18.4 with its caller's share; 24 tokens of Qwen2.5-0.5B at 150 rows 16579 -> 15984, of the 1.5B shape at 700 30916 -> 30566.) ──
+    const int last = (state ? max_len : kv_len_arg) - 1 - n0;
+    if (last < 0) return;
+    const int pos_now = *(state ? &state->pos : reinterpret_cast<const int *>(q));  // (without a cursor any word will do)
+    u32x4 kreg[NRG], vreg[NRG];
 #pragma unroll
-    for (int i = 0; i < NRG_MAX; i++) {
-        const int row = (i * ATT_WAVES + wave) * RPI + sub;
-        const bool ok = i < nrg && row < cnt;
-        kreg[i] = ok ? ld128_stream(kbase + (size_t)row * HD) : u32x4{0u, 0u, 0u, 0u};
-        vreg[i] = ok ? ld128_stream(vbase + (size_t)row * HD) : u32x4{0u, 0u, 0u, 0u};
+    for (int i = 0; i < NRG; i++) {
+        const int row = min((i * ATT_WAVES + wave) * RPI + sub, last);
+        kreg[i] = ld128_stream(kbase + (size_t)row * HD);
+        vreg[i] = ld128_stream(vbase + (size_t)row * HD);
     }
+    const int kv_len = state ? pos_now + 1 : kv_len_arg;
+    const int nsplit = (kv_len + chunk - 1) / chunk;  // live splits; the grid may be larger
+    const int cnt = min(kv_len, n0 + chunk) - n0;
     const bool fused = fuse.qkv_raw != nullptr;
     const int pos = kv_len - 1;
     const bool owner = fused && split == nsplit - 1;  // this chunk holds the new row
@@ -251,6 +254,7 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
         for (int i = tid; i < G * HD; i += ATT_THREADS)
             qs[i / HD][i % HD] = i < g_here * HD ? q[((size_t)b * H + kvhd * g_total + g0) * HD + i] : 0.f;
     }
+    if (split >= nsplit) return;  // (only here: the loads above would be put behind an earlier exit)
     __syncthreads();
 
     float qv[G][8];
@@ -262,21 +266,19 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
     // ── scores = (Q.K^T) * scale; rows outside the live range (and the not-yet-written new
     //    row) are dropped here ──
 #pragma unroll
-    for (int i = 0; i < NRG_MAX; i++) {
-        if (i < nrg) {
-            const int row = (i * ATT_WAVES + wave) * RPI + sub;
-            const bool live = row < cnt && !(owner && row == new_row);
-            if (!live) vreg[i] = u32x4{0u, 0u, 0u, 0u};  // the new row's slot is not written yet
-            float kf[8];
-            unpack8(kreg[i], kf);
+    for (int i = 0; i < NRG; i++) {
+        const int row = (i * ATT_WAVES + wave) * RPI + sub;
+        const bool live = row < cnt && !(owner && row == new_row);
+        if (!live) vreg[i] = u32x4{0u, 0u, 0u, 0u};  // the new row's slot is not written yet
+        float kf[8];
+        unpack8(kreg[i], kf);
 #pragma unroll
-            for (int gi = 0; gi < G; gi++) {
-                float p = 0.f;
+        for (int gi = 0; gi < G; gi++) {
+            float p = 0.f;
 #pragma unroll
-                for (int e = 0; e < 8; e++) p = fmaf(kf[e], qv[gi][e], p);
-                p = row_group_sum<LPR>(p);
-                if (dl == 0 && live) sc[gi * chunk + row] = p * scale;
-            }
+            for (int e = 0; e < 8; e++) p = fmaf(kf[e], qv[gi][e], p);
+            p = row_group_sum<LPR>(p);
+            if (dl == 0 && live) sc[gi * chunk + row] = p * scale;
         }
     }
     if (owner && wave == 0) {  // the new row's score from the rounded values in LDS
@@ -318,17 +320,15 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
 #pragma unroll
         for (int e = 0; e < 8; e++) acc[gi][e] = 0.f;
 #pragma unroll
-    for (int i = 0; i < NRG_MAX; i++) {
-        if (i < nrg) {
-            const int row = (i * ATT_WAVES + wave) * RPI + sub;
-            float vf[8];
-            unpack8(vreg[i], vf);
+    for (int i = 0; i < NRG; i++) {
+        const int row = (i * ATT_WAVES + wave) * RPI + sub;
+        float vf[8];
+        unpack8(vreg[i], vf);
 #pragma unroll
-            for (int gi = 0; gi < G; gi++) {
-                const float p = row < cnt ? sc[gi * chunk + row] : 0.f;
+        for (int gi = 0; gi < G; gi++) {
+            const float p = row < cnt ? sc[gi * chunk + row] : 0.f;
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[gi][e] = fmaf(p, vf[e], acc[gi][e]);
-            }
+            for (int e = 0; e < 8; e++) acc[gi][e] = fmaf(p, vf[e], acc[gi][e]);
         }
     }
     if (owner && wave == 0 && sub == 0) {
@@ -793,17 +793,22 @@ int launch_attn(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
     float *part_ml = part_o + pairs * nsplit * G * HD;
     AttnFuse f{a.qkv_raw, a.qw, a.kw, a.cos_tab, a.sin_tab, a.eps};
     if (a.phase != AttnArgs::FOLD_ONLY) {
-        static bool lds_limit_raised = false;  // per instantiation; large groups need more than 64 KiB
-        if (lds > 64 * 1024 && !lds_limit_raised) {
-            HM_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(&gqa_decode_attn_kernel<HD, GB>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-            lds_limit_raised = true;
-        }
         HM_REQUIRE(ctx, lds <= 96 * 1024, "gqa_decode_attn: LDS need %zu too large", lds);
-        hipLaunchKernelGGL((gqa_decode_attn_kernel<HD, GB>), die.splits ? dim3(homura::die_grid(die.groups, nsplit)) : dim3(nsplit, a.kvh * NG, a.B),
-                           dim3(ATT_THREADS), lds, ctx->stream, a.q, const_cast<uint16_t *>(a.kcache),
-                           const_cast<uint16_t *>(a.vcache), a.out, part_o, part_ml, a.kvh, a.max_len,
-                           a.kv_len, chunk, a.scale, a.state, (int)front, f, G, die);
+        constexpr int GROUP = ATT_WAVES * (WAVE / (HD / 8));  // rows
+        auto go = [&](auto steps) -> int {
+            constexpr int NRG = decltype(steps)::value * 32 / GROUP;
+            static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gqa_decode_attn_kernel<HD, GB, NRG>),
+                                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+            HM_HIP(ctx, raised);
+            hipLaunchKernelGGL((gqa_decode_attn_kernel<HD, GB, NRG>), die.splits ? dim3(homura::die_grid(die.groups, nsplit)) : dim3(nsplit, a.kvh * NG, a.B),
+                               dim3(ATT_THREADS), lds, ctx->stream, a.q ? a.q : a.qkv_raw, const_cast<uint16_t *>(a.kcache),
+                               const_cast<uint16_t *>(a.vcache), a.out, part_o, part_ml, a.kvh, a.max_len,
+                               a.kv_len, chunk, a.scale, a.state, (int)front, f, G, die);
+            return HM_OK;
+        };
+        const int rc = chunk == 32 ? go(std::integral_constant<int, 1>{}) : chunk == 64 ? go(std::integral_constant<int, 2>{})
+                     : chunk == 96 ? go(std::integral_constant<int, 3>{}) : go(std::integral_constant<int, 4>{});
+        if (rc != HM_OK) return rc;
         HM_LAUNCH_CHECK(ctx);
     }
     // nsplit is the grid's split count: 1 means no call can ever need a fold
