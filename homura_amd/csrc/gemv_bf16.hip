@@ -694,6 +694,10 @@ __global__ __launch_bounds__(WAVE * W * G) void gemv_bf16_nk_rolling_kernel(Gemv
     // (the sets of rows of a workgroup end together: its last sub-group's rows may lie past N)
     const int groups = (N + G * R - 1) / (G * R);
     auto finish = [&](int set, int row) {
+        if ((wave - first + 1) * WAVE * 8 > K) {  // (a weight that is no number does not reach the row by way of a zero)
+#pragma unroll
+            for (int r = 0; r < R; r++) wv[set][r] = ok ? wv[set][r] : u32x4{0u, 0u, 0u, 0u};
+        }
         float acc[R];
 #pragma unroll
         for (int r = 0; r < R; r++) acc[r] = wave_sum(dot8(wv[set][r], xv, 0.f));

@@ -48,15 +48,19 @@ __global__ __launch_bounds__(GTHREADS) void gemv_k8_kernel(const float *__restri
     f32x4 xr[NC][4], ar[NS][4], nr[NN][4];
     u32x4 qw[NC][R];
     uint32_t sub[NC][R], dd[NC][R];
-    const float *second = fuse.x2 ? fuse.x2 : fuse.res_in;
+    // All chunks but the last are whole. There a piece past the row's end reads the last one again and drops it, and an operand that is not there is the
+    // row itself, which nobody uses: behind a condition the compiler waited for a load ahead of all others, a trip to memory of its own (24 tokens of
+    // Qwen2.5-1.5B, Q4_K_M mix, 28850 -> 27000 us).
+    const float *second = fuse.x2 ? fuse.x2 : fuse.res_in ? fuse.res_in : x, *norm = fuse.norm_w ? fuse.norm_w : x;
+    auto live = [&](int c) { return c < NC - 1 || ((c * WPS + wis) * WAVE + lane) * 16 < K; };
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-        const int k = ((c * WPS + wis) * WAVE + lane) * 16;
+        const int k = min(((c * WPS + wis) * WAVE + lane) * 16, K - 16);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            xr[c][j] = k < K ? *reinterpret_cast<const f32x4 *>(x + k + 4 * j) : zero4;
-            if constexpr (MODE >= 1) ar[c][j] = (second && k < K) ? *reinterpret_cast<const f32x4 *>(second + k + 4 * j) : zero4;
-            if constexpr (MODE == 2) nr[c][j] = (fuse.norm_w && k < K) ? *reinterpret_cast<const f32x4 *>(fuse.norm_w + k + 4 * j) : zero4;
+            xr[c][j] = *reinterpret_cast<const f32x4 *>(x + k + 4 * j);
+            if constexpr (MODE >= 1) ar[c][j] = *reinterpret_cast<const f32x4 *>(second + k + 4 * j);
+            if constexpr (MODE == 2) nr[c][j] = *reinterpret_cast<const f32x4 *>(norm + k + 4 * j);
         }
     }
 #pragma unroll
@@ -75,6 +79,12 @@ __global__ __launch_bounds__(GTHREADS) void gemv_k8_kernel(const float *__restri
     // every request above goes out before any arithmetic below (left alone, the compiler requests three rows,
     // waits for the activations and deals the other rows' requests out between the products)
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        xr[NC - 1][j] = live(NC - 1) ? xr[NC - 1][j] : zero4;
+        if constexpr (MODE >= 1) ar[NC - 1][j] = live(NC - 1) ? ar[NC - 1][j] : zero4;
+        if constexpr (MODE == 2) nr[NC - 1][j] = live(NC - 1) ? nr[NC - 1][j] : zero4;
+    }
     // the light ops of the quantised plan in front of this product (reference src/hf/emitter_quant.rs:713-791,
     // :985-1103), arithmetic as in the stand-alone kernels
     if constexpr (MODE >= 1) {

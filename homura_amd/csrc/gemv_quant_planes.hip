@@ -363,21 +363,33 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
     f32x4 xr[NC][XV], ar[FUSED ? NC : 1][FUSED ? XV : 1], nr[MODE == 2 ? NC : 1][MODE == 2 ? XV : 1];
     u32x4 qw[NC][R];
     uint32_t sc[NC][R];
-    const float *second = fuse.x2 ? fuse.x2 : fuse.res_in;
+    // All chunks but the last are whole. There a unit past the row's end reads the last one again and drops it, and an operand that is not there is
+    // the row itself, which nobody uses: behind a condition the compiler waited for a load ahead of all others, a trip to memory of its own.
+    // Rows of three chunks and more, which it does not wait in, leave those requests out: reading again costs them more. us for 24 tokens, waiting / here
+    // (no conditions at any length): Qwen2.5-0.5B Q4_0 17100 / 16250, TinyLlama Q8_0 18150 / 17750, Qwen2.5-1.5B Q8_0 25450 / 25160 (25740).
+    constexpr bool STRAIGHT = NC <= 2;
+    const float *second = fuse.x2 ? fuse.x2 : fuse.res_in, *norm = fuse.norm_w;
+    if (STRAIGHT && !second) second = x;
+    if (STRAIGHT && !norm) norm = x;
+    auto live = [&](int c) { return c < NC - 1 || ((c * WPS + wis) * L + ul) * KPL < K; };
+    auto ask = [&](const float *p, int k, f32x4 &v) {
+        if constexpr (STRAIGHT) v = *reinterpret_cast<const f32x4 *>(p + min(k, K - KPL + k % KPL));
+        else v = p && k < K ? *reinterpret_cast<const f32x4 *>(p + k) : zero4;
+    };
 #pragma unroll
     for (int c = 0; c < NC; c++) {
         const int k = ((c * WPS + wis) * L + ul) * KPL;
 #pragma unroll
         for (int j = 0; j < XV; j++) {
-            xr[c][j] = k < K ? *reinterpret_cast<const f32x4 *>(x + k + 4 * j) : zero4;
-            if constexpr (FUSED) ar[c][j] = (second && k < K) ? *reinterpret_cast<const f32x4 *>(second + k + 4 * j) : zero4;
-            if constexpr (MODE == 2) nr[c][j] = (fuse.norm_w && k < K) ? *reinterpret_cast<const f32x4 *>(fuse.norm_w + k + 4 * j) : zero4;
+            ask(x, k + 4 * j, xr[c][j]);
+            if constexpr (FUSED) ask(second, k + 4 * j, ar[c][j]);
+            if constexpr (MODE == 2) ask(norm, k + 4 * j, nr[c][j]);
         }
     }
 #pragma unroll
     for (int c = 0; c < NC; c++) {
         const int k = ((c * WPS + wis) * L + ul) * KPL;
-        const int kc = k < K ? k : 0;  // units past the row end re-read its first one against activations of zero
+        const int kc = min(k, K - KPL);  // units past the row end re-read its last one against activations of zero
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int row = min(row0 + r * (WAVE / L) + sub, N - 1);  // rows past the end re-read the last one
@@ -392,6 +404,12 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above goes out before any arithmetic below
+#pragma unroll
+    for (int j = 0; j < XV && STRAIGHT; j++) {
+        xr[NC - 1][j] = live(NC - 1) ? xr[NC - 1][j] : zero4;
+        if constexpr (FUSED) ar[NC - 1][j] = live(NC - 1) ? ar[NC - 1][j] : zero4;
+        if constexpr (MODE == 2) nr[NC - 1][j] = live(NC - 1) ? nr[NC - 1][j] : zero4;
+    }
     // the light ops of the quantised plan in front of this product (reference src/hf/emitter_quant.rs:985-1103)
     if constexpr (FUSED) {
         if (fuse.x2) {
@@ -442,7 +460,6 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
     for (int r = 0; r < R; r++) a[r] = 0.f;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-        const bool live = ((c * WPS + wis) * L + ul) * KPL < K;
         float xv[KPL], sx = 0.f, sx_first = 0.f;
 #pragma unroll
         for (int j = 0; j < XV; j++)
@@ -464,7 +481,7 @@ __global__ __launch_bounds__(PTHREADS) void gemv_planes_splitk_kernel(const floa
         for (int r = 0; r < R; r++) {
             float d = f16_bits_to_f32((uint16_t)sc[c][r]);
             // a unit past the row's end (there is none but in the last chunk): an infinite scale times its zero activations would be NaN
-            if (RAW && c == NC - 1 && !live) d = 0.f;
+            if (c == NC - 1 && !live(c)) d = 0.f;
             const uint32_t w[4] = {qw[c][r].x, qw[c][r].y, qw[c][r].z, qw[c][r].w};
             float t = 0.f;
             if (QT == 0) {

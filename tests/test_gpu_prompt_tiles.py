@@ -200,6 +200,30 @@ def test_q8_0_row_with_an_infinite_scale(ctx, K):
         buf.free()
 
 
+# one, two and four wavefronts a row, one chunk to three, units past the row's end in the last one (Q4_0: rows that are cut at all)
+@pytest.mark.parametrize("block", [0, -1])
+@pytest.mark.parametrize("fmt,K", [("q8_0", k) for k in (544, 1056, 2080, 4128, 6176, 8960)] + [("q4_0", k) for k in (4128, 6176, 8960)])
+def test_planes_row_with_an_infinite_scale(ctx, fmt, K, block):
+    """As above from planes, the infinite scale in the first block or in the last."""
+    N, size = 5, 34 if fmt == "q8_0" else 18
+    raw = (synth.q8_0_blocks if fmt == "q8_0" else synth.q4_0_blocks)(51, N * K // 32, 0.01).reshape(N, K // 32, size).copy()
+    x = np.abs(synth.normal_f32(52, K)) + np.float32(0.1)
+    dx, dout = ctx.to_device(x), ctx.empty(N)
+    got = []
+    for inf in (False, True):
+        if inf:
+            raw[2, block, :2], raw[2, block, 2:] = (0x00, 0x7C), 3 if fmt == "q8_0" else 0xCC
+        dw = ctx.to_device(raw)
+        planes = ctx.pack_quant_planes(DTYPE_Q8_0 if fmt == "q8_0" else DTYPE_Q4_0, dw, N, K)
+        (ctx.gemv_q8_0_planes if fmt == "q8_0" else ctx.gemv_q4_0_planes)(dx, planes, dout, 1, K, N)
+        got.append(dout.download(np.float32, (N,)))
+        dw.free()
+        planes.free()
+    assert got[1][2] == np.inf and np.array_equal(np.delete(got[0], 2), np.delete(got[1], 2))
+    for buf in (dx, dout):
+        buf.free()
+
+
 @pytest.mark.parametrize("n", [127, 255, 256, 300, 1025, 2048])
 def test_selective_scan_in_segments(ctx, n):
     """A chunk scanned in segments leaves the logits that the same tokens give one portion of at most 100 after the other
