@@ -7,7 +7,8 @@
 // cover a row, 64/(HD/8) rows per wavefront instruction. Scores live in LDS; softmax is f32.
 // Partial (o, max, sum) triples go to the workspace and are folded per (batch, kv head) in an order that does not depend on timing: by
 // the last workgroup of a head's splits where those sit on one die (die_fold.h), else by a second, tiny kernel.
-// Algorithmic HBM traffic: 2 * kv_len * HD * 2 bytes per (batch, kv head).
+// Algorithmic HBM traffic: 2 * kv_len * HD * 2 bytes per (batch, kv head), in the decode plan up to a chunk's rows more: it asks for the last live
+// chunk before it knows where that ends.
 #include "attention.h"
 
 #include <type_traits>
@@ -124,7 +125,7 @@ template <int HD, int G, int NRG>
 __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
     const float *__restrict__ q, uint16_t *__restrict__ kcache, uint16_t *__restrict__ vcache,
     float *__restrict__ out, float *part_o, float *part_ml, int kvh,
-    int max_len, int kv_len_arg, int chunk, float scale, const DecodeState *__restrict__ state,
+    int max_len, int kv_len_arg, int chunk, int sure, float scale, const DecodeState *__restrict__ state,
     int lds_front, AttnFuse fuse, int g_total, DieFold die) {
     constexpr int LPR = HD / 8;      // lanes per row
     constexpr int RPI = WAVE / LPR;  // rows per wavefront instruction
@@ -155,12 +156,19 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
     const uint16_t *kbase = kcache + head_base + (size_t)n0 * HD + dl * 8;
     const uint16_t *vbase = vcache + head_base + (size_t)n0 * HD + dl * 8;
 
-    // ── every K and V row of the chunk is requested before anything waits, the live length among it: rows past it are dropped below, and
-    //    splits past it leave. (Addresses held inside the cache rather than loads behind conditions: the compiler waited for the first of those
-    //    ahead of the others, a second trip to memory, and the length was a third. 0.8 to 0.9 us a call: 4 sequences x 14 heads on 2 x 64, 700 rows
-    //    19.3 -> 18.4 with its caller's share; 24 tokens of Qwen2.5-0.5B at 150 rows 16579 -> 15984, of the 1.5B shape at 700 30916 -> 30566.) ──
-    const int last = (state ? max_len : kv_len_arg) - 1 - n0;
+    // ── every K and V row of the chunk is requested before anything waits, in the splits that begin inside the `sure` rows the live length among
+    //    it: rows past it are dropped below. (Addresses held inside the cache rather than loads behind conditions: the compiler waited for the
+    //    first of those ahead of the others, a second trip to memory, and the length was a third.) Splits behind those rows look at the length
+    //    first and leave if they are past it: rows that nobody needs cost those that are needed their share of the memory, more so
+    //    the more KV heads there are. us a decode step at 150 / 1500 / 5000 live rows with conditions / every split asking at once / here: 12 heads on 2 x 128
+    //    28 layers 919 / 929 / 1107, 900 / 904 / 1095, 895 / 902 / 1088; 16 on 8 x 128, 28 layers 648 / 660 / 861, 642 / 644 / 875, 623 / 634 / 836; 32 x 64, 12 layers
+    //    491 / 498 / 615, 493 / 496 / 623, 481 / 489 / 588; 32 x 128, 6 layers 362 / 377 / 454, 376 / 378 / 484, 361 / 369 / 442. ──
+    int last = (state ? max_len : kv_len_arg) - 1 - n0;
     if (last < 0) return;
+    if (n0 >= sure) {
+        last = min(last, state->pos - n0);
+        if (last < 0) return;
+    }
     const int pos_now = *(state ? &state->pos : reinterpret_cast<const int *>(q));  // (without a cursor any word will do)
     u32x4 kreg[NRG], vreg[NRG];
 #pragma unroll
@@ -254,7 +262,7 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
         for (int i = tid; i < G * HD; i += ATT_THREADS)
             qs[i / HD][i % HD] = i < g_here * HD ? q[((size_t)b * H + kvhd * g_total + g0) * HD + i] : 0.f;
     }
-    if (split >= nsplit) return;  // (only here: the loads above would be put behind an earlier exit)
+    if (split >= nsplit) return;  // (rows that were not live after all; only here: the loads above would be put behind an earlier exit)
     __syncthreads();
 
     float qv[G][8];
@@ -795,6 +803,7 @@ int launch_attn(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
     if (a.phase != AttnArgs::FOLD_ONLY) {
         HM_REQUIRE(ctx, lds <= 96 * 1024, "gqa_decode_attn: LDS need %zu too large", lds);
         constexpr int GROUP = ATT_WAVES * (WAVE / (HD / 8));  // rows
+        const int sure = a.state ? a.sure : 0x7fffffff;
         auto go = [&](auto steps) -> int {
             constexpr int NRG = decltype(steps)::value * 32 / GROUP;
             static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gqa_decode_attn_kernel<HD, GB, NRG>),
@@ -803,7 +812,7 @@ int launch_attn(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
             hipLaunchKernelGGL((gqa_decode_attn_kernel<HD, GB, NRG>), die.splits ? dim3(homura::die_grid(die.groups, nsplit)) : dim3(nsplit, a.kvh * NG, a.B),
                                dim3(ATT_THREADS), lds, ctx->stream, a.q ? a.q : a.qkv_raw, const_cast<uint16_t *>(a.kcache),
                                const_cast<uint16_t *>(a.vcache), a.out, part_o, part_ml, a.kvh, a.max_len,
-                               a.kv_len, chunk, a.scale, a.state, (int)front, f, G, die);
+                               a.kv_len, chunk, sure, a.scale, a.state, (int)front, f, G, die);
             return HM_OK;
         };
         const int rc = chunk == 32 ? go(std::integral_constant<int, 1>{}) : chunk == 64 ? go(std::integral_constant<int, 2>{})

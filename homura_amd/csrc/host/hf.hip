@@ -5,8 +5,8 @@
 #include <cmath>
 #include <cstdlib>
 
+#include "../../../include/homura_amd_bench.h"
 #include "../attention.h"
-#include "../light_ops.h"
 #include "../decode_fused.h"
 #include "../kquant_planes8.h"
 #include "../gemm_kquant_i8.h"
@@ -52,6 +52,12 @@ int attn_span_for(int live, int max_len) {
     int span = live <= ATTN_UNSPLIT ? ATTN_UNSPLIT : 2048;
     while (span < live && span < max_len) span *= 2;
     return std::min(span, max_len);
+}
+// The fewest live rows that a span serves
+int attn_span_from(int span, int max_len) {
+    int from = 1;
+    for (int s = attn_span_for(1, max_len); s < span && s < max_len; s = attn_span_for(from, max_len)) from = s + 1;
+    return from;
 }
 int attn_chunk_for(int span, int fixed) { return fixed ? fixed : span > ATTN_UNSPLIT && span <= 2048 ? 64 : 128; }
 
@@ -838,6 +844,7 @@ int HfModel::emit_transformer_plan() {
                 a.scale = (float)(1.0 / std::sqrt((double)hd));  // f64 -> f32 constant, emitter.rs:719
                 a.state = sc.plan->state();
                 a.span = sc.plan->attn_span();
+                a.sure = attn_span_from(a.span, a.max_len);
                 a.fixed_chunk = attn_chunk_for(a.span, att_chunk_fixed);
                 a.phase = phase;
                 return a;
@@ -1453,6 +1460,7 @@ int HfModel::emit_transformer_plan_quant() {
                 a.scale = (float)(1.0 / std::sqrt((double)hd));
                 a.state = sc.plan->state();
                 a.span = sc.plan->attn_span();
+                a.sure = attn_span_from(a.span, a.max_len);
                 a.fixed_chunk = attn_chunk_for(a.span, att_chunk_fixed);
                 a.phase = phase;
                 return a;
@@ -2577,3 +2585,11 @@ int HfModel::reset_kv_cache() {
 }
 
 }  // namespace homura
+
+extern "C" int hm_test_attn_rows(int live, int max_len, int *span, int *chunk, int *sure) {
+    if (live < 1 || max_len < live || !span || !chunk || !sure) return HM_ERR_INVALID;
+    *span = homura::attn_span_for(live, max_len);
+    *chunk = homura::attn_chunk_for(*span, 0);
+    *sure = homura::attn_span_from(*span, max_len);
+    return HM_OK;
+}

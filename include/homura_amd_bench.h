@@ -60,6 +60,10 @@ int hm_test_fill_lds(hm_ctx *ctx, uint32_t word);
  * weight format on a chip of `cus` CUs, and the most that the product of m <= rows rows writes (all its K slices). Host only. */
 int hm_test_prompt_product(int hm_dtype, int rows, int m, int k, int n, int cus, long long *floats_held, long long *floats_written);
 
+/* Test support: the rows that the decode attention's grid covers in a step of `live` live rows over a cache of max_len, the rows of a split, and
+ * the rows that its splits ask for without having looked at the live length. Host only. */
+int hm_test_attn_rows(int live, int max_len, int *span, int *chunk, int *sure);
+
 /* Test support: the tile and K slices (at most max_parts) of a product of gemm_tiles_mfma.hip on a chip of `cus` CUs; the few-rows kernel's
  * tile of 32 or 64 rows by 32 or 64 columns where that takes it. kind 0: two f16 pieces with column factors, 1: with block scales, 2: one bf16 piece.
  * k a multiple of 64. Host only. */
