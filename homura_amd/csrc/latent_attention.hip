@@ -3,6 +3,7 @@
 
 #include <algorithm>
 
+#include "../../include/homura_amd_bench.h"
 #include "row_pieces.h"
 
 namespace {
@@ -578,12 +579,20 @@ __global__ __launch_bounds__(256) void latent_rows_wave_kernel(LatentRowsArgs a)
             sn = *reinterpret_cast<const f32x4 *>(a.sin_tab + (size_t)pos * s.rot_dims + i0);
         }
     }
-    float ss = 0.f;
+    // The squares in the order of the workgroup kernels, to the bit: a lane's four columns are a quad of those kernels' threads, a row of sixteen
+    // lanes one of their wavefronts (wg_sum256), so that a token's cache row is the same whichever kernel writes it.
+    f32x4 sq = zero;
 #pragma unroll
     for (int j = 0; j < VEC; j++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) ss += v[j][k] * v[j][k];
-    const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)rank + a.eps);
+        for (int k = 0; k < 4; k++) sq[k] = fmaf(v[j][k], v[j][k], sq[k]);
+    float ss = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+    ss += dpp_move<0xB1, 0xF>(ss, 0.f);
+    ss += dpp_move<0x4E, 0xF>(ss, 0.f);
+    ss += dpp_move<0x141, 0xF>(ss, 0.f);
+    ss += dpp_move<0x140, 0xF>(ss, 0.f);
+    auto row_total = [&](int r) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ss), 16 * r)); };
+    const float inv = 1.0f / sqrtf(((row_total(0) + row_total(1)) + (row_total(2) + row_total(3))) / (float)rank + a.eps);
     uint16_t *row = cache ? a.ring + (size_t)(pos % s.ring_rows) * s.row_elems() : a.q_split + (size_t)t * a.q_pieces * pad;
     const int width = cache ? s.row_width() : pad, pieces = cache ? s.pieces : a.q_pieces;
 #pragma unroll
@@ -911,3 +920,31 @@ int latent_kv_rows_launch(hm_ctx *ctx, const LatentShape &s, const RowSource &kv
 }
 
 }  // namespace homura
+
+extern "C" int hm_test_latent_rows(hm_ctx *ctx, const float *down, int ld, int parts, const float *q_norm, const float *kv_norm, const float *cos_tab,
+                                   const float *sin_tab, int q_rank, int rank, int rot, int pieces, int n, int past, float eps, uint16_t *q_split,
+                                   uint16_t *ring) {
+    HM_CHECK_CTX(ctx);
+    homura::LatentRowsArgs a;
+    a.s.heads = a.s.dim = a.s.vdim = 1;
+    a.s.rank = rank;
+    a.s.rot_dim = a.s.rot_dims = rot;
+    a.s.rank_pad = (rank + 31) / 32 * 32;
+    a.s.rot_pad = (rot + 31) / 32 * 32;
+    a.s.pieces = a.q_pieces = pieces;
+    a.s.ring_rows = past + n;
+    a.down = homura::RowSource{down, ld, parts, (size_t)n * ld, nullptr};
+    a.q_norm = q_norm;
+    a.kv_norm = kv_norm;
+    a.cos_tab = cos_tab;
+    a.sin_tab = sin_tab;
+    a.q_rank = q_rank;
+    a.q_rank_pad = (q_rank + 31) / 32 * 32;
+    a.n = n;
+    a.past = past;
+    a.eps = eps;
+    a.q_split = q_split;
+    a.ring = ring;
+    const int rc = homura::latent_rows_launch(ctx, a);
+    return rc == HM_OK ? hm_sync(ctx) : rc;
+}

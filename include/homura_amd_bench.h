@@ -90,6 +90,12 @@ int hm_test_qkv_product(hm_ctx *ctx, const void *x, const float *norm_w, int dty
                         const float *bias, const float *qw, const float *kw, const float *cos, const float *sin, float *q, uint16_t *kcache,
                         uint16_t *vcache, int max_len, int past, float eps, int *pays);
 
+/* Test support: the latents' rows of a prompt: down [parts][n][ld] f32 (q latent, padded to a multiple of 32 | kv latent | rotated key), norms, tables
+ * [past + n][rot], to q_split [n][pieces * q_rank padded] and ring [past + n][pieces * (rank padded + rot padded)]. Rows that are no
+ * whole vectors (an odd ld) take the kernel of a workgroup a row. */
+int hm_test_latent_rows(hm_ctx *ctx, const float *down, int ld, int parts, const float *q_norm, const float *kv_norm, const float *cos_tab,
+                        const float *sin_tab, int q_rank, int rank, int rot, int pieces, int n, int past, float eps, uint16_t *q_split, uint16_t *ring);
+
 /* Test support: a gate|up product of one bf16 piece with its activation, a [m][k], b [n][k] as (gate, up) pairs of rows, out [m][n / 2] bf16; kind 0
  * silu(g) u, 1 the clamped sigmoid gate. *pays: whether the prompt pass of a list-of-layers model would take it. */
 int hm_test_gated_product(hm_ctx *ctx, const uint16_t *a, const uint16_t *b, uint16_t *out, int m, int k, int n, int kind, float limit, float slope,

@@ -496,3 +496,33 @@ def test_gate_rows_from_slices_and_whole(ctx, n, dtype):
 def test_decode_products_behind_a_norm(ctx, width, ff):
     cfg = bf.config([bf.scan(inner=64, state=16, ff=ff), bf.recurrence(width=66, blocks=2, ff=ff), bf.attn(heads=3)], width=width)
     check(ctx, cfg, 9, "bf16", prefill_min=0)
+
+
+# one to eight vectors a lane, in one slice and in several, ranks that fill no whole wavefront, one and three pieces
+@pytest.mark.parametrize("q_rank,rank,rot,parts,pieces,n,past", [(768, 512, 64, 1, 1, 33, 0), (100, 36, 8, 1, 3, 5, 2), (512, 132, 128, 1, 1, 7, 0),
+                                                                  (2048, 1024, 64, 1, 1, 9, 3), (1536, 512, 64, 1, 3, 2, 0), (4, 4, 0, 1, 1, 1, 0),
+                                                                  (256, 512, 32, 3, 1, 6, 1), (1024, 260, 16, 8, 3, 4, 0)])
+def test_latent_rows_have_the_same_bits_from_either_kernel(ctx, q_rank, rank, rot, parts, pieces, n, past):
+    """A wavefront a row, and a workgroup a row (which a row stride of no whole vectors takes; the decode step writes its cache row with the same
+    code): the same values in another place give the same bits."""
+    rng = np.random.default_rng(q_rank + rank + parts)
+    pad = lambda w: (w + 31) // 32 * 32
+    q_pad, wide = pad(q_rank), pad(q_rank) + rank + rot
+    values = rng.standard_normal((parts, n, wide)).astype(np.float32)
+    q_norm, kv_norm = (1 + 0.1 * rng.standard_normal((2, max(q_pad, pad(rank))))).astype(np.float32)
+    cos, sin = rng.standard_normal((2, past + n, max(rot, 4))).astype(np.float32)
+    dev = [ctx.to_device(v) for v in (q_norm, kv_norm, cos.reshape(-1)[:(past + n) * max(rot, 4)], sin.reshape(-1)[:(past + n) * max(rot, 4)])]
+    got = []
+    for ld in (wide + 3 & ~3, (wide + 3 & ~3) + 1):
+        down = np.full((parts, n, ld), np.nan, np.float32)
+        down[:, :, :wide] = values
+        d = ctx.to_device(down)
+        q, ring = (ctx.to_device(np.full(size + 64, 0x7B7B, np.uint16)) for size in (n * pieces * q_pad, (past + n) * pieces * (pad(rank) + pad(rot))))
+        ctx._check(ctx.lib.hm_test_latent_rows(ctx.h, d.ptr, ld, parts, *(b.ptr for b in dev), q_rank, rank, rot, pieces, n, past, 1e-6, q.ptr, ring.ptr))
+        got.append((q.download(np.uint16), ring.download(np.uint16)))
+        for b in (d, q, ring):
+            b.free()
+    for b in dev:
+        b.free()
+    for wave, group in zip(*got):
+        assert np.all(wave[-64:] == 0x7B7B) and np.array_equal(wave, group)
