@@ -96,6 +96,7 @@ SIGNATURES = {
     "hm_test_prompt_rows": (_I, [_P, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P, _P, C.POINTER(_I)]),
     "hm_test_qkv_tail": (_I, [_P] * 8 + [_I] * 6 + [C.c_float]),
     "hm_test_gated_rows": (_I, [_P, _P, _P, _I, _P, _I, _I, _I, _I, _P, _P, C.POINTER(_I)]),
+    "hm_test_gated_down": (_I, [_P, _P, _P, _I, _P, _P] + [_I] * 4 + [_P]),
     "hm_test_qkv_product": (_I, [_P, _P, _P, _I, _P] + [_I] * 6 + [_P] * 8 + [_I] * 2 + [C.c_float, C.POINTER(_I)]),
     "hm_test_gated_product": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, C.c_float, C.c_float, C.POINTER(_I)]),
     "hm_test_attn_rows": (_I, [_I, _I] + [C.POINTER(_I)] * 3),

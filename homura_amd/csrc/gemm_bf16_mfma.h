@@ -64,8 +64,9 @@ int gemm_pieces_scaled_nk(hm_ctx *ctx, const uint16_t *d_a_split, const uint16_t
 // unscale[n]; block-scaled integers (d_scales) carry their factors in the scales, unscale is NULL then, and npad >= half_scale_cols(N). K % 64 == 0.
 // (gemm_half_wide: its widest tiles, gemm_pieces_mfma.hip; stages of 32 k)
 // gated (gate_scale with it): neighbouring columns are (gate, up) pairs, and silu(gate) up times gate_scale [N / 2] leaves as two f16
-// pieces, gated [M][2 (N / 2)], instead of d_c: one slice, N % 2 == 0. gemm_half_gated_pays: whether that is the quicker way, or slices and
+// pieces, the second times HALF_LOW (row_pieces.h), gated [M][2 (N / 2)], instead of d_c: one slice, N % 2 == 0. gemm_half_gated_pays: whether that is the quicker way, or slices and
 // silu_mul_half_launch behind them.
+// low: the second pieces come so, as the gated rows hold them.
 // tail (with head_dim 64 or 128): the product is a q|k|v projection of M = tail->S rows, and its workgroups hand their head rows on as
 // qkv_post_launch does: q [M][N] at tail->qkv, k and v in the caches, nothing to d_c. One slice. gemm_half_tail_pays as above.
 struct QkvPostArgs;
@@ -74,6 +75,7 @@ struct HalfProduct {
     const float *gate_scale = nullptr;
     uint16_t *gated = nullptr;
     const QkvPostArgs *tail = nullptr;
+    bool low = false;
 };
 bool gemm_half_tail_pays(bool scaled, int head_dim, int M, int K, int N, int cus, int max_parts);
 bool gemm_half_gated_pays(bool scaled, int M, int K, int N, int cus, int max_parts);

@@ -9,9 +9,12 @@
 //   a norm's output       |x_k| <= sqrt(dim) |w_k|                      one e per column, folded into the norm's weights
 //   attention's output    a mean of value rows, |v_j| <= sqrt(dim) |W_v[j] o w|_2 + |b_j| (Cauchy-Schwarz)   one e per value column
 //   SiLU(gate) up         |g_j u_j| <= dim |W_g[j] o w|_2 |W_u[j] o w|_2   one e per column, so that the gate|up product can write the
-//                         rows itself. Rows of normal values lie 2^10 to 2^11 below that (2^-28 of themselves is lost, f32's own rounding
-//                         2^-24). A row whose gates all lie far below zero is
-//                         off by no more than that. Where a column's factor would cost the down weights bits: one e per row, from its maximum
+//                         rows itself. Rows of normal values lie 2^10 to 2^12 below that, and rows of small gates anywhere below those, so the
+//                         second pieces are held 2^12 higher (HALF_LOW, row_pieces.h): 23 to 24 bits of values down to 2^-18 of a normal
+//                         row's, gates near -15; below, a bit less a binade. Where the row kernel writes the rows there is a factor per row
+//                         on top, from its largest value, and where a column's factor would cost the down weights bits, that one alone.
+//                         (Down product, error of a row relative to itself, gates at -12 / -20, from the product and from the row kernel: 4e-7 / 4e-6 to
+//                         1.2e-5, and 4e-7 / 1e-6. Second pieces as they are and no row factors: 1e-5 / 2e-2.)
 // What is multiplied into a column of the activations is divided out of that column of the weights, so a product needs one
 // factor per output row of the weights, 2^-r, which also puts the row's largest weight at 2^14 .. 2^15. All factors are powers
 // of two. A matrix takes this way only if every one of its weights is then an f16 exactly (bf16 weights: 31 binades of a row,

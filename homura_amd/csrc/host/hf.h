@@ -188,7 +188,7 @@ class HfModel : public DecoderModel {
     // The projections as f16 for the prompt pass (half_weights.h), built by finalize() within the prompt pass's weight budget. Per
     // layer: the groups' matrices (q|k|v, o, gate|up, down; rows interleaved as in the packed bf16 matrices) followed by their row
     // factors or block scales, the two norms' weights times their columns' factors, the value rows' factors, and the gated rows' column
-    // factors (none: those rows have factors of their own). A group that is
+    // factors (none: only factors by row). A group that is
     // ok without a matrix has it made in half_scratch_ for every chunk (a budget made smaller behind the first prompt).
     struct HalfLayer {
         Buffer w[4], norms, values, gated;

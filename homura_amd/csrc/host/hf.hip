@@ -2387,6 +2387,7 @@ int HfModel::prefill_chunk(const int32_t *d_ids, int n, float *h_logits) {
                 hp.gated = gated;
             }
             hp.tail = tail;
+            hp.low = g == 3;
             return gemm_half_nk(ctx_, rows, reinterpret_cast<const uint16_t *>(w), hp, quant ? f : nullptr, quant ? half_scale_cols(N) : 0, out, n, K,
                                 N, MP, &parts);
         }
@@ -2525,8 +2526,7 @@ int HfModel::prefill_chunk(const int32_t *d_ids, int n, float *h_logits) {
         if (rc == HM_OK) rc = project(l, 4, 2, lp.gate_up, hidden, gate_up, split, gated);
         i8 = i8_planes(l, 3, 6, 1, inter);
         if (rc == HM_OK && !gated && h3)
-            rc = silu_mul_half_launch(ctx_, gate_up, parts, split, by_column ? nullptr : p.row_unscale.as<float>(), n, inter,
-                                      by_column ? half_[l].gated.as<float>() : nullptr);
+            rc = silu_mul_half_launch(ctx_, gate_up, parts, split, p.row_unscale.as<float>(), n, inter, by_column ? half_[l].gated.as<float>() : nullptr);
         else if (rc == HM_OK && !gated) rc = silu_mul_split_launch(ctx_, gate_up, parts, split, np, n, inter, q8k(l, 6), q8k(l, 6) ? capture_at(l, 3) : nullptr,
                                                     i8 ? q8 : nullptr, i8 ? q8s : nullptr);
         if (rc == HM_OK) rc = project(l, 6, 1, lp.down, inter, proj_out, gated ? gated : split, nullptr);
@@ -2534,7 +2534,7 @@ int HfModel::prefill_chunk(const int32_t *d_ids, int n, float *h_logits) {
         if (rc != HM_OK) return rc;
         x = resid;
         res = proj_out;
-        res_scale = h3 && !by_column ? p.row_unscale.as<float>() : nullptr;
+        res_scale = h3 && !gated ? p.row_unscale.as<float>() : nullptr;
         res_parts = parts;
     }
     if (h_logits) {  // LM head (reference src/hf/emitter.rs:828-862) for every row

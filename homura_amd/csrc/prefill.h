@@ -58,8 +58,8 @@ int silu_mul_split_launch(hm_ctx *ctx, const float *d_gu, int parts, uint16_t *d
                           float *d_q8_scale = nullptr);
 
 // The same rows as two f16 pieces, each row times a power of two that puts its largest value at 2^14 .. 2^15; row_unscale [rows]
-// receives the inverse. With d_col_scale [inter] every column times its factor instead (half_gated_scales), and no row factors
-// (d_row_unscale NULL). inter <= SILU_HALF_MAX.
+// receives the inverse. With d_col_scale [inter] every column times its factor first (half_gated_scales). The second pieces are held times HALF_LOW
+// (row_pieces.h; HalfProduct::low). inter <= SILU_HALF_MAX.
 constexpr int SILU_HALF_MAX = 16384;
 int silu_mul_half_launch(hm_ctx *ctx, const float *d_gu, int parts, uint16_t *d_out_half, float *d_row_unscale, int rows, int inter,
                          const float *d_col_scale = nullptr);

@@ -83,6 +83,10 @@ int hm_test_prompt_rows(hm_ctx *ctx, int front, const void *x, const float *norm
 int hm_test_gated_rows(hm_ctx *ctx, const void *x, const float *norm_w, int dtype, const void *w, int fused, int m, int k, int inter,
                        uint16_t *out, float *scale, int *pays);
 
+/* Test support: those rows through the down product: down [k][inter], the same dtype (inter a multiple of 64), out [m][k] f32. */
+int hm_test_gated_down(hm_ctx *ctx, const void *x, const float *norm_w, int dtype, const void *w, const void *down, int fused, int m, int k,
+                       int inter, float *out);
+
 /* Test support: the q|k|v projection of the prompt pass in f16 pieces and its tail: x [S][k] f32 through RMSNorm (norm_w [k], eps), w
  * [(H + 2 kvh) hd][k] bf16 rows or Q8_0 / Q4_0 blocks; bias, and qw with kw, may be NULL. fused 1: the product's workgroups do the tail, 0: its slices go
  * through the row kernel. q [S][(H + 2 kvh) hd] (its q columns), caches [kvh][max_len][hd] rows past .. *pays: what the prompt pass would take. */

@@ -34,6 +34,18 @@ def weights(dtype, n, k, rng):
     return b, (q * d.astype(np.float64)[..., None]).reshape(n, k)
 
 
+def blocks(dtype, w):
+    """[n, k] values as Q8_0 / Q4_0 blocks, and what these stand for."""
+    n, k = w.shape
+    b, top = w.reshape(n, k // 32, 32), 127 if dtype == DTYPE_Q8_0 else 7
+    d = (np.abs(b).max(-1) / top).astype(np.float16)
+    q = np.rint(b / d.astype(np.float64)[..., None]).clip(-top, top)
+    raw = np.empty((n, k // 32, 34 if dtype == DTYPE_Q8_0 else 18), np.uint8)
+    raw[..., :2] = d[..., None].view(np.uint8)
+    raw[..., 2:] = q.astype(np.int8).view(np.uint8) if dtype == DTYPE_Q8_0 else (q[..., :16] + 8).astype(np.uint8) | (q[..., 16:] + 8).astype(np.uint8) << 4
+    return raw, (q * d.astype(np.float64)[..., None]).reshape(n, k)
+
+
 def product(ctx, front, x, norm_w, dtype, raw, n, half=1):
     m, k = x.shape[0], x.shape[1] // (2 if front == 1 else 1)
     dx, dn, dw = ctx.to_device(x), ctx.to_device(norm_w), ctx.to_device(raw)
@@ -341,6 +353,52 @@ def test_gated_rows_from_the_product(ctx, dtype, m, k, inter):
         for b in (out, scale):
             b.free()
     for b in (dx, dn, dw):
+        b.free()
+
+
+# the few-rows kernel's tiles (up to 32 and to 64 rows), 64 x 64 .. 64 x 192 and 128 x 128, 128 x 256 behind the gated rows
+@pytest.mark.parametrize("m,k,inter", [(7, 128, 320), (37, 896, 1088), (70, 320, 1152), (181, 1024, 3072), (700, 192, 2112), (2048, 1024, 1024)])
+@pytest.mark.parametrize("dtype", [DTYPE_BF16, DTYPE_Q8_0, DTYPE_Q4_0])
+def test_rows_of_small_gates(ctx, dtype, m, k, inter):
+    """Two rows whose gates all lie at -12 and at -20, each off a single column of the input so that the gates themselves are exact to f32's
+    rounding: their gated values are some 2^14 and 2^25 below what their columns' bounds allow for, and leave the down product as exact,
+    relative to themselves, as any other row: 2e-6, the bound of a row above five times over, and three roundings of a gate (the input's, the product's, the
+    block's scale), by which alone exp(gate) moves by that much of itself. The rows that the product wrote have column
+    factors only: what f16's smallest number leaves of the second piece, 2^-37 of the factor's inverse each, comes on top, in the norm of a sum of
+    independent roundings (one part in a million at -12)."""
+    print(f"dtype {dtype} {m} x {k} x {inter}", flush=True)
+    rng = np.random.default_rng(m + k + inter)
+    norm_w = np.ones(k, np.float32)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[3], x[m - 1] = 0, 0
+    x[3, 5], x[m - 1, 70] = -1, -1
+    gate = 0.02 * rng.standard_normal((inter, k))
+    gate[:, 5], gate[:, 70] = 12 * k ** -0.5, 20 * k ** -0.5
+    raw_g, gate = bf16(gate.astype(np.float32)) if dtype == DTYPE_BF16 else blocks(dtype, gate)
+    raw_u, up = weights(dtype, inter, k, rng)
+    raw_d, down = weights(dtype, k, inter, rng)
+    raw = np.ascontiguousarray(np.stack([raw_g, raw_u], 1).reshape(2 * inter, *raw_g.shape[1:]))
+    gate, up, down, rows = (v.astype(np.float64) for v in (gate, up, down, rows_of(0, x, norm_w)))
+    g = rows @ gate.T
+    y = g / (1 + np.exp(-g)) * (rows @ up.T)
+    want = y @ down.T
+    assert -14 < g[3].min() <= g[3].max() < -10 and -23 < g[m - 1].min() <= g[m - 1].max() < -17
+    bound = 1.01 ** 2 * k * np.linalg.norm(gate, axis=1) * np.linalg.norm(up, axis=1)
+    small = np.where((rows != 0).sum(1) == 1, -g.min(1), 0)
+    unscale = 2.0 ** (np.floor(np.log2(bound)) - 14)
+    floor = np.linalg.norm(down * 2.0 ** -37 * unscale) + np.sqrt(inter * k) * 2.0 ** -38 * np.abs(down * unscale).max()
+    dev = [ctx.to_device(v) for v in (x, norm_w, raw, raw_d)]
+    for fused in (1, 0):
+        out = ctx.to_device(np.full(m * k + 64, -77.0, np.float32))
+        ctx._check(ctx.lib.hm_test_gated_down(ctx.h, dev[0].ptr, dev[1].ptr, dtype, dev[2].ptr, dev[3].ptr, fused, m, k, inter, out.ptr))
+        got = out.download(np.float32)
+        out.free()
+        assert np.all(got[m * k:] == -77.0), "wrote past the end"
+        size, off = np.linalg.norm(want, axis=1), np.linalg.norm(got[:m * k].reshape(m, k) - want, axis=1)
+        print("fused" if fused else "row kernel", "small gates", (off / size)[[3, m - 1]], "all", np.max(np.delete(off / size, [3, m - 1])), flush=True)
+        assert floor < 5e-8 * size[3]
+        assert np.all(off <= (2e-6 + 3 * 2.0 ** -24 * small) * size + fused * floor)
+    for b in dev:
         b.free()
 
 
