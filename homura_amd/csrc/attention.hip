@@ -56,7 +56,8 @@ __device__ __forceinline__ float row_group_sum(float v) {
 // Splits folded by the last of their workgroups (die_fold.h): `splits` of the grid per group of heads, 0: in a launch of its own
 struct DieFold {
     int splits, groups;
-    unsigned int *arrived;
+    unsigned long long *arrived;
+    int *apart;
 };
 
 // The whole workgroup: heads <= 8 heads whose nsplit <= DIE_SPLITS_MAX partial results (o [HD]; max and sum) lie `all` heads apart, one head
@@ -375,7 +376,7 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_kernel(
         pml[tid * 2] = s_m[tid];
         pml[tid * 2 + 1] = s_l[tid];
     }
-    if (!die.splits || !homura::last_on_die(die.arrived, group, nsplit)) return;
+    if (!die.splits || !homura::last_on_die(die.arrived, group, nsplit, die.apart)) return;
     fold_here<HD>(part_o + (pair * nsplit * g_total + g0) * HD, part_ml + (pair * nsplit * g_total + g0) * 2,
                   out + ((size_t)b * H + kvhd * g_total + g0) * HD, g_here, nsplit, g_total);
 }
@@ -617,7 +618,7 @@ __global__ __launch_bounds__(ATT_THREADS) void gqa_decode_attn_stream_kernel(
         pml[tid * 2] = s_m[tid];
         pml[tid * 2 + 1] = s_l[tid];
     }
-    if (!die.splits || !homura::last_on_die(die.arrived, group, nsplit)) return;
+    if (!die.splits || !homura::last_on_die(die.arrived, group, nsplit, die.apart)) return;
     fold_here<HD>(part_o + pair * nsplit * G * HD, part_ml + pair * nsplit * G * 2, out + ((size_t)b * H + kvhd * G) * HD, G, nsplit, G);
 }
 
@@ -785,8 +786,8 @@ __global__ void kv_append_kernel(uint16_t *__restrict__ kc, uint16_t *__restrict
 // single heads slower again).
 constexpr int heads_a_workgroup(int g) { return g <= 4 ? g : 2; }
 DieFold die_fold(hm_ctx *ctx, long long groups, int nsplit, int chunk, int hd) {
-    if (!homura::die_fold_pays(ctx, groups, nsplit, 4.0 * groups * nsplit * chunk * hd)) return DieFold{0, 0, nullptr};
-    return DieFold{nsplit, (int)groups, ctx->counters};
+    if (!homura::die_fold_pays(ctx, groups, nsplit, 4.0 * groups * nsplit * chunk * hd)) return DieFold{0, 0, nullptr, nullptr};
+    return DieFold{nsplit, (int)groups, ctx->counters, ctx->dies_apart};
 }
 
 template <int HD, int G>
@@ -819,6 +820,7 @@ int launch_attn(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
                      : chunk == 96 ? go(std::integral_constant<int, 3>{}) : go(std::integral_constant<int, 4>{});
         if (rc != HM_OK) return rc;
         HM_LAUNCH_CHECK(ctx);
+        ctx->die_folds += die.splits > 0;
     }
     // nsplit is the grid's split count: 1 means no call can ever need a fold
     if (nsplit > 1 && !die.splits && a.phase != AttnArgs::SPLIT_ONLY) {
@@ -840,6 +842,7 @@ int launch_attn_stream(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
                        dim3(ATT_THREADS), 0, ctx->stream, a.q, a.kcache, a.vcache, a.out, part_o,
                        part_ml, a.kvh, a.max_len, a.kv_len, chunk, a.scale, die);
     HM_LAUNCH_CHECK(ctx);
+    ctx->die_folds += die.splits > 0;
     if (nsplit > 1 && !die.splits) {
         const int rc = launch_fold<HD, G>(ctx, a, part_o, part_ml, nsplit, chunk, (const DecodeState *)nullptr);
         if (rc != HM_OK) return rc;

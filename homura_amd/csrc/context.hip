@@ -1,6 +1,9 @@
 // Context, device memory and stream plumbing behind the C boundary.
 #include "hm_common.h"
+
+#include "../../include/homura_amd_bench.h"
 #include "attention.h"
+#include "die_fold.h"
 
 #include <cstdlib>
 #include <mutex>
@@ -24,10 +27,11 @@ int hm_set_error(hm_ctx *ctx, int code, const char *fmt, ...) {
 }
 
 __global__ void note_die_kernel(unsigned int *die) {
-    if (threadIdx.x == 0) die[blockIdx.x] = __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 0xF;
+    if (threadIdx.x == 0) die[blockIdx.x] = (unsigned int)homura::die_id();
 }
 
-// Grids of a few sizes, so that they begin on different dies: every workgroup where the one eight ids before it was.
+// Grids of a few sizes, so that they begin on different dies: every workgroup where the one eight ids before it was. (Every launch that relies on it
+// checks it for itself, last_on_die.)
 // HOMURA_FOLD_LAUNCH=1: not looked at, folds are launches of their own (for comparisons).
 static bool find_dies_round_robin(hm_ctx *ctx) {
     const char *e = std::getenv("HOMURA_FOLD_LAUNCH");
@@ -80,15 +84,16 @@ hm_ctx *hm_init(int device) {
         return nullptr;
     }
     ctx->workspace_bytes = (size_t)64 << 20;
-    ctx->num_counters = 1 << 16;
+    ctx->num_counters = 1 << 15;
     if (hipMalloc(&ctx->workspace, ctx->workspace_bytes) != hipSuccess ||
-        hipMalloc((void **)&ctx->counters, ctx->num_counters * sizeof(unsigned int)) !=
-            hipSuccess) {
+        hipMalloc((void **)&ctx->counters, ctx->num_counters * sizeof(*ctx->counters)) != hipSuccess ||
+        hipHostMalloc((void **)&ctx->dies_apart, sizeof(int), hipHostMallocDefault) != hipSuccess) {
         hm_set_error(nullptr, HM_ERR_OOM, "workspace allocation failed");
         hm_destroy(ctx);
         return nullptr;
     }
-    (void)hipMemsetAsync(ctx->counters, 0, ctx->num_counters * sizeof(unsigned int), ctx->stream);
+    *ctx->dies_apart = 0;
+    (void)hipMemsetAsync(ctx->counters, 0, ctx->num_counters * sizeof(*ctx->counters), ctx->stream);
     (void)hipStreamSynchronize(ctx->stream);
     ctx->dies_round_robin = find_dies_round_robin(ctx);
     if (gqa_attn_fixed_scratch_setup(ctx) != HM_OK) {
@@ -105,6 +110,7 @@ void hm_destroy(hm_ctx *ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->workspace) (void)hipFree(ctx->workspace);
     if (ctx->counters) (void)hipFree(ctx->counters);
+    if (ctx->dies_apart) (void)hipHostFree(ctx->dies_apart);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -156,8 +162,7 @@ int hm_download(hm_ctx *ctx, void *h_dst, const void *d_src, size_t bytes) {
     if (bytes == 0) return HM_OK;
     HM_REQUIRE(ctx, h_dst && d_src, "hm_download: NULL pointer");
     HM_HIP(ctx, hipMemcpyAsync(h_dst, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    HM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return HM_OK;
+    return hm_sync(ctx);
 }
 
 int hm_copy(hm_ctx *ctx, void *d_dst, const void *d_src, size_t bytes) {
@@ -192,7 +197,24 @@ int hm_fill_zero(hm_ctx *ctx, void *d_dst, size_t bytes) {
 int hm_sync(hm_ctx *ctx) {
     HM_CHECK_CTX(ctx);
     HM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (__atomic_load_n(ctx->dies_apart, __ATOMIC_RELAXED) != 0)
+        return hm_set_error(ctx, HM_ERR_STATE, "workgroups that share results ran on different accelerator dies, which this context found dealt in "
+                                               "turn when it was made: what attention gave is not valid. Make it with HOMURA_FOLD_LAUNCH=1.");
     return HM_OK;
+}
+
+int hm_test_die_folds(hm_ctx *ctx, long long *launches) {
+    HM_CHECK_CTX(ctx);
+    HM_REQUIRE(ctx, launches != nullptr, "hm_test_die_folds: NULL pointer");
+    *launches = ctx->die_folds;
+    return HM_OK;
+}
+
+int hm_test_die_arrivals(hm_ctx *ctx, int group) {
+    HM_CHECK_CTX(ctx);
+    HM_REQUIRE(ctx, group >= 0 && (size_t)(group + 1) * homura::DIE_COUNTER_STRIDE <= ctx->num_counters, "hm_test_die_arrivals: group %d", group);
+    const unsigned long long came = 0x0101;
+    return hm_upload(ctx, ctx->counters + (size_t)group * homura::DIE_COUNTER_STRIDE, &came, sizeof(came));
 }
 
 void *hm_stream(hm_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }

@@ -3,7 +3,8 @@
 // Workgroups are dealt to the eight dies round-robin, so those with the same blockIdx.x % 8 share an L2 (hm_init looks whether they do:
 // hm_ctx::dies_round_robin). A group of splits that sits on one die can hand its results over through that L2 without a fence: every
 // workgroup stores its results, waits until the L2 has them, and counts itself in; the one that finds all others counted reads them back
-// past its L1 and folds. Nobody waits for anybody. A launch of its own for the fold costs a kernel boundary and two trips to memory;
+// past its L1 and folds. Nobody waits for anybody. The counting says by die who came: a launch whose groups were dealt
+// otherwise after all tells the host, which fails the next synchronisation instead of handing out what was folded from another die's memory. A launch of its own for the fold costs a kernel boundary and two trips to memory;
 // between dies the hand-over itself takes them (a counter and stores through memory made the attention launch 4.9 us longer to
 // save 4.1 of fold).
 #pragma once
@@ -13,7 +14,8 @@ namespace homura {
 
 constexpr int DIES = 8, DIE_SPLITS_MAX = 32;
 // A counter has a cache line of its own: two dies counting in one line pass it to and fro (256 workgroups' arrivals 3.7 us instead of 0.6).
-constexpr int DIE_COUNTER_STRIDE = 64;
+// Its bytes are the arrivals from the eight dies.
+constexpr int DIE_COUNTER_STRIDE = 32;
 
 // Group p's split s is workgroup (p / 8 * splits + s) * 8 + p % 8 of a one-dimensional grid.
 __host__ __device__ inline int die_grid(int groups, int splits) { return (groups + DIES - 1) / DIES * splits * DIES; }
@@ -35,16 +37,22 @@ inline bool die_fold_pays(const hm_ctx *ctx, long long groups, int splits, doubl
     return groups >= DIES / 2 && (most * splits <= ctx->num_cus / DIES || most * DIES == groups) && bytes / 6.2e6 * ((double)(most * DIES) / groups - 1) <= 1;
 }
 
+__device__ __forceinline__ int die_id() { return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 0xF; }  // XCC_ID
+
 // Called by all threads behind their last store of results; true in every thread of the workgroup that is the last of n to come here.
-// The counter is left at zero.
-__device__ __forceinline__ bool last_on_die(unsigned int *counters, int group, int n) {
+// The counter is left at zero. If they came from several dies nobody is, and `apart` (memory of the host's) is set.
+__device__ __forceinline__ bool last_on_die(unsigned long long *counters, int group, int n, int *apart) {
     __shared__ int last;
-    unsigned int *counter = counters + (size_t)group * DIE_COUNTER_STRIDE;
+    unsigned long long *counter = counters + (size_t)group * DIE_COUNTER_STRIDE;
+    const int shift = die_id() % DIES * 8;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the L2 has this wavefront's stores
     __syncthreads();
     if (threadIdx.x == 0) {
-        last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned int)(n - 1);
-        if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long came = __hip_atomic_fetch_add(counter, 1ull << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool all = (int)((came * 0x0101010101010101ull) >> 56) == n - 1;  // (the sum of its bytes, at most 31)
+        last = all && came >> shift == (unsigned)(n - 1);
+        if (all) __hip_atomic_store(counter, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (all && !last) __hip_atomic_store(apart, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     __syncthreads();
     return last != 0;

@@ -18,11 +18,14 @@ struct hm_ctx {
     // Workspace for kernels that need partial results (split-K / split-KV); allocated once.
     void *workspace = nullptr;
     size_t workspace_bytes = 0;
-    // 4-byte counters used by "last workgroup finishes" reductions (die_fold.h); always left at zero.
-    unsigned int *counters = nullptr;
+    // 8-byte counters used by "last workgroup finishes" reductions (die_fold.h); always left at zero.
+    unsigned long long *counters = nullptr;
     size_t num_counters = 0;
     // Workgroups whose ids are equal modulo eight run on one accelerator die (found by running some when the context is made).
     bool dies_round_robin = false;
+    // Pinned host word that a launch sets which found it otherwise (die_fold.h); hm_sync and hm_download fail from then on.
+    int *dies_apart = nullptr;
+    long long die_folds = 0;  // launches that were given such a fold
     // Device address, on this context's device, of the fixed array behind hm_gqa_decode_attn_noalloc.
     void *attn_fixed_scratch = nullptr;
     std::string last_error;

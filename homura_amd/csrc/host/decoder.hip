@@ -79,7 +79,7 @@ int DecoderModel::run_kv_once(const int64_t *h_ids, int n_ids, float *h_logits) 
         const void *status = pending_status_words();
         rc = move_words_launch(ctx_, stage, plan_->slot(logits_slot)->ptr(), row_bytes / 4, status ? stage + row_bytes : nullptr, status);
         if (rc != HM_OK) return rc;
-        HM_HIP(ctx_, hipStreamSynchronize(ctx_->stream));
+        if ((rc = hm_sync(ctx_)) != HM_OK) return rc;
         std::memcpy(h_logits + (size_t)i * vocab_size(), stage, row_bytes);
         if (status && (rc = check_status_words(reinterpret_cast<const uint32_t *>(stage + row_bytes))) != HM_OK) return rc;
     }

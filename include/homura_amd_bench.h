@@ -60,6 +60,11 @@ int hm_test_fill_lds(hm_ctx *ctx, uint32_t word);
  * weight format on a chip of `cus` CUs, and the most that the product of m <= rows rows writes (all its K slices). Host only. */
 int hm_test_prompt_product(int hm_dtype, int rows, int m, int k, int n, int cus, long long *floats_held, long long *floats_written);
 
+/* Test support: a group of splits that folds on its die (die_fold.h) finds one arrival from each of two dies that were not there. */
+int hm_test_die_arrivals(hm_ctx *ctx, int group);
+/* Test support: attention launches of this context so far whose splits fold on their die. */
+int hm_test_die_folds(hm_ctx *ctx, long long *launches);
+
 /* Test support: the rows that the decode attention's grid covers in a step of `live` live rows over a cache of max_len, the rows of a split, and
  * the rows that its splits ask for without having looked at the live length. Host only. */
 int hm_test_attn_rows(int live, int max_len, int *span, int *chunk, int *sure);

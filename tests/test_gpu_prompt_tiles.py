@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from homura_amd import DTYPE_F32, DTYPE_Q4_0, DTYPE_Q8_0, synth, synth_model
+from homura_amd.runtime import HomuraError
 
 pytestmark = pytest.mark.gpu
 
@@ -360,6 +361,37 @@ def test_fold_keeps_an_infinite_value(ctx, H, kvh, hd, kv_len):
     assert np.all(got[:, 5] == np.inf) and np.all(np.isfinite(np.delete(got, 5, 1)))
     for buf in (dq, dk, dv, do):
         buf.free()
+
+
+def die_folds(c):
+    n = C.c_longlong()
+    c._check(c.lib.hm_test_die_folds(c.h, C.byref(n)))
+    return n.value
+
+
+# the kernel that holds its chunk in registers, and the one that walks it
+@pytest.mark.parametrize("B,H,kvh,hd,kv_len", [(1, 16, 8, 128, 1000), (8, 12, 2, 128, 4096)])
+def test_splits_from_several_dies_are_not_folded_silently(ctx, B, H, kvh, hd, kv_len):
+    """Arrivals from two dies in a group that is dealt to one: the launch ends as ever, the synchronisations behind it fail and go on failing,
+    and another context takes no harm."""
+    c = type(ctx)(0)
+    dq, dk, dv, do = c.to_device(np.ones((B, H, hd), np.float32)), *(c.to_device(np.zeros((B, kvh, kv_len, hd), np.uint16)) for _ in range(2)), c.empty(B * H * hd)
+    call = lambda: c.gqa_decode_attn(dq, dk, dv, do, B, H, kvh, hd, kv_len, kv_len, hd ** -0.5)
+    before = die_folds(c)
+    call()
+    assert die_folds(c) == before + 1
+    assert np.all(do.download(np.float32) == 0)
+    c._check(c.lib.hm_test_die_arrivals(c.h, 3))
+    call()
+    for _ in range(2):
+        with pytest.raises(HomuraError, match="HOMURA_FOLD_LAUNCH"):
+            c.sync()
+        with pytest.raises(HomuraError, match="HOMURA_FOLD_LAUNCH"):
+            do.download(np.float32)
+    for buf in (dq, dk, dv, do):
+        buf.free()
+    c.close()
+    ctx.sync()
 
 
 # Groups of splits that sit on one die each: one to eight heads of a workgroup (four, two or one share of the splits a thread), two to
