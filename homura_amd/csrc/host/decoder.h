@@ -101,8 +101,9 @@ class DecoderModel {
     int check_ids(const int64_t *ids, int n, std::vector<int32_t> &out);
 
     // Pinned host memory that kernels read and write: of run_kv, a logits row and the status words, which arrive with one
-    // synchronisation; a prompt's ids; a generation's draws and tokens. Every call synchronises before it returns, or before it uses a
-    // block again.
+    // synchronisation; a prompt's ids; a generation's draws and tokens. A call that succeeds synchronises before it returns. One that fails may
+    // leave kernels behind that read a prompt's ids or the draws, so these are written behind a synchronisation; the other blocks are written by kernels
+    // only, in stream order, and read behind a synchronisation of their own.
     struct Pinned {
         void *p = nullptr;
         size_t bytes = 0;

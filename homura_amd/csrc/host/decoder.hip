@@ -234,6 +234,7 @@ int DecoderModel::generate_once(const int64_t *h_prompt, int n_prompt, int max_n
         const bool own_pick = greedy && !penalties;
         if (!greedy) {
             if ((rc = pinned_for(draws_, (size_t)max_new * 4)) != HM_OK) return rc;
+            if (n_prompt == 1 && (rc = hm_sync(ctx_)) != HM_OK) return rc;  // (a call that failed may have left a kernel that reads them)
             for (int i = 0; i < max_new; i++) draws_.as<float>()[i] = hm_rng_next_f32(&rng);
             if (s.draws_cap < max_new) {
                 s.draws = Buffer::alloc(ctx_, {max_new}, DType::F32);
