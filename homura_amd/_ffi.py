@@ -100,7 +100,7 @@ SIGNATURES = {
     "hm_test_qkv_product": (_I, [_P, _P, _P, _I, _P] + [_I] * 6 + [_P] * 8 + [_I] * 2 + [C.c_float, C.POINTER(_I)]),
     "hm_test_gated_product": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, C.c_float, C.c_float, C.POINTER(_I)]),
     "hm_test_die_arrivals": (_I, [_P, _I]),
-    "hm_test_die_folds": (_I, [_P, C.POINTER(C.c_longlong)]),
+    "hm_test_routes": (_I, [_P, C.POINTER(C.c_longlong)]),
     "hm_test_attn_rows": (_I, [_I, _I] + [C.POINTER(_I)] * 3),
     "hm_test_latent_rows": (_I, [_P, _P, _I, _I] + [_P] * 4 + [_I] * 6 + [C.c_float, _P, _P]),
     "hm_test_product_tiles": (_I, [_I] * 6 + [C.POINTER(_I)] * 3),

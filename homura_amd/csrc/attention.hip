@@ -820,7 +820,7 @@ int launch_attn(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
                      : chunk == 96 ? go(std::integral_constant<int, 3>{}) : go(std::integral_constant<int, 4>{});
         if (rc != HM_OK) return rc;
         HM_LAUNCH_CHECK(ctx);
-        ctx->die_folds += die.splits > 0;
+        ctx->routes.die_folds += die.splits > 0;
     }
     // nsplit is the grid's split count: 1 means no call can ever need a fold
     if (nsplit > 1 && !die.splits && a.phase != AttnArgs::SPLIT_ONLY) {
@@ -842,7 +842,7 @@ int launch_attn_stream(hm_ctx *ctx, const AttnArgs &a, int nsplit, int chunk) {
                        dim3(ATT_THREADS), 0, ctx->stream, a.q, a.kcache, a.vcache, a.out, part_o,
                        part_ml, a.kvh, a.max_len, a.kv_len, chunk, a.scale, die);
     HM_LAUNCH_CHECK(ctx);
-    ctx->die_folds += die.splits > 0;
+    ctx->routes.die_folds += die.splits > 0;
     if (nsplit > 1 && !die.splits) {
         const int rc = launch_fold<HD, G>(ctx, a, part_o, part_ml, nsplit, chunk, (const DecodeState *)nullptr);
         if (rc != HM_OK) return rc;

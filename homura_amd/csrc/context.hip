@@ -203,10 +203,12 @@ int hm_sync(hm_ctx *ctx) {
     return HM_OK;
 }
 
-int hm_test_die_folds(hm_ctx *ctx, long long *launches) {
+int hm_test_routes(hm_ctx *ctx, long long *counts) {
     HM_CHECK_CTX(ctx);
-    HM_REQUIRE(ctx, launches != nullptr, "hm_test_die_folds: NULL pointer");
-    *launches = ctx->die_folds;
+    HM_REQUIRE(ctx, counts != nullptr, "hm_test_routes: NULL pointer");
+    counts[0] = ctx->routes.die_folds;
+    counts[1] = ctx->routes.gates_whole;
+    counts[2] = ctx->routes.gates_sliced;
     return HM_OK;
 }
 

@@ -25,7 +25,9 @@ struct hm_ctx {
     bool dies_round_robin = false;
     // Pinned host word that a launch sets which found it otherwise (die_fold.h); hm_sync and hm_download fail from then on.
     int *dies_apart = nullptr;
-    long long die_folds = 0;  // launches that were given such a fold
+    // Which way work went, for tests: attention launches with such a fold; gate rows of scans and recurrences straight from their projection, and
+    // through the convolution
+    struct { long long die_folds = 0, gates_whole = 0, gates_sliced = 0; } routes;
     // Device address, on this context's device, of the fixed array behind hm_gqa_decode_attn_noalloc.
     void *attn_fixed_scratch = nullptr;
     std::string last_error;

@@ -1315,6 +1315,7 @@ int BlockModel::prefill_mixer(int run, int layer, const float *cos_tab, const fl
         c.pieces = np;
         c.channels = c.block_width = c.block_pad = d.inner;
         const bool whole = in.parts == 1;  // sums of K slices are taken once, by the convolution
+        (whole ? ctx_->routes.gates_whole : ctx_->routes.gates_sliced)++;
         if (!whole) {
             c.side = p.f3.as<float>();
             c.side_cols = d.inner;
@@ -1367,6 +1368,7 @@ int BlockModel::prefill_mixer(int run, int layer, const float *cos_tab, const fl
     c.block_width = d.block;
     c.block_pad = d.block_pad;
     const bool whole = in.parts == 1;
+    (whole ? ctx_->routes.gates_whole : ctx_->routes.gates_sliced)++;
     if (!whole) {
         c.side = p.f3.as<float>();
         c.side_cols = d.width;

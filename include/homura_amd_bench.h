@@ -62,8 +62,9 @@ int hm_test_prompt_product(int hm_dtype, int rows, int m, int k, int n, int cus,
 
 /* Test support: a group of splits that folds on its die (die_fold.h) finds one arrival from each of two dies that were not there. */
 int hm_test_die_arrivals(hm_ctx *ctx, int group);
-/* Test support: attention launches of this context so far whose splits fold on their die. */
-int hm_test_die_folds(hm_ctx *ctx, long long *launches);
+/* Test support: counts[3] of what went which way in this context so far: attention launches whose splits fold on their die; gate rows of scans and
+ * recurrences (layers of a prompt's portions) straight from their projection, and through the convolution. */
+int hm_test_routes(hm_ctx *ctx, long long *counts);
 
 /* Test support: the rows that the decode attention's grid covers in a step of `live` live rows over a cache of max_len, the rows of a split, and
  * the rows that its splits ask for without having looked at the live length. Host only. */

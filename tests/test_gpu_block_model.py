@@ -3,6 +3,7 @@ and in portions, decoding, windows and their edges, reuse of the cache, generati
 and is held to 2e-5 of the logits' spread; `bf16` is the serving precision."""
 from __future__ import annotations
 
+import ctypes as C
 import json
 
 import numpy as np
@@ -485,9 +486,14 @@ def test_latent_rows_of_a_prompt(ctx, name, dtype):
 @pytest.mark.parametrize("n", [70, 300])
 def test_gate_rows_from_slices_and_whole(ctx, n, dtype):
     """The gates of the scan and the recurrence straight from their projection, and from the convolution where it came in K slices (1100 wide)."""
+    routes = (C.c_longlong * 3)()
     for width in (1100, 96):
+        ctx._check(ctx.lib.hm_test_routes(ctx.h, routes))
+        whole, sliced = routes[1:]
         cfg = bf.config([bf.scan(inner=64, state=16), bf.scan(inner=130, state=33), bf.recurrence(), bf.recurrence(width=66, blocks=2)], width=width)
         check(ctx, cfg, n, dtype, cuts=(n // 3,))
+        ctx._check(ctx.lib.hm_test_routes(ctx.h, routes))
+        assert (routes[1] > whole, routes[2] > sliced) == (width == 96, width == 1100)
 
 
 # one to four wavefronts a row, the last of them part of the way; one round of rows, several with a last one of few rows; the paired, the

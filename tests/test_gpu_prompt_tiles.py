@@ -364,9 +364,9 @@ def test_fold_keeps_an_infinite_value(ctx, H, kvh, hd, kv_len):
 
 
 def die_folds(c):
-    n = C.c_longlong()
-    c._check(c.lib.hm_test_die_folds(c.h, C.byref(n)))
-    return n.value
+    n = (C.c_longlong * 3)()
+    c._check(c.lib.hm_test_routes(c.h, n))
+    return n[0]
 
 
 # the kernel that holds its chunk in registers, and the one that walks it
@@ -400,7 +400,8 @@ def test_splits_from_several_dies_are_not_folded_silently(ctx, B, H, kvh, hd, kv
                                                (8, 12, 2, 128, 4096), (8, 14, 2, 64, 5000), (4, 64, 8, 128, 4001), (16, 5, 1, 64, 4096),
                                                (6, 14, 2, 64, 777)])
 def test_splits_folded_on_their_die(ctx, monkeypatch, B, H, kvh, hd, kv_len):
-    """Eager twice and replayed three times (the arrivals are counted anew every time), with other work between. A softmax over f32 sums:
+    """Eager twice and replayed three times (the arrivals are counted anew every time), with other work between, in a context that folds so and in
+    one that does not. A softmax over f32 sums:
     2^-20 of the largest value holds a few thousand additions, and the long caches' two-piece operands 2^-17 of their terms."""
     rng = np.random.default_rng(kv_len + H)
     q = rng.standard_normal((B, H, hd)).astype(np.float32)
@@ -415,8 +416,10 @@ def test_splits_folded_on_their_die(ctx, monkeypatch, B, H, kvh, hd, kv_len):
     for c in (ctx, apart):
         dq, dk, dv, do, other = c.to_device(q), c.to_device(k), c.to_device(v), c.empty(B * H * hd), c.empty(256 * hd)
         call = lambda out: c.gqa_decode_attn(dq, dk, dv, out, B, H, kvh, hd, kv_len, kv_len, hd ** -0.5)
+        before = die_folds(c)
         for _ in range(2):
             call(do)
+        assert die_folds(c) - before == (2 if c is ctx else 0)
         got.append(do.download(np.float32, (B, H, hd)))
         graph = C.c_void_p()
         c._check(c.lib.hm_graph_begin(c.h))
