@@ -1,7 +1,6 @@
 // Context, device memory and stream plumbing behind the C boundary.
 #include "hm_common.h"
 
-#include "../../include/homura_amd_bench.h"
 #include "attention.h"
 #include "die_fold.h"
 
@@ -201,22 +200,6 @@ int hm_sync(hm_ctx *ctx) {
         return hm_set_error(ctx, HM_ERR_STATE, "workgroups that share results ran on different accelerator dies, which this context found dealt in "
                                                "turn when it was made: what attention gave is not valid. Make it with HOMURA_FOLD_LAUNCH=1.");
     return HM_OK;
-}
-
-int hm_test_routes(hm_ctx *ctx, long long *counts) {
-    HM_CHECK_CTX(ctx);
-    HM_REQUIRE(ctx, counts != nullptr, "hm_test_routes: NULL pointer");
-    counts[0] = ctx->routes.die_folds;
-    counts[1] = ctx->routes.gates_whole;
-    counts[2] = ctx->routes.gates_sliced;
-    return HM_OK;
-}
-
-int hm_test_die_arrivals(hm_ctx *ctx, int group) {
-    HM_CHECK_CTX(ctx);
-    HM_REQUIRE(ctx, group >= 0 && (size_t)(group + 1) * homura::DIE_COUNTER_STRIDE <= ctx->num_counters, "hm_test_die_arrivals: group %d", group);
-    const unsigned long long came = 0x0101;
-    return hm_upload(ctx, ctx->counters + (size_t)group * homura::DIE_COUNTER_STRIDE, &came, sizeof(came));
 }
 
 void *hm_stream(hm_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }

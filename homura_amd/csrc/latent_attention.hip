@@ -3,7 +3,6 @@
 
 #include <algorithm>
 
-#include "../../include/homura_amd_bench.h"
 #include "row_pieces.h"
 
 namespace {
@@ -920,31 +919,3 @@ int latent_kv_rows_launch(hm_ctx *ctx, const LatentShape &s, const RowSource &kv
 }
 
 }  // namespace homura
-
-extern "C" int hm_test_latent_rows(hm_ctx *ctx, const float *down, int ld, int parts, const float *q_norm, const float *kv_norm, const float *cos_tab,
-                                   const float *sin_tab, int q_rank, int rank, int rot, int pieces, int n, int past, float eps, uint16_t *q_split,
-                                   uint16_t *ring) {
-    HM_CHECK_CTX(ctx);
-    homura::LatentRowsArgs a;
-    a.s.heads = a.s.dim = a.s.vdim = 1;
-    a.s.rank = rank;
-    a.s.rot_dim = a.s.rot_dims = rot;
-    a.s.rank_pad = (rank + 31) / 32 * 32;
-    a.s.rot_pad = (rot + 31) / 32 * 32;
-    a.s.pieces = a.q_pieces = pieces;
-    a.s.ring_rows = past + n;
-    a.down = homura::RowSource{down, ld, parts, (size_t)n * ld, nullptr};
-    a.q_norm = q_norm;
-    a.kv_norm = kv_norm;
-    a.cos_tab = cos_tab;
-    a.sin_tab = sin_tab;
-    a.q_rank = q_rank;
-    a.q_rank_pad = (q_rank + 31) / 32 * 32;
-    a.n = n;
-    a.past = past;
-    a.eps = eps;
-    a.q_split = q_split;
-    a.ring = ring;
-    const int rc = homura::latent_rows_launch(ctx, a);
-    return rc == HM_OK ? hm_sync(ctx) : rc;
-}
