@@ -625,7 +625,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void gemv_bf16_nk_splitk_kernel(GemvA
 // of the normed row in registers and stay: a workgroup takes G sets of R rows, then the next G R that are its, asked for ahead of the sums
 // of those at hand. The sums are those of the kernel above, bit for bit.
 // us a decode step, that kernel (eight rows a workgroup from 8192 outputs on, four below) / here: Qwen2.5-1.5B 1354 / 1266, Qwen2.5-0.5B 854 / 773,
-// TinyLlama 960 / 927, Nokuvik 1024 wide 1631 / 1475, Ludalix 1024 wide 1268 / 1203. What is in flight is enough with eight wavefronts a CU; more
+// TinyLlama 960 / 927, Nokuvik 1024 wide 1631 / 1475, Ludalix 1024 wide 1268 / 1203. What is in flight is enough with 4 W wavefronts a CU; more
 // rows, sets or workgroups wait behind one another's prologues.
 template <int W, int G, int R, int PRO>
 __global__ __launch_bounds__(WAVE * W * G) void gemv_bf16_nk_rolling_kernel(GemvArgs a, int epi) {
