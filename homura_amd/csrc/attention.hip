@@ -68,6 +68,7 @@ template <int HD>
 __device__ __forceinline__ void fold_here(const float *po, const float *pml, float *__restrict__ out, int heads, int nsplit, int all) {
     constexpr int AHEAD = 8;  // splits asked for at a time
     static_assert(homura::DIE_SPLITS_MAX == 32 && ATT_THREADS == 8 * 32 && 8 * HD / 4 <= ATT_THREADS, "a split a lane of half a wavefront");
+    static_assert(HD * 4 % homura::DIE_LINE == 0, "a split's outputs are whole cache lines (the workspaces begin with one)");
     __shared__ float s_w[8][32];
     __shared__ f32x4 s_o[ATT_THREADS];
     const int tid = threadIdx.x, h = tid >> 5, sp = tid & 31, vecs = heads * (HD / 4);

@@ -60,8 +60,9 @@ __device__ __forceinline__ bool last_on_die(unsigned long long *counters, int gr
 
 // A result that another workgroup of the die stored: from the L2, whatever this CU's L1 holds
 __device__ __forceinline__ float from_die(const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// Four at once, for results in cache lines that no workgroup of this launch has read before (a kernel begins with an empty L1, and its own
-// stores go through it).
+// Four at once, for results in cache lines of their own that no workgroup of this launch has read before (a kernel begins with an empty L1, and
+// its own stores go through it). Past the L1 as above, eight bytes at a time: 8 sequences x 12 heads on 2 x 128, 4096 rows 11.83 -> 12.09 us.
+constexpr int DIE_LINE = 128;  // bytes
 __device__ __forceinline__ f32x4 from_die4(const float *p) { return __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p)); }
 
 }  // namespace homura
