@@ -14,7 +14,8 @@
  *    (The reference's kernels return void and panic in Rust; a GPU call can fail, so the
  *    boundary carries a status.)
  *  - one hm_ctx = one GPU + one HIP stream; all kernels are enqueued on that stream and are
- *    asynchronous; hm_download() and hm_sync() are the blocking calls. One host thread per
+ *    asynchronous; hm_download() and hm_sync() are the blocking calls. (They fail with HM_ERR_STATE for good once an
+ *    attention launch has found its workgroups placed otherwise than hm_init did; HOMURA_FOLD_LAUNCH=1 does without that.) One host thread per
  *    context at a time (the reference serialises runs under a Mutex, src/hf/model.rs:205).
  *  - activations, norms, logits are f32; bf16 values travel as uint16_t (top half of an f32,
  *    reference src/hf/safetensors.rs:105-115); quantised weights are raw GGUF block bytes.
